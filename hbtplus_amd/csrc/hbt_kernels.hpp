@@ -33,7 +33,8 @@ enum { NC_SRC = 0, NC_PART = 1, NC_BOUND = 2, NC_SORT = 3, NC_CROSS = 4, NC_ROWS
 struct __align__(32) Item {
   float4 pm;   // x, y, z, mass (a node: centre of mass and total mass)
   int2 ax;     // float bits of len^2 (0 for a leaf), skip (first item after the subtree)
-  int2 sb;     // skip as a byte offset from the segment's first item (32 * skip), unused
+  int2 sb;     // skip as a byte offset from the segment's first item (32 * skip); float bits of the
+               // squared distance below which the FP32 walk opens the node (0 for a leaf)
 };
 
 struct Work {
@@ -756,9 +757,35 @@ __device__ __forceinline__ float node_len(const Seg &S, int v) {
   return (float)ldexp(S.Len, -e);
 }
 
+// The squared distance below which the FP32 walk opens a node: the smallest
+// float r2 for which lsq > r2 * theta2 (rounded to float) fails, so that
+// r2 < open_below(lsq, theta2) is that test for every r2 >= 0 (the product is
+// monotonic in r2).  The quotient is off by a step or two; where the product
+// is subnormal a plateau can be longer, and the bits are bisected.
+__device__ __forceinline__ float open_below(float lsq, float theta2) {
+#pragma clang fp contract(off)
+  if (!(lsq > 0.f)) return 0.f;
+  auto opens = [&](u32 bits) { return lsq > __uint_as_float(bits) * theta2; };
+  const float t0 = lsq / theta2;
+  if (!(t0 >= 0.f)) return 0.f;  // theta2 is NaN: nothing opens
+  u32 t = __float_as_uint(t0);
+  for (int i = 0; i < 3 && t < 0x7f800000u && opens(t); i++) t++;
+  for (int i = 0; i < 3 && t > 0u && !opens(t - 1u); i++) t--;
+  const bool low = t < 0x7f800000u && opens(t), high = t > 0u && !opens(t - 1u);
+  if (low || high) {
+    u32 a = 0u, b = 0x7f800000u;  // the answer lies in [a, b]
+    while (a < b) {
+      const u32 m = (a + b) >> 1;
+      if (opens(m)) a = m + 1u; else b = m;
+    }
+    t = a;
+  }
+  return __uint_as_float(t);
+}
+
 // Writes leaves and node headers in pre-order.  pre = exclusive prefix of
 // popcount(bits) over the segment's sorted sources.
-__global__ void __launch_bounds__(BLOCK) items_kernel(Work W) {
+__global__ void __launch_bounds__(BLOCK) items_kernel(Work W, DevParams P) {
   SLOT_LOOP(s, W) {
     int k;
     int l = seg_lane_local(W, s, k);
@@ -776,9 +803,10 @@ __global__ void __launch_bounds__(BLOCK) items_kernel(Work W) {
                                  make_int2(0, pos + 1), make_int2(32 * (pos + 1), 0)};
         if (l + 1 == S.n_src) {
           W.seg[k].n_items = pos + 1;
-          // sentinel after the last item: massless, never opened, its skip is
-          // itself, so a group walk that has finished reads it and stays put
-          W.items[ib + pos + 1] = Item{make_float4(0.f, 0.f, 0.f, 0.f), make_int2(0, pos + 1),
+          // sentinel after the last item: massless, far from every target,
+          // never opened, its skip is itself, so a group walk that has
+          // finished reads it, adds nothing and stays put
+          W.items[ib + pos + 1] = Item{make_float4(1e18f, 1e18f, 1e18f, 0.f), make_int2(0, pos + 1),
                                        make_int2(32 * (pos + 1), 0)};
         }
         const int lo = W.nlo[s];
@@ -790,7 +818,7 @@ __global__ void __launch_bounds__(BLOCK) items_kernel(Work W) {
           const float len = node_len(S, v);
           const float lsq = len * len;
           W.items[ib + npos] = Item{make_float4(0.f, 0.f, 0.f, 0.f), make_int2(__float_as_int(lsq), hpos + 1),
-                                    make_int2(32 * (hpos + 1), 0)};
+                                    make_int2(32 * (hpos + 1), __float_as_int(open_below(lsq, P.theta2)))};
           W.npos[s] = (int)(ib + npos);
         }
       }
@@ -1206,6 +1234,35 @@ __device__ __forceinline__ int group_field(int v) {
   return __builtin_amdgcn_ds_swizzle(v, AND | (K << 5));
 }
 
+// Lane K of the caller's row of 16 lanes, read by every lane of the row (DPP
+// row_newbcast: a source modifier of the consuming vector instruction, no LDS
+// crossbar).  Every lane of the wave must be active.
+template <int K>
+__device__ __forceinline__ int row_field(int v) {
+  return __builtin_amdgcn_mov_dpp(v, 0x150 + K, 0xf, 0xf, true);
+}
+// the same value in an instruction of its own
+template <int K>
+__device__ __forceinline__ int row_field_again(int v) {
+  return __builtin_amdgcn_update_dpp(v, v, 0x150 + K, 0xf, 0xf, false);
+}
+
+// Lane mask m with every GROUP-lane field that holds a set bit filled (GROUP =
+// 16 or 32), on the scalar unit.
+template <int GROUP>
+__device__ __forceinline__ u64 fill_fields(u64 m) {
+  static_assert(GROUP == 16 || GROUP == 32, "16- or 32-lane fields");
+  if (GROUP == 32) return ((u32)m ? 0xffffffffull : 0ull) | ((m >> 32) ? ~0xffffffffull : 0ull);
+  // one bit per quad of lanes, filled per four quads, each bit widened to four again
+  u64 q, r;
+  u32 w;
+  asm("s_quadmask_b64 %0, %1" : "=s"(q) : "s"(m) : "scc");
+  asm("s_wqm_b32 %0, %1" : "=s"(w) : "s"((u32)q) : "scc");
+  asm("s_bitreplicate_b64_b32 %0, %1" : "=s"(r) : "s"(w));
+  asm("s_bitreplicate_b64_b32 %0, %1" : "=s"(q) : "s"((u32)r));
+  return q;
+}
+
 // Per-target arithmetic of one item in FP32: sep2 = squared separation,
 // opens = the opening test, add = the softened monopole term, the terms summed
 // in FP64 (WIDE: the FAST precision; one conversion and one FP64 add per term,
@@ -1214,6 +1271,7 @@ __device__ __forceinline__ int group_field(int v) {
 template <bool STRADDLE, bool WIDE>
 struct FastTerm {
   using real = float;
+  static constexpr bool WIDE_F32 = WIDE;
   float h2, hinv;
   typename std::conditional<WIDE, double, float>::type acc;
   __device__ __forceinline__ void init(const DevParams &P, bool live, float tmass) {
@@ -1245,6 +1303,10 @@ struct FastTerm {
 #pragma clang fp contract(off)
     return __builtin_amdgcn_fcmpf(lsq, r2 * P.theta2, 2 /* ordered > */);
   }
+  // the same against the row's item v (its bound on r2)
+  __device__ __forceinline__ u64 opens_row(const DevParams &, int v, float r2) const {
+    return __builtin_amdgcn_fcmpf(r2, __int_as_float(row_field<7>(v)), 4 /* ordered < */);
+  }
   __device__ __forceinline__ void add(float m, float r2) {
 #pragma clang fp contract(off)
     acc += kernel_term_f(m, r2, h2, hinv);
@@ -1259,12 +1321,27 @@ struct FastTerm {
     const float added = accept ? term : 0.f;
     acc += added;
   }
+  // the lanes' terms of the row's item v, negated: the Newtonian form for every
+  // lane, the spline only in steps where a lane of amask lies within the
+  // softening length (the mass is read again there, so that the common product
+  // takes it as a DPP operand)
+  __device__ __forceinline__ float row_term(u64 amask, int v, float r2) const {
+#pragma clang fp contract(off)
+    float term = __int_as_float(row_field<3>(v)) * __builtin_amdgcn_rsqf(r2);
+    const u64 near = amask & __builtin_amdgcn_fcmpf(r2, h2, 12 /* unordered or < */);
+    if (near != 0ull) {
+      const float m = __int_as_float(row_field_again<3>(v));
+      if (__builtin_amdgcn_inverse_ballot_w64(near)) term = -kernel_term_f(m, r2, h2, hinv);
+    }
+    return term;
+  }
   __device__ __forceinline__ double result() const { return (double)acc; }
 };
 
 // Reference arithmetic (src/gravity_tree.cpp:79-164): FP64 over float data.
 struct ReplayTerm {
   using real = double;
+  static constexpr bool WIDE_F32 = false;
   double h, hinv, pot;
   __device__ __forceinline__ void init(const DevParams &P, bool live, float tmass) {
 #pragma clang fp contract(off)
@@ -1287,6 +1364,9 @@ struct ReplayTerm {
 #pragma clang fp contract(off)
     return __builtin_amdgcn_fcmp((double)lsq, r2 * (double)P.theta2, 2 /* ordered > */);
   }
+  __device__ __forceinline__ u64 opens_row(const DevParams &P, int v, double r2) const {
+    return opens_mask(P, __int_as_float(row_field<4>(v)), r2);
+  }
   __device__ __forceinline__ void add(float m, double r2) {
 #pragma clang fp contract(off)
     pot += kernel_term_d((double)m, sqrt(r2), h, hinv);
@@ -1303,8 +1383,9 @@ struct ReplayTerm {
 // group-uniform index compile to scalar loads when GROUP = 64, and both
 // possible successors of item j (j+1 and skip(j)) are fetched while j is
 // evaluated.  Smaller groups read with vector loads at a 32-bit byte offset
-// from the scalar base, one dword of the item per lane, and spread the six
-// fields over the group with crossbar swizzles; every lane of the wave takes
+// from the scalar base, one dword of the item per lane, and spread the fields
+// over the group -- 16 and 32 lanes with DPP row broadcasts, 8 lanes with
+// crossbar swizzles; every lane of the wave takes
 // part in every step (lanes off their path discard the result), the dwords of
 // both possible successors are fetched as soon as skip(j) is known, the
 // group's vote takes the group's field of the opened-lane mask, and the
@@ -1350,6 +1431,91 @@ __device__ double walk_group(const Item *__restrict__ it, const DevParams &P, in
       j = go ? j1 : js;
       q = go ? q1 : qs;
       a = go ? a1 : as;
+    }
+  } else if constexpr (GROUP >= 16) {
+    // Vector issue bounds this loop: a step is about 20 vector instructions,
+    // and products, sums and moves of vector registers issue in half the time
+    // of compares, selects, conversions, FMAs and DPP forms (measured: 2.4
+    // against 4.4 cycles per wave; the reciprocal root 8.3), so item fields
+    // are DPP operands where an instruction can take them, the vote runs on
+    // the scalar unit and selects are moves under an exec mask.  With the
+    // items read through ds_swizzle and 8 lanes the 200,000-subhalo share's
+    // walks took 91.8 ms; so, with 16 lanes, 78.2 ms (86 cycles of a SIMD per
+    // wave step), the 4M-particle host's 14.9 -> 11.8 ms.
+    // lane r of every 8 fetches dword r of its group's item; a row of 16 lanes shares the group's item, so its fields are
+    // DPP row broadcasts inside the instructions that use them.  Positions are
+    // byte offsets from the segment's first item plus the lane's dword offset
+    // (< 32): J = 32 j + dw, and a skip becomes JS = 32 skip + dw.  A finished
+    // group sits on the sentinel item (skip = itself, massless, far away, never
+    // opened), where steps change nothing, so the exit is tested every UNROLL
+    // steps; a lane without a target is never on its path.
+    // (the address is the wave's: kept in scalar registers)
+    using Global = const __attribute__((address_space(1))) char;
+    Global *base = (Global *)(((u64)(u32)__builtin_amdgcn_readfirstlane((int)((u64)it >> 32)) << 32) |
+                              (u32)__builtin_amdgcn_readfirstlane((int)(u64)it));
+    auto dword = [base](unsigned off) { return *(const __attribute__((address_space(1))) int *)(base + off); };
+    auto dword_next = [base](unsigned off) { return *(const __attribute__((address_space(1))) int *)(base + off + 32); };
+    const unsigned dw = 4u * (threadIdx.x & 7u);
+    const unsigned endb = 32u * (unsigned)end;
+    unsigned J = 32u * (unsigned)j + dw;
+    unsigned untilb = live ? 32u * (unsigned)ib + dw : UINT_MAX;
+    int v = dword(J);
+    const u64 full = __builtin_amdgcn_read_exec();
+    constexpr int UNROLL = COUNT ? 1 : 4;
+    while (__any(J < endb)) {
+#pragma unroll
+      for (int u = 0; u < UNROLL; u++) {
+        const unsigned JS = (unsigned)row_field<6>(v) + dw;
+        // both possible successors are fetched under the work on item j
+        // (j + 1 = end + 1 reads the next region or the buffer's two spare items)
+        const int v1 = dword_next(J), vs = dword(JS);
+        const float4 q = make_float4(__int_as_float(row_field<0>(v)), __int_as_float(row_field<1>(v)),
+                                     __int_as_float(row_field<2>(v)), __int_as_float(row_field<3>(v)));
+        const u64 pmask = __builtin_amdgcn_uicmp(untilb, J, 37 /* unsigned <= */);
+        const typename Term::real r2 = t.sep2(P, q, tx, ty, tz);
+        const u64 omask = pmask & t.opens_row(P, v, r2);
+        const u64 amask = pmask & ~omask;
+        if (COUNT) {
+          if (J < endb && leader) wc.ns += GROUP;
+          if ((threadIdx.x & (WAVE - 1)) == 0) wc.nw++;
+          const bool on = J < endb;
+          wc.no += on && __builtin_amdgcn_inverse_ballot_w64(omask) ? 1u : 0u;
+          wc.ni += on && __builtin_amdgcn_inverse_ballot_w64(amask) ? 1u : 0u;
+        }
+        const u64 gmask = fill_fields<GROUP>(omask);
+        if constexpr (Term::WIDE_F32) {
+          // under the accepting lanes' exec mask, and under that of the groups
+          // that step into item j, plain moves and adds (half the issue time of
+          // selects)
+          const float term = t.row_term(amask, v, r2);
+          double wide;
+          asm volatile("s_mov_b64 exec, %3\n\t"
+                       "v_mov_b32 %0, %4\n\t"
+                       "v_cvt_f64_f32 %2, %5\n\t"
+                       "v_add_f64 %1, %1, -%2\n\t"
+                       "s_mov_b64 exec, %6"
+                       : "+v"(untilb), "+v"(t.acc), "=&v"(wide)
+                       : "s"(amask), "v"(JS), "v"(term), "s"(full));
+          // v is written two instructions before its next use, a DPP read
+          unsigned Jn = JS;
+          int vn = vs;
+          asm volatile("s_mov_b64 exec, %2\n\t"
+                       "v_mov_b32 %0, %3\n\t"
+                       "v_add_u32 %1, 32, %4\n\t"
+                       "s_mov_b64 exec, %5"
+                       : "+v"(vn), "+v"(Jn)
+                       : "s"(gmask), "v"(v1), "v"(J), "s"(full));
+          J = Jn;
+          v = vn;
+        } else {
+          const bool go = __builtin_amdgcn_inverse_ballot_w64(gmask);
+          J = go ? J + 32u : JS;
+          v = go ? v1 : vs;
+          const bool accept = __builtin_amdgcn_inverse_ballot_w64(amask);
+          if (accept) t.add(q.w, r2);
+          untilb = accept ? JS : untilb;
+        }
+      }
     }
   } else {
     // lane r of every 8 fetches dword r of its group's item (r = 5, 7 are

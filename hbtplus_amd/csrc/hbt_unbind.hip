@@ -149,8 +149,10 @@ struct hbt_ctx {
   int prof_mode = 0;
   int walk_mode = 0;  // 0: group-shared traversal, 1: independent per-lane walks
   // lanes per traversal group by size bin, graph capture of the pass sequence
-  // (extra passes of a graph launch on a converged level are no-ops)
-  hbt_tuning tune = {{8, 8, 8}, {0, 1 << 30}, 2, 0, 16};
+  // (extra passes of a graph launch on a converged level are no-ops), XCD runs
+  // (64 blocks: the share's walks 78 ms against 82 in runs of 16, and no size
+  // from one 24,000-particle list up was slower)
+  hbt_tuning tune = {{16, 16, 16}, {0, 1 << 30}, 2, 0, 64};
   hipEvent_t evw0 = nullptr, evw1 = nullptr;
   double walk_ms = 0;
   int64_t walk_launches = 0;
@@ -850,7 +852,7 @@ struct Runner {
     if (any_wave()) emit_wave_kernel<<<gwave, BLOCK, 0, c->stream>>>(W, tl_cur, nt_big, nt_cur, copy_sp ? 1 : 0);
     RETCHK(seg_scan(PopLoad{W.ibase, W.bits}, PreStore{W.ibase, W.pre}, PreAdd{W.ibase, W.pre},
                     count_row(NC_SRC)));
-    items_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
+    items_kernel<<<gs, BLOCK, 0, c->stream>>>(W, P);
     if (any_big()) {
       moments_tile_kernel<<<gtile, BLOCK, 0, c->stream>>>(W, tl_cur, nt_big);
       moments_super_kernel<<<gtile, BLOCK, 0, c->stream>>>(W, tl_cur, nt_big);

@@ -587,3 +587,26 @@ def test_particle_type_outside_the_table_is_an_error(gpu):
     cat.cols["type"][5] = 6
     with pytest.raises(RuntimeError, match="particle types outside"):
         gpu(cat.params).unbind_batch(cat)
+
+
+@pytest.mark.parametrize("open_angle", [0.0, 1e-12, 0.45, 30.0])
+@pytest.mark.parametrize("at_edges", [False, True])
+def test_walk_group_forms_agree(gpu, open_angle, at_edges):
+    """the row-broadcast walk of 16- and 32-lane groups (opening test against
+    each item's bound on r^2, exit tested every few steps) and the 8- and
+    64-lane walks (opening test on len^2) give the same bytes, over opening
+    angles from 0 (every node opened) to one at which the root is accepted, in
+    FAST, plain FP32 and REPLAY, with and without segments across a box face"""
+    cat = synth.config2(seed=75, nsub=60, hi=3000, at_edges=at_edges)
+    for prec in (abi.HBT_PREC_FAST, abi.HBT_PREC_FP32, abi.HBT_PREC_REPLAY):
+        U = gpu(_with(cat.params, precision=prec, open_angle=open_angle))
+        got = []
+        for groups in ((8, 8, 8), (16, 16, 16), (32, 32, 32), (64, 64, 64), (16, 32, 16)):
+            t = U.get_tuning()
+            t["walk_group"] = groups
+            t["bin_edge"] = (100, 700)
+            U.set_tuning(t)
+            got.append(U.unbind_batch(cat))
+        for other in got[1:]:
+            for x, y in zip(got[0], other):
+                assert np.array_equal(x.view(np.uint8), y.view(np.uint8)), (prec, groups)
