@@ -1,0 +1,63 @@
+"""Kernels at the sizes where they can go wrong: remainders and edges of tiles
+and waves, smallest and largest of a form's range, values that take its other
+branches, against the CPU oracle."""
+import numpy as np
+import pytest
+
+import oracle
+from hbtplus_amd import abi
+
+pytestmark = pytest.mark.gpu
+
+U53, U24 = 2.0 ** -53, 2.0 ** -24
+
+
+def _pair_sums_of_float_separations(p, seg, pos, m):
+    """The pair sums in double over separations rounded and wrapped in float32,
+    as the FP32 modes form them."""
+    out = np.zeros(int(seg[-1]))
+    h, box, half = 2.8 * float(p["softening"][0]), np.float32(p["box_size"][0]), np.float32(p["box_size"][0] / 2)
+    for lo, hi in zip(seg[:-1], seg[1:]):
+        d = pos[None, lo:hi, :] - pos[lo:hi, None, :]
+        assert d.dtype == np.float32
+        if p["periodic"][0]:
+            d = np.where(d > half, d - box, np.where(d < -half, d + box, d))
+        r = np.sqrt((d.astype(np.float64) ** 2).sum(-1))
+        u = r / h
+        safe = np.maximum(u, 0.5)
+        spline = np.where(u < 0.5, -2.8 + u * u * (16 / 3 + u * u * (6.4 * u - 9.6)),
+                          -3.2 + 1 / (15 * safe) + u * u * (32 / 3 + u * (-16 + u * (9.6 - 32 / 15 * u)))) / h
+        t = np.where(u < 1, spline, -1 / np.maximum(r, h)) * m[None, lo:hi].astype(np.float64)
+        np.fill_diagonal(t, 0)
+        out[lo:hi] = t.sum(1)
+    return out * float(p["G"][0])
+
+
+@pytest.mark.parametrize("where", ["inside", "across_a_face", "not_periodic"])
+def test_direct_potential_sizes(gpu, where):
+    """group sizes around the wave (64) and the chunk (256) and the unrolled
+    four; groups inside the box, split by a face (wrapped chunks) and without a
+    box; coincident particles.  All terms have one sign, so a sum of n terms of
+    up to 16 roundings each is within n + 16 roundings of the exact one: of the
+    oracle's for FP64, for FP32 of the double sum over float separations"""
+    sizes = [1, 2, 3, 4, 5, 63, 64, 65, 127, 255, 256, 257, 511, 513, 1023, 1030]
+    rng = np.random.default_rng(31)
+    seg = np.concatenate([[0], np.cumsum(sizes)])
+    box = 1.0e4
+    pos = rng.normal(size=(seg[-1], 3)) * 20.0 + {"inside": box / 2, "across_a_face": 0.0, "not_periodic": 0.0}[where]
+    pos[seg[5] + 1] = pos[seg[5]]  # a coincident pair, and pairs inside the softening length
+    pos[seg[8]:seg[8] + 10] = pos[seg[8]] + rng.normal(size=(10, 3)) * 0.3
+    pos = (pos % box if where != "not_periodic" else pos).astype(np.float32)
+    x, y, z = (pos[:, j].copy() for j in range(3))
+    m = rng.uniform(1e-5, 2e-4, len(x)).astype(np.float32)
+    p = abi.make_params(periodic=int(where != "not_periodic"), box_size=box)
+    U = gpu(p)
+    refs = {abi.HBT_DIRECT_FP64: oracle.direct_potential(p, seg, x, y, z, m, abi.HBT_DIRECT_FP64)}
+    refs[abi.HBT_DIRECT_FP32] = refs[abi.HBT_DIRECT_FP32_KAHAN] = _pair_sums_of_float_separations(p, seg, pos, m)
+    n = np.repeat(sizes, sizes).astype(np.float64)
+    for mode, ref in refs.items():
+        got = U.direct_potential(seg, x, y, z, m, mode)
+        lone = n == 1
+        assert np.all(got[lone] == 0) and np.all(ref[lone] == 0)
+        rel = np.abs(got[~lone] / ref[~lone] - 1)
+        assert np.all(rel <= (n[~lone] + 16) * (U53 if mode == abi.HBT_DIRECT_FP64 else U24)), (mode, rel.max())
