@@ -5,7 +5,8 @@ import numpy as np
 import pytest
 
 import oracle
-from hbtplus_amd import abi
+from hbtplus_amd import abi, synth
+from test_gpu_props import assert_props
 
 pytestmark = pytest.mark.gpu
 
@@ -61,3 +62,34 @@ def test_direct_potential_sizes(gpu, where):
         assert np.all(got[lone] == 0) and np.all(ref[lone] == 0)
         rel = np.abs(got[~lone] / ref[~lone] - 1)
         assert np.all(rel <= (n[~lone] + 16) * (U53 if mode == abi.HBT_DIRECT_FP64 else U24)), (mode, rel.max())
+
+
+@pytest.mark.parametrize("hz,periodic", [(0.0, 0), (0.1, 1)])
+def test_properties_sizes(gpu, hz, periodic):
+    """bound lists of 0 to 3 entries and around the wave, the block and the
+    tile: profiles bit for bit, shapes within 2 ulps of the oracle's"""
+    sizes = [0, 1, 2, 3, 63, 64, 65, 255, 256, 257, 1023, 1024, 1025, 2049, 5000]
+    rng = np.random.default_rng(37)
+    n = int(np.sum(sizes))
+    pos = rng.normal(size=(n, 3)) * 30.0 + (0.0 if periodic else 500.0)
+    cols = {k: (pos[:, j] % 1000.0).astype(np.float32) for j, k in enumerate("xyz")}
+    for k in ("vx", "vy", "vz"):
+        cols[k] = rng.normal(size=n).astype(np.float32)
+    cols.update(id=np.arange(n, dtype=np.int64), mass=rng.uniform(1e-4, 2e-4, n).astype(np.float32),
+                type=np.ones(n, np.int32))
+    subs = np.zeros(len(sizes), abi.SUB_DTYPE)
+    subs["count"] = subs["nbound"] = sizes
+    subs["parent"] = -1
+    subs["offset"] = subs["out_offset"] = np.cumsum(sizes) - sizes
+    index = rng.permutation(n).astype(np.int64)  # lists of scattered columns
+    for s in subs:
+        l = index[s["out_offset"]:s["out_offset"] + s["nbound"]]
+        if len(l):
+            s["mostbound_pos"] = [cols[k][l[0]] for k in "xyz"]
+            s["mbound"] = cols["mass"][l].astype(np.float64).sum()
+    p = abi.make_params(hz=hz, periodic=periodic, box_size=1000.0)
+    U = gpu(p)
+    cat = synth.Catalogue(cols, subs, p)
+    h = U.upload(cat)
+    got = U.properties_device(h, (U._dev(subs.view(np.uint8)), U._dev(index), None))
+    assert_props(oracle.subhalo_properties(p, cols, subs, index, np.zeros(len(subs), abi.PROPS_DTYPE)), got)
