@@ -24,14 +24,125 @@ __global__ void tree_sources_kernel(Work W, int n, const float *x, const float *
   }
 }
 
-__global__ void walk_points_kernel(Work W, DevParams P, int64_t nt, const float *tx, const float *ty,
-                                   const float *tz, const float *tm, double *out) {
-  // the targets may lie anywhere: a periodic box always takes the wrapped walk
+// The targets in an order that follows the tree, so that neighbouring lanes
+// walk together: a target's bucket is the place of its octant digits among the
+// sources' sorted digits, BUCKET sources to a bucket, and a counting sort puts
+// the buckets in order (the order inside one is arbitrary; no result depends
+// on it).  Walked lane by lane in the caller's order, 120,000 targets spent
+// 1.44 of their call's 1.68 ms in the walk; in tree order, 16 lanes together
+// and without the wrap's FP64 separations where nothing wraps, 0.60 of 0.91.
+constexpr int BUCKET_BITS = 4;
+constexpr int64_t TGT_SLICE = 1 << 24;  // targets per round (their scratch is 12 bytes each)
+
+struct TgtArgs {
+  const float *x, *y, *z, *m;
+  double *out;
+  int n;
+  int *bucket, *rank, *order;  // [n]
+  int *count;                  // [buckets] targets per bucket
+  u64 *first;                  // [buckets] exclusive prefix of count
+  u32 *box;                    // [6] targets' bounding box, ordered-integer encoding
+};
+
+struct TgtLoad {
+  const int *count;
+  __device__ u64 operator()(int, int l) const { return (u64)count[l]; }
+};
+struct TgtStore {
+  u64 *first;
+  __device__ void operator()(int, int l, u64 x) const { first[l] = x; }
+};
+struct TgtAdd {
+  u64 *first;
+  __device__ void operator()(int, int l, u64 x) const { first[l] += x; }
+};
+
+__global__ void __launch_bounds__(BLOCK) tgt_clear_kernel(Work W, TgtArgs A, int nb) {
+  const int i = blockIdx.x * BLOCK + threadIdx.x;
+  if (i < 6) A.box[i] = i < 3 ? 0xffffffffu : 0u;
+  if (i == 0) W.ncount[NC_SORT * W.nseg] = nb;  // the scan's element count
+  for (int j = i; j < nb; j += gridDim.x * BLOCK) A.count[j] = 0;
+}
+
+// Bucket of each target, its place among the bucket's targets, the box of all.
+__global__ void __launch_bounds__(BLOCK) tgt_bucket_kernel(Work W, TgtArgs A) {
+  const Seg &S = W.seg[0];
+  u32 mn[3] = {0xffffffffu, 0xffffffffu, 0xffffffffu}, mx[3] = {0u, 0u, 0u};
+  for (int i0 = blockIdx.x * BLOCK; i0 < A.n; i0 += gridDim.x * BLOCK) {  // uniform across the block
+    const int i = i0 + (int)threadIdx.x;
+    int b = -1;
+    if (i < A.n) {
+#pragma clang fp contract(off)
+      const float x = A.x[i], y = A.y[i], z = A.z[i];
+      const u32 o[3] = {f2ord(x), f2ord(y), f2ord(z)};
+      for (int j = 0; j < 3; j++) { mn[j] = min(mn[j], o[j]); mx[j] = max(mx[j], o[j]); }
+      double c0 = S.center[0], c1 = S.center[1], c2 = S.center[2], lh = 0.5 * S.Len;
+      u64 key = 0;
+      for (int d = 0; d < S.D; d++) {
+        lh *= 0.5;
+        int sub = 0;
+        if (x > c0) { c0 += lh; sub |= 1; } else c0 -= lh;
+        if (y > c1) { c1 += lh; sub |= 2; } else c1 -= lh;
+        if (z > c2) { c2 += lh; sub |= 4; } else c2 -= lh;
+        key = (key << 3) | (u64)sub;
+      }
+      key <<= 3 * (MAX_DEPTH - S.D);
+      int lo = 0, hi = S.n_src;  // first source whose digits are not below the target's
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (W.k0[mid] < key) lo = mid + 1; else hi = mid;
+      }
+      b = lo >> BUCKET_BITS;
+      A.bucket[i] = b;
+    }
+    // the lanes in the first lane's bucket take their places with one atomic
+    const int lead = __builtin_amdgcn_readfirstlane(b);
+    const u64 same = __ballot(b == lead && b >= 0);
+    if (b >= 0) {
+      const int lane = threadIdx.x & (WAVE - 1);
+      int r = 0;
+      if (b == lead) {
+        const int head = __ffsll((long long)same) - 1;
+        if (lane == head) r = atomicAdd(&A.count[b], __popcll(same));
+        r = __shfl(r, head, WAVE) + __popcll(same & ((1ull << lane) - 1ull));
+      } else {
+        r = atomicAdd(&A.count[b], 1);
+      }
+      A.rank[i] = r;
+    }
+  }
+  fold_box(mn, mx, A.box, A.box + 3);
+}
+
+__global__ void __launch_bounds__(BLOCK) tgt_order_kernel(TgtArgs A) {
+  for (int i = blockIdx.x * BLOCK + threadIdx.x; i < A.n; i += gridDim.x * BLOCK)
+    A.order[A.first[A.bucket[i]] + A.rank[i]] = i;
+}
+
+// One target per lane, in tree order.  The FP32 walk wraps separations only
+// where some target and source can be more than half a box apart (sources'
+// and targets' boxes; a node's centre may lie a rounding outside its sources').
+__global__ void __launch_bounds__(BLOCK) walk_points_kernel(Work W, DevParams P, TgtArgs A,
+                                                            const Item *__restrict__ it) {
   Seg S = W.seg[0];
-  S.straddle = P.periodic;
-  unsigned ni = 0, no = 0;
-  for (int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x; i < nt; i += (int64_t)gridDim.x * BLOCK)
-    out[i] = walk_dispatch<false>(W, P, S, tx[i], ty[i], tz[i], tm ? tm[i] : 0.f, ni, no);
+  bool wrap = false;
+  if (P.periodic)
+    for (int j = 0; j < 3; j++) {
+      const double s0 = ord2f(S.bmin[j]), s1 = ord2f(S.bmax[j]), t0 = ord2f(A.box[j]), t1 = ord2f(A.box[3 + j]);
+      const double far = t1 - s0 > s1 - t0 ? t1 - s0 : s1 - t0;
+      if (!(far <= (double)P.box_half * (1.0 - 1e-6)) || !(t0 <= t1)) wrap = true;  // also where one is not a number
+    }
+  S.straddle = wrap ? 1 : 0;
+  WalkCount wc;
+  for (int i0 = blockIdx.x * BLOCK + (threadIdx.x & ~(WAVE - 1)); i0 < A.n; i0 += gridDim.x * BLOCK) {
+    const int i = i0 + (int)(threadIdx.x & (WAVE - 1));
+    const bool live = i < A.n;
+    const int t = live ? A.order[i] : 0;
+    const float x = A.x[t], y = A.y[t], z = A.z[t], tm = A.m ? A.m[t] : 0.f;
+    const double pot = P.replay ? walk_group_dispatch<16, false, true>(it, P, S, 0, S.n_items, live, x, y, z, tm, wc)
+                                : walk_group_dispatch<16, false, false>(it, P, S, 0, S.n_items, live, x, y, z, tm, wc);
+    if (live) A.out[t] = pot * (double)P.G / (double)P.a;
+  }
 }
 
 }  // namespace
@@ -52,6 +163,8 @@ extern "C" int hbt_tree_potential(hbt_ctx *ctx, int64_t n_src, const float *sx, 
   Level L;
   build_level(N, std::vector<int>{0}, ctx->tune, nullptr, 1, L);
   RETCHK(ensure_slots(ctx, L.nslots, 1, (int64_t)L.tiles.size()));
+  if (n_tgt > 0)
+    RETCHK(ctx->tgt.ensure(((size_t)(n_src >> BUCKET_BITS) + 1) * 12 + 24 + (size_t)std::min(n_tgt, TGT_SLICE) * 12));
   RETCHK(stage_level(ctx, L));
   Runner R;
   R.c = ctx;
@@ -69,9 +182,29 @@ extern "C" int hbt_tree_potential(hbt_ctx *ctx, int64_t n_src, const float *sx, 
   tree_only_setup_kernel<<<1, 1, 0, st>>>(R.W, (int)n_src);
   tree_sources_kernel<<<grid_for(n_src, ctx->cus), BLOCK, 0, st>>>(R.W, (int)n_src, sx, sy, sz, smass);
   RETCHK(R.build_tree(false));
-  if (n_tgt > 0)
-    walk_points_kernel<<<grid_for(n_tgt, ctx->cus), BLOCK, 0, st>>>(R.W, R.P, n_tgt, tx, ty, tz,
-                                                                    target_mass, out_phi);
+  const int nb = (int)(n_src >> BUCKET_BITS) + 1;  // a target's place among the sources is 0 .. n_src
+  for (int64_t t0 = 0; t0 < n_tgt; t0 += TGT_SLICE) {
+    TgtArgs A;
+    A.n = (int)std::min<int64_t>(TGT_SLICE, n_tgt - t0);
+    A.x = tx + t0; A.y = ty + t0; A.z = tz + t0;
+    A.m = target_mass ? target_mass + t0 : nullptr;
+    A.out = out_phi + t0;
+    A.first = ctx->tgt.as<u64>();
+    A.count = (int *)(A.first + nb);
+    A.box = (u32 *)(A.count + nb);
+    A.bucket = (int *)(A.box + 6);
+    A.rank = A.bucket + A.n;
+    A.order = A.rank + A.n;
+    const int *n = R.count_row(NC_SORT);
+    tgt_clear_kernel<<<grid_for(nb, ctx->cus), BLOCK, 0, st>>>(R.W, A, nb);
+    tgt_bucket_kernel<<<grid_for(A.n, ctx->cus), BLOCK, 0, st>>>(R.W, A);
+    // the level's tile table starts at the buckets' tiles (fewer buckets than sources)
+    const int nt = (nb + TILE - 1) / TILE, g = std::min(nt, ctx->cus * 8);
+    scan_tiles_kernel<u64><<<g, BLOCK, 0, st>>>(R.tl_cur, nt, n, ctx->tsum.as<u64>(), TgtLoad{A.count}, TgtStore{A.first});
+    if (nt > 1) scan_add_kernel<u64><<<g, BLOCK, 0, st>>>(R.tl_cur, nt, n, ctx->tsum.as<u64>(), TgtAdd{A.first});
+    tgt_order_kernel<<<grid_for(A.n, ctx->cus), BLOCK, 0, st>>>(A);
+    walk_points_kernel<<<(int)std::min<int64_t>((A.n + BLOCK - 1) / BLOCK, (int64_t)1 << 20), BLOCK, 0, st>>>(R.W, R.P, A, R.W.items);
+  }
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(st));
   return HBT_OK;

@@ -171,6 +171,7 @@ struct hbt_ctx {
   uint32_t rand_seed = 1;
   int64_t rand_pos = 0;
   DBuf Er, draws, randtab;              // refinement energies; a level's draws; chunk jump matrices
+  DBuf tgt;                             // hbt_tree_potential: its targets in tree order
   DBuf kick, kickin, kickcnt;           // lists compacted by KickNullParticles, their ranges and counts
   DView rwin;                           // the level's window of the stream (staged)
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -181,7 +182,7 @@ struct hbt_ctx {
                     &bits, &pre, &nlo, &nhi, &npos, &items, &scan64, &pk, &gk,
                     &isb, &seg_of_slot, &cross, &cross2, &tcount, &seg, &lvlbuf, &ncount, &tsum, &tpart, &active, &counters,
                     &st_cols, &st_subs, &st_out_i, &st_out_e, &st_phi, &segact, &actbuf, &gaps, &pack, &idtab, &idpart, &idcnt,
-                    &Er, &draws, &randtab, &kick, &kickin, &kickcnt})
+                    &Er, &draws, &randtab, &tgt, &kick, &kickin, &kickcnt})
       b->release();
     if (h_active) (void)hipHostFree(h_active);
     if (h_stage) (void)hipHostFree(h_stage);
