@@ -30,7 +30,8 @@ __global__ void tree_sources_kernel(Work W, int n, const float *x, const float *
 // the buckets in order (the order inside one is arbitrary; no result depends
 // on it).  Walked lane by lane in the caller's order, 120,000 targets spent
 // 1.44 of their call's 1.68 ms in the walk; in tree order, 16 lanes together
-// and without the wrap's FP64 separations where nothing wraps, 0.60 of 0.91.
+// and without the wrap's FP64 separations where nothing wraps, 0.60 of 0.91
+// (and 0.32 of 0.65 where several waves share a chunk).
 constexpr int BUCKET_BITS = 4;
 constexpr int64_t TGT_SLICE = 1 << 24;  // targets per round (their scratch is 12 bytes each)
 
@@ -119,12 +120,10 @@ __global__ void __launch_bounds__(BLOCK) tgt_order_kernel(TgtArgs A) {
     A.order[A.first[A.bucket[i]] + A.rank[i]] = i;
 }
 
-// One target per lane, in tree order.  The FP32 walk wraps separations only
-// where some target and source can be more than half a box apart (sources'
-// and targets' boxes; a node's centre may lie a rounding outside its sources').
-__global__ void __launch_bounds__(BLOCK) walk_points_kernel(Work W, DevParams P, TgtArgs A,
-                                                            const Item *__restrict__ it) {
-  Seg S = W.seg[0];
+// The FP32 walk wraps separations only where some target and source can be
+// more than half a box apart (sources' and targets' boxes; a node's centre may
+// lie a rounding outside its sources').
+__device__ __forceinline__ bool targets_wrap(const Seg &S, const DevParams &P, const TgtArgs &A) {
   bool wrap = false;
   if (P.periodic)
     for (int j = 0; j < 3; j++) {
@@ -132,7 +131,14 @@ __global__ void __launch_bounds__(BLOCK) walk_points_kernel(Work W, DevParams P,
       const double far = t1 - s0 > s1 - t0 ? t1 - s0 : s1 - t0;
       if (!(far <= (double)P.box_half * (1.0 - 1e-6)) || !(t0 <= t1)) wrap = true;  // also where one is not a number
     }
-  S.straddle = wrap ? 1 : 0;
+  return wrap;
+}
+
+// One target per lane, in tree order.
+__global__ void __launch_bounds__(BLOCK) walk_points_kernel(Work W, DevParams P, TgtArgs A,
+                                                            const Item *__restrict__ it) {
+  Seg S = W.seg[0];
+  S.straddle = targets_wrap(S, P, A) ? 1 : 0;
   WalkCount wc;
   for (int i0 = blockIdx.x * BLOCK + (threadIdx.x & ~(WAVE - 1)); i0 < A.n; i0 += gridDim.x * BLOCK) {
     const int i = i0 + (int)(threadIdx.x & (WAVE - 1));
@@ -143,6 +149,27 @@ __global__ void __launch_bounds__(BLOCK) walk_points_kernel(Work W, DevParams P,
                                 : walk_group_dispatch<16, false, false>(it, P, S, 0, S.n_items, live, x, y, z, tm, wc);
     if (live) A.out[t] = pot * (double)P.G / (double)P.a;
   }
+}
+
+// The same with PARTS waves to 64 targets, one chunk per workgroup.
+template <int PARTS>
+__global__ void __launch_bounds__(PARTS *WAVE) walk_points_split_kernel(Work W, DevParams P, TgtArgs A,
+                                                                        const Item *__restrict__ it) {
+  __shared__ double part[PARTS - 1][WAVE];
+  const Seg &S = W.seg[0];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int i = blockIdx.x * WAVE + (int)(threadIdx.x & (WAVE - 1));
+  const bool live = i < A.n;
+  const int t = live ? A.order[i] : 0;
+  const float x = A.x[t], y = A.y[t], z = A.z[t], tm = A.m ? A.m[t] : 0.f;
+  const int M = S.n_items;
+  const int mid = A.bucket[A.order[min((int)blockIdx.x * WAVE + WAVE / 2, A.n - 1)]] << BUCKET_BITS;
+  const int own = __builtin_amdgcn_readfirstlane((int)((int64_t)M * min(mid, S.n_src) / S.n_src));
+  double pot;
+  if (targets_wrap(S, P, A)) pot = walk_part<PARTS, FastTerm<true, true>>(it, P, w, own, M, live, x, y, z, tm);
+  else pot = walk_part<PARTS, FastTerm<false, true>>(it, P, w, own, M, live, x, y, z, tm);
+  pot = add_parts<PARTS>(pot, part);
+  if (w == 0 && live) A.out[t] = pot * (double)P.G / (double)P.a;
 }
 
 }  // namespace
@@ -203,7 +230,15 @@ extern "C" int hbt_tree_potential(hbt_ctx *ctx, int64_t n_src, const float *sx, 
     scan_tiles_kernel<u64><<<g, BLOCK, 0, st>>>(R.tl_cur, nt, n, ctx->tsum.as<u64>(), TgtLoad{A.count}, TgtStore{A.first});
     if (nt > 1) scan_add_kernel<u64><<<g, BLOCK, 0, st>>>(R.tl_cur, nt, n, ctx->tsum.as<u64>(), TgtAdd{A.first});
     tgt_order_kernel<<<grid_for(A.n, ctx->cus), BLOCK, 0, st>>>(A);
-    walk_points_kernel<<<(int)std::min<int64_t>((A.n + BLOCK - 1) / BLOCK, (int64_t)1 << 20), BLOCK, 0, st>>>(R.W, R.P, A, R.W.items);
+    const int chunks = (A.n + WAVE - 1) / WAVE;
+    switch (R.P.replay || !R.P.wide_sum ? 1 : walk_parts(chunks, ctx->cus)) {
+      case 16: walk_points_split_kernel<16><<<chunks, 16 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items); break;
+      case 8: walk_points_split_kernel<8><<<chunks, 8 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items); break;
+      case 4: walk_points_split_kernel<4><<<chunks, 4 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items); break;
+      case 2: walk_points_split_kernel<2><<<chunks, 2 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items); break;
+      default:
+        walk_points_kernel<<<(A.n + BLOCK - 1) / BLOCK, BLOCK, 0, st>>>(R.W, R.P, A, R.W.items);
+    }
   }
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(st));

@@ -472,6 +472,19 @@ int walk_grid(int64_t nslots, int xcd_run) {
   return (int)std::max<int64_t>(g, 1);
 }
 
+// Waves that share a chunk's walk (1, 2, 4, 8 or 16): about eight waves per
+// SIMD.  From six without sharing on a second wave no longer pays: a list of
+// 420,000 (6,563 chunks) walks 1.71 ms alone and 1.78 shared by two, 50 lists of
+// together 5,900 chunks 0.81 and 0.62, one list of 24,000 (375) 0.53 and, by 16,
+// 0.147.
+int walk_parts(int64_t chunks, int cus) {
+  const int64_t simds = 4 * (int64_t)cus;
+  if (chunks >= 6 * simds) return 1;
+  int parts = 2;
+  while (parts < 16 && chunks * parts < 8 * simds) parts *= 2;
+  return parts;
+}
+
 int grid_for(int64_t n, int cus) {
   int64_t g = (n + BLOCK - 1) / BLOCK;
   int64_t cap = (int64_t)cus * 16;
@@ -902,8 +915,20 @@ struct Runner {
     }
   }
 
+  template <int PARTS>
+  void launch_split_walk() {
+    walk_split_kernel<PARTS><<<(int)(W.nact / WAVE), PARTS * WAVE, 0, c->stream>>>(W, P, W.items);
+  }
+
   void launch_walk(bool count) {
-    if (c->walk_mode == 0) {
+    // few chunks: several waves to a chunk (FP64 sums of FP32 terms only)
+    const int parts = (c->walk_mode == 0 && !count && !P.replay && P.wide_sum) ? walk_parts(W.nact / WAVE, c->cus) : 1;
+    if (parts > 1) {
+      if (parts == 2) launch_split_walk<2>();
+      else if (parts == 4) launch_split_walk<4>();
+      else if (parts == 8) launch_split_walk<8>();
+      else launch_split_walk<16>();
+    } else if (c->walk_mode == 0) {
       const int *g = c->tune.walk_group;
       const int uniform = (g[0] == g[1] && g[1] == g[2]) ? g[0] : 0;
       switch (uniform) {

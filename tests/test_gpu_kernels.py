@@ -128,3 +128,17 @@ def test_tree_potential_target_orders(gpu, n_src, periodic):
                 assert np.array_equal(ref[ok], got[ok]), (kind, nt)
             else:
                 assert np.abs(got[ok] / ref[ok] - 1).max() < 1e-5, (kind, nt)
+
+
+@pytest.mark.parametrize("at_edges", [False, True])
+def test_shared_walk_changes_no_bit(gpu, at_edges):
+    """a level of more than 6,144 chunks of targets is walked one wave to a
+    chunk, each of its subhalos alone by up to 16 waves sharing the items: the
+    FP64 sums are exact for terms this far apart (masses over a factor of 30,
+    lists up to 20,000), so records, lists and energies agree byte for byte"""
+    cat = synth.config2(seed=81, nsub=2600, hi=2.0e4, at_edges=at_edges)
+    assert np.sum((cat.subs["count"] + 63) // 64) > 6144
+    cat.cols["mass"] = (1e-4 * np.random.default_rng(5).uniform(1, 30, cat.n_particles)).astype(np.float32)
+    U = gpu(cat.params)
+    for a, b in zip(U.unbind_batch(cat), U.unbind_batch(cat, plain=True)):
+        assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
