@@ -149,6 +149,132 @@ __device__ __forceinline__ int merge_levels(int n) {
   return m;
 }
 
+// ---- sorting networks of one wave ---------------------------------------------
+// Lane l holds elements R l .. R l + R - 1 (padding sorts last), a bitonic
+// network up to the power of two that covers them, partners less than R apart
+// swapped in the lane and the others read across lanes.
+
+// Lane x ^ M of the wave (within 32 lanes through the crossbar's bit mode,
+// whose pattern is part of the instruction).
+template <int M>
+__device__ __forceinline__ u32 lane_xor(u32 v) {
+  if constexpr (M < 32) return (u32)__builtin_amdgcn_ds_swizzle((int)v, 0x1f | (M << 10));
+  else return (u32)__shfl_xor((int)v, M, WAVE);
+}
+template <int M>
+__device__ __forceinline__ u64 lane_xor(u64 v) {
+  return ((u64)lane_xor<M>((u32)(v >> 32)) << 32) | lane_xor<M>((u32)v);
+}
+
+__device__ __forceinline__ void sort_keep(bool keep_small, u64 ko, u32 vo, u64 &k, u32 &v) {
+  const bool other_less = pair_less(ko, vo, k, v);
+  if (keep_small ? other_less : !other_less) {
+    k = ko;
+    v = vo;
+  }
+}
+
+// Elements a < b of one lane: the lower keeps the smaller in an ascending run.
+__device__ __forceinline__ void sort_pair(bool up, u64 &ka, u32 &va, u64 &kb, u32 &vb) {
+  if (pair_less(kb, vb, ka, va) == up) {
+    const u64 tk = ka; ka = kb; kb = tk;
+    const u32 tv = va; va = vb; vb = tv;
+  }
+}
+
+// The network's stage (SIZE, J): partners J apart in runs of SIZE.
+template <int R, int SIZE, int J>
+__device__ __forceinline__ void sort_stage(u64 (&k)[R], u32 (&v)[R], int lane) {
+  const int e0 = R * lane;
+  if constexpr (J >= R) {
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int e = e0 + r;
+      // the lower element of a pair keeps the smaller one in an ascending run
+      sort_keep(((e & J) == 0) == ((e & SIZE) == 0), lane_xor<J / R>(k[r]), lane_xor<J / R>(v[r]), k[r], v[r]);
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < R; r++)
+      if ((r & J) == 0) sort_pair(((e0 + r) & SIZE) == 0, k[r], v[r], k[r | J], v[r | J]);
+  }
+  if constexpr (J > 1) sort_stage<R, SIZE, J / 2>(k, v, lane);
+}
+
+// Sorts the wave's R * WAVE elements, of which the first `cnt` matter (the
+// rest are padding): runs of SIZE, then of twice that, up to cnt.
+template <int R, int SIZE = 2>
+__device__ __forceinline__ void sort_wave(u64 (&k)[R], u32 (&v)[R], int lane, int cnt) {
+  if (SIZE / 2 >= cnt) return;  // uniform across the wave
+  sort_stage<R, SIZE, SIZE / 2>(k, v, lane);
+  if constexpr (SIZE < R * WAVE) sort_wave<R, SIZE * 2>(k, v, lane, cnt);
+}
+
+// Outputs among the first d of the merge of A (la) and B (lb) that come from A.
+template <class GetA, class GetB>
+__device__ __forceinline__ int merge_split(GetA a, GetB b, int la, int lb, int d) {
+  int lo = d > lb ? d - lb : 0, hi = d < la ? d : la;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    u64 ka, kb;
+    u32 va, vb;
+    a(mid, ka, va);
+    b(d - 1 - mid, kb, vb);
+    if (pair_less(ka, va, kb, vb)) lo = mid + 1; else hi = mid;
+  }
+  return lo;
+}
+
+// Sorts a tile of cnt <= TILE elements held four per thread (element 4 i + r
+// in thread i, padding ~0 / ~0 past cnt) into sk / sv: each wave sorts its 256
+// in registers, then merges in LDS join 2 and 4 of those runs, each thread
+// finding its split of its pair of runs and its four outputs.  One LDS network
+// over the whole tile is a chain of 55 barriers: 25 us for a tile alone, 10 so.
+__device__ __forceinline__ void sort_tile(u64 (&k)[ITEMS], u32 (&v)[ITEMS], int cnt, u64 *sk, u32 *sv) {
+  constexpr int RUN = ITEMS * WAVE;
+  const int i0 = ITEMS * (int)threadIdx.x;
+  const int w0 = i0 & ~(RUN - 1);
+  if (w0 < cnt) sort_wave<ITEMS>(k, v, threadIdx.x & (WAVE - 1), min(RUN, cnt - w0));
+#pragma unroll
+  for (int r = 0; r < ITEMS; r++) { sk[i0 + r] = k[r]; sv[i0 + r] = v[r]; }
+  __syncthreads();
+  for (int width = RUN; width < cnt; width *= 2) {  // uniform across the block
+    const int a0 = i0 & ~(2 * width - 1), d = i0 - a0;
+    const u64 *ka = sk + a0, *kb = ka + width;
+    const u32 *va = sv + a0, *vb = va + width;
+    const int lb = min(width, max(0, cnt - a0 - width));  // past cnt there is padding only
+    const bool merge = lb > 0;
+    if (merge) {
+      int i = merge_split([&](int x, u64 &kk, u32 &vv) { kk = ka[x]; vv = va[x]; },
+                          [&](int x, u64 &kk, u32 &vv) { kk = kb[x]; vv = vb[x]; }, width, width, d);
+      int j = d - i;
+      u64 x = i < width ? ka[i] : ~0ull, y = j < width ? kb[j] : ~0ull;
+      u32 xv = i < width ? va[i] : ~0u, yv = j < width ? vb[j] : ~0u;
+#pragma unroll
+      for (int r = 0; r < ITEMS; r++) {
+        const bool take_a = j >= width || (i < width && !pair_less(y, yv, x, xv));
+        k[r] = take_a ? x : y;
+        v[r] = take_a ? xv : yv;
+        if (take_a) {
+          i++;
+          x = i < width ? ka[i] : ~0ull;
+          xv = i < width ? va[i] : ~0u;
+        } else {
+          j++;
+          y = j < width ? kb[j] : ~0ull;
+          yv = j < width ? vb[j] : ~0u;
+        }
+      }
+    }
+    __syncthreads();
+    if (merge) {
+#pragma unroll
+      for (int r = 0; r < ITEMS; r++) { sk[i0 + r] = k[r]; sv[i0 + r] = v[r]; }
+    }
+    __syncthreads();
+  }
+}
+
 // Sorts each tile's live elements [start, min(start+TILE, n[seg])) from
 // (k0, v0) into the buffer from which the segment's merge levels end in
 // (k0, v0): (k1, v1) when it needs an odd number of levels, else in place.
@@ -182,29 +308,15 @@ tile_sort_kernel(const Tile *__restrict__ tiles, int ntiles, const int64_t *__re
         if (threadIdx.x == 0) { kout[off] = k0[off]; vout[off] = v0[off]; }
         continue;
       }
-      int P = 1;
-      while (P < cnt) P <<= 1;
-      for (int i = threadIdx.x; i < P; i += BLOCK) {
-        if (i < cnt) { sk[i] = k0[off + i]; sv[i] = v0[off + i]; }
-        else { sk[i] = ~0ull; sv[i] = 0xffffffffu; }
+      u64 k[ITEMS];
+      u32 v[ITEMS];
+#pragma unroll
+      for (int r = 0; r < ITEMS; r++) {
+        const int e = ITEMS * (int)threadIdx.x + r;
+        k[r] = e < cnt ? k0[off + e] : ~0ull;
+        v[r] = e < cnt ? v0[off + e] : ~0u;
       }
-      __syncthreads();
-      for (int k = 2; k <= P; k <<= 1) {
-        for (int j = k >> 1; j > 0; j >>= 1) {
-          for (int p = threadIdx.x; p < (P >> 1); p += BLOCK) {
-            // 2 j (p / j) + p % j, with j a power of two
-            const int i = ((p & ~(j - 1)) << 1) | (p & (j - 1));
-            const int q = i + j;
-            const bool up = (i & k) == 0;
-            u64 ka = sk[i], kb = sk[q];
-            u32 va = sv[i], vb = sv[q];
-            if (pair_less(kb, vb, ka, va) == up) {
-              sk[i] = kb; sk[q] = ka; sv[i] = vb; sv[q] = va;
-            }
-          }
-          __syncthreads();
-        }
-      }
+      sort_tile(k, v, cnt, sk, sv);
       for (int i = threadIdx.x; i < cnt; i += BLOCK) { kout[off + i] = sk[i]; vout[off + i] = sv[i]; }
       __syncthreads();
     }
@@ -212,79 +324,30 @@ tile_sort_kernel(const Tile *__restrict__ tiles, int ntiles, const int64_t *__re
   }
 }
 
-// One-wave tiles of up to R * WAVE elements: lane l holds elements R l ..
-// R l + R - 1 (padding sorts last), a bitonic network up to the power of two
-// that covers the segment, partners less than R apart swapped in the lane and
-// the others read across lanes.  Such segments need no merge level, so the
-// result stays in (k0, v0).
-__device__ __forceinline__ void sort_keep(bool keep_small, u64 ko, u32 vo, u64 &k, u32 &v) {
-  const bool other_less = pair_less(ko, vo, k, v);
-  if (keep_small ? other_less : !other_less) {
-    k = ko;
-    v = vo;
-  }
-}
-
-// Elements a < b of one lane: the lower keeps the smaller in an ascending run.
-__device__ __forceinline__ void sort_pair(bool up, u64 &ka, u32 &va, u64 &kb, u32 &vb) {
-  if (pair_less(kb, vb, ka, va) == up) {
-    const u64 tk = ka; ka = kb; kb = tk;
-    const u32 tv = va; va = vb; vb = tv;
-  }
-}
-
+// One-wave tiles of up to R * WAVE elements.  Such segments need no merge
+// level, so the result stays in (k0, v0).
 template <int R>
 __device__ __forceinline__ void sort_wave_tile(const Tile &tl, const int64_t *__restrict__ base,
                                                const int *__restrict__ n, u64 *k0, u32 *v0) {
-  static_assert(R == 1 || R == 4, "one or four elements per lane");
   const int lane = threadIdx.x & (WAVE - 1);
-  const int e0 = R * lane;
-  {
-    const int cnt = min(R * WAVE, n[tl.seg]);
-    if (cnt <= 1) return;  // uniform across the wave
-    const int64_t off = base[tl.seg];
-    u64 k[R];
-    u32 v[R];
+  const int cnt = min(R * WAVE, n[tl.seg]);
+  if (cnt <= 1) return;  // uniform across the wave
+  const int64_t off = base[tl.seg];
+  u64 k[R];
+  u32 v[R];
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-      const int e = e0 + r;
-      k[r] = e < cnt ? k0[off + e] : ~0ull;
-      v[r] = e < cnt ? v0[off + e] : 0xffffffffu;
-    }
-    int P = 2;
-    while (P < cnt) P <<= 1;
-    for (int size = 2; size <= P; size <<= 1) {
-      for (int j = size >> 1; j > 0; j >>= 1) {  // uniform across the wave
-        if (j >= R) {
+  for (int r = 0; r < R; r++) {
+    const int e = R * lane + r;
+    k[r] = e < cnt ? k0[off + e] : ~0ull;
+    v[r] = e < cnt ? v0[off + e] : 0xffffffffu;
+  }
+  sort_wave<R>(k, v, lane, cnt);
 #pragma unroll
-          for (int r = 0; r < R; r++) {
-            const int e = e0 + r;
-            const u64 ko = __shfl_xor(k[r], j / R, WAVE);
-            const u32 vo = __shfl_xor(v[r], j / R, WAVE);
-            // the lower element of a pair keeps the smaller one in an ascending run
-            sort_keep(((e & j) == 0) == ((e & size) == 0), ko, vo, k[r], v[r]);
-          }
-        } else if (R == 4) {
-          const bool up = (e0 & size) == 0;  // size > j: the same for the lane's pairs
-          if (j == 2) {
-            sort_pair(up, k[0], v[0], k[R > 2 ? 2 : 0], v[R > 2 ? 2 : 0]);
-            sort_pair(up, k[R > 1 ? 1 : 0], v[R > 1 ? 1 : 0], k[R > 3 ? 3 : 0], v[R > 3 ? 3 : 0]);
-          } else {
-            // at size 2 the lane's two pairs run in opposite directions
-            sort_pair(up, k[0], v[0], k[R > 1 ? 1 : 0], v[R > 1 ? 1 : 0]);
-            sort_pair(size == 2 ? !up : up, k[R > 2 ? 2 : 0], v[R > 2 ? 2 : 0], k[R > 3 ? 3 : 0],
-                      v[R > 3 ? 3 : 0]);
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      const int e = e0 + r;
-      if (e < cnt) {
-        k0[off + e] = k[r];
-        v0[off + e] = v[r];
-      }
+  for (int r = 0; r < R; r++) {
+    const int e = R * lane + r;
+    if (e < cnt) {
+      k0[off + e] = k[r];
+      v0[off + e] = v[r];
     }
   }
 }
@@ -310,21 +373,6 @@ sort_wave_kernel(const Tile *__restrict__ tiles, int t0, int tmid, int ntiles, c
 // MERGE_PER outputs.  Keys with their values are distinct, so the merged order
 // is unique.
 constexpr int MERGE_PER = TILE / BLOCK;
-
-// Outputs among the first d of the merge of A (la) and B (lb) that come from A.
-template <class GetA, class GetB>
-__device__ __forceinline__ int merge_split(GetA a, GetB b, int la, int lb, int d) {
-  int lo = d > lb ? d - lb : 0, hi = d < la ? d : la;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    u64 ka, kb;
-    u32 va, vb;
-    a(mid, ka, va);
-    b(d - 1 - mid, kb, vb);
-    if (pair_less(ka, va, kb, vb)) lo = mid + 1; else hi = mid;
-  }
-  return lo;
-}
 
 __global__ void __launch_bounds__(BLOCK)
 merge_pass_kernel(const Tile *__restrict__ tiles, int ntiles, const int64_t *__restrict__ base,
