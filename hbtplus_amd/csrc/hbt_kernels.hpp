@@ -4,15 +4,14 @@
 // runs for every active segment (subhalo) of a level at once:
 //   pass_setup        full pass over Elist[0,Nlast) or correction pass over the
 //                     freshly removed block Elist[Nbound,Nlast) (:312-356)
-//   bbox / tree_params / keys
-//                     root cube and per-particle octant digits computed with the
-//                     reference's double-precision centre iteration
-//                     (src/oct_tree.tpp:118-224)
-//   (segmented sort of the keys)
-//   delta / emit / items / moments
-//                     compressed octree in pre-order with skip pointers; node
-//                     moments accumulated in double over float children in son
-//                     order (src/gravity_tree.cpp:18-77)
+//   tree_one          a segment of one tile: its whole tree in one launch
+//   bbox / keys_sort / (merge levels) / emit / items_tile / moments_super, _cross
+//                     the others: root cube and per-particle octant digits
+//                     computed with the reference's double-precision centre
+//                     iteration (src/oct_tree.tpp:118-224), their segmented sort,
+//                     and from the sorted digits the compressed octree in pre-order
+//                     with skip pointers; node moments accumulated in double over
+//                     float children in son order (src/gravity_tree.cpp:18-77)
 //   walk              stackless walk per target (src/gravity_tree.cpp:79-175)
 //   partition_*       parallel replica of PartitionBindingEnergy (:21-58)
 //   frames            FP64 AverageVelocity/AveragePosition, convergence (:357-421)
@@ -480,7 +479,13 @@ __global__ void pass_setup_kernel(Work W, DevParams P) {
 }
 
 // ---------------------------------------------------------------------------
-// Tree: bounding box, root cube, keys
+// Tree.  Segments of one tile (cap <= TILE) build theirs in one launch, a wave
+// or a workgroup each, everything between the sources and the finished items in
+// LDS (tree_one_kernel).  Larger ones go through their tiles: box, digits and
+// tile sort, merge levels, nodes, pre-order positions, items and moments.  The
+// trees of 200,000 subhalos' passes take 9.1 ms this way (5.5 of it the larger
+// segments'), 50,000 small ones' 6.1; with every stage a launch over all
+// segments, through memory, 12.4 and 8.4.
 
 // Folds every thread's box (ordered-integer encoding of the floats) over the
 // block and into lo[3], hi[3].  Atomics on one address are served one after
@@ -515,7 +520,10 @@ __global__ void __launch_bounds__(BLOCK) bbox_kernel(Work W, const Tile *tiles, 
   for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
     const Tile tl = tiles[t];
     Seg &S = W.seg[tl.seg];
-    if (threadIdx.x == 0) W.tcount[t] = 0;  // node lists of the pass's moments
+    if (threadIdx.x == 0) {
+      W.tcount[t] = 0;  // node lists of the pass's moments
+      if (tl.start == 0) W.ncount[NC_CROSS * W.nseg + tl.seg] = 0;
+    }
     const int cnt = min(TILE, S.n_src - tl.start);
     if (cnt <= 0) continue;  // uniform
     const int64_t b = S.ibase;
@@ -530,122 +538,127 @@ __global__ void __launch_bounds__(BLOCK) bbox_kernel(Work W, const Tile *tiles, 
   }
 }
 
-// One-wave tiles (up to R * WAVE sources, lane l taking sources l + WAVE r):
-// a segment's only tile, so its box is stored directly.
-template <int R>
-__device__ __forceinline__ void bbox_wave_tile(const Work &W, const Tile &tl, int t) {
-  const int lane = threadIdx.x & (WAVE - 1);
-  {
-    Seg &S = W.seg[tl.seg];
-    if (lane == 0) W.tcount[t] = 0;
-    const int cnt = min(R * WAVE, S.n_src);
-    if (cnt <= 0) return;  // uniform across the wave
-    const int64_t b = S.ibase;
-    unsigned int mn[3] = {0xffffffffu, 0xffffffffu, 0xffffffffu}, mx[3] = {0u, 0u, 0u};
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      const int e = lane + WAVE * r;
-      if (e < cnt) {
-        const float4 q = W.pos[b + W.el[b + S.src_lo + e]];
-        const unsigned int o[3] = {f2ord(q.x), f2ord(q.y), f2ord(q.z)};
-        for (int j = 0; j < 3; j++) { mn[j] = min(mn[j], o[j]); mx[j] = max(mx[j], o[j]); }
-      }
-    }
-    for (int d = WAVE / 2; d > 0; d >>= 1)
-      for (int j = 0; j < 3; j++) {
-        mn[j] = min(mn[j], (unsigned int)__shfl_xor((int)mn[j], d, WAVE));
-        mx[j] = max(mx[j], (unsigned int)__shfl_xor((int)mx[j], d, WAVE));
-      }
-    if (lane == 0)
-      for (int j = 0; j < 3; j++) { S.bmin[j] = mn[j]; S.bmax[j] = mx[j]; }
-  }
-}
-
-// Tiles t0 <= t < tmid take four sources per lane, tmid <= t < ntiles one.
-__global__ void __launch_bounds__(BLOCK) bbox_wave_kernel(Work W, const Tile *tiles, int t0, int tmid, int ntiles) {
-  WAVE_TILE_LOOP(t, t0, ntiles) {
-    const Tile tl = tiles[t];
-    if (t < tmid) bbox_wave_tile<4>(W, tl, t);
-    else bbox_wave_tile<1>(W, tl, t);
-  }
-}
-
 // Root cube exactly as OctTree_t::Build (src/oct_tree.tpp:118-139) and the
 // depth schedule: node length halves while >= TreeNodeResolution
 // (src/gravity_tree.cpp:37-40); a node created at depth >= max(1, dlen) is
 // below the resolution floor (src/oct_tree.tpp:200).
-__global__ void tree_params_kernel(Work W, DevParams P) {
-  SEG_LOOP(k, W) {
+struct RootCube {
+  double center[3], Len;
+  int dlen, D;
+  bool deep;  // D truncated at MAX_DEPTH
+};
+
+__device__ __forceinline__ RootCube root_cube(const DevParams &P, const u32 bmin[3], const u32 bmax[3]) {
 #pragma clang fp contract(off)
-    Seg &S = W.seg[k];
-    W.ncount[NC_CROSS * W.nseg + k] = 0;
-    if (S.n_src <= 0) continue;
-    double xmin[3], xmax[3];
-    for (int j = 0; j < 3; j++) { xmin[j] = ord2f(S.bmin[j]); xmax[j] = ord2f(S.bmax[j]); }
-    double Len = xmax[0] - xmin[0];
-    for (int j = 1; j < 3; j++)
-      if ((xmax[j] - xmin[j]) > Len) Len = xmax[j] - xmin[j];
-    for (int j = 0; j < 3; j++) S.center[j] = 0.5 * (xmax[j] + xmin[j]);
-    S.Len = Len;
-    int dlen = 0;
-    while (dlen < 1100 && ldexp(Len, -dlen) >= (double)P.res) dlen++;
-    S.dlen = dlen;
-    int D = dlen < 1 ? 1 : dlen;
-    if (D > MAX_DEPTH) { D = MAX_DEPTH; S.flags |= F_DEEP; }
-    S.D = D;
-    // a correction pass builds its tree over the block just removed, which
-    // lies inside the latest full pass's sources but not inside the previous
-    // correction pass's: the latest full pass bounds the depth of later passes
-    if (!(S.flags & F_CORR)) S.Dfull = D;
-    // the FP32 walk drops the periodic wrap unless some target-source pair can
-    // be more than half a box apart: a correction pass's sources (the block
-    // just removed) may lie on one side of the box edge while its targets lie
-    // on both, so its flag also takes the latest full pass's, whose sources
-    // hold both sets
-    const int st = (P.periodic && Len > 0.5 * (double)P.box_half) ? 1 : 0;
-    if (!(S.flags & F_CORR)) S.sfull = st;
-    // a shuffled list's sampled sources may span less than its targets: the
-    // straddle of the whole list (prelude) bounds every pass
-    S.straddle = st | S.sfull | S.sall;
-  }
+  RootCube R;
+  double xmin[3], xmax[3];
+  for (int j = 0; j < 3; j++) { xmin[j] = ord2f(bmin[j]); xmax[j] = ord2f(bmax[j]); }
+  double Len = xmax[0] - xmin[0];
+  for (int j = 1; j < 3; j++)
+    if ((xmax[j] - xmin[j]) > Len) Len = xmax[j] - xmin[j];
+  for (int j = 0; j < 3; j++) R.center[j] = 0.5 * (xmax[j] + xmin[j]);
+  R.Len = Len;
+  int dlen = 0;
+  while (dlen < 1100 && ldexp(Len, -dlen) >= (double)P.res) dlen++;
+  R.dlen = dlen;
+  int D = dlen < 1 ? 1 : dlen;
+  R.deep = D > MAX_DEPTH;
+  R.D = R.deep ? MAX_DEPTH : D;
+  return R;
 }
 
-// Octant digits of each source for depths 1..D: the reference's insertion
+// The root cube into the segment's state, by one thread.
+__device__ __forceinline__ void store_root_cube(const DevParams &P, const RootCube &R, Seg &S) {
+  for (int j = 0; j < 3; j++) S.center[j] = R.center[j];
+  S.Len = R.Len;
+  S.dlen = R.dlen;
+  if (R.deep) S.flags |= F_DEEP;
+  S.D = R.D;
+  // a correction pass builds its tree over the block just removed, which
+  // lies inside the latest full pass's sources but not inside the previous
+  // correction pass's: the latest full pass bounds the depth of later passes
+  if (!(S.flags & F_CORR)) S.Dfull = R.D;
+  // the FP32 walk drops the periodic wrap unless some target-source pair can
+  // be more than half a box apart: a correction pass's sources (the block
+  // just removed) may lie on one side of the box edge while its targets lie
+  // on both, so its flag also takes the latest full pass's, whose sources
+  // hold both sets
+  const int st = (P.periodic && R.Len > 0.5 * (double)P.box_half) ? 1 : 0;
+  if (!(S.flags & F_CORR)) S.sfull = st;
+  // a shuffled list's sampled sources may span less than its targets: the
+  // straddle of the whole list (prelude) bounds every pass
+  S.straddle = st | S.sfull | S.sall;
+}
+
+// Octant digits of a source for depths 1..D: the reference's insertion
 // descends with lenhalf *= 0.5 and centre +/- lenhalf in double and compares
 // the float coordinate with strict '>' (src/oct_tree.tpp:151-184).  Digits
 // are packed most significant first in bits 62..0.
-__global__ void __launch_bounds__(BLOCK) keys_kernel(Work W) {
-  SLOT_LOOP(s, W) {
+__device__ __forceinline__ u64 octant_key(const double center[3], double Len, int D, float x, float y, float z) {
 #pragma clang fp contract(off)
-    int k;
-    int l = seg_lane_local(W, s, k);
-    if (l < 0) continue;
-    const Seg &S = W.seg[k];
-    if (l >= S.n_src) continue;
-    const int64_t b = S.ibase;
-    const int li = W.el[b + S.src_lo + l];
-    const float4 q = W.pos[b + li];
-    const float x = q.x, y = q.y, z = q.z;
-    double c0 = S.center[0], c1 = S.center[1], c2 = S.center[2];
-    double lh = 0.5 * S.Len;
-    u64 key = 0;
-    for (int d = 0; d < S.D; d++) {
-      lh *= 0.5;
-      int sub = 0;
-      if (x > c0) { c0 += lh; sub |= 1; } else c0 -= lh;
-      if (y > c1) { c1 += lh; sub |= 2; } else c1 -= lh;
-      if (z > c2) { c2 += lh; sub |= 4; } else c2 -= lh;
-      key = (key << 3) | (u64)sub;
+  double c0 = center[0], c1 = center[1], c2 = center[2], lh = 0.5 * Len;
+  u64 key = 0;
+  for (int d = 0; d < D; d++) {
+    lh *= 0.5;
+    int sub = 0;
+    if (x > c0) { c0 += lh; sub |= 1; } else c0 -= lh;
+    if (y > c1) { c1 += lh; sub |= 2; } else c1 -= lh;
+    if (z > c2) { c2 += lh; sub |= 4; } else c2 -= lh;
+    key = (key << 3) | (u64)sub;
+  }
+  return key << (3 * (MAX_DEPTH - D));
+}
+
+// A tile's digits, sorted, into the buffer from which the merge levels end in
+// (k0, v0); the root cube from the box, into the segment's state by its first
+// tile.  In one kernel the keys reach memory sorted: digits and sort in kernels
+// of their own wrote and read 12 bytes per source in between.
+__global__ void __launch_bounds__(BLOCK) keys_sort_kernel(Work W, DevParams P, const Tile *__restrict__ tiles,
+                                                          int ntiles) {
+  __shared__ u64 sk[TILE];
+  __shared__ u32 sv[TILE];
+  __shared__ RootCube cube;
+  for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    const Tile tl = tiles[t];
+    Seg &S = W.seg[tl.seg];
+    const int n = S.n_src;
+    const int cnt = min(TILE, n - tl.start);
+    if (cnt <= 0) continue;  // uniform
+    if (threadIdx.x == 0) {
+      cube = root_cube(P, S.bmin, S.bmax);
+      if (tl.start == 0) store_root_cube(P, cube, S);
     }
-    key <<= 3 * (MAX_DEPTH - S.D);
-    W.k0[s] = key;
-    W.v0[s] = (u32)li;
-    W.bits[s] = 0u;  // node-start masks, set by emit_kernel
+    const int64_t off = S.ibase + tl.start;
+    u32 v[ITEMS];
+    float4 q[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++) {
+      const int e = ITEMS * (int)threadIdx.x + r;
+      v[r] = e < cnt ? (u32)W.el[off + S.src_lo + e] : ~0u;
+    }
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++)
+      if (v[r] != ~0u) q[r] = W.pos[S.ibase + v[r]];
+    __syncthreads();
+    u64 k[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++)
+      k[r] = v[r] != ~0u ? octant_key(cube.center, cube.Len, cube.D, q[r].x, q[r].y, q[r].z) : ~0ull;
+    sort_tile(k, v, cnt, sk, sv);
+    const bool odd = (merge_levels(n) & 1) != 0;
+    u64 *kout = odd ? W.k1 : W.k0;
+    u32 *vout = odd ? W.v1 : W.v0;
+    for (int i = threadIdx.x; i < cnt; i += BLOCK) {
+      kout[off + i] = sk[i];
+      vout[off + i] = sv[i];
+      W.bits[off + i] = 0u;  // node-start masks, set by emit_kernel
+    }
+    __syncthreads();
   }
 }
 
 // ---------------------------------------------------------------------------
-// Tree: structure from sorted keys.  Pair l joins sorted sources l and l+1;
+// Structure from sorted keys.  Pair l joins sorted sources l and l+1;
 // delta = number of leading digits they share (D when the keys are equal: the
 // two are in one cell at the depth of the resolution floor).  A node of the
 // compressed octree is a maximal run of sources whose pairs all have
@@ -670,10 +683,6 @@ __device__ __forceinline__ int prefix_lower(const u64 *key, int lo, int hi, int 
   return lo;
 }
 
-// Per pair l of sorted sources: its delta, and the node of which it is the
-// leftmost split.  The neighbouring pairs' deltas come from the keys.  In a
-// full pass the sorted order also becomes the spatial target order.
-//
 // The keys of a tile (and one on either side) are staged in LDS, so the
 // binary searches for a node's first and last sources run there; a search
 // goes to device memory only for the part of its range outside the tile (the
@@ -699,32 +708,38 @@ struct KeyWin {
   }
 };
 
-// One source l (slot s) of segment S: the work of emit for it.
-__device__ __forceinline__ void emit_one(const Work &W, const Seg &S, const KeyWin &K, int l, int full_copy_sp) {
-  const int n = S.n_src;
-  const int64_t s = S.ibase + l;
-  if (full_copy_sp && !(S.flags & (F_CORR | F_SAMP | F_REFINE))) W.sp[s] = (int)W.v0[s];
-  W.nlo[s] = -1;
-  const int v = (l + 1 < n) ? key_delta(K.at(l), K.at(l + 1), S.D) : -1;
-  W.dl[s] = (signed char)v;
-  if (v < 0) return;
-  const int vl = l > 0 ? key_delta(K.at(l - 1), K.at(l), S.D) : -1;
-  if (vl == v) return;  // source l-1 is in the node, in another child
-  const int vr = l + 2 < n ? key_delta(K.at(l + 1), K.at(l + 2), S.D) : -1;
+// The same interface over keys that are all in LDS.
+struct KeyAll {
+  const u64 *sk;
+  __device__ __forceinline__ u64 at(int i) const { return sk[i]; }
+  __device__ __forceinline__ int lower(int a, int h, int v, u64 p) const { return prefix_lower(sk, a, h, v, p); }
+};
+
+// The node whose leftmost split is pair l of n sources: sources lo..hi at
+// depth v; false if l is no node's leftmost split.  v: the pair's delta (-1:
+// l is the last source).
+template <class Keys>
+__device__ __forceinline__ bool node_of_pair(const Keys &K, int l, int n, int D, int &lo, int &hi, int &v) {
+  v = (l + 1 < n) ? key_delta(K.at(l), K.at(l + 1), D) : -1;
+  if (v < 0) return false;
+  const int vl = l > 0 ? key_delta(K.at(l - 1), K.at(l), D) : -1;
+  if (vl == v) return false;  // source l-1 is in the node, in another child
+  const int vr = l + 2 < n ? key_delta(K.at(l + 1), K.at(l + 2), D) : -1;
   const u64 p = key_prefix(K.at(l), v);
-  int lo = l, hi = l + 1;
+  lo = l;
+  hi = l + 1;
   if (vl > v) {
     lo = K.lower(0, l - 1, v, p);
     // leftmost split iff sources lo and l are in the same child
-    if (key_delta(K.at(lo), K.at(l), S.D) <= v) return;
+    if (key_delta(K.at(lo), K.at(l), D) <= v) return false;
   }
   if (vr >= v) hi = K.lower(l + 2, n - 1, v, p + 1) - 1;
-  W.nlo[s] = lo;
-  W.nhi[s] = hi;
-  atomicOr(&W.bits[S.ibase + lo], 1u << v);
+  return true;
 }
 
-// Workgroup form: one tile of TILE sources, window t0 - 1 .. t0 + TILE + 1.
+// Per pair l of sorted sources: its delta, and the node of which it is the
+// leftmost split.  In a full pass the sorted order also becomes the spatial
+// target order.  One tile of TILE sources, window t0 - 1 .. t0 + TILE + 1.
 __global__ void __launch_bounds__(BLOCK) emit_kernel(Work W, const Tile *__restrict__ tiles, int ntiles,
                                                      int full_copy_sp) {
   __shared__ u64 sk[TILE + 3];
@@ -734,37 +749,31 @@ __global__ void __launch_bounds__(BLOCK) emit_kernel(Work W, const Tile *__restr
     const int n = S.n_src;
     const int cnt = min(TILE, n - tl.start);
     if (cnt <= 0) continue;  // uniform across the block
+    const bool copy_sp = full_copy_sp && !(S.flags & (F_CORR | F_SAMP | F_REFINE));
     KeyWin K{sk, W.k0 + S.ibase, tl.start > 0 ? tl.start - 1 : 0, min(n - 1, tl.start + TILE + 1)};
     for (int i = K.w_lo + (int)threadIdx.x; i <= K.w_hi; i += BLOCK) sk[i - K.w_lo] = K.key[i];
     __syncthreads();
-    for (int i = threadIdx.x; i < cnt; i += BLOCK) emit_one(W, S, K, tl.start + i, full_copy_sp);
+    for (int i = threadIdx.x; i < cnt; i += BLOCK) {
+      const int l = tl.start + i;
+      const int64_t s = S.ibase + l;
+      if (copy_sp) W.sp[s] = (int)W.v0[s];
+      int lo, hi, v;
+      const bool node = node_of_pair(K, l, n, S.D, lo, hi, v);
+      W.dl[s] = (signed char)v;
+      W.nlo[s] = node ? lo : -1;
+      if (node) {
+        W.nhi[s] = hi;
+        atomicOr(&W.bits[S.ibase + lo], 1u << v);
+      }
+    }
     __syncthreads();  // the next tile restages sk
   }
 }
 
-// One-wave form: a segment of at most SMALL_CAP sources, all of its keys in
-// the wave's LDS.
-__global__ void __launch_bounds__(BLOCK) emit_wave_kernel(Work W, const Tile *__restrict__ tiles, int t0,
-                                                          int ntiles, int full_copy_sp) {
-  __shared__ u64 sk[BLOCK / WAVE][SMALL_CAP];
-  const int lane = threadIdx.x & (WAVE - 1), wv = threadIdx.x / WAVE;
-  WAVE_TILE_LOOP(t, t0, ntiles) {
-    const Tile tl = tiles[t];
-    const Seg &S = W.seg[tl.seg];
-    const int n = min(SMALL_CAP, S.n_src);
-    if (n <= 0) continue;  // uniform across the wave
-    KeyWin K{sk[wv], W.k0 + S.ibase, 0, n - 1};
-    for (int i = lane; i < n; i += WAVE) sk[wv][i] = K.key[i];
-    wave_sync();
-    for (int i = lane; i < n; i += WAVE) emit_one(W, S, K, i, full_copy_sp);
-    wave_sync();  // the next tile restages the wave's keys
-  }
-}
-
 // Node length at depth v: Len halved while >= resolution, stored as float.
-__device__ __forceinline__ float node_len(const Seg &S, int v) {
-  const int e = v < S.dlen ? v : S.dlen;
-  return (float)ldexp(S.Len, -e);
+__device__ __forceinline__ float node_len(double Len, int dlen, int v) {
+  const int e = v < dlen ? v : dlen;
+  return (float)ldexp(Len, -e);
 }
 
 // The squared distance below which the FP32 walk opens a node: the smallest
@@ -793,47 +802,36 @@ __device__ __forceinline__ float open_below(float lsq, float theta2) {
   return __uint_as_float(t);
 }
 
-// Writes leaves and node headers in pre-order.  pre = exclusive prefix of
-// popcount(bits) over the segment's sorted sources.
-__global__ void __launch_bounds__(BLOCK) items_kernel(Work W, DevParams P) {
-  SLOT_LOOP(s, W) {
-    int k;
-    int l = seg_lane_local(W, s, k);
-    if (l >= 0) {
-      const Seg &S = W.seg[k];
-      if (l < S.n_src) {
-        const int64_t b = S.ibase, ib = 2 * b;
-        const u32 bl = W.bits[s];
-        const int pos = l + W.pre[s] + __popc(bl);
-        const int li = (int)W.v0[s];
-        // a sampled tree's leaves carry mass * MassFactor (EnergySnapshot_t::GetMass, :79)
-        const float4 q = W.pos[b + li];
-        const float m = (S.flags & F_SAMP) ? q.w * S.mf : q.w;
-        W.items[ib + pos] = Item{make_float4(q.x, q.y, q.z, m),
-                                 make_int2(0, pos + 1), make_int2(32 * (pos + 1), 0)};
-        if (l + 1 == S.n_src) {
-          W.seg[k].n_items = pos + 1;
-          // sentinel after the last item: massless, far from every target,
-          // never opened, its skip is itself, so a group walk that has
-          // finished reads it, adds nothing and stays put
-          W.items[ib + pos + 1] = Item{make_float4(1e18f, 1e18f, 1e18f, 0.f), make_int2(0, pos + 1),
-                                       make_int2(32 * (pos + 1), 0)};
-        }
-        const int lo = W.nlo[s];
-        if (lo >= 0) {
-          const int v = W.dl[s], hi = W.nhi[s];
-          const u32 blo = W.bits[b + lo];
-          const int npos = lo + W.pre[b + lo] + __popc(blo & ((1u << v) - 1u));
-          const int hpos = hi + W.pre[b + hi] + __popc(W.bits[b + hi]);
-          const float len = node_len(S, v);
-          const float lsq = len * len;
-          W.items[ib + npos] = Item{make_float4(0.f, 0.f, 0.f, 0.f), make_int2(__float_as_int(lsq), hpos + 1),
-                                    make_int2(32 * (hpos + 1), __float_as_int(open_below(lsq, P.theta2)))};
-          W.npos[s] = (int)(ib + npos);
-        }
-      }
+// The opening lengths of a tree's depths, filled by the first NLEVEL threads.
+struct DepthTable {
+  float lsq[NLEVEL], below[NLEVEL];
+  __device__ __forceinline__ void fill(int v, double Len, int dlen, float theta2) {
+    if (v < NLEVEL) {
+      const float len = node_len(Len, dlen, v);
+      lsq[v] = len * len;
+      below[v] = open_below(lsq[v], theta2);
     }
   }
+};
+
+__device__ __forceinline__ Item leaf_item(const float4 &pm, int pos) {
+  return Item{pm, make_int2(0, pos + 1), make_int2(32 * (pos + 1), 0)};
+}
+__device__ __forceinline__ Item node_item(const float4 &pm, int skip, float lsq, float below) {
+  return Item{pm, make_int2(__float_as_int(lsq), skip), make_int2(32 * skip, __float_as_int(below))};
+}
+// Sentinel after the last item: massless, far from every target, never
+// opened, its skip is itself, so a group walk that has finished reads it, adds
+// nothing and stays put.
+__device__ __forceinline__ Item sentinel_item(int pos) {
+  return Item{make_float4(1e18f, 1e18f, 1e18f, 0.f), make_int2(0, pos), make_int2(32 * pos, 0)};
+}
+
+// A leaf: a sampled tree's leaves carry mass * MassFactor (EnergySnapshot_t::GetMass, :79).
+__device__ __forceinline__ float4 leaf_pm(const Work &W, const Seg &S, int li) {
+  float4 q = W.pos[S.ibase + li];
+  if (S.flags & F_SAMP) q.w = q.w * S.mf;
+  return q;
 }
 
 // Node moments: mass and centre of mass accumulated in double over the float
@@ -866,20 +864,242 @@ __device__ __forceinline__ void node_moments(const Work &W, int64_t ib, int g) {
                                g, (int)(ib + W.items[g].ax.y));
 }
 
-// Node moments in two or three launches.  moments_tile_kernel: one workgroup
-// per tile stages the tile's items in LDS (its leaves, the headers of the
-// nodes whose leftmost leaf it holds: fewer than 2 TILE + MAX_DEPTH), computes
-// the nodes whose leaves all lie in the tile deepest first (their children do
-// too), depth by depth with a workgroup barrier between depths, and lists the
-// pairs of the nodes whose leaves cross a tile edge (at most one per depth per
-// edge): in W.cross, by super-tile (SUPER_TILES tiles), when the node lies in
-// one, else in W.cross2 by segment.  moments_super_kernel: one workgroup per
-// super-tile computes its listed nodes, deepest first; moments_cross_kernel
-// (only for segments of more than one super-tile): one workgroup per segment
-// computes the rest, deepest first.  A node's children are inside a tile (done
-// by the first launch) or listed at the same or a lower level and deeper.
-// Each node sums its children in son order (sum_children), so the results do
-// not depend on which launch computes a node.
+// A team: the threads that build one tile's tree (one wave, or the workgroup),
+// R elements each.
+template <int T_, int R_>
+struct Team {
+  static constexpr int T = T_, R = R_, CAP = T_ * R_;
+  static_assert(T_ == WAVE || T_ == BLOCK, "a wave or a workgroup");
+  static __device__ __forceinline__ int id() { return T == WAVE ? threadIdx.x & (WAVE - 1) : threadIdx.x; }
+  static __device__ __forceinline__ void sync() {
+    if (T == WAVE) wave_sync();
+    else __syncthreads();
+  }
+  template <class X>
+  static __device__ __forceinline__ X exclusive_scan(X x, X *total) {
+    if (T == BLOCK) return block_exclusive_scan(x, total);
+    const X inc = wave_inclusive_scan(x);
+    *total = __shfl(inc, WAVE - 1, WAVE);
+    return inc - x;
+  }
+};
+
+// The nodes whose leaves all lie in the tile, computed deepest first: depth
+// counts and places, and the LDS items they work on.
+template <int NI, int NN>
+struct TileNodes {
+  float4 pm[NI];
+  unsigned short skip[NI];
+  unsigned short node[NN];       // nodes (item index) grouped by depth, deepest first
+  int count[NLEVEL], first[NLEVEL + 1];
+};
+
+// Fills in the moments of a tile's nodes.  at[r] < 0: no node in thread's slot
+// r; otherwise its LDS item and its depth v[r] (headers' skips and every leaf
+// are in place).  Called by the whole team; leaves the team synchronised.
+template <class TM, int R, int NI, int NN>
+__device__ __forceinline__ void tile_moments(TileNodes<NI, NN> &N, const int (&at)[R], const int (&v)[R]) {
+  for (int d = TM::id(); d < NLEVEL; d += TM::T) N.count[d] = 0;
+  TM::sync();
+  int rank[R];
+#pragma unroll
+  for (int r = 0; r < R; r++)
+    if (at[r] >= 0) rank[r] = atomicAdd(&N.count[v[r]], 1);
+  TM::sync();
+  if (TM::id() == 0) {
+    int o = 0;
+    for (int d = MAX_DEPTH; d >= 0; d--) { N.first[d] = o; o += N.count[d]; }
+    N.first[NLEVEL] = o;
+  }
+  TM::sync();
+#pragma unroll
+  for (int r = 0; r < R; r++)
+    if (at[r] >= 0) N.node[N.first[v[r]] + rank[r]] = (unsigned short)at[r];
+  TM::sync();
+  for (int d = MAX_DEPTH; d >= 0; d--) {
+    const int p0 = N.first[d], p1 = d > 0 ? N.first[d - 1] : N.first[NLEVEL];
+    if (p0 == p1) continue;  // uniform
+    for (int p = p0 + TM::id(); p < p1; p += TM::T) {
+      const int g = N.node[p];
+      N.pm[g] = sum_children([&](int c) { return N.pm[c]; }, [&](int c) { return (int)N.skip[c]; }, g, N.skip[g]);
+    }
+    TM::sync();
+  }
+}
+
+// LDS of a one-tile tree: the sorted keys with what places the items, then, in
+// the same memory, the items.
+template <int CAP>
+struct OneTile {
+  union {
+    struct {
+      u64 key[CAP];
+      u32 val[CAP];
+      u32 bits[CAP];
+      unsigned short pre[CAP];
+    } s;
+    TileNodes<2 * CAP, CAP> n;
+  };
+  DepthTable depth;
+  u32 box[6][BLOCK / WAVE];
+};
+
+// The whole tree of a segment of at most CAP sources: box, root cube, digits,
+// sort, nodes, pre-order positions, items and moments, between one read of the
+// sources and one write of the items.  A chain of LDS steps bounds it: a tree of
+// 300 alone takes 19 us, in launches of their own, each waiting on its chain of
+// loads per source, the stages took 36 and their gaps.  LDS (40 KB) and registers
+// (held to 128) each let four waves run per SIMD.
+template <class TM>
+__device__ __forceinline__ void tree_one(const Work &W, const DevParams &P, const Tile &tl, int full_copy_sp,
+                                         OneTile<TM::CAP> &L) {
+  constexpr int R = TM::R, CAP = TM::CAP;
+  Seg &S = W.seg[tl.seg];
+  const int n = min(CAP, S.n_src);
+  if (n <= 0) return;  // uniform across the team
+  const int64_t b = S.ibase;
+  const int id = TM::id();
+  u32 v[R];
+  float4 q[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const int e = R * id + r;
+    v[r] = e < n ? (u32)W.el[b + S.src_lo + e] : ~0u;
+  }
+  u32 mn[3] = {0xffffffffu, 0xffffffffu, 0xffffffffu}, mx[3] = {0u, 0u, 0u};
+#pragma unroll
+  for (int r = 0; r < R; r++)
+    if (v[r] != ~0u) {
+      q[r] = W.pos[b + v[r]];
+      const u32 o[3] = {f2ord(q[r].x), f2ord(q[r].y), f2ord(q[r].z)};
+      for (int j = 0; j < 3; j++) { mn[j] = min(mn[j], o[j]); mx[j] = max(mx[j], o[j]); }
+    }
+  for (int d = WAVE / 2; d > 0; d >>= 1)
+    for (int j = 0; j < 3; j++) {
+      mn[j] = min(mn[j], (u32)__shfl_xor((int)mn[j], d, WAVE));
+      mx[j] = max(mx[j], (u32)__shfl_xor((int)mx[j], d, WAVE));
+    }
+  if (TM::T > WAVE) {
+    if ((threadIdx.x & (WAVE - 1)) == 0)
+      for (int j = 0; j < 3; j++) { L.box[j][threadIdx.x / WAVE] = mn[j]; L.box[3 + j][threadIdx.x / WAVE] = mx[j]; }
+    TM::sync();
+    for (int w = 0; w < TM::T / WAVE; w++)
+      for (int j = 0; j < 3; j++) { mn[j] = min(mn[j], L.box[j][w]); mx[j] = max(mx[j], L.box[3 + j][w]); }
+  }
+  const RootCube cube = root_cube(P, mn, mx);
+  L.depth.fill(id, cube.Len, cube.dlen, P.theta2);
+  const bool copy_sp = full_copy_sp && !(S.flags & (F_CORR | F_SAMP | F_REFINE));
+  u64 k[R];
+#pragma unroll
+  for (int r = 0; r < R; r++)
+    k[r] = v[r] != ~0u ? octant_key(cube.center, cube.Len, cube.D, q[r].x, q[r].y, q[r].z) : ~0ull;
+  if constexpr (TM::T == WAVE) {
+    sort_wave<R>(k, v, id, n);
+#pragma unroll
+    for (int r = 0; r < R; r++) { L.s.key[R * id + r] = k[r]; L.s.val[R * id + r] = v[r]; }
+  } else {
+    sort_tile(k, v, n, L.s.key, L.s.val);
+  }
+#pragma unroll
+  for (int r = 0; r < R; r++) L.s.bits[id + r * TM::T] = 0u;
+  TM::sync();
+  // nodes, by their leftmost split
+  int lo[R], hi[R], dv[R], at[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const int l = id + r * TM::T;
+    at[r] = -1;
+    if (l < n && node_of_pair(KeyAll{L.s.key}, l, n, cube.D, lo[r], hi[r], dv[r])) {
+      at[r] = 0;
+      atomicOr(&L.s.bits[lo[r]], 1u << dv[r]);
+    }
+  }
+  TM::sync();
+  // pre-order: the nodes that start before each source
+  int own = 0, nodes;
+#pragma unroll
+  for (int r = 0; r < R; r++) own += __popc(L.s.bits[R * id + r]);
+  int run = TM::exclusive_scan(own, &nodes);
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    L.s.pre[R * id + r] = (unsigned short)run;
+    run += __popc(L.s.bits[R * id + r]);
+  }
+  TM::sync();
+  int leaf[R], nskip[R];
+  float4 pm[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const int l = id + r * TM::T;
+    leaf[r] = -1;
+    if (l < n) {
+      const int li = (int)L.s.val[l];
+      if (copy_sp) W.sp[b + l] = li;
+      leaf[r] = l + L.s.pre[l] + __popc(L.s.bits[l]);
+      pm[r] = leaf_pm(W, S, li);
+    }
+    if (at[r] >= 0) {
+      at[r] = lo[r] + L.s.pre[lo[r]] + __popc(L.s.bits[lo[r]] & ((1u << dv[r]) - 1u));
+      nskip[r] = hi[r] + L.s.pre[hi[r]] + __popc(L.s.bits[hi[r]]) + 1;
+    }
+  }
+  TM::sync();  // the items take the keys' place
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    if (leaf[r] >= 0) {
+      L.n.pm[leaf[r]] = pm[r];
+      L.n.skip[leaf[r]] = (unsigned short)(leaf[r] + 1);
+    }
+    if (at[r] >= 0) L.n.skip[at[r]] = (unsigned short)nskip[r];
+  }
+  tile_moments<TM>(L.n, at, dv);
+  Item *out = W.items + 2 * b;
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    if (leaf[r] >= 0) out[leaf[r]] = leaf_item(pm[r], leaf[r]);
+    if (at[r] >= 0) out[at[r]] = node_item(L.n.pm[at[r]], nskip[r], L.depth.lsq[dv[r]], L.depth.below[dv[r]]);
+  }
+  if (id == 0) {
+    const int ni = n + nodes;
+    out[ni] = sentinel_item(ni);
+    store_root_cube(P, cube, S);
+    S.n_items = ni;
+  }
+  TM::sync();  // the next tile reuses the LDS
+}
+
+// Tiles t0 <= t < ntiles, one team each.
+template <int R>
+__global__ void __launch_bounds__(BLOCK, 4) tree_one_wave_kernel(Work W, DevParams P, const Tile *__restrict__ tiles,
+                                                              int t0, int ntiles, int full_copy_sp) {
+  using TM = Team<WAVE, R>;
+  __shared__ OneTile<TM::CAP> L[BLOCK / WAVE];
+  WAVE_TILE_LOOP(t, t0, ntiles) tree_one<TM>(W, P, tiles[t], full_copy_sp, L[threadIdx.x / WAVE]);
+}
+__global__ void __launch_bounds__(BLOCK, 4) tree_one_kernel(Work W, DevParams P, const Tile *__restrict__ tiles, int t0,
+                                                         int ntiles, int full_copy_sp) {
+  using TM = Team<BLOCK, ITEMS>;
+  __shared__ OneTile<TM::CAP> L;
+  for (int t = t0 + (int)blockIdx.x; t < ntiles; t += gridDim.x) tree_one<TM>(W, P, tiles[t], full_copy_sp, L);
+}
+
+// items_tile_kernel: one workgroup per tile places
+// the tile's leaves and the nodes whose leaves all lie in it in LDS (leaves plus
+// the headers of the nodes whose leftmost leaf it holds: fewer than 2 TILE +
+// MAX_DEPTH), computes those nodes deepest first (their children are there too)
+// and writes both out; of the nodes whose leaves cross a tile edge (at most one
+// per depth per edge) it writes the header and lists the pair: in W.cross, by
+// super-tile (SUPER_TILES tiles), when the node lies in one, else in W.cross2 by
+// segment.  moments_super_kernel: one workgroup per super-tile computes its
+// listed nodes, deepest first; moments_cross_kernel (only for segments of more
+// than one super-tile): one workgroup per segment computes the rest, deepest
+// first.  A node's children are inside a tile (done by the first launch) or
+// listed at the same or a lower level and deeper.  Each node sums its children
+// in son order (sum_children), so the results do not depend on which launch
+// computes a node.  With the items placed in LDS they reach memory once and
+// finished, 32 bytes each; placed by a launch of its own and staged again for
+// the moments they were written, read and half written again (200,000 subhalos:
+// 5.2 ms with the smaller segments', 2.0 now).
 constexpr int TILE_ITEMS = 2 * TILE + MAX_DEPTH + 2;
 constexpr int SUPER_TILES = 64;
 constexpr int SUPER = SUPER_TILES * TILE;
@@ -896,110 +1116,99 @@ __device__ __forceinline__ void list_crossing(const Work &W, int t, const Tile &
   }
 }
 
-__global__ void __launch_bounds__(BLOCK) moments_tile_kernel(Work W, const Tile *__restrict__ tiles, int ntiles) {
-  __shared__ float4 spm[TILE_ITEMS];
-  __shared__ int sskip[TILE_ITEMS];
-  __shared__ int snode[TILE];            // local nodes (LDS item index), grouped by depth
-  __shared__ int sdepth[MAX_DEPTH + 2];  // nodes per depth, then the next free place
-  __shared__ int sfirst[MAX_DEPTH + 2];  // first place of each depth
+// pre = exclusive prefix of popcount(bits) over the segment's sorted sources.
+__global__ void __launch_bounds__(BLOCK, 4) items_tile_kernel(Work W, DevParams P, const Tile *__restrict__ tiles,
+                                                           int ntiles) {
+  using TM = Team<BLOCK, ITEMS>;
+  struct Place { u32 bits[TILE]; int pre[TILE]; };
+  __shared__ union { Place p; TileNodes<TILE_ITEMS, TILE> n; } L;
+  __shared__ DepthTable depth;
   for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
     const Tile tl = tiles[t];
     const Seg &S = W.seg[tl.seg];
     const int n = S.n_src;
-    const int cnt = min(TILE, n - 1 - tl.start);  // pairs l with l + 1 < n
-    if (cnt <= 0) continue;  // uniform across the block
-    const int64_t b = S.ibase, ib = 2 * b;
-    const int t_lo = tl.start, t_hi = tl.start + TILE - 1;
     const int nl = min(TILE, n - tl.start);
-    const int lastl = tl.start + nl - 1;
-    const int first = tl.start + W.pre[b + tl.start];
-    const int last = lastl + W.pre[b + lastl] + __popc(W.bits[b + lastl]);
-    const int nit = last - first + 1;
-    int *ncross = W.ncount + NC_CROSS * W.nseg + tl.seg;
-    if (nit > TILE_ITEMS) {
-      // not expected (leaves plus the headers of the nodes starting in the
-      // tile); the same depth order over device memory
-      for (int v = min(max(S.D, S.Dfull), MAX_DEPTH); v >= 0; v--) {
-        for (int i = threadIdx.x; i < cnt; i += BLOCK) {
-          const int64_t s = b + tl.start + i;
-          if (W.dl[s] != v || W.nlo[s] < 0) continue;
-          if (W.nlo[s] >= t_lo && W.nhi[s] <= t_hi) node_moments(W, ib, W.npos[s]);
-          else list_crossing(W, t, tl, b, tl.start + i, W.nlo[s], W.nhi[s], ncross);
-        }
-        __syncthreads();
-      }
-      continue;  // uniform across the block
-    }
-    // one batch of loads per thread: its PER pairs (4-aligned slots; the
-    // group stays inside the segment's wave-aligned slots) and its items
-    constexpr int PER = TILE / BLOCK, IPER = (TILE_ITEMS + BLOCK - 1) / BLOCK;
-    static_assert(PER == 4, "pairs are loaded four at a time");
-    const int p0 = PER * (int)threadIdx.x;
-    int plo[PER], phi[PER], ppos[PER], pdl[PER];
-    if (p0 < cnt) {
-      const int64_t s = b + tl.start + p0;
-      const int4 a = *reinterpret_cast<const int4 *>(W.nlo + s);
-      const int4 h = *reinterpret_cast<const int4 *>(W.nhi + s);
-      const int4 g = *reinterpret_cast<const int4 *>(W.npos + s);
-      const char4 d = *reinterpret_cast<const char4 *>(W.dl + s);
+    if (nl <= 0) continue;  // uniform across the block
+    const int64_t b = S.ibase, ib = 2 * b, s0 = b + tl.start;
+    const int t_lo = tl.start, t_hi = tl.start + TILE - 1;
+    depth.fill(threadIdx.x, S.Len, S.dlen, P.theta2);
+    // one batch of loads per thread: four neighbouring sources and pairs
+    // (4-aligned slots inside the segment's wave-aligned slots)
+    static_assert(ITEMS == 4, "sources are loaded four at a time");
+    const int p0 = ITEMS * (int)threadIdx.x;
+    int plo[ITEMS], phi[ITEMS], pdl[ITEMS], li[ITEMS], pre[ITEMS];
+    u32 bits[ITEMS];
+    if (p0 < nl) {
+      const int4 a = *reinterpret_cast<const int4 *>(W.nlo + s0 + p0);
+      const int4 h = *reinterpret_cast<const int4 *>(W.nhi + s0 + p0);
+      const int4 x = *reinterpret_cast<const int4 *>(W.v0 + s0 + p0);
+      const int4 e = *reinterpret_cast<const int4 *>(W.pre + s0 + p0);
+      const int4 m = *reinterpret_cast<const int4 *>(W.bits + s0 + p0);
+      const char4 d = *reinterpret_cast<const char4 *>(W.dl + s0 + p0);
       plo[0] = a.x; plo[1] = a.y; plo[2] = a.z; plo[3] = a.w;
       phi[0] = h.x; phi[1] = h.y; phi[2] = h.z; phi[3] = h.w;
-      ppos[0] = g.x; ppos[1] = g.y; ppos[2] = g.z; ppos[3] = g.w;
+      li[0] = x.x; li[1] = x.y; li[2] = x.z; li[3] = x.w;
+      pre[0] = e.x; pre[1] = e.y; pre[2] = e.z; pre[3] = e.w;
+      bits[0] = (u32)m.x; bits[1] = (u32)m.y; bits[2] = (u32)m.z; bits[3] = (u32)m.w;
       pdl[0] = d.x; pdl[1] = d.y; pdl[2] = d.z; pdl[3] = d.w;
     }
+    float4 pm[ITEMS];
 #pragma unroll
-    for (int j = 0; j < PER; j++)
-      if (p0 + j >= cnt) plo[j] = -1;
-    float4 qpm[IPER];
-    int qsk[IPER];
-#pragma unroll
-    for (int k = 0; k < IPER; k++) {
-      // past the tile's items the last one is read again (and not stored)
-      const int i = min((int)threadIdx.x + k * BLOCK, nit - 1);
-      qpm[k] = W.items[ib + first + i].pm;
-      qsk[k] = W.items[ib + first + i].ax.y - first;
-    }
-#pragma unroll
-    for (int k = 0; k < IPER; k++) {
-      const int i = (int)threadIdx.x + k * BLOCK;
-      if (i < nit) {
-        spm[i] = qpm[k];
-        sskip[i] = qsk[k];
+    for (int j = 0; j < ITEMS; j++) {
+      if (p0 + j < nl) {
+        pm[j] = leaf_pm(W, S, li[j]);
+        L.p.bits[p0 + j] = bits[j];
+        L.p.pre[p0 + j] = pre[j];
+      } else {
+        plo[j] = -1;
       }
     }
-    for (int v = threadIdx.x; v <= MAX_DEPTH + 1; v += BLOCK) sdepth[v] = 0;
     __syncthreads();
-    int rank[PER];
+    const int first = t_lo + L.p.pre[0];  // the tile's first item
+    int *ncross = W.ncount + NC_CROSS * W.nseg + tl.seg;
+    int leaf[ITEMS], at[ITEMS], nskip[ITEMS];
 #pragma unroll
-    for (int j = 0; j < PER; j++) {
+    for (int j = 0; j < ITEMS; j++) {
+      const int l = t_lo + p0 + j;
+      leaf[j] = p0 + j < nl ? l + pre[j] + __popc(bits[j]) : -1;
+      at[j] = -1;
       if (plo[j] < 0) continue;
-      if (plo[j] >= t_lo && phi[j] <= t_hi) rank[j] = atomicAdd(&sdepth[pdl[j]], 1);
-      else list_crossing(W, t, tl, b, tl.start + p0 + j, plo[j], phi[j], ncross);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      int o = 0;
-      for (int v = MAX_DEPTH; v >= 0; v--) { sfirst[v] = o; o += sdepth[v]; }
-      sfirst[MAX_DEPTH + 1] = o;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < PER; j++)
-      if (plo[j] >= t_lo && phi[j] <= t_hi) snode[sfirst[pdl[j]] + rank[j]] = (int)(ppos[j] - ib) - first;
-    __syncthreads();
-    // depths deepest first: places sfirst[v] .. sfirst[v] + count, in order
-    for (int v = MAX_DEPTH; v >= 0; v--) {
-      const int p0 = sfirst[v], p1 = (v > 0 ? sfirst[v - 1] : sfirst[MAX_DEPTH + 1]);
-      if (p0 == p1) continue;  // uniform
-      for (int p = p0 + (int)threadIdx.x; p < p1; p += BLOCK) {
-        const int g = snode[p];
-        spm[g] = sum_children([&](int c) { return spm[c]; }, [&](int c) { return sskip[c]; }, g, sskip[g]);
+      const bool lo_in = plo[j] >= t_lo, hi_in = phi[j] <= t_hi;
+      const u32 blo = lo_in ? L.p.bits[plo[j] - t_lo] : W.bits[b + plo[j]];
+      const int elo = lo_in ? L.p.pre[plo[j] - t_lo] : W.pre[b + plo[j]];
+      const u32 bhi = hi_in ? L.p.bits[phi[j] - t_lo] : W.bits[b + phi[j]];
+      const int ehi = hi_in ? L.p.pre[phi[j] - t_lo] : W.pre[b + phi[j]];
+      const int pos = plo[j] + elo + __popc(blo & ((1u << pdl[j]) - 1u));
+      nskip[j] = phi[j] + ehi + __popc(bhi) + 1;
+      if (lo_in && hi_in) {
+        at[j] = pos - first;
+      } else {
+        W.items[ib + pos] = node_item(make_float4(0.f, 0.f, 0.f, 0.f), nskip[j], depth.lsq[pdl[j]], depth.below[pdl[j]]);
+        W.npos[b + l] = (int)(ib + pos);
+        list_crossing(W, t, tl, b, l, plo[j], phi[j], ncross);
       }
-      __syncthreads();
     }
-    for (int p = threadIdx.x; p < sfirst[MAX_DEPTH + 1]; p += BLOCK) {
-      const int g = snode[p];
-      W.items[ib + first + g].pm = spm[g];
+    __syncthreads();  // the items take the places' memory
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) {
+      if (leaf[j] >= 0) {
+        L.n.pm[leaf[j] - first] = pm[j];
+        L.n.skip[leaf[j] - first] = (unsigned short)(leaf[j] + 1 - first);
+      }
+      if (at[j] >= 0) L.n.skip[at[j]] = (unsigned short)(nskip[j] - first);
+    }
+    tile_moments<TM>(L.n, at, pdl);
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) {
+      if (leaf[j] >= 0) {
+        W.items[ib + leaf[j]] = leaf_item(pm[j], leaf[j]);
+        if (t_lo + p0 + j + 1 == n) {
+          W.seg[tl.seg].n_items = leaf[j] + 1;
+          W.items[ib + leaf[j] + 1] = sentinel_item(leaf[j] + 1);
+        }
+      }
+      if (at[j] >= 0)
+        W.items[ib + first + at[j]] = node_item(L.n.pm[at[j]], nskip[j], depth.lsq[pdl[j]], depth.below[pdl[j]]);
     }
     __syncthreads();
   }
@@ -1036,79 +1245,6 @@ __global__ void __launch_bounds__(BLOCK) moments_cross_kernel(Work W, const Tile
     if (ng == 0) continue;  // uniform
     const Seg &S = W.seg[tl.seg];
     moments_of_list(W, S, W.cross2 + S.ibase, ng);
-  }
-}
-
-// One-wave tiles: the whole tree of a segment of at most R * WAVE sources
-// (fewer than 2 R WAVE items) in LDS; lane l holds pairs l + WAVE r, and the
-// depths that hold nodes are taken deepest first with a wave barrier between
-// them.
-template <int R>
-__global__ void __launch_bounds__(BLOCK) moments_wave_kernel(Work W, const Tile *__restrict__ tiles, int t0,
-                                                             int ntiles) {
-  constexpr int NI = 2 * R * WAVE;
-  __shared__ float4 spm[BLOCK / WAVE][NI];
-  __shared__ int sskip[BLOCK / WAVE][NI];
-  const int lane = threadIdx.x & (WAVE - 1), wv = threadIdx.x / WAVE;
-  WAVE_TILE_LOOP(t, t0, ntiles) {
-    const Tile tl = tiles[t];
-    const Seg &S = W.seg[tl.seg];
-    const int cnt = min(R * WAVE, S.n_src) - 1;  // pairs
-    if (cnt <= 0) continue;  // uniform across the wave
-    const int64_t b = S.ibase, ib = 2 * b;
-    const int nit = S.n_items;
-    int lo[R], pos[R], v[R];
-    unsigned int dm = 0;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      const int e = lane + WAVE * r;
-      lo[r] = -1;
-      pos[r] = 0;
-      v[r] = 0;
-      if (e < cnt) {
-        lo[r] = W.nlo[b + e];
-        pos[r] = W.npos[b + e];
-        v[r] = W.dl[b + e];
-      }
-      if (lo[r] >= 0) dm |= 1u << v[r];
-    }
-    for (int d = WAVE / 2; d > 0; d >>= 1) dm |= (unsigned int)__shfl_xor((int)dm, d, WAVE);
-    if (nit > NI) {
-      // not expected (a compressed octree has fewer nodes than leaves): the
-      // same depth order over device memory
-      while (dm) {
-        const int d = 31 - __clz(dm);
-        dm &= ~(1u << d);
-#pragma unroll
-        for (int r = 0; r < R; r++)
-          if (lo[r] >= 0 && v[r] == d) node_moments(W, ib, pos[r]);
-        __threadfence();
-        wave_sync();
-      }
-      continue;
-    }
-    for (int i = lane; i < nit; i += WAVE) {
-      const Item q = W.items[ib + i];
-      spm[wv][i] = q.pm;
-      sskip[wv][i] = q.ax.y;
-    }
-    wave_sync();
-    while (dm) {  // uniform across the wave
-      const int d = 31 - __clz(dm);
-      dm &= ~(1u << d);
-#pragma unroll
-      for (int r = 0; r < R; r++)
-        if (lo[r] >= 0 && v[r] == d) {
-          const int g = pos[r] - (int)ib;
-          spm[wv][g] = sum_children([&](int c) { return spm[wv][c]; }, [&](int c) { return sskip[wv][c]; }, g,
-                                    sskip[wv][g]);
-        }
-      wave_sync();
-    }
-#pragma unroll
-    for (int r = 0; r < R; r++)
-      if (lo[r] >= 0) W.items[pos[r]].pm = spm[wv][pos[r] - (int)ib];
-    wave_sync();  // the next tile reuses the wave's LDS
   }
 }
 
@@ -1806,18 +1942,18 @@ __global__ void __launch_bounds__(PARTS *WAVE) walk_split_kernel(Work W, DevPara
 
 // Instrumented passes: the elements a segmented sort ordered (counters[8])
 // and the elements times the merge levels each needed (counters[9]).
-__global__ void sort_count_kernel(const int *n, int nseg, unsigned long long *counters) {
+__global__ void sort_count_kernel(Work W, const int *n, int above) {
   unsigned long long e = 0, el = 0;
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nseg; k += gridDim.x * blockDim.x) {
-    const int c = n[k] > 0 ? n[k] : 0;
+  SEG_LOOP(k, W) {
+    const int c = W.seg[k].cap > above && n[k] > 0 ? n[k] : 0;
     e += (unsigned long long)c;
     el += (unsigned long long)c * (unsigned long long)merge_levels(c);
   }
   e = wave_reduce_sum(e);
   el = wave_reduce_sum(el);
   if ((threadIdx.x & (WAVE - 1)) == 0 && (e | el)) {
-    atomicAdd(&counters[8], e);
-    atomicAdd(&counters[9], el);
+    atomicAdd(&W.counters[8], e);
+    atomicAdd(&W.counters[9], el);
   }
 }
 

@@ -73,21 +73,10 @@ __global__ void __launch_bounds__(BLOCK) tgt_bucket_kernel(Work W, TgtArgs A) {
     const int i = i0 + (int)threadIdx.x;
     int b = -1;
     if (i < A.n) {
-#pragma clang fp contract(off)
       const float x = A.x[i], y = A.y[i], z = A.z[i];
       const u32 o[3] = {f2ord(x), f2ord(y), f2ord(z)};
       for (int j = 0; j < 3; j++) { mn[j] = min(mn[j], o[j]); mx[j] = max(mx[j], o[j]); }
-      double c0 = S.center[0], c1 = S.center[1], c2 = S.center[2], lh = 0.5 * S.Len;
-      u64 key = 0;
-      for (int d = 0; d < S.D; d++) {
-        lh *= 0.5;
-        int sub = 0;
-        if (x > c0) { c0 += lh; sub |= 1; } else c0 -= lh;
-        if (y > c1) { c1 += lh; sub |= 2; } else c1 -= lh;
-        if (z > c2) { c2 += lh; sub |= 4; } else c2 -= lh;
-        key = (key << 3) | (u64)sub;
-      }
-      key <<= 3 * (MAX_DEPTH - S.D);
+      const u64 key = octant_key(S.center, S.Len, S.D, x, y, z);
       int lo = 0, hi = S.n_src;  // first source whose digits are not below the target's
       while (lo < hi) {
         const int mid = (lo + hi) >> 1;
@@ -208,7 +197,7 @@ extern "C" int hbt_tree_potential(hbt_ctx *ctx, int64_t n_src, const float *sx, 
                                                                       ctx->seg_of_slot.as<int>());
   tree_only_setup_kernel<<<1, 1, 0, st>>>(R.W, (int)n_src);
   tree_sources_kernel<<<grid_for(n_src, ctx->cus), BLOCK, 0, st>>>(R.W, (int)n_src, sx, sy, sz, smass);
-  RETCHK(R.build_tree(false));
+  RETCHK(R.build_tree(false, true));  // the targets' order reads the sorted digits
   const int nb = (int)(n_src >> BUCKET_BITS) + 1;  // a target's place among the sources is 0 .. n_src
   for (int64_t t0 = 0; t0 < n_tgt; t0 += TGT_SLICE) {
     TgtArgs A;

@@ -678,7 +678,7 @@ struct Runner {
   bool swap_sp = true;         // swap the spatial list with its compacted copy (direct launches)
   int nt_big = 0;              // tiles of segments of more than SMALL_CAP slots (a prefix)
   int nt_tiny = 0;             // then those of more than TINY_CAP; the rest are of at most TINY_CAP
-  int gsmall = 1, gtiny = 1, gwave = 1;  // one-wave tile grids (four tiles per workgroup)
+  int gwave = 1;               // one-wave tile grid (four tiles per workgroup)
   int gwseg = 1;               // segment-wave grid
   int gw;                      // walk grid: every slot block once
   // the tile table a pass uses: the level's, or that of its active segments
@@ -708,11 +708,10 @@ struct Runner {
     gw = walk_grid(W.nact, c->tune.xcd_run);
     nt_big = tiles_above(SMALL_CAP);
     nt_tiny = tiles_above(TINY_CAP);
-    gtile = (int)std::max<int64_t>(1, std::min<int64_t>(nt_big, (int64_t)c->cus * 8));
-    gsmall = wave_grid(nt_tiny - nt_big);
-    gtiny = wave_grid(nt_cur - nt_tiny);
+    gtile = tile_grid(nt_big);
     gwave = wave_grid(nt_cur - nt_big);
   }
+  int tile_grid(int nt) const { return (int)std::max<int64_t>(1, std::min<int64_t>(nt, (int64_t)c->cus * 8)); }
 
   // tile kernels: the workgroup form over the large segments' tiles, the
   // one-wave form over the rest
@@ -721,8 +720,6 @@ struct Runner {
                                                        (int64_t)c->cus * 16));
   }
   bool any_big() const { return nt_big > 0; }
-  bool any_small() const { return nt_tiny > nt_big; }
-  bool any_tiny() const { return nt_cur > nt_tiny; }
   bool any_wave() const { return nt_cur > nt_big; }
 
   // Lists the segments still active after a pass: their wave-sized slot
@@ -834,23 +831,20 @@ struct Runner {
   }
 
   int sort_pairs(const int *n) {  // sorts (k0,v0) by the counts n[seg], result in (k0,v0)
-    const Tile *tl = tl_cur;
-    const int nt = nt_cur;
+    RETCHK(sort_begin());
+    if (any_big()) tile_sort_kernel<<<gtile, BLOCK, 0, c->stream>>>(tl_cur, nt_big, W.ibase, n, W.k0, W.v0, W.k1, W.v1);
+    if (any_wave()) sort_wave_kernel<<<gwave, BLOCK, 0, c->stream>>>(tl_cur, nt_big, nt_tiny, nt_cur, W.ibase, n, W.k0, W.v0);
+    merge_sorted(n, nt_cur);
+    return sort_end(n);
+  }
+
+  // instrumentation: a sort's device time, or the elements it sorted and their
+  // merge levels
+  int sort_begin() {
     if (c->prof_mode == 1) HIPCHK(hipEventRecord(c->evs0, c->stream));
-    if (any_big()) tile_sort_kernel<<<gtile, BLOCK, 0, c->stream>>>(tl, nt_big, W.ibase, n, W.k0, W.v0, W.k1, W.v1);
-    if (any_wave()) sort_wave_kernel<<<gwave, BLOCK, 0, c->stream>>>(tl, nt_big, nt_tiny, nt, W.ibase, n, W.k0, W.v0);
-    // one launch per merge level of the largest segment of the level, over
-    // the tiles of the segments whose capacity exceeds the level's width
-    // (segments are ordered largest first, so those tiles are a prefix)
-    int level = 0;
-    for (int w = TILE; w < max_n; w *= 2, level++) {
-      const int ntw = tiles_above(w);
-      if (ntw == 0) break;
-      const int gmerge = (int)std::max<int64_t>(1, std::min<int64_t>(ntw, (int64_t)c->cus * 16));
-      merge_pass_kernel<<<gmerge, BLOCK, 0, c->stream>>>(tl, ntw, W.ibase, n, level, W.k0, W.v0, W.k1, W.v1);
-    }
-    // instrumentation: the sort's device time, or the elements it sorted and
-    // their merge levels
+    return HBT_OK;
+  }
+  int sort_end(const int *n, int above = 0) {  // above: only segments of more slots were sorted
     if (c->prof_mode == 1) {
       HIPCHK(hipEventRecord(c->evs1, c->stream));
       HIPCHK(hipEventSynchronize(c->evs1));
@@ -859,7 +853,7 @@ struct Runner {
       c->sort_ms += ms;
       c->sort_calls++;
     } else if (c->prof_mode == 2) {
-      sort_count_kernel<<<gseg, BLOCK, 0, c->stream>>>(n, W.nseg, W.counters);
+      sort_count_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, n, above);
     }
     return HBT_OK;
   }
@@ -877,29 +871,50 @@ struct Runner {
   }
   const int *count_row(int row) const { return W.ncount + (size_t)row * W.nseg; }
 
-  // tree over the pass's sources: keys, sort, structure, moments
-  void bbox() {
-    if (any_big()) bbox_kernel<<<gtile, BLOCK, 0, c->stream>>>(W, tl_cur, nt_big);
-    if (any_wave()) bbox_wave_kernel<<<gwave, BLOCK, 0, c->stream>>>(W, tl_cur, nt_big, nt_tiny, nt_cur);
+  // The merge levels after a tile sort of the first nt_first tiles.
+  void merge_sorted(const int *n, int nt_first) {
+    // one launch per merge level of the largest segment of the level, over
+    // the tiles of the segments whose capacity exceeds the level's width
+    // (segments are ordered largest first, so those tiles are a prefix)
+    int level = 0;
+    for (int w = TILE; w < max_n; w *= 2, level++) {
+      const int ntw = std::min(tiles_above(w), nt_first);
+      if (ntw == 0) break;
+      const int gmerge = (int)std::max<int64_t>(1, std::min<int64_t>(ntw, (int64_t)c->cus * 16));
+      merge_pass_kernel<<<gmerge, BLOCK, 0, c->stream>>>(tl_cur, ntw, W.ibase, n, level, W.k0, W.v0, W.k1, W.v1);
+    }
+  }
+  // Root cubes and sorted octant digits of the segments of the first nt tiles.
+  int sorted_digits(int nt) {
+    const int g = tile_grid(nt);
+    bbox_kernel<<<g, BLOCK, 0, c->stream>>>(W, tl_cur, nt);
+    RETCHK(sort_begin());
+    keys_sort_kernel<<<g, BLOCK, 0, c->stream>>>(W, P, tl_cur, nt);
+    merge_sorted(count_row(NC_SRC), nt);
+    return sort_end(count_row(NC_SRC), nt < nt_cur ? TILE : 0);
   }
 
-  int build_tree(bool copy_sp) {
-    bbox();
-    tree_params_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P);
-    keys_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
-    RETCHK(sort_pairs(count_row(NC_SRC)));
-    if (any_big()) emit_kernel<<<gtile, BLOCK, 0, c->stream>>>(W, tl_cur, nt_big, copy_sp ? 1 : 0);
-    if (any_wave()) emit_wave_kernel<<<gwave, BLOCK, 0, c->stream>>>(W, tl_cur, nt_big, nt_cur, copy_sp ? 1 : 0);
-    RETCHK(seg_scan(PopLoad{W.ibase, W.bits}, PreStore{W.ibase, W.pre}, PreAdd{W.ibase, W.pre},
-                    count_row(NC_SRC)));
-    items_kernel<<<gs, BLOCK, 0, c->stream>>>(W, P);
-    if (any_big()) {
-      moments_tile_kernel<<<gtile, BLOCK, 0, c->stream>>>(W, tl_cur, nt_big);
-      moments_super_kernel<<<gtile, BLOCK, 0, c->stream>>>(W, tl_cur, nt_big);
-      if (max_n > SUPER) moments_cross_kernel<<<gtile, BLOCK, 0, c->stream>>>(W, tl_cur, nt_big);
+  // Tree over the pass's sources.  Segments of at most one tile take one launch
+  // (tree_one), unless the caller goes on to read the sorted digits.
+  int build_tree(bool copy_sp, bool keep_digits = false) {
+    const int cp = copy_sp ? 1 : 0;
+    const int nm = keep_digits ? nt_cur : tiles_above(TILE);
+    if (nm > 0) {
+      const int g = tile_grid(nm);
+      RETCHK(sorted_digits(nm));
+      emit_kernel<<<g, BLOCK, 0, c->stream>>>(W, tl_cur, nm, cp);
+      u64 *ts = c->tsum.as<u64>();
+      scan_tiles_kernel<u64><<<g, BLOCK, 0, c->stream>>>(tl_cur, nm, count_row(NC_SRC), ts, PopLoad{W.ibase, W.bits},
+                                                         PreStore{W.ibase, W.pre});
+      scan_add_kernel<u64><<<g, BLOCK, 0, c->stream>>>(tl_cur, nm, count_row(NC_SRC), ts, PreAdd{W.ibase, W.pre});
+      items_tile_kernel<<<g, BLOCK, 0, c->stream>>>(W, P, tl_cur, nm);
+      moments_super_kernel<<<g, BLOCK, 0, c->stream>>>(W, tl_cur, nm);
+      if (max_n > SUPER) moments_cross_kernel<<<g, BLOCK, 0, c->stream>>>(W, tl_cur, nm);
     }
-    if (any_small()) moments_wave_kernel<4><<<gsmall, BLOCK, 0, c->stream>>>(W, tl_cur, nt_big, nt_tiny);
-    if (any_tiny()) moments_wave_kernel<1><<<gtiny, BLOCK, 0, c->stream>>>(W, tl_cur, nt_tiny, nt_cur);
+    const int nb = std::max(nm, nt_big), ns = std::max(nm, nt_tiny);
+    if (nb > nm) tree_one_kernel<<<tile_grid(nb - nm), BLOCK, 0, c->stream>>>(W, P, tl_cur, nm, nb, cp);
+    if (ns > nb) tree_one_wave_kernel<4><<<wave_grid(ns - nb), BLOCK, 0, c->stream>>>(W, P, tl_cur, nb, ns, cp);
+    if (nt_cur > ns) tree_one_wave_kernel<1><<<wave_grid(nt_cur - ns), BLOCK, 0, c->stream>>>(W, P, tl_cur, ns, nt_cur, cp);
     return HBT_OK;
   }
 
@@ -1056,10 +1071,7 @@ struct Runner {
   int prelude() {
     if (L->ndraws <= 0) return HBT_OK;
     prelude_setup_kernel<<<gseg, BLOCK, 0, c->stream>>>(W);
-    bbox();
-    tree_params_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P);
-    keys_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
-    RETCHK(sort_pairs(count_row(NC_SRC)));
+    RETCHK(sorted_digits(nt_cur));
     prelude_sp_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
     HIPCHK(hipGetLastError());
     return HBT_OK;

@@ -6,6 +6,7 @@ import pytest
 
 import oracle
 from hbtplus_amd import abi, synth
+from helpers import assert_exact, assert_tolerant
 from test_gpu_props import assert_props
 
 pytestmark = pytest.mark.gpu
@@ -141,4 +142,36 @@ def test_shared_walk_changes_no_bit(gpu, at_edges):
     cat.cols["mass"] = (1e-4 * np.random.default_rng(5).uniform(1, 30, cat.n_particles)).astype(np.float32)
     U = gpu(cat.params)
     for a, b in zip(U.unbind_batch(cat), U.unbind_batch(cat, plain=True)):
+        assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
+
+
+@pytest.mark.parametrize("coincident", [False, True])
+def test_tree_forms(gpu, coincident):
+    """a list's first n particles at the sizes where its trees change form: one
+    wave (64, 256), one workgroup (1,024), tiles, super-tiles (65,536); REPLAY
+    against the oracle bit for bit, and where runs of particles share one place
+    (whole subtrees at the resolution floor, whose inner order the reference
+    draws at random) its tolerant criteria"""
+    base = synth.config1(seed=93, n_nfw=56600, n_cont=10000)
+    if coincident:
+        for c in ("x", "y", "z"):
+            base.cols[c][1:2001:2] = base.cols[c][:2000:2]
+            base.cols[c][4000:4300] = base.cols[c][4000]
+    sizes = [2, 3, 7, 62, 64, 65, 130, 254, 256, 257, 700, 1022, 1024, 1025, 2048, 2049, 5000, 65536, 65537, 66600]
+    cols = {c: np.concatenate([a[:n] for n in sizes]) for c, a in base.cols.items()}
+    cols["id"] = np.arange(sum(sizes), dtype=np.int64)
+    cols["mass"] *= np.repeat(66600 / np.float32(sizes), sizes)  # each list as bound as the whole
+    subs = np.repeat(base.subs[:1], len(sizes))
+    subs["count"] = subs["nbound_prev"] = sizes
+    subs["offset"] = np.cumsum([0] + sizes[:-1])
+    p = base.params.copy()
+    p["precision"] = abi.HBT_PREC_REPLAY
+    cat = synth.Catalogue(cols, subs, p, "tree forms")
+    ref = oracle.unbind_batch(cat, nthreads=16)
+    got = gpu(p).unbind_batch(cat)
+    if coincident:
+        assert_tolerant(ref, got)
+    else:
+        assert_exact(ref, got)
+    for a, b in zip(got, gpu(p).unbind_batch(cat, plain=True)):
         assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
