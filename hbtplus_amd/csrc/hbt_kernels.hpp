@@ -13,9 +13,10 @@
 //                     with skip pointers; node moments accumulated in double over
 //                     float children in son order (src/gravity_tree.cpp:18-77)
 //   walk              stackless walk per target (src/gravity_tree.cpp:79-175)
-//   partition_*       parallel replica of PartitionBindingEnergy (:21-58)
+//   post_one          a segment of one tile: the rest of the pass in one launch
+//   partition_*       the others: parallel replica of PartitionBindingEnergy (:21-58)
 //   frames            FP64 AverageVelocity/AveragePosition, convergence (:357-421)
-//   finalize          permuted list, kinematics, particle-type counts (:405-431)
+//   output            permuted list, kinematics, particle-type counts (:405-431)
 #pragma once
 #include "hbt_device.hpp"
 #include "../../include/hbt_unbind.h"
@@ -40,12 +41,13 @@ struct Work {
   // per level
   Seg *seg;
   int nseg;
+  int nmulti;                // segments of more than one tile
   int64_t nslots;
   // the slots a pass visits: all (act_chunk null, nact = nslots) or the
   // wave-sized chunks of the segments still active (nact = 64 * chunks)
   const int *act_chunk;
   int64_t nact;
-  int *segact;               // [nseg] 1: the segment stays active after the pass
+  int *segact;               // [nseg] nonzero: the segment stays active after the pass (its Nlast)
   const int *seg_of_slot;
   const int64_t *ibase;
   int *ncount;               // [NC_ROWS][nseg] element counts of the pass's scans and sorts
@@ -113,12 +115,16 @@ __device__ __forceinline__ int64_t slot_at(const Work &W, int64_t i) {
   for (int64_t s##_i = (int64_t)blockIdx.x * BLOCK + threadIdx.x, s = slot_at((W), s##_i);    \
        s##_i < (W).nact; s##_i += (int64_t)gridDim.x * BLOCK, s = slot_at((W), s##_i))
 
+// The segments of more than one tile come first in a level.
+#define MULTI_SEG_LOOP(k, W) \
+  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < (W).nmulti; k += gridDim.x * blockDim.x)
+
 #define SEG_LOOP(k, W) \
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < (W).nseg; k += gridDim.x * blockDim.x)
 
-// One wave per segment (k is wave-uniform).
-#define WAVE_SEG_LOOP(k, W)                                                     \
-  for (int k = (int)((blockIdx.x * blockDim.x + threadIdx.x) / WAVE); k < (W).nseg; \
+// One wave per segment of the first n (k is wave-uniform).
+#define WAVE_SEG_LOOP(k, n)                                                     \
+  for (int k = (int)((blockIdx.x * blockDim.x + threadIdx.x) / WAVE); k < (n); \
        k += (int)(gridDim.x * blockDim.x / WAVE))
 
 // Sums of C values over the tiles t0 .. t0+nt-1 of part: the wave's lanes take
@@ -2044,7 +2050,7 @@ __global__ void __launch_bounds__(BLOCK) partition_k_kernel(Work W) {
 }
 
 __global__ void partition_hole_kernel(Work W) {
-  SEG_LOOP(k, W) {
+  MULTI_SEG_LOOP(k, W) {
     Seg &S = W.seg[k];
     if (!(S.flags & F_ACTIVE)) continue;
     const int64_t b = S.ibase;
@@ -2084,7 +2090,7 @@ __global__ void __launch_bounds__(BLOCK) partition_move_kernel(Work W) {
 
 // Nbound after the partition; disruption test (:357-379).
 __global__ void partition_done_kernel(Work W, DevParams P) {
-  SEG_LOOP(k, W) {
+  MULTI_SEG_LOOP(k, W) {
     Seg &S = W.seg[k];
     S.ncopy = (S.flags & F_ACTIVE) ? S.nlast : 0;  // bound_flags_kernel copies the new Elist back
     if (!(S.flags & F_ACTIVE)) continue;
@@ -2118,16 +2124,19 @@ __global__ void __launch_bounds__(BLOCK) disrupt_find_kernel(Work W) {
   }
 }
 
+__device__ __forceinline__ void swap_entries(const Work &W, int64_t a, int64_t c) {
+  auto sw = [](auto *v, int64_t i, int64_t j) { const auto t = v[i]; v[i] = v[j]; v[j] = t; };
+  sw(W.gidx, a, c); sw(W.pos, a, c); sw(W.vel, a, c);
+}
+
 __global__ void disrupt_swap_kernel(Work W) {
-  SEG_LOOP(k, W) {
+  MULTI_SEG_LOOP(k, W) {
     Seg &S = W.seg[k];
     if (!(S.flags & F_SHUF) || (S.flags & (F_DISR | F_FINAL)) != (F_DISR | F_FINAL)) continue;
     const int q = S.swapq;
     S.swapq = INT_MAX;
     if (q == INT_MAX || q == 0) continue;
-    const int64_t a = S.ibase, c = S.ibase + q;
-    auto sw = [](auto *v, int64_t i, int64_t j) { const auto t = v[i]; v[i] = v[j]; v[j] = t; };
-    sw(W.gidx, a, c); sw(W.pos, a, c); sw(W.vel, a, c);
+    swap_entries(W, S.ibase, S.ibase + q);
   }
 }
 
@@ -2267,53 +2276,13 @@ frames_partial_kernel(Work W, DevParams P, const Tile *tiles, int ntiles, double
   }
 }
 
-// One-wave tiles of up to R * WAVE entries: pass r of the wave takes entries
-// WAVE r .. WAVE r + WAVE - 1, lane l entry WAVE r + l, as wave r of the
-// workgroup form does, and the totals of the passes are added to zero in
-// order, as the workgroup form adds its waves' totals, so both give the same
-// bits.
-template <int R>
-__device__ __forceinline__ void frames_wave_tile(const Work &W, const DevParams &P, const Tile &tl, int t,
-                                                 double *part) {
-#pragma clang fp contract(off)
-  const int lane = threadIdx.x & (WAVE - 1);
-  {
-    const Seg &S = W.seg[tl.seg];
-    const int cnt = (S.flags & F_ACTIVE) ? min(R * WAVE, S.nbound) : 0;
-    if (cnt <= 0) return;  // uniform across the wave
-    const int64_t b = S.ibase;
-    const float4 p0 = W.pos[b + W.el[b]];
-    const double o[3] = {p0.x, p0.y, p0.z};
-    double acc[FRAME_SUMS] = {0, 0, 0, 0, 0, 0, 0};
-    for (int r = 0; r < R; r++) {
-      double v[FRAME_SUMS] = {0, 0, 0, 0, 0, 0, 0};
-      const int e = lane + WAVE * r;
-      if (e < cnt) frame_accum(W, P, b, W.el[b + e], o, v);
-      for (int c = 0; c < FRAME_SUMS; c++) acc[c] += wave_total(v[c]);
-    }
-    if (lane == 0)
-      for (int c = 0; c < FRAME_SUMS; c++) part[(int64_t)t * FRAME_SUMS + c] = acc[c];
-  }
-}
-
-// Tiles t0 <= t < tmid take four entries per lane, tmid <= t < ntiles one.
-__global__ void __launch_bounds__(BLOCK)
-frames_partial_wave_kernel(Work W, DevParams P, const Tile *tiles, int t0, int tmid, int ntiles, double *part) {
-  WAVE_TILE_LOOP(t, t0, ntiles) {
-    const Tile tl = tiles[t];
-    if (t < tmid) frames_wave_tile<4>(W, P, tl, t, part);
-    else frames_wave_tile<1>(W, P, tl, t, part);
-  }
-}
-
 // Correction switch, new frame, convergence (:380-421) for one segment, given
-// the FP64 sums over its bound block.
-__device__ void frame_update(Work &W, const DevParams &P, Seg &S, double msum, double s1, double s2,
+// its most-bound entry and the FP64 sums over its bound block.
+__device__ void frame_update(Work &W, const DevParams &P, Seg &S, int l0, double msum, double s1, double s2,
                              double s3, double q1, double q2, double q3) {
 #pragma clang fp contract(off)
   const int64_t b = S.ibase;
   const int nb = S.nbound;
-  const int l0 = W.el[b];
   const float4 p0 = W.pos[b + l0], v0 = W.vel[b + l0];
   const double o[3] = {p0.x, p0.y, p0.z};
   // correction switch (uses the frame of the pass just done); with sampling
@@ -2353,9 +2322,7 @@ __device__ void frame_update(Work &W, const DevParams &P, Seg &S, double msum, d
   } else {
     S.sort_lo = nb;
     S.nsort = S.nlast - nb;
-    atomicAdd(&W.active[0], 1);
-    atomicMax(&W.active[1], S.nlast);  // bounds every count of the next pass
-    W.segact[&S - W.seg] = 1;
+    W.segact[&S - W.seg] = max(1, S.nlast);
   }
   W.ncount[NC_SORT * W.nseg + (int)(&S - W.seg)] = S.nsort;
 }
@@ -2402,15 +2369,12 @@ __global__ void __launch_bounds__(BLOCK) frames_runs_kernel(Work W, const Tile *
   }
 }
 
-// One thread per segment: the wave's updates of the active count and of the
-// largest Nlast (frame_update) then combine into one atomic each.  (One wave
-// per segment, as output_combine_kernel does, measured slower here.)  A bound
-// block of more than SUPER_TILES tiles is summed over the runs of
-// frames_runs_kernel.
+// One thread per segment.  A bound block of more than SUPER_TILES tiles is
+// summed over the runs of frames_runs_kernel.
 __global__ void frames_combine_kernel(Work W, DevParams P, const int *first_tile, const double *part,
                                       const double *gpart) {
 #pragma clang fp contract(off)
-  SEG_LOOP(k, W) {
+  MULTI_SEG_LOOP(k, W) {
     Seg &S = W.seg[k];
     if (!(S.flags & F_ACTIVE)) continue;
     double v[FRAME_SUMS] = {0, 0, 0, 0, 0, 0, 0};
@@ -2419,7 +2383,7 @@ __global__ void frames_combine_kernel(Work W, DevParams P, const int *first_tile
       sum_tiles_in_order<FRAME_SUMS>(part, first_tile[k], nt, 1, v);
     else
       sum_tiles_in_order<FRAME_SUMS>(gpart, first_tile[k], (nt + SUPER_TILES - 1) / SUPER_TILES, SUPER_TILES, v);
-    frame_update(W, P, S, v[0], v[1], v[2], v[3], v[4], v[5], v[6]);
+    frame_update(W, P, S, W.el[S.ibase], v[0], v[1], v[2], v[3], v[4], v[5], v[6]);
   }
 }
 
@@ -2452,14 +2416,30 @@ __global__ void frames_serial_kernel(Work W, DevParams P) {
         }
       }
     }
-    frame_update(W, P, S, msum, s1, s2, s3, q1, q2, q3);
+    frame_update(W, P, S, W.el[b], msum, s1, s2, s3, q1, q2, q3);
   }
 }
 
 // ---------------------------------------------------------------------------
 // Outputs for segments that finished in this pass, early exits and orphans.
 
-// per-slot: output list and energies
+// Output list and energies of entry l.  li: Elist's entry at l, for l < ulen.
+__device__ __forceinline__ void output_entry(const Work &W, const Seg &S, int l, int li) {
+  const int64_t o = S.out_off + l;
+  if ((S.flags & F_CONV) && !(S.flags & F_ORPHAN)) {
+    if (l >= S.ulen) li = l;
+    W.out_index[o] = W.gidx[S.ibase + li];
+    W.out_energy[o] = l < S.ulen ? W.E[S.ibase + li] : __builtin_nanf("");
+  } else {
+    // disrupted, early, orphan: the list keeps its order -- an orphan's
+    // own list as it came in, even when a shuffled copy of it was unbound
+    // (:434-446)
+    const bool orig = (S.flags & F_ORPHAN) && (S.flags & F_SHUF) && l < S.count;
+    W.out_index[o] = orig ? own_entry(W, S, l) : W.gidx[S.ibase + l];
+    W.out_energy[o] = __builtin_nanf("");
+  }
+}
+
 __global__ void __launch_bounds__(BLOCK) output_list_kernel(Work W, int early) {
   SLOT_LOOP(s, W) {
     int k;
@@ -2468,19 +2448,7 @@ __global__ void __launch_bounds__(BLOCK) output_list_kernel(Work W, int early) {
     const Seg &S = W.seg[k];
     const bool fin = early ? (S.flags & F_EARLY) != 0 : (S.flags & F_FINAL) != 0;
     if (!fin || l >= S.len) continue;
-    const int64_t o = S.out_off + l;
-    if ((S.flags & F_CONV) && !(S.flags & F_ORPHAN)) {
-      const int li = l < S.ulen ? W.el[s] : l;
-      W.out_index[o] = W.gidx[S.ibase + li];
-      W.out_energy[o] = l < S.ulen ? W.E[S.ibase + li] : __builtin_nanf("");
-    } else {
-      // disrupted, early, orphan: the list keeps its order -- an orphan's
-      // own list as it came in, even when a shuffled copy of it was unbound
-      // (:434-446)
-      const bool orig = (S.flags & F_ORPHAN) && (S.flags & F_SHUF) && l < S.count;
-      W.out_index[o] = orig ? own_entry(W, S, l) : W.gidx[s];
-      W.out_energy[o] = __builtin_nanf("");
-    }
+    output_entry(W, S, l, W.el[s]);
   }
 }
 
@@ -2612,9 +2580,8 @@ __device__ __forceinline__ int record_span(const Seg &S) { return (S.flags & F_C
 // The record sums of slot li: kinematics of a bound entry, and its type
 // count and mass unless it is a null particle of a small subhalo.
 __device__ __forceinline__ void record_accum(const Work &W, const DevParams &P, const Seg &S, int64_t b, int li,
-                                             bool conv, int nb, bool skip_null, double (&v)[REC_SUMS]) {
+                                             int nb, bool skip_null, double (&v)[REC_SUMS]) {
 #pragma clang fp contract(off)
-  if (conv && !W.isb[b + li]) return;
   if (nb > 1) kin_accum(W, P, S, li, v);
   if (skip_null && W.g_id[W.gidx[b + li]] == -1) return;
   const int ty = __float_as_int(W.vel[b + li].w);
@@ -2642,7 +2609,8 @@ output_partial_kernel(Work W, DevParams P, const Tile *tiles, int ntiles, double
     const bool skip_null = nb <= 100;
     double v[REC_SUMS];
     for (int c = 0; c < REC_SUMS; c++) v[c] = 0;
-    for (int i = threadIdx.x; i < cnt; i += BLOCK) record_accum(W, P, S, b, tl.start + i, conv, nb, skip_null, v);
+    for (int i = threadIdx.x; i < cnt; i += BLOCK)
+      if (!conv || W.isb[b + tl.start + i]) record_accum(W, P, S, b, tl.start + i, nb, skip_null, v);
     for (int c = 0; c < REC_SUMS; c++) {
       const double r = wave_total(v[c]);
       if ((threadIdx.x & (WAVE - 1)) == 0) sh[c][threadIdx.x / WAVE] = r;
@@ -2657,57 +2625,287 @@ output_partial_kernel(Work W, DevParams P, const Tile *tiles, int ntiles, double
   }
 }
 
-// One-wave tiles of up to R * WAVE slots, the same bits as the workgroup
-// form (see frames_partial_wave_kernel).
-template <int R>
-__device__ __forceinline__ void output_wave_tile(const Work &W, const DevParams &P, const Tile &tl, int t,
-                                                 double *part) {
-#pragma clang fp contract(off)
-  const int lane = threadIdx.x & (WAVE - 1);
-  {
-    const Seg &S = W.seg[tl.seg];
-    const bool fin = (S.flags & F_FINAL) != 0;
-    const int cnt = fin ? min(R * WAVE, record_span(S)) : 0;
-    if (cnt <= 0) return;  // uniform across the wave
-    const int64_t b = S.ibase;
-    const int nb = S.nbound;
-    double acc[REC_SUMS];
-    for (int c = 0; c < REC_SUMS; c++) acc[c] = 0;
-    for (int r = 0; r < R; r++) {
-      double v[REC_SUMS];
-      for (int c = 0; c < REC_SUMS; c++) v[c] = 0;
-      const int e = lane + WAVE * r;
-      if (e < cnt) record_accum(W, P, S, b, e, (S.flags & F_CONV) != 0, nb, nb <= 100, v);
-      for (int c = 0; c < REC_SUMS; c++) acc[c] += wave_total(v[c]);
-    }
-    if (lane == 0)
-      for (int c = 0; c < REC_SUMS; c++) part[(int64_t)t * REC_SUMS + c] = acc[c];
-  }
+// The record of a segment that finished, from its sums.
+__device__ __forceinline__ void write_record_sums(Work &W, const DevParams &P, Seg &S, const double (&v)[REC_SUMS]) {
+  int nt[HBT_TYPE_MAX];
+  float mts[HBT_TYPE_MAX];
+  for (int q = 0; q < HBT_TYPE_MAX; q++) { nt[q] = (int)v[6 + q]; mts[q] = (float)v[12 + q]; }
+  write_record(W, P, S, v[0], v[1], v[2], v[3], v[4], v[5], nt, mts);
 }
 
-// Tiles t0 <= t < tmid take four slots per lane, tmid <= t < ntiles one.
-__global__ void __launch_bounds__(BLOCK)
-output_partial_wave_kernel(Work W, DevParams P, const Tile *tiles, int t0, int tmid, int ntiles, double *part) {
-  WAVE_TILE_LOOP(t, t0, ntiles) {
-    const Tile tl = tiles[t];
-    if (t < tmid) output_wave_tile<4>(W, P, tl, t, part);
-    else output_wave_tile<1>(W, P, tl, t, part);
-  }
-}
-
-__global__ void __launch_bounds__(BLOCK) output_combine_kernel(Work W, DevParams P, const int *first_tile,
+// The first nseg segments, a wave each.
+__global__ void __launch_bounds__(BLOCK) output_combine_kernel(Work W, DevParams P, int nseg, const int *first_tile,
                                                                const double *part) {
-#pragma clang fp contract(off)
-  WAVE_SEG_LOOP(k, W) {
+  WAVE_SEG_LOOP(k, nseg) {
     Seg &S = W.seg[k];
     if (!(S.flags & F_FINAL)) continue;  // uniform across the wave
     double v[REC_SUMS];
     wave_sum_tiles<REC_SUMS>(part, first_tile[k], (record_span(S) + TILE - 1) / TILE, v);
-    if ((threadIdx.x & (WAVE - 1)) != 0) continue;
-    int nt[HBT_TYPE_MAX];
-    float mts[HBT_TYPE_MAX];
-    for (int q = 0; q < HBT_TYPE_MAX; q++) { nt[q] = (int)v[6 + q]; mts[q] = (float)v[12 + q]; }
-    write_record(W, P, S, v[0], v[1], v[2], v[3], v[4], v[5], nt, mts);
+    if ((threadIdx.x & (WAVE - 1)) == 0) write_record_sums(W, P, S, v);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Everything after the walk for a segment of one tile, in one launch: the
+// partition, the spatial list, the frame, the energy sort and, where the
+// segment finished, its outputs, a wave or a workgroup each (the teams of
+// tree_one), Elist and energies in LDS in between.  REPLAY sums in the
+// reference's order between two stages of it.  As fifteen launches over every
+// slot, each behind its own loads of segment, list and record, this took 7.0 ms
+// of a batch of 200,000 subhalos' passes (3.8 now) and 35 of a 300-particle
+// list's 50 us a pass (15 now); the record's 18 FP64 sums bound it, so their
+// registers are kept to four waves per SIMD.
+enum { POST_PART = 1, POST_FRAME = 2, POST_SORT = 4, POST_RECORD = 8 };
+constexpr int POST_ALL = POST_PART | POST_FRAME | POST_SORT | POST_RECORD;
+
+template <int CAP>
+struct OnePost {
+  union {
+    struct { unsigned short p[CAP + 1], g[CAP + 1]; } part;  // p_k, g_k of the partition
+    struct { u64 key[CAP]; u32 val[CAP]; } sort;
+  };
+  float E[CAP];             // by Elist position, until the energy sort
+  unsigned short el[CAP];   // Elist
+  unsigned char bound[CAP]; // by list entry
+  double sums[REC_SUMS][BLOCK / WAVE];
+  int K;
+};
+
+// Sums of C values over the elements 0 .. cnt-1 of a tile, add(e, v) adding
+// element e's; in the team's first thread.  Up to BLOCK elements, which any team
+// may hold, both forms add the totals of 64 neighbouring ones to zero in order:
+// the same bits.
+template <class TM, int C, class Add>
+__device__ __forceinline__ void tile_sums(int cnt, double (&out)[C], double (*sh)[BLOCK / WAVE], Add add) {
+#pragma clang fp contract(off)
+  if constexpr (TM::T == WAVE) {
+    double sum = 0;
+    for (int e0 = 0; e0 < cnt; e0 += WAVE) {
+      double v[C];
+      for (int c = 0; c < C; c++) v[c] = 0;
+      if (e0 + TM::id() < cnt) add(e0 + TM::id(), v);
+      for (int c = 0; c < C; c++) {
+        const double t = wave_total(v[c]);
+        if (TM::id() == c) sum += t;  // lane c keeps sum c
+      }
+    }
+    for (int c = 0; c < C; c++) out[c] = readlane_double(sum, c);
+  } else {
+    double v[C];
+    for (int c = 0; c < C; c++) v[c] = 0;
+    for (int e = TM::id(); e < cnt; e += TM::T) add(e, v);
+    for (int c = 0; c < C; c++) {
+      const double r = wave_total(v[c]);
+      if ((threadIdx.x & (WAVE - 1)) == 0) sh[c][threadIdx.x / WAVE] = r;
+    }
+    TM::sync();
+    if (TM::id() < C) {
+      double r = 0;
+      for (int w = 0; w < BLOCK / WAVE; w++) r += sh[TM::id()][w];
+      sh[TM::id()][0] = r;
+    }
+    TM::sync();
+    if (TM::id() == 0)
+      for (int c = 0; c < C; c++) out[c] = sh[c][0];
+  }
+}
+
+template <class TM, int STAGE>
+__device__ __forceinline__ void post_one(Work &W, const DevParams &P, const Tile &tl, int *sp_out,
+                                         OnePost<TM::CAP> &L) {
+  constexpr int R = TM::R, CAP = TM::CAP, T = TM::T;
+  Seg &S = W.seg[tl.seg];
+  const int64_t b = S.ibase;
+  const int id = TM::id();
+  int n = min(CAP, S.nlast);
+  if constexpr ((STAGE & POST_PART) != 0) {
+    if (!(S.flags & F_ACTIVE)) return;  // uniform across the team
+    int li[R], cls[R], rank[R];
+    float e[R];
+    u32 own = 0, all;  // low half: E > 0, high half: E < 0
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int l = R * id + r;
+      li[r] = l < n ? W.el[b + l] : 0;
+      e[r] = l < n ? W.E[b + li[r]] : 0.f;
+      cls[r] = (l < 1 || l >= n) ? 0 : e[r] > 0.f ? 1 : e[r] < 0.f ? 2 : 0;
+      own += cls[r] == 1 ? 1u : cls[r] == 2 ? 0x10000u : 0u;
+    }
+    const u32 before = TM::exclusive_scan(own, &all);
+    const int nP = (int)(all & 0xffffu), nG = (int)(all >> 16);
+    int p = (int)(before & 0xffffu), g = (int)(before >> 16);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int l = R * id + r;
+      if (cls[r] == 1) L.part.p[rank[r] = ++p] = (unsigned short)l;
+      if (cls[r] == 2) L.part.g[rank[r] = nG - g++] = (unsigned short)l;
+    }
+    if (id == 0) L.K = 0;
+    TM::sync();
+    const int m = min(nP, nG);
+    for (int k = 1 + id; k <= m; k += T)
+      if (L.part.p[k] < L.part.g[k] && (k == m || L.part.p[k + 1] >= L.part.g[k + 1])) L.K = k;
+    TM::sync();
+    const int K = L.K, pK = K ? L.part.p[K] : 0;
+    const bool extra = K + 1 <= nG && L.part.g[K + 1] > pK;
+    const int hole = extra ? L.part.g[K + 1] : pK, moves = extra ? K + 1 : K;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int l = R * id + r;
+      if (l >= n) continue;
+      int dest = l;
+      if (l == 0) dest = hole;
+      else if (cls[r] == 1 && rank[r] <= K) dest = L.part.g[rank[r]];
+      else if (cls[r] == 2 && rank[r] <= moves) dest = rank[r] == 1 ? 0 : L.part.p[rank[r] - 1];
+      L.el[dest] = (unsigned short)li[r];
+      L.E[dest] = e[r];
+    }
+    for (int i = id; i < CAP; i += T) L.bound[i] = 0;
+    TM::sync();
+    // Nbound after the partition; disruption test (:357-379): the original
+    // element 0 ends in the last hole (Etmp, :37-38 and :50-51)
+    const int nb = n == 0 ? 0 : hole + (L.E[hole] < 0.f ? 1 : 0);
+    const bool disrupted = nb < P.min_part;
+    if (id == 0) {
+      S.nbound = nb;
+      S.nsort = 0;
+      if (disrupted) {
+        S.flags = (S.flags & ~F_ACTIVE) | F_DISR | F_FINAL;
+        S.nbound = 1;
+        S.nlast = 1;
+      }
+    }
+    if (disrupted) {
+      if (S.flags & F_SHUF) {
+        // the old most-bound particle back in front (see disrupt_find_kernel)
+        int q = INT_MAX;
+        for (int l = id; l < S.ulen; l += T)
+          if (W.g_id[W.gidx[b + l]] == S.old_mb_id) q = min(q, l);
+        if (id == 0) L.K = INT_MAX;
+        TM::sync();
+        if (q != INT_MAX) atomicMin(&L.K, q);
+        TM::sync();
+        if (id == 0 && L.K != INT_MAX) swap_entries(W, b, b + L.K);
+      }
+      n = 0;  // its Elist is not read again
+    } else {
+      for (int l = id; l < nb; l += T) L.bound[L.el[l]] = 1;
+      TM::sync();
+      int q[R], keep[R], kept = 0, total;
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        const int l = R * id + r;
+        q[r] = l < n ? W.sp[b + l] : 0;
+        keep[r] = l < n ? L.bound[q[r]] : 0;
+        kept += keep[r];
+      }
+      int at = TM::exclusive_scan(kept, &total);
+      TM::sync();  // the list may be compacted in place
+#pragma unroll
+      for (int r = 0; r < R; r++)
+        if (keep[r]) sp_out[b + at++] = q[r];
+      if (P.refine)  // the outputs after a refinement read the flags
+        for (int l = id; l < n; l += T) W.isb[b + L.el[l]] = l < nb ? 1 : 0;
+    }
+    if constexpr ((STAGE & POST_FRAME) != 0) {
+      if (!disrupted) {
+        const int l0 = L.el[0];
+        const float4 p0 = W.pos[b + l0];
+        const double o[3] = {p0.x, p0.y, p0.z};
+        double v[FRAME_SUMS];
+        tile_sums<TM, FRAME_SUMS>(nb, v, L.sums,
+                                  [&](int i, double (&x)[FRAME_SUMS]) { frame_accum(W, P, b, L.el[i], o, x); });
+        if (id == 0) frame_update(W, P, S, l0, v[0], v[1], v[2], v[3], v[4], v[5], v[6]);
+      }
+    }
+    TM::sync();
+  }
+  if constexpr ((STAGE & POST_SORT) != 0) {
+    const int flags = S.flags, nsort = S.nsort, lo = S.sort_lo;
+    if constexpr ((STAGE & POST_PART) == 0) {
+      if (nsort <= 0 && !(flags & F_FINAL)) return;  // uniform across the team
+      if (flags & F_DISR) n = 0;
+      for (int l = id; l < n; l += T) {
+        const int li = W.el[b + l];
+        L.el[l] = (unsigned short)li;
+        L.E[l] = W.E[b + li];
+      }
+      TM::sync();
+    }
+    // energy sort of Elist[lo, lo + nsort) (see energy_keys_kernel)
+    if (nsort > 0) {
+      u64 k[R];
+      u32 v[R];
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        const int i = R * id + r, at = lo + i;
+        const bool live = i < nsort;
+        k[r] = live ? ((at >= S.nbound ? 1ull : 0ull) << 63) | ((u64)f2ord(L.E[at]) << 31) | (u64)(unsigned)at : ~0ull;
+        v[r] = live ? L.el[at] : ~0u;
+      }
+      if constexpr (T == WAVE) {
+        sort_wave<R>(k, v, id, nsort);
+        TM::sync();
+#pragma unroll
+        for (int r = 0; r < R; r++)
+          if (R * id + r < nsort) L.el[lo + R * id + r] = (unsigned short)v[r];
+      } else {
+        sort_tile(k, v, nsort, L.sort.key, L.sort.val);
+        for (int i = id; i < nsort; i += T) L.el[lo + i] = (unsigned short)L.sort.val[i];
+      }
+      TM::sync();
+    }
+  }
+  for (int l = id; l < n; l += T) W.el[b + l] = L.el[l];
+  if constexpr ((STAGE & POST_SORT) != 0) {
+    if (S.flags & F_FINAL) {  // uniform across the team
+      for (int l = id; l < S.len; l += T) output_entry(W, S, l, l < n ? L.el[l] : l < S.ulen ? W.el[b + l] : 0);
+      if constexpr ((STAGE & POST_RECORD) != 0) {
+        const bool conv = (S.flags & F_CONV) != 0;
+        const int nb = S.nbound;
+        double v[REC_SUMS];
+        tile_sums<TM, REC_SUMS>(record_span(S), v, L.sums, [&](int i, double (&x)[REC_SUMS]) {
+          if (!conv || L.bound[i]) record_accum(W, P, S, b, i, nb, nb <= 100, x);
+        });
+        if (id == 0) write_record_sums(W, P, S, v);
+      }
+    }
+  }
+  TM::sync();  // the next tile reuses the LDS
+}
+
+// Tiles t0 <= t < ntiles, one team each.
+template <int R, int STAGE>
+__global__ void __launch_bounds__(BLOCK, 4) post_one_wave_kernel(Work W, DevParams P, const Tile *__restrict__ tiles,
+                                                              int t0, int ntiles, int *sp_out) {
+  using TM = Team<WAVE, R>;
+  __shared__ OnePost<TM::CAP> L[BLOCK / WAVE];
+  WAVE_TILE_LOOP(t, t0, ntiles) post_one<TM, STAGE>(W, P, tiles[t], sp_out, L[threadIdx.x / WAVE]);
+}
+template <int STAGE>
+__global__ void __launch_bounds__(BLOCK, 4) post_one_kernel(Work W, DevParams P, const Tile *__restrict__ tiles, int t0,
+                                                         int ntiles, int *sp_out) {
+  using TM = Team<BLOCK, ITEMS>;
+  __shared__ OnePost<TM::CAP> L;
+  for (int t = t0 + (int)blockIdx.x; t < ntiles; t += gridDim.x) post_one<TM, STAGE>(W, P, tiles[t], sp_out, L);
+}
+
+// Segments active after the pass, and the largest Nlast among them: by blocks,
+// since the atomics on two addresses are served one after another.
+__global__ void __launch_bounds__(BLOCK) count_active_kernel(Work W) {
+  int cnt = 0, most = 0;
+  SEG_LOOP(k, W) {
+    const int a = W.segact[k];
+    cnt += a > 0 ? 1 : 0;
+    most = max(most, a);
+  }
+  for (int d = WAVE / 2; d > 0; d >>= 1) {
+    cnt += __shfl_xor(cnt, d, WAVE);
+    most = max(most, __shfl_xor(most, d, WAVE));
+  }
+  if ((threadIdx.x & (WAVE - 1)) == 0 && cnt) {
+    atomicAdd(&W.active[0], cnt);
+    atomicMax(&W.active[1], most);  // bounds every count of the next pass
   }
 }
 

@@ -10,10 +10,9 @@
 // Primitives:
 //   segmented sort of (u64 key, u32 value) pairs by (key, value):
 //     tile_sort_kernel    : LDS bitonic sort of each tile
-//     sort_wave_kernel    : the same for segments of at most SMALL_CAP, one per wave
 //     merge_pass_kernel   : one bottom-up merge level (co-rank by binary search)
 //   segmented exclusive scan (load/store functors):
-//     scan_tiles_kernel / scan_add_kernel, scan_wave_kernel
+//     scan_tiles_kernel / scan_add_kernel
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -324,45 +323,6 @@ tile_sort_kernel(const Tile *__restrict__ tiles, int ntiles, const int64_t *__re
   }
 }
 
-// One-wave tiles of up to R * WAVE elements.  Such segments need no merge
-// level, so the result stays in (k0, v0).
-template <int R>
-__device__ __forceinline__ void sort_wave_tile(const Tile &tl, const int64_t *__restrict__ base,
-                                               const int *__restrict__ n, u64 *k0, u32 *v0) {
-  const int lane = threadIdx.x & (WAVE - 1);
-  const int cnt = min(R * WAVE, n[tl.seg]);
-  if (cnt <= 1) return;  // uniform across the wave
-  const int64_t off = base[tl.seg];
-  u64 k[R];
-  u32 v[R];
-#pragma unroll
-  for (int r = 0; r < R; r++) {
-    const int e = R * lane + r;
-    k[r] = e < cnt ? k0[off + e] : ~0ull;
-    v[r] = e < cnt ? v0[off + e] : 0xffffffffu;
-  }
-  sort_wave<R>(k, v, lane, cnt);
-#pragma unroll
-  for (int r = 0; r < R; r++) {
-    const int e = R * lane + r;
-    if (e < cnt) {
-      k0[off + e] = k[r];
-      v0[off + e] = v[r];
-    }
-  }
-}
-
-// Tiles t0 <= t < tmid take four elements per lane, tmid <= t < ntiles one.
-__global__ void __launch_bounds__(BLOCK)
-sort_wave_kernel(const Tile *__restrict__ tiles, int t0, int tmid, int ntiles, const int64_t *__restrict__ base,
-                 const int *__restrict__ n, u64 *k0, u32 *v0) {
-  WAVE_TILE_LOOP(t, t0, ntiles) {
-    const Tile tl = tiles[t];
-    if (t < tmid) sort_wave_tile<4>(tl, base, n, k0, v0);
-    else sort_wave_tile<1>(tl, base, n, k0, v0);
-  }
-}
-
 // Merge level `level` (runs of width TILE << level merged pairwise).  A
 // segment that needs m levels takes part in levels 0..m-1 and ping-pongs
 // between the two buffers so that level m-1 writes (k0, v0); segments with
@@ -460,50 +420,6 @@ scan_tiles_kernel(const Tile *__restrict__ tiles, int ntiles, const int *__restr
       off += v[i];
     }
     if (threadIdx.x == 0) tile_sum[t] = total;
-  }
-}
-
-// Pass 1 for one-wave tiles of up to R * WAVE elements (a segment's only
-// tile: its prefixes are final); lane l holds elements R l .. R l + R - 1.
-template <int R, class T, class Load, class Store>
-__device__ __forceinline__ void scan_wave_tile(const Tile &tl, int t, const int *__restrict__ n,
-                                               T *__restrict__ tile_sum, Load load, Store store) {
-  const int lane = threadIdx.x & (WAVE - 1);
-  {
-    const int cnt = min(R * WAVE, n[tl.seg]);
-    if (cnt <= 0) {  // uniform across the wave
-      if (lane == 0) tile_sum[t] = T(0);
-      return;
-    }
-    T v[R];
-    T sum = 0;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      const int e = R * lane + r;
-      v[r] = e < cnt ? load(tl.seg, e) : T(0);
-      sum += v[r];
-    }
-    const T inc = wave_inclusive_scan(sum);
-    T off = inc - sum;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      const int e = R * lane + r;
-      if (e < cnt) store(tl.seg, e, off);
-      off += v[r];
-    }
-    if (lane == WAVE - 1) tile_sum[t] = inc;
-  }
-}
-
-// Tiles t0 <= t < tmid take four elements per lane, tmid <= t < ntiles one.
-template <class T, class Load, class Store>
-__global__ void __launch_bounds__(BLOCK)
-scan_wave_kernel(const Tile *__restrict__ tiles, int t0, int tmid, int ntiles, const int *__restrict__ n,
-                 T *__restrict__ tile_sum, Load load, Store store) {
-  WAVE_TILE_LOOP(t, t0, ntiles) {
-    const Tile tl = tiles[t];
-    if (t < tmid) scan_wave_tile<4, T>(tl, t, n, tile_sum, load, store);
-    else scan_wave_tile<1, T>(tl, t, n, tile_sum, load, store);
   }
 }
 

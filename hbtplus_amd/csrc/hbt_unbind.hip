@@ -534,11 +534,11 @@ struct BoundLoad {
 __global__ void partition_counts_kernel(Work W, const int *first_tile, const u64 *tile_sum) {
   constexpr int FEW = 16;
   const int lane = threadIdx.x & (WAVE - 1);
-  for (int k0 = blockIdx.x * blockDim.x + (threadIdx.x & ~(WAVE - 1)); k0 < W.nseg; k0 += gridDim.x * blockDim.x) {
+  for (int k0 = blockIdx.x * blockDim.x + (threadIdx.x & ~(WAVE - 1)); k0 < W.nmulti; k0 += gridDim.x * blockDim.x) {
     const int k = k0 + lane;
     int t0 = 0, nt = 0;
     bool active = false;
-    if (k < W.nseg) {
+    if (k < W.nmulti) {
       Seg &S = W.seg[k];
       active = (S.flags & F_ACTIVE) != 0;
       if (active) {
@@ -674,12 +674,12 @@ struct Runner {
   Work W;
   DevParams P;
   Level *L;
-  int gs, gseg, gtile, gblk;  // slot, segment-thread, tile and segment-block grids
+  int gs, gseg, gblk;          // slot, segment-thread and segment-block grids
   bool swap_sp = true;         // swap the spatial list with its compacted copy (direct launches)
-  int nt_big = 0;              // tiles of segments of more than SMALL_CAP slots (a prefix)
+  int nt_multi = 0;            // tiles of segments of more than one (a prefix)
+  int nt_big = 0;              // then those of segments of more than SMALL_CAP slots
   int nt_tiny = 0;             // then those of more than TINY_CAP; the rest are of at most TINY_CAP
-  int gwave = 1;               // one-wave tile grid (four tiles per workgroup)
-  int gwseg = 1;               // segment-wave grid
+  int64_t nact_multi = 0;      // visited slots of segments of more than one tile (a prefix)
   int gw;                      // walk grid: every slot block once
   // the tile table a pass uses: the level's, or that of its active segments
   // (then W.act_chunk lists their slots); caps and first tiles of the listed
@@ -706,21 +706,18 @@ struct Runner {
   void set_grids() {
     gs = grid_for(W.nact, c->cus);
     gw = walk_grid(W.nact, c->tune.xcd_run);
+    nt_multi = tiles_above(TILE);
     nt_big = tiles_above(SMALL_CAP);
     nt_tiny = tiles_above(TINY_CAP);
-    gtile = tile_grid(nt_big);
-    gwave = wave_grid(nt_cur - nt_big);
+    nact_multi = 0;
+    for (size_t i = 0; i < cur_cap.size() && cur_cap[i] > TILE; i++) nact_multi += (cur_cap[i] + WAVE - 1) / WAVE * WAVE;
   }
   int tile_grid(int nt) const { return (int)std::max<int64_t>(1, std::min<int64_t>(nt, (int64_t)c->cus * 8)); }
 
-  // tile kernels: the workgroup form over the large segments' tiles, the
-  // one-wave form over the rest
   int wave_grid(int ntiles) const {
     return (int)std::max<int64_t>(1, std::min<int64_t>((ntiles + BLOCK / WAVE - 1) / (BLOCK / WAVE),
                                                        (int64_t)c->cus * 16));
   }
-  bool any_big() const { return nt_big > 0; }
-  bool any_wave() const { return nt_cur > nt_big; }
 
   // Lists the segments still active after a pass: their wave-sized slot
   // chunks, their tiles (a table of its own, with a first-tile index per
@@ -830,12 +827,12 @@ struct Runner {
     return lo < (int)cur_cap.size() ? cur_first[lo] : nt_cur;
   }
 
-  int sort_pairs(const int *n) {  // sorts (k0,v0) by the counts n[seg], result in (k0,v0)
+  // Sorts the pairs (k0, v0) of the first nt tiles by the counts n[seg], in place.
+  int sort_pairs(const int *n, int nt) {
     RETCHK(sort_begin());
-    if (any_big()) tile_sort_kernel<<<gtile, BLOCK, 0, c->stream>>>(tl_cur, nt_big, W.ibase, n, W.k0, W.v0, W.k1, W.v1);
-    if (any_wave()) sort_wave_kernel<<<gwave, BLOCK, 0, c->stream>>>(tl_cur, nt_big, nt_tiny, nt_cur, W.ibase, n, W.k0, W.v0);
-    merge_sorted(n, nt_cur);
-    return sort_end(n);
+    tile_sort_kernel<<<tile_grid(nt), BLOCK, 0, c->stream>>>(tl_cur, nt, W.ibase, n, W.k0, W.v0, W.k1, W.v1);
+    merge_sorted(n, nt);
+    return sort_end(n, nt < nt_cur ? TILE : 0);
   }
 
   // instrumentation: a sort's device time, or the elements it sorted and their
@@ -844,7 +841,7 @@ struct Runner {
     if (c->prof_mode == 1) HIPCHK(hipEventRecord(c->evs0, c->stream));
     return HBT_OK;
   }
-  int sort_end(const int *n, int above = 0) {  // above: only segments of more slots were sorted
+  int sort_end(const int *n, int above) {  // above: only segments of more slots were sorted
     if (c->prof_mode == 1) {
       HIPCHK(hipEventRecord(c->evs1, c->stream));
       HIPCHK(hipEventSynchronize(c->evs1));
@@ -858,16 +855,13 @@ struct Runner {
     return HBT_OK;
   }
 
-  // segmented exclusive scan over the counts n[seg]; the tile totals stay in tsum
+  // Segmented exclusive scan over the counts n[seg] of the first nt tiles; the
+  // tile totals stay in tsum.
   template <class Load, class Store, class Add>
-  int seg_scan(Load ld, Store st, Add ad, const int *n) {
+  void seg_scan(Load ld, Store st, Add ad, const int *n, int nt) {
     u64 *ts = c->tsum.as<u64>();
-    if (any_big()) scan_tiles_kernel<u64><<<gtile, BLOCK, 0, c->stream>>>(tl_cur, nt_big, n, ts, ld, st);
-    if (any_wave()) scan_wave_kernel<u64><<<gwave, BLOCK, 0, c->stream>>>(tl_cur, nt_big, nt_tiny, nt_cur, n, ts, ld, st);
-    // only segments of more than one tile have tiles after their first
-    const int nmulti = tiles_above(TILE);
-    if (nmulti > 0) scan_add_kernel<u64><<<gtile, BLOCK, 0, c->stream>>>(tl_cur, nmulti, n, ts, ad);
-    return HBT_OK;
+    scan_tiles_kernel<u64><<<tile_grid(nt), BLOCK, 0, c->stream>>>(tl_cur, nt, n, ts, ld, st);
+    scan_add_kernel<u64><<<tile_grid(nt), BLOCK, 0, c->stream>>>(tl_cur, nt, n, ts, ad);
   }
   const int *count_row(int row) const { return W.ncount + (size_t)row * W.nseg; }
 
@@ -898,15 +892,12 @@ struct Runner {
   // (tree_one), unless the caller goes on to read the sorted digits.
   int build_tree(bool copy_sp, bool keep_digits = false) {
     const int cp = copy_sp ? 1 : 0;
-    const int nm = keep_digits ? nt_cur : tiles_above(TILE);
+    const int nm = keep_digits ? nt_cur : nt_multi;
     if (nm > 0) {
       const int g = tile_grid(nm);
       RETCHK(sorted_digits(nm));
       emit_kernel<<<g, BLOCK, 0, c->stream>>>(W, tl_cur, nm, cp);
-      u64 *ts = c->tsum.as<u64>();
-      scan_tiles_kernel<u64><<<g, BLOCK, 0, c->stream>>>(tl_cur, nm, count_row(NC_SRC), ts, PopLoad{W.ibase, W.bits},
-                                                         PreStore{W.ibase, W.pre});
-      scan_add_kernel<u64><<<g, BLOCK, 0, c->stream>>>(tl_cur, nm, count_row(NC_SRC), ts, PreAdd{W.ibase, W.pre});
+      seg_scan(PopLoad{W.ibase, W.bits}, PreStore{W.ibase, W.pre}, PreAdd{W.ibase, W.pre}, count_row(NC_SRC), nm);
       items_tile_kernel<<<g, BLOCK, 0, c->stream>>>(W, P, tl_cur, nm);
       moments_super_kernel<<<g, BLOCK, 0, c->stream>>>(W, tl_cur, nm);
       if (max_n > SUPER) moments_cross_kernel<<<g, BLOCK, 0, c->stream>>>(W, tl_cur, nm);
@@ -967,66 +958,98 @@ struct Runner {
     launch_walk(c->prof_mode == 2);
     if (c->prof_mode == 2) tree_items_kernel<<<gseg, BLOCK, 0, c->stream>>>(W);
     if (c->prof_mode == 1) HIPCHK(hipEventRecord(c->evw1, c->stream));
-    // partition
-    RETCHK(seg_scan(PartLoad{W.ibase, W.el, W.E}, S64Store{W.ibase, W.scan64},
-                    S64Add{W.ibase, W.scan64}, count_row(NC_PART)));
-    partition_counts_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, ft_cur, c->tsum.as<u64>());
-    partition_rank_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
-    partition_k_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
-    partition_hole_kernel<<<gseg, BLOCK, 0, c->stream>>>(W);
-    partition_move_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
-    partition_done_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P);
-    if (P.max_sample > 0) {
-      disrupt_find_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
-      disrupt_swap_kernel<<<gseg, BLOCK, 0, c->stream>>>(W);
-    }
-    // spatial target list keeps the bound particles
-    bound_flags_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
-    RETCHK(seg_scan(BoundLoad{W.ibase, W.sp, W.isb}, PreStore{W.ibase, W.pre},
-                    PreAdd{W.ibase, W.pre}, count_row(NC_BOUND)));
-    spatial_compact_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
+    // everything else, for the segments of one tile and for the others; REPLAY
+    // sums the frames of both in the reference's order in between
+    int *sp_out = swap_sp ? W.el2 : W.sp;
+    if (P.replay) post_one<POST_PART>(sp_out);
+    else post_one<POST_ALL>(sp_out);
+    if (nt_multi > 0) RETCHK(partition());
     // the compacted list (in el2) becomes the spatial list and the old one
     // the next pass's scratch; only the active segments read either, and
     // they are rewritten every pass.  A captured pass sequence replays fixed
     // pointers, so it copies the list back instead.
     if (swap_sp) std::swap(W.sp, W.el2);
-    else spatial_copy_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
-    // frames, convergence (the frame sums read the bound block only, in Elist order)
     if (P.replay) {
       frames_serial_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P);
-    } else {
-      if (any_big()) frames_partial_kernel<<<gtile, BLOCK, 0, c->stream>>>(W, P, tl_cur, nt_big, c->tpart.as<double>());
-      if (any_wave())
-        frames_partial_wave_kernel<<<gwave, BLOCK, 0, c->stream>>>(W, P, tl_cur, nt_big, nt_tiny, nt_cur,
-                                                                   c->tpart.as<double>());
-      // the run sums go after the tile partials in the same buffer
-      double *gpart = c->tpart.as<double>() + (int64_t)(nt_cur + 1) * FRAME_SUMS;
-      if (max_n > SUPER)
-        frames_runs_kernel<<<grid_for(nt_cur, c->cus), BLOCK, 0, c->stream>>>(W, tl_cur, nt_cur, c->tpart.as<double>(),
-                                                                             gpart);
-      frames_combine_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P, ft_cur, c->tpart.as<double>(), gpart);
+      post_one<POST_SORT>(sp_out);
     }
-    // energy sort of the removed block, and of the bound block on convergence
-    energy_keys_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
-    RETCHK(sort_pairs(count_row(NC_SORT)));
-    energy_writeback_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
-    outputs();
+    if (nt_multi > 0) {
+      if (!P.replay) frames();
+      // energy sort of the removed block, and of the bound block on convergence
+      Work M = multi();
+      energy_keys_kernel<<<gmulti(), BLOCK, 0, c->stream>>>(M);
+      RETCHK(sort_pairs(count_row(NC_SORT), nt_multi));
+      energy_writeback_kernel<<<gmulti(), BLOCK, 0, c->stream>>>(M);
+      output_list_kernel<<<gmulti(), BLOCK, 0, c->stream>>>(M, 0);
+      if (!P.replay) output_records(W.nmulti, nt_multi);
+    }
+    if (P.replay) output_record_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P, 0);
+    count_active_kernel<<<std::min(gseg, 64), BLOCK, 0, c->stream>>>(W);
     HIPCHK(hipGetLastError());
     return HBT_OK;
   }
 
-  // The outputs of the record and its list for the segments flagged F_FINAL.
-  void outputs() {
-    output_list_kernel<<<gs, BLOCK, 0, c->stream>>>(W, 0);
-    if (P.replay) {
-      output_record_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P, 0);
-    } else {
-      if (any_big()) output_partial_kernel<<<gtile, BLOCK, 0, c->stream>>>(W, P, tl_cur, nt_big, c->tpart.as<double>());
-      if (any_wave())
-        output_partial_wave_kernel<<<gwave, BLOCK, 0, c->stream>>>(W, P, tl_cur, nt_big, nt_tiny, nt_cur,
-                                                                   c->tpart.as<double>());
-      output_combine_kernel<<<gwseg, BLOCK, 0, c->stream>>>(W, P, ft_cur, c->tpart.as<double>());
+  // The segments of one tile after their walk.
+  template <int STAGE>
+  void post_one(int *sp_out) {
+    const int m = nt_multi, b = nt_big, s = nt_tiny, n = nt_cur;
+    if (b > m) post_one_kernel<STAGE><<<tile_grid(b - m), BLOCK, 0, c->stream>>>(W, P, tl_cur, m, b, sp_out);
+    if (s > b) post_one_wave_kernel<4, STAGE><<<wave_grid(s - b), BLOCK, 0, c->stream>>>(W, P, tl_cur, b, s, sp_out);
+    if (n > s) post_one_wave_kernel<1, STAGE><<<wave_grid(n - s), BLOCK, 0, c->stream>>>(W, P, tl_cur, s, n, sp_out);
+  }
+
+  // The slots of the segments of more than one tile.
+  Work multi() const {
+    Work M = W;
+    M.nact = nact_multi;
+    return M;
+  }
+  int gmulti() const { return grid_for(nact_multi, c->cus); }
+  int gmseg() const { return grid_for(W.nmulti, c->cus); }
+
+  // Partition, bound flags and compacted spatial list of the larger segments.
+  int partition() {
+    Work M = multi();
+    const int g = gmulti(), gk = gmseg();
+    seg_scan(PartLoad{W.ibase, W.el, W.E}, S64Store{W.ibase, W.scan64}, S64Add{W.ibase, W.scan64}, count_row(NC_PART),
+             nt_multi);
+    partition_counts_kernel<<<gk, BLOCK, 0, c->stream>>>(M, ft_cur, c->tsum.as<u64>());
+    partition_rank_kernel<<<g, BLOCK, 0, c->stream>>>(M);
+    partition_k_kernel<<<g, BLOCK, 0, c->stream>>>(M);
+    partition_hole_kernel<<<gk, BLOCK, 0, c->stream>>>(M);
+    partition_move_kernel<<<g, BLOCK, 0, c->stream>>>(M);
+    partition_done_kernel<<<gk, BLOCK, 0, c->stream>>>(M, P);
+    if (P.max_sample > 0) {
+      disrupt_find_kernel<<<g, BLOCK, 0, c->stream>>>(M);
+      disrupt_swap_kernel<<<gk, BLOCK, 0, c->stream>>>(M);
     }
+    // spatial target list keeps the bound particles
+    bound_flags_kernel<<<g, BLOCK, 0, c->stream>>>(M);
+    seg_scan(BoundLoad{W.ibase, W.sp, W.isb}, PreStore{W.ibase, W.pre}, PreAdd{W.ibase, W.pre}, count_row(NC_BOUND),
+             nt_multi);
+    spatial_compact_kernel<<<g, BLOCK, 0, c->stream>>>(M);
+    if (!swap_sp) spatial_copy_kernel<<<g, BLOCK, 0, c->stream>>>(M);
+    return HBT_OK;
+  }
+
+  // Frames, convergence of the larger segments (the frame sums read the bound
+  // block only, in Elist order).
+  void frames() {
+    double *part = c->tpart.as<double>();
+    frames_partial_kernel<<<tile_grid(nt_multi), BLOCK, 0, c->stream>>>(W, P, tl_cur, nt_multi, part);
+    // the run sums go after the tile partials in the same buffer
+    double *gpart = part + (int64_t)(nt_cur + 1) * FRAME_SUMS;
+    if (max_n > SUPER)
+      frames_runs_kernel<<<grid_for(nt_multi, c->cus), BLOCK, 0, c->stream>>>(W, tl_cur, nt_multi, part, gpart);
+    frames_combine_kernel<<<gmseg(), BLOCK, 0, c->stream>>>(W, P, ft_cur, part, gpart);
+  }
+
+  // The records of the finished ones among the first nseg segments, which hold
+  // the first nt tiles.
+  void output_records(int nseg, int nt) {
+    double *part = c->tpart.as<double>();
+    output_partial_kernel<<<tile_grid(nt), BLOCK, 0, c->stream>>>(W, P, tl_cur, nt, part);
+    output_combine_kernel<<<grid_for((int64_t)nseg * WAVE, c->cus), BLOCK, 0, c->stream>>>(W, P, nseg, ft_cur, part);
   }
 
   // RefineBindingEnergyOrder for the segments that converged with more than
@@ -1041,10 +1064,12 @@ struct Runner {
     RETCHK(build_tree(false));
     launch_walk(false);
     refine_keys_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
-    RETCHK(sort_pairs(count_row(NC_SORT)));
+    RETCHK(sort_pairs(count_row(NC_SORT), nt_cur));
     energy_writeback_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
     refine_done_kernel<<<gseg, BLOCK, 0, c->stream>>>(W);
-    outputs();
+    output_list_kernel<<<gs, BLOCK, 0, c->stream>>>(W, 0);
+    if (P.replay) output_record_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P, 0);
+    else output_records(W.nseg, nt_cur);
     HIPCHK(hipGetLastError());
     return HBT_OK;
   }
@@ -1060,7 +1085,7 @@ struct Runner {
     rand_gen_kernel<<<g, BLOCK, 0, c->stream>>>(c->randtab.as<uint32_t>(), c->rwin.as<uint32_t>(), L->ndraws,
                                                   c->draws.as<int>());
     shuffle_keys_kernel<<<gs, BLOCK, 0, c->stream>>>(W, c->draws.as<int>());
-    RETCHK(sort_pairs(count_row(NC_SRC)));
+    RETCHK(sort_pairs(count_row(NC_SRC), nt_cur));
     shuffle_links_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
     shuffle_apply_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
     HIPCHK(hipGetLastError());
@@ -1123,6 +1148,7 @@ Work make_work(hbt_ctx *c, const Level &L, const hbt_particles *parts, hbt_subha
   Work W{};
   W.seg = c->seg.as<Seg>();
   W.nseg = (int)L.seg.size();
+  while (W.nmulti < W.nseg && L.seg[W.nmulti].cap > TILE) W.nmulti++;
   W.nslots = L.nslots;
   W.act_chunk = nullptr;
   W.nact = L.nslots;
@@ -1192,7 +1218,6 @@ int run_level(hbt_ctx *c, Level &L, const hbt_particles *parts, hbt_subhalo *sub
   R.max_n = L.maxcap;
   R.list_all();
   R.gseg = grid_for(nseg, c->cus);
-  R.gwseg = (int)std::min<int64_t>(((int64_t)nseg * WAVE + BLOCK - 1) / BLOCK, (int64_t)c->cus * 8);
   const int gsb = (int)std::min<int64_t>(nseg, (int64_t)c->cus * 8);
   R.gblk = gsb;
   seg_expand_kernel<<<R.gseg, BLOCK, 0, c->stream>>>(R.W.seg, c->segin.as<SegIn>(), (int)nseg);

@@ -175,3 +175,30 @@ def test_tree_forms(gpu, coincident):
         assert_exact(ref, got)
     for a, b in zip(got, gpu(p).unbind_batch(cat, plain=True)):
         assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
+
+
+@pytest.mark.parametrize("prec", [abi.HBT_PREC_REPLAY, abi.HBT_PREC_FAST])
+@pytest.mark.parametrize("refine", [0, 1])
+def test_one_tile_passes_with_a_sample(gpu, prec, refine):
+    """lists of up to a few tiles with a sample of 20: most are shuffled, their
+    trees hold 20 sources, and with the refinement their outputs wait for it;
+    REPLAY equals the oracle, FAST meets the band rule, and the captured pass
+    sequence (no list swap) and the plain form give the batched bytes"""
+    cat = synth.config2(seed=95, nsub=400, hi=3000)
+    cat.params["max_sample_size"] = 20
+    cat.params["refine_mostbound_particle"] = refine
+    cat.params["precision"] = prec
+    ref = oracle.unbind_batch(cat, nthreads=8, rand_state={"seed": 1, "draws": 0})
+    U = gpu(cat.params)
+    got = U.unbind_batch(cat)
+    if prec == abi.HBT_PREC_REPLAY:
+        assert_exact(ref, got)
+    else:
+        assert_tolerant(ref, got, refined=20 if refine else 0)
+    for form in ("graph", "plain"):
+        U.set_rand_state(1, 0)
+        t = U.get_tuning()
+        t["use_graph"] = int(form == "graph")
+        U.set_tuning(t)
+        for a, b in zip(got, U.unbind_batch(cat, plain=form == "plain")):
+            assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), form
