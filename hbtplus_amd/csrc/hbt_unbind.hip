@@ -133,7 +133,7 @@ struct hbt_ctx {
   int cus = 256;
   // per-slot work arrays
   DBuf gidx, pos, vel, E, el, el2, sp, k0, k1, v0, v1, dl, bits, pre, nlo, nhi,
-      npos, items, scan64, pk, gk, isb, seg_of_slot, cross, cross2, tcount;
+      npos, items, scan64, isb, seg_of_slot, cross, cross2, tcount;
   // per-level tables: staged through one pinned host buffer and one copy
   DBuf lvlbuf;
   void *h_stage = nullptr;
@@ -179,8 +179,7 @@ struct hbt_ctx {
   int64_t last_evals = 0, last_passes = 0;
   ~hbt_ctx() {
     for (DBuf *b : {&gidx, &pos, &vel, &E, &el, &el2, &sp, &k0, &k1, &v0, &v1, &dl,
-                    &bits, &pre, &nlo, &nhi, &npos, &items, &scan64, &pk, &gk,
-                    &isb, &seg_of_slot, &cross, &cross2, &tcount, &seg, &lvlbuf, &ncount, &tsum, &tpart, &active, &counters,
+                    &bits, &pre, &nlo, &nhi, &npos, &items, &scan64, &isb, &seg_of_slot, &cross, &cross2, &tcount, &seg, &lvlbuf, &ncount, &tsum, &tpart, &active, &counters,
                     &st_cols, &st_subs, &st_out_i, &st_out_e, &st_phi, &segact, &actbuf, &gaps, &pack, &idtab, &idpart, &idcnt,
                     &Er, &draws, &randtab, &tgt, &kick, &kickin, &kickcnt})
       b->release();
@@ -506,68 +505,6 @@ struct PreAdd {
   const int64_t *ibase; int *pre;
   __device__ void operator()(int k, int l, u64 x) const { pre[ibase[k] + l] += (int)x; }
 };
-struct PartLoad {
-  const int64_t *ibase; const int *el; const float *E;
-  __device__ u64 operator()(int k, int l) const {
-    if (l < 1) return 0;
-    const float e = E[ibase[k] + el[ibase[k] + l]];
-    return (u64)(e > 0.f ? 1u : 0u) | ((u64)(e < 0.f ? 1u : 0u) << 32);
-  }
-};
-struct S64Store {
-  const int64_t *ibase; u64 *out;
-  __device__ void operator()(int k, int l, u64 x) const { out[ibase[k] + l] = x; }
-};
-struct S64Add {
-  const int64_t *ibase; u64 *out;
-  __device__ void operator()(int k, int l, u64 x) const { out[ibase[k] + l] += x; }
-};
-struct BoundLoad {
-  const int64_t *ibase; const int *sp; const unsigned char *isb;
-  __device__ u64 operator()(int k, int l) const { return (u64)isb[ibase[k] + sp[ibase[k] + l]]; }
-};
-
-
-// Partition totals of each active segment: the sum of its tile totals, by its
-// own lane for a few tiles and by the whole wave, segment after segment, for
-// more (one lane over the 5,200 tiles of a 5.3M-particle host: 0.29 ms).
-__global__ void partition_counts_kernel(Work W, const int *first_tile, const u64 *tile_sum) {
-  constexpr int FEW = 16;
-  const int lane = threadIdx.x & (WAVE - 1);
-  for (int k0 = blockIdx.x * blockDim.x + (threadIdx.x & ~(WAVE - 1)); k0 < W.nmulti; k0 += gridDim.x * blockDim.x) {
-    const int k = k0 + lane;
-    int t0 = 0, nt = 0;
-    bool active = false;
-    if (k < W.nmulti) {
-      Seg &S = W.seg[k];
-      active = (S.flags & F_ACTIVE) != 0;
-      if (active) {
-        t0 = first_tile[k];
-        nt = (W.ncount[NC_PART * W.nseg + k] + TILE - 1) / TILE;
-      } else {
-        S.nP = S.nG = 0;
-      }
-    }
-    u64 t = 0;
-    if (nt <= FEW)
-      for (int u = t0; u < t0 + nt; u++) t += tile_sum[u];
-    for (u64 many = __ballot(nt > FEW); many; many &= many - 1) {
-      const int who = __ffsll((long long)many) - 1;
-      const int a = __shfl(t0, who, WAVE), n = __shfl(nt, who, WAVE);
-      u64 v = 0;
-      for (int u = lane; u < n; u += WAVE) v += tile_sum[a + u];
-      for (int d = WAVE / 2; d > 0; d >>= 1) v += __shfl_xor(v, d, WAVE);
-      if (lane == who) t = v;
-    }
-    if (active) {
-      Seg &S = W.seg[k];
-      S.nP = (int)(t & 0xffffffffu);
-      S.nG = (int)(t >> 32);
-      S.K = 0;
-    }
-  }
-}
-
 // A host's output region holds its own list and every nested particle (the
 // planned capacity); only its subhalos' unbound tails arrive, so the slots
 // past its final list are set to -1 and NaN.  gap: (subhalo, capacity, first
@@ -963,7 +900,7 @@ struct Runner {
     int *sp_out = swap_sp ? W.el2 : W.sp;
     if (P.replay) post_one<POST_PART>(sp_out);
     else post_one<POST_ALL>(sp_out);
-    if (nt_multi > 0) RETCHK(partition());
+    if (nt_multi > 0) partition();
     // the compacted list (in el2) becomes the spatial list and the old one
     // the next pass's scratch; only the active segments read either, and
     // they are rewritten every pass.  A captured pass sequence replays fixed
@@ -974,7 +911,6 @@ struct Runner {
       post_one<POST_SORT>(sp_out);
     }
     if (nt_multi > 0) {
-      if (!P.replay) frames();
       // energy sort of the removed block, and of the bound block on convergence
       Work M = multi();
       energy_keys_kernel<<<gmulti(), BLOCK, 0, c->stream>>>(M);
@@ -1007,40 +943,29 @@ struct Runner {
   int gmulti() const { return grid_for(nact_multi, c->cus); }
   int gmseg() const { return grid_for(W.nmulti, c->cus); }
 
-  // Partition, bound flags and compacted spatial list of the larger segments.
-  int partition() {
-    Work M = multi();
-    const int g = gmulti(), gk = gmseg();
-    seg_scan(PartLoad{W.ibase, W.el, W.E}, S64Store{W.ibase, W.scan64}, S64Add{W.ibase, W.scan64}, count_row(NC_PART),
-             nt_multi);
-    partition_counts_kernel<<<gk, BLOCK, 0, c->stream>>>(M, ft_cur, c->tsum.as<u64>());
-    partition_rank_kernel<<<g, BLOCK, 0, c->stream>>>(M);
-    partition_k_kernel<<<g, BLOCK, 0, c->stream>>>(M);
-    partition_hole_kernel<<<gk, BLOCK, 0, c->stream>>>(M);
-    partition_move_kernel<<<g, BLOCK, 0, c->stream>>>(M);
-    partition_done_kernel<<<gk, BLOCK, 0, c->stream>>>(M, P);
-    if (P.max_sample > 0) {
-      disrupt_find_kernel<<<g, BLOCK, 0, c->stream>>>(M);
-      disrupt_swap_kernel<<<gk, BLOCK, 0, c->stream>>>(M);
-    }
-    // spatial target list keeps the bound particles
-    bound_flags_kernel<<<g, BLOCK, 0, c->stream>>>(M);
-    seg_scan(BoundLoad{W.ibase, W.sp, W.isb}, PreStore{W.ibase, W.pre}, PreAdd{W.ibase, W.pre}, count_row(NC_BOUND),
-             nt_multi);
-    spatial_compact_kernel<<<g, BLOCK, 0, c->stream>>>(M);
-    if (!swap_sp) spatial_copy_kernel<<<g, BLOCK, 0, c->stream>>>(M);
-    return HBT_OK;
-  }
-
-  // Frames, convergence of the larger segments (the frame sums read the bound
-  // block only, in Elist order).
-  void frames() {
+  // Partition, bound flags, compacted spatial list, frames and convergence of
+  // the larger segments.
+  void partition() {
+    const int nt = nt_multi, g = tile_grid(nt);
+    u64 *ts = c->tsum.as<u64>();
     double *part = c->tpart.as<double>();
-    frames_partial_kernel<<<tile_grid(nt_multi), BLOCK, 0, c->stream>>>(W, P, tl_cur, nt_multi, part);
+    part_signs_kernel<<<g, BLOCK, 0, c->stream>>>(W, tl_cur, nt, ts);
+    part_list_kernel<<<g, BLOCK, 0, c->stream>>>(W, tl_cur, nt, ts);
+    part_hole_kernel<<<std::min(W.nmulti, c->cus * 8), BLOCK, 0, c->stream>>>(W, P, ft_cur, ts);
+    if (P.max_sample > 0) {
+      Work M = multi();
+      disrupt_find_kernel<<<gmulti(), BLOCK, 0, c->stream>>>(M);
+      disrupt_swap_kernel<<<gmseg(), BLOCK, 0, c->stream>>>(M);
+    }
+    part_move_kernel<<<g, BLOCK, 0, c->stream>>>(W, tl_cur, nt, ts);
+    bound_masks_kernel<<<g, BLOCK, 0, c->stream>>>(W, tl_cur, nt, ts);
+    if (P.replay) part_finish_kernel<false><<<g, BLOCK, 0, c->stream>>>(W, P, tl_cur, nt, ts, W.el2, part);
+    else part_finish_kernel<true><<<g, BLOCK, 0, c->stream>>>(W, P, tl_cur, nt, ts, W.el2, part);
+    if (!swap_sp) spatial_copy_kernel<<<gmulti(), BLOCK, 0, c->stream>>>(multi());
+    if (P.replay) return;
     // the run sums go after the tile partials in the same buffer
     double *gpart = part + (int64_t)(nt_cur + 1) * FRAME_SUMS;
-    if (max_n > SUPER)
-      frames_runs_kernel<<<grid_for(nt_multi, c->cus), BLOCK, 0, c->stream>>>(W, tl_cur, nt_multi, part, gpart);
+    if (max_n > SUPER) frames_runs_kernel<<<grid_for(nt, c->cus), BLOCK, 0, c->stream>>>(W, tl_cur, nt, part, gpart);
     frames_combine_kernel<<<gmseg(), BLOCK, 0, c->stream>>>(W, P, ft_cur, part, gpart);
   }
 
@@ -1130,8 +1055,6 @@ int ensure_slots(hbt_ctx *c, int64_t S, int64_t nseg, int64_t ntiles) {
   RETCHK(c->cross.ensure(s * 4));
   RETCHK(c->cross2.ensure(s * 4));
   RETCHK(c->tcount.ensure((size_t)(ntiles + 1) * 4));
-  RETCHK(c->pk.ensure((s + 1) * 4));
-  RETCHK(c->gk.ensure((s + 1) * 4));
   RETCHK(c->isb.ensure(s));
   RETCHK(c->seg_of_slot.ensure(s * 4));
   RETCHK(c->ncount.ensure((size_t)(NC_ROWS * nseg + 1) * 4));
@@ -1179,8 +1102,6 @@ Work make_work(hbt_ctx *c, const Level &L, const hbt_particles *parts, hbt_subha
   W.cross = c->cross.as<int>();
   W.cross2 = c->cross2.as<int>();
   W.tcount = c->tcount.as<int>();
-  W.scan64 = c->scan64.as<u64>();
-  W.pk = c->pk.as<int>(); W.gk = c->gk.as<int>();
   W.isb = c->isb.as<unsigned char>();
   W.active = c->active.as<int>();
   W.counters = c->counters.as<unsigned long long>();
