@@ -609,21 +609,46 @@ __device__ __forceinline__ u64 octant_key(const double center[3], double Len, in
   return key << (3 * (MAX_DEPTH - D));
 }
 
-// A tile's digits, sorted, into the buffer from which the merge levels end in
+// Sorted runs of RUN elements (a workgroup of RUN_THREADS), a segment's merge
+// levels starting there: longer than a tile, since a level reads and writes
+// every element once more, but a workgroup's phases overlap only with another's.
+// Digits, energies and merge levels of 200,000 subhalos' passes take 5.5 ms with
+// runs of 1,024, 5.3 with 2,048 and 5.7 with 4,096 (7.2 with 1,024 sorted as keys
+// with values, the energy keys by a launch of their own).
+constexpr int RUN_THREADS = 512, RUN = ITEMS * RUN_THREADS;
+
+// The runs with elements (count n(segment)) among the block's tiles
+// (blockIdx.x + k gridDim.x, a multiple of RUN into their segments), checked
+// RUN_THREADS at a time: an operation on a few entries per segment skips the
+// others without a chain of header loads.  f(tile) for each.
+template <class Count, class F>
+__device__ __forceinline__ void for_runs(const Tile *__restrict__ tiles, int ntiles, Count n, F f) {
+  __shared__ int live[RUN_THREADS], nlive;
+  for (int tb = blockIdx.x; tb < ntiles; tb += gridDim.x * RUN_THREADS) {
+    if (threadIdx.x == 0) nlive = 0;
+    __syncthreads();
+    const int tc = tb + (int)threadIdx.x * (int)gridDim.x;
+    if (tc < ntiles && tiles[tc].start % RUN == 0 && n(tiles[tc].seg) > tiles[tc].start) live[atomicAdd(&nlive, 1)] = tc;
+    __syncthreads();
+    const int m = nlive;
+    for (int i = 0; i < m; i++) f(tiles[live[i]]);
+    __syncthreads();
+  }
+}
+
+// A run's digits, sorted, into the buffer from which the merge levels end in
 // (k0, v0); the root cube from the box, into the segment's state by its first
-// tile.  In one kernel the keys reach memory sorted: digits and sort in kernels
+// run.  In one kernel the keys reach memory sorted: digits and sort in kernels
 // of their own wrote and read 12 bytes per source in between.
-__global__ void __launch_bounds__(BLOCK) keys_sort_kernel(Work W, DevParams P, const Tile *__restrict__ tiles,
-                                                          int ntiles) {
-  __shared__ u64 sk[TILE];
-  __shared__ u32 sv[TILE];
+__global__ void __launch_bounds__(RUN_THREADS, 8) keys_sort_kernel(Work W, DevParams P, const Tile *__restrict__ tiles,
+                                                                   int ntiles) {
+  __shared__ u64 sk[RUN];
+  __shared__ u32 sv[RUN];
   __shared__ RootCube cube;
-  for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    const Tile tl = tiles[t];
+  for_runs(tiles, ntiles, [&](int k) { return W.ncount[NC_SRC * W.nseg + k]; }, [&](const Tile &tl) {
     Seg &S = W.seg[tl.seg];
     const int n = S.n_src;
-    const int cnt = min(TILE, n - tl.start);
-    if (cnt <= 0) continue;  // uniform
+    const int cnt = min(RUN, n - tl.start);
     if (threadIdx.x == 0) {
       cube = root_cube(P, S.bmin, S.bmax);
       if (tl.start == 0) store_root_cube(P, cube, S);
@@ -644,17 +669,17 @@ __global__ void __launch_bounds__(BLOCK) keys_sort_kernel(Work W, DevParams P, c
 #pragma unroll
     for (int r = 0; r < ITEMS; r++)
       k[r] = v[r] != ~0u ? octant_key(cube.center, cube.Len, cube.D, q[r].x, q[r].y, q[r].z) : ~0ull;
-    sort_tile(k, v, cnt, sk, sv);
-    const bool odd = (merge_levels(n) & 1) != 0;
+    sort_tile_spare<RUN_THREADS>(k, v, cnt, 3 * (MAX_DEPTH - cube.D), sk, sv);
+    const bool odd = (merge_levels(n, RUN) & 1) != 0;
     u64 *kout = odd ? W.k1 : W.k0;
     u32 *vout = odd ? W.v1 : W.v0;
-    for (int i = threadIdx.x; i < cnt; i += BLOCK) {
+    for (int i = threadIdx.x; i < cnt; i += RUN_THREADS) {
       kout[off + i] = sk[i];
       vout[off + i] = sv[i];
       W.bits[off + i] = 0u;  // node-start masks, set by emit_kernel
     }
     __syncthreads();
-  }
+  });
 }
 
 // ---------------------------------------------------------------------------
@@ -993,13 +1018,9 @@ __device__ __forceinline__ void tree_one(const Work &W, const DevParams &P, cons
 #pragma unroll
   for (int r = 0; r < R; r++)
     k[r] = v[r] != ~0u ? octant_key(cube.center, cube.Len, cube.D, q[r].x, q[r].y, q[r].z) : ~0ull;
-  if constexpr (TM::T == WAVE) {
-    sort_wave<R>(k, v, id, n);
-#pragma unroll
-    for (int r = 0; r < R; r++) { L.s.key[R * id + r] = k[r]; L.s.val[R * id + r] = v[r]; }
-  } else {
-    sort_tile(k, v, n, L.s.key, L.s.val);
-  }
+  const int spare = 3 * (MAX_DEPTH - cube.D);
+  if constexpr (TM::T == WAVE) sort_wave_spare<R>(k, v, id, n, spare, L.s.key, L.s.val);
+  else sort_tile_spare<TM::T>(k, v, n, spare, L.s.key, L.s.val);
 #pragma unroll
   for (int r = 0; r < R; r++) L.s.bits[id + r * TM::T] = 0u;
   TM::sync();
@@ -1942,12 +1963,12 @@ __global__ void __launch_bounds__(PARTS *WAVE) walk_split_kernel(Work W, DevPara
 
 // Instrumented passes: the elements a segmented sort ordered (counters[8])
 // and the elements times the merge levels each needed (counters[9]).
-__global__ void sort_count_kernel(Work W, const int *n, int above) {
+__global__ void sort_count_kernel(Work W, const int *n, int above, int run) {
   unsigned long long e = 0, el = 0;
   SEG_LOOP(k, W) {
     const int c = W.seg[k].cap > above && n[k] > 0 ? n[k] : 0;
     e += (unsigned long long)c;
-    el += (unsigned long long)c * (unsigned long long)merge_levels(c);
+    el += (unsigned long long)c * (unsigned long long)merge_levels(c, run);
   }
   e = wave_reduce_sum(e);
   el = wave_reduce_sum(el);
@@ -2275,33 +2296,68 @@ __global__ void __launch_bounds__(BLOCK) spatial_copy_kernel(Work W) {
   }
 }
 
-// Sort keys for Elist[sort_lo, sort_lo + nsort) by energy: (block, ordered E,
-// position) -> local index.  The block bit keeps the bound block Elist[0, nbound)
-// and the removed block Elist[nbound, nlast) apart, so one segmented sort
-// orders each block by energy in place; position breaks ties (a stable order).
-__global__ void __launch_bounds__(BLOCK) energy_keys_kernel(Work W) {
-  SLOT_LOOP(s, W) {
-    int k;
-    int l = seg_lane_local(W, s, k);
-    if (l < 0) continue;
-    const Seg &S = W.seg[k];
-    if (l >= S.nsort) continue;
-    const int64_t b = S.ibase;
-    const int at = S.sort_lo + l;
-    const int li = W.el[b + at];
-    const u64 block = at >= S.nbound ? 1ull : 0ull;
-    W.k0[s] = (block << 63) | ((u64)f2ord(W.E[b + li]) << 31) | (u64)(unsigned)at;
-    W.v0[s] = (u32)li;
-  }
+// What orders Elist by energy: (block, E), position breaking ties (a stable
+// order).  The block bit keeps the bound block Elist[0, nbound) and the removed
+// block Elist[nbound, nlast) apart, so one segmented sort orders each in place.
+// Position `at` of a run or tile of 2^BITS from position `first`, as one word ...
+template <int BITS>
+__device__ __forceinline__ u64 energy_word(int at, int first, int nbound, float E) {
+  return ((u64)(at >= nbound ? 1u : 0u) << (32 + BITS)) | ((u64)f2ord(E) << BITS) | (u64)(unsigned)(at - first);
+}
+// ... and as the key of the merge levels over the whole segment.
+template <int BITS>
+__device__ __forceinline__ u64 energy_key(u64 w, int first) {
+  return ((w >> (32 + BITS)) << 63) | (((w >> BITS) & 0xffffffffull) << 31) |
+         (u64)(unsigned)(first + (int)(w & ((1ull << BITS) - 1)));
 }
 
-__global__ void __launch_bounds__(BLOCK) energy_writeback_kernel(Work W) {
+// Energies of Elist[sort_lo, sort_lo + nsort), sorted by runs: into Elist where
+// that is all, else into the buffer from which the merge levels end in (k0, v0).
+__global__ void __launch_bounds__(RUN_THREADS, 8) energy_sort_kernel(Work W, const Tile *__restrict__ tiles,
+                                                                     int ntiles) {
+  constexpr int BITS = log2_of(RUN);
+  __shared__ u64 sk[RUN];
+  __shared__ int sv[RUN];
+  for_runs(tiles, ntiles, [&](int k) { return W.ncount[NC_SORT * W.nseg + k]; }, [&](const Tile &tl) {
+    const Seg &S = W.seg[tl.seg];
+    const int64_t b = S.ibase;
+    const int n = S.nsort, first = S.sort_lo + tl.start, nb = S.nbound;
+    const int cnt = min(RUN, n - tl.start);
+    u64 x[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++) {
+      const int e = ITEMS * (int)threadIdx.x + r;
+      const int li = e < cnt ? W.el[b + first + e] : -1;
+      sv[e] = li;
+      x[r] = e < cnt ? energy_word<BITS>(first + e, first, nb, W.E[b + li]) : ~0ull;
+    }
+    sort_tile_words<RUN_THREADS>(x, cnt, sk);
+    const int m = merge_levels(n, RUN);
+    u64 *kout = (m & 1) != 0 ? W.k1 : W.k0;
+    u32 *vout = (m & 1) != 0 ? W.v1 : W.v0;
+    for (int i = threadIdx.x; i < cnt; i += RUN_THREADS) {
+      const u64 w = sk[i];
+      const int li = sv[w & (RUN - 1)];
+      if (m == 0) {
+        W.el[b + first + i] = li;
+      } else {
+        kout[b + tl.start + i] = energy_key<BITS>(w, first);
+        vout[b + tl.start + i] = (u32)li;
+      }
+    }
+    __syncthreads();
+  });
+}
+
+// The merged order into Elist, for segments that more than `run` elements were
+// sorted of.
+__global__ void __launch_bounds__(BLOCK) energy_writeback_kernel(Work W, int run) {
   SLOT_LOOP(s, W) {
     int k;
     int l = seg_lane_local(W, s, k);
     if (l < 0) continue;
     const Seg &S = W.seg[k];
-    if (l >= S.nsort) continue;
+    if (l >= S.nsort || S.nsort <= run) continue;
     W.el[S.ibase + S.sort_lo + l] = (int)W.v0[s];
   }
 }
@@ -2783,7 +2839,7 @@ template <int CAP>
 struct OnePost {
   union {
     struct { unsigned short p[CAP + 1], g[CAP + 1]; } part;  // p_k, g_k of the partition
-    struct { u64 key[CAP]; u32 val[CAP]; } sort;
+    u64 key[CAP];                                            // energy sort of a workgroup
   };
   float E[CAP];             // by Elist position, until the energy sort
   unsigned short el[CAP];   // Elist
@@ -2953,27 +3009,30 @@ __device__ __forceinline__ void post_one(Work &W, const DevParams &P, const Tile
       }
       TM::sync();
     }
-    // energy sort of Elist[lo, lo + nsort) (see energy_keys_kernel)
+    // energy sort of Elist[lo, lo + nsort)
     if (nsort > 0) {
-      u64 k[R];
-      u32 v[R];
+      constexpr int BITS = log2_of(CAP);
+      u64 x[R];
 #pragma unroll
       for (int r = 0; r < R; r++) {
-        const int i = R * id + r, at = lo + i;
-        const bool live = i < nsort;
-        k[r] = live ? ((at >= S.nbound ? 1ull : 0ull) << 63) | ((u64)f2ord(L.E[at]) << 31) | (u64)(unsigned)at : ~0ull;
-        v[r] = live ? L.el[at] : ~0u;
+        const int i = R * id + r;
+        x[r] = i < nsort ? energy_word<BITS>(lo + i, lo, S.nbound, L.E[lo + i]) : ~0ull;
       }
       if constexpr (T == WAVE) {
-        sort_wave<R>(k, v, id, nsort);
-        TM::sync();
-#pragma unroll
-        for (int r = 0; r < R; r++)
-          if (R * id + r < nsort) L.el[lo + R * id + r] = (unsigned short)v[r];
+        sort_words<R>(x, id, nsort);
       } else {
-        sort_tile(k, v, nsort, L.sort.key, L.sort.val);
-        for (int i = id; i < nsort; i += T) L.el[lo + i] = (unsigned short)L.sort.val[i];
+        sort_tile_words<T>(x, nsort, L.key);
+#pragma unroll
+        for (int r = 0; r < R; r++) x[r] = L.key[R * id + r];
       }
+      unsigned short li[R];
+#pragma unroll
+      for (int r = 0; r < R; r++)
+        if (R * id + r < nsort) li[r] = L.el[lo + (int)(x[r] & (CAP - 1))];
+      TM::sync();
+#pragma unroll
+      for (int r = 0; r < R; r++)
+        if (R * id + r < nsort) L.el[lo + R * id + r] = li[r];
       TM::sync();
     }
   }

@@ -242,7 +242,7 @@ extern "C" int hbt_mask_subhalos(hbt_ctx *ctx, const hbt_particles *particles, c
     tile_sort_kernel<<<gt, BLOCK, 0, st>>>(dt, nt, A.gbase, A.gn, A.k0, A.v0, ctx->k1.as<u64>(), ctx->v1.as<u32>());
     int level = 0;
     for (int w = TILE; w < maxn; w *= 2, level++)
-      merge_pass_kernel<<<gm, BLOCK, 0, st>>>(dt, nt, A.gbase, A.gn, level, A.k0, A.v0, ctx->k1.as<u64>(),
+      merge_pass_kernel<<<gm, BLOCK, 0, st>>>(dt, nt, A.gbase, A.gn, TILE, level, A.k0, A.v0, ctx->k1.as<u64>(),
                                               ctx->v1.as<u32>());
     mask_owner_kernel<<<grid_for(off, ctx->cus), BLOCK, 0, st>>>(A);
     u64 *ts = ctx->tsum.as<u64>();

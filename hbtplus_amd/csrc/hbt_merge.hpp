@@ -507,7 +507,7 @@ extern "C" int hbt_merge_subhalos(hbt_ctx *ctx, const hbt_particles *snapshot, c
     tile_sort_kernel<<<gt, BLOCK, 0, st>>>(dt, nt, U.gbase, U.gn, U.k0, U.v0, ctx->k1.as<u64>(), ctx->v1.as<u32>());
     int level = 0;
     for (int w = TILE; w < maxn; w *= 2, level++)
-      merge_pass_kernel<<<gm, BLOCK, 0, st>>>(dt, nt, U.gbase, U.gn, level, U.k0, U.v0, ctx->k1.as<u64>(),
+      merge_pass_kernel<<<gm, BLOCK, 0, st>>>(dt, nt, U.gbase, U.gn, TILE, level, U.k0, U.v0, ctx->k1.as<u64>(),
                                               ctx->v1.as<u32>());
     merge_keep_kernel<<<grid_for(slots, ctx->cus), BLOCK, 0, st>>>(U);
     u64 *ts = ctx->tsum.as<u64>();

@@ -346,7 +346,7 @@ extern "C" int hbt_subhalo_properties(hbt_ctx *ctx, const hbt_particles *particl
   tile_sort_kernel<<<gt, BLOCK, 0, st>>>(dt, ntiles, A.ibase, A.n, A.k0, A.v0, A.k1, A.v1);
   int level = 0;
   for (int w = TILE; w < maxn; w *= 2, level++)
-    merge_pass_kernel<<<gm, BLOCK, 0, st>>>(dt, ntiles, A.ibase, A.n, level, A.k0, A.v0, A.k1, A.v1);
+    merge_pass_kernel<<<gm, BLOCK, 0, st>>>(dt, ntiles, A.ibase, A.n, TILE, level, A.k0, A.v0, A.k1, A.v1);
   // running mass in distance order
   double *ts = (double *)ctx->tsum.as<u64>();
   scan_tiles_kernel<double><<<gt, BLOCK, 0, st>>>(dt, ntiles, A.n, ts, CumLoad{A.ibase, A.v0, A.m},

@@ -649,7 +649,13 @@ struct Runner {
     nact_multi = 0;
     for (size_t i = 0; i < cur_cap.size() && cur_cap[i] > TILE; i++) nact_multi += (cur_cap[i] + WAVE - 1) / WAVE * WAVE;
   }
-  int tile_grid(int nt) const { return (int)std::max<int64_t>(1, std::min<int64_t>(nt, (int64_t)c->cus * 8)); }
+  // A block per tile, at most eight per CU; less: a few blocks fewer, so that
+  // kernels which work at every 4th or 64th tile of a segment spread over all of
+  // them (a stride of a power of two gave one list of 4 million's super-tiles to
+  // 32 blocks).
+  int tile_grid(int nt, int less = 0) const {
+    return (int)std::max<int64_t>(1, std::min<int64_t>(nt, (int64_t)c->cus * 8 - less));
+  }
 
   int wave_grid(int ntiles) const {
     return (int)std::max<int64_t>(1, std::min<int64_t>((ntiles + BLOCK / WAVE - 1) / (BLOCK / WAVE),
@@ -768,8 +774,8 @@ struct Runner {
   int sort_pairs(const int *n, int nt) {
     RETCHK(sort_begin());
     tile_sort_kernel<<<tile_grid(nt), BLOCK, 0, c->stream>>>(tl_cur, nt, W.ibase, n, W.k0, W.v0, W.k1, W.v1);
-    merge_sorted(n, nt);
-    return sort_end(n, nt < nt_cur ? TILE : 0);
+    merge_sorted(n, nt, TILE);
+    return sort_end(n, 0, TILE);
   }
 
   // instrumentation: a sort's device time, or the elements it sorted and their
@@ -778,7 +784,7 @@ struct Runner {
     if (c->prof_mode == 1) HIPCHK(hipEventRecord(c->evs0, c->stream));
     return HBT_OK;
   }
-  int sort_end(const int *n, int above) {  // above: only segments of more slots were sorted
+  int sort_end(const int *n, int above, int run) {  // above: only segments of more slots were sorted
     if (c->prof_mode == 1) {
       HIPCHK(hipEventRecord(c->evs1, c->stream));
       HIPCHK(hipEventSynchronize(c->evs1));
@@ -787,7 +793,7 @@ struct Runner {
       c->sort_ms += ms;
       c->sort_calls++;
     } else if (c->prof_mode == 2) {
-      sort_count_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, n, above);
+      sort_count_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, n, above, run);
     }
     return HBT_OK;
   }
@@ -802,17 +808,17 @@ struct Runner {
   }
   const int *count_row(int row) const { return W.ncount + (size_t)row * W.nseg; }
 
-  // The merge levels after a tile sort of the first nt_first tiles.
-  void merge_sorted(const int *n, int nt_first) {
+  // The merge levels after a sort of the first nt_first tiles in runs of `run`.
+  void merge_sorted(const int *n, int nt_first, int run) {
     // one launch per merge level of the largest segment of the level, over
     // the tiles of the segments whose capacity exceeds the level's width
     // (segments are ordered largest first, so those tiles are a prefix)
     int level = 0;
-    for (int w = TILE; w < max_n; w *= 2, level++) {
+    for (int w = run; w < max_n; w *= 2, level++) {
       const int ntw = std::min(tiles_above(w), nt_first);
       if (ntw == 0) break;
       const int gmerge = (int)std::max<int64_t>(1, std::min<int64_t>(ntw, (int64_t)c->cus * 16));
-      merge_pass_kernel<<<gmerge, BLOCK, 0, c->stream>>>(tl_cur, ntw, W.ibase, n, level, W.k0, W.v0, W.k1, W.v1);
+      merge_pass_kernel<<<gmerge, BLOCK, 0, c->stream>>>(tl_cur, ntw, W.ibase, n, run, level, W.k0, W.v0, W.k1, W.v1);
     }
   }
   // Root cubes and sorted octant digits of the segments of the first nt tiles.
@@ -820,9 +826,9 @@ struct Runner {
     const int g = tile_grid(nt);
     bbox_kernel<<<g, BLOCK, 0, c->stream>>>(W, tl_cur, nt);
     RETCHK(sort_begin());
-    keys_sort_kernel<<<g, BLOCK, 0, c->stream>>>(W, P, tl_cur, nt);
-    merge_sorted(count_row(NC_SRC), nt);
-    return sort_end(count_row(NC_SRC), nt < nt_cur ? TILE : 0);
+    keys_sort_kernel<<<tile_grid(nt, 1), RUN_THREADS, 0, c->stream>>>(W, P, tl_cur, nt);
+    merge_sorted(count_row(NC_SRC), nt, RUN);
+    return sort_end(count_row(NC_SRC), nt < nt_cur ? TILE : 0, RUN);
   }
 
   // Tree over the pass's sources.  Segments of at most one tile take one launch
@@ -836,7 +842,7 @@ struct Runner {
       emit_kernel<<<g, BLOCK, 0, c->stream>>>(W, tl_cur, nm, cp);
       seg_scan(PopLoad{W.ibase, W.bits}, PreStore{W.ibase, W.pre}, PreAdd{W.ibase, W.pre}, count_row(NC_SRC), nm);
       items_tile_kernel<<<g, BLOCK, 0, c->stream>>>(W, P, tl_cur, nm);
-      moments_super_kernel<<<g, BLOCK, 0, c->stream>>>(W, tl_cur, nm);
+      moments_super_kernel<<<tile_grid(nm, 1), BLOCK, 0, c->stream>>>(W, tl_cur, nm);
       if (max_n > SUPER) moments_cross_kernel<<<g, BLOCK, 0, c->stream>>>(W, tl_cur, nm);
     }
     const int nb = std::max(nm, nt_big), ns = std::max(nm, nt_tiny);
@@ -913,9 +919,11 @@ struct Runner {
     if (nt_multi > 0) {
       // energy sort of the removed block, and of the bound block on convergence
       Work M = multi();
-      energy_keys_kernel<<<gmulti(), BLOCK, 0, c->stream>>>(M);
-      RETCHK(sort_pairs(count_row(NC_SORT), nt_multi));
-      energy_writeback_kernel<<<gmulti(), BLOCK, 0, c->stream>>>(M);
+      RETCHK(sort_begin());
+      energy_sort_kernel<<<tile_grid(nt_multi, 1), RUN_THREADS, 0, c->stream>>>(W, tl_cur, nt_multi);
+      merge_sorted(count_row(NC_SORT), nt_multi, RUN);
+      RETCHK(sort_end(count_row(NC_SORT), TILE, RUN));
+      if (max_n > RUN) energy_writeback_kernel<<<gmulti(), BLOCK, 0, c->stream>>>(M, RUN);
       output_list_kernel<<<gmulti(), BLOCK, 0, c->stream>>>(M, 0);
       if (!P.replay) output_records(W.nmulti, nt_multi);
     }
@@ -990,7 +998,7 @@ struct Runner {
     launch_walk(false);
     refine_keys_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
     RETCHK(sort_pairs(count_row(NC_SORT), nt_cur));
-    energy_writeback_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
+    energy_writeback_kernel<<<gs, BLOCK, 0, c->stream>>>(W, 0);
     refine_done_kernel<<<gseg, BLOCK, 0, c->stream>>>(W);
     output_list_kernel<<<gs, BLOCK, 0, c->stream>>>(W, 0);
     if (P.replay) output_record_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P, 0);

@@ -202,3 +202,23 @@ def test_one_tile_passes_with_a_sample(gpu, prec, refine):
         U.set_tuning(t)
         for a, b in zip(got, U.unbind_batch(cat, plain=form == "plain")):
             assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), form
+
+
+@pytest.mark.parametrize("softening", [0.0108, 0.5])
+def test_digit_sorts(gpu, softening):
+    """octant digits of 19 depths leave a word no room for the place in the
+    run, and are sorted as pairs, those of 13 as words; a few equal digits (pairs
+    of sources closer than the smallest cell) are ordered by their values.
+    REPLAY against the oracle bit for bit, at the sizes of each sort"""
+    base = synth.config1(seed=97, n_nfw=8000, n_cont=1000)
+    sizes = [3, 60, 250, 1000, 2000, 2100, 9000]
+    cols = {c: np.concatenate([a[:n] for n in sizes]) for c, a in base.cols.items()}
+    cols["id"] = np.arange(sum(sizes), dtype=np.int64)
+    cols["mass"] *= np.repeat(9000 / np.float32(sizes), sizes)
+    subs = np.repeat(base.subs[:1], len(sizes))
+    subs["count"] = subs["nbound_prev"] = sizes
+    subs["offset"] = np.cumsum([0] + sizes[:-1])
+    p = base.params.copy()
+    p["precision"], p["softening"] = abi.HBT_PREC_REPLAY, softening
+    cat = synth.Catalogue(cols, subs, p, "digit sorts")
+    assert_exact(oracle.unbind_batch(cat, nthreads=8), gpu(p).unbind_batch(cat))
