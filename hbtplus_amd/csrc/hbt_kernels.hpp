@@ -75,7 +75,7 @@ struct Work {
   Item *items;               // [2*nslots] tree items in pre-order
   unsigned char *isb;
   int *active;               // [4]: segments active after the pass, the largest Nlast among them
-  unsigned long long *counters;  // [4]: interactions, opened nodes, targets (instrumented passes)
+  unsigned long long *counters;  // interactions, opened nodes, targets (instrumented passes); [4] evaluations
   // caller outputs
   hbt_subhalo *subs;
   int64_t *out_index;
@@ -250,9 +250,9 @@ __device__ __forceinline__ int own_entry(const Work &W, const Seg &S, int l) {
   return W.g_index ? (int)W.g_index[o] : (int)o;
 }
 
-// Column positions of the segments' own particles (phase bit 1), and local
-// copies of the listed particles' columns (phase bit 2), slot-parallel.  A
-// shuffled list is permuted between the two phases.
+// Column positions of the segments' own particles (phase bit 1), local copies
+// of the listed particles' columns and the initial Elist (phase bit 2),
+// slot-parallel.  A shuffled list is permuted between the two phases.
 __global__ void __launch_bounds__(BLOCK) gather_kernel(Work W, int phase) {
   SLOT_LOOP(s, W) {
     int k;
@@ -266,6 +266,7 @@ __global__ void __launch_bounds__(BLOCK) gather_kernel(Work W, int phase) {
       g = W.gidx[s];
     }
     if (!(phase & 2)) continue;
+    if (l < W.seg[k].ulen) W.el[s] = l;
     if (W.g_packed) {
       W.pos[s] = W.g_packed[2 * (int64_t)g];
       W.vel[s] = W.g_packed[2 * (int64_t)g + 1];
@@ -279,7 +280,10 @@ __global__ void __launch_bounds__(BLOCK) gather_kernel(Work W, int phase) {
 // Unbind entry (src/subhalo_unbind.cpp:263-309): early exits, initial Elist;
 // the shuffle's sort count (steps 1..ulen-1) of a shuffled list.
 __global__ void seg_init_kernel(Work W, DevParams P) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) W.active[3] = 0;  // refinements pending in the level
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    W.active[3] = 0;    // refinements pending in the level
+    W.counters[4] = 0;  // evaluations, summed after the last level
+  }
   SEG_LOOP(k, W) {
     Seg &S = W.seg[k];
     hbt_subhalo &r = W.subs[S.sub];
@@ -420,15 +424,6 @@ __global__ void __launch_bounds__(BLOCK) prelude_sp_kernel(Work W) {
     if (S.draw_off < 0 || !(S.flags & F_ACTIVE) || l >= S.ulen) continue;
     W.sp[s] = (int)W.v0[s];
     if (l == 0) S.sall = S.straddle;
-  }
-}
-
-__global__ void el_init_kernel(Work W) {
-  SLOT_LOOP(s, W) {
-    int k;
-    int l = seg_lane_local(W, s, k);
-    if (l < 0) continue;
-    if (l < W.seg[k].ulen) W.el[s] = l;
   }
 }
 
@@ -2617,14 +2612,14 @@ __device__ __forceinline__ void output_entry(const Work &W, const Seg &S, int l,
   }
 }
 
-__global__ void __launch_bounds__(BLOCK) output_list_kernel(Work W, int early) {
+// Lists of the segments that finished in the pass.
+__global__ void __launch_bounds__(BLOCK) output_list_kernel(Work W) {
   SLOT_LOOP(s, W) {
     int k;
     int l = seg_lane_local(W, s, k);
     if (l < 0) continue;
     const Seg &S = W.seg[k];
-    const bool fin = early ? (S.flags & F_EARLY) != 0 : (S.flags & F_FINAL) != 0;
-    if (!fin || l >= S.len) continue;
+    if (!(S.flags & F_FINAL) || l >= S.len) continue;
     output_entry(W, S, l, W.el[s]);
   }
 }
@@ -2713,33 +2708,47 @@ __device__ __forceinline__ void kin_accum(const Work &W, const DevParams &P, con
   v[5] += m;
 }
 
-// Serial form (REPLAY and early exits): one thread per finished segment,
-// sums in list order as the reference does with one thread.
-__global__ void output_record_kernel(Work W, DevParams P, int early) {
+// Serial form (REPLAY and early exits): sums in list order as the reference
+// does with one thread.
+__device__ __forceinline__ void record_serial(Work &W, const DevParams &P, Seg &S) {
 #pragma clang fp contract(off)
+  const int64_t b = S.ibase;
+  const bool conv = (S.flags & F_CONV) != 0;
+  const int nb = S.nbound;
+  const bool skip_null = !(S.flags & F_EARLY) && nb <= 100;
+  double v[6] = {0, 0, 0, 0, 0, 0};
+  int nt[HBT_TYPE_MAX] = {0, 0, 0, 0, 0, 0};
+  float mts[HBT_TYPE_MAX] = {0, 0, 0, 0, 0, 0};
+  for (int i = 0; i < nb; i++) {
+    const int li = conv ? W.el[b + i] : i;
+    if (nb > 1) kin_accum(W, P, S, li, v);
+  }
+  for (int i = 0; i < nb; i++) {
+    const int li = conv ? W.el[b + i] : i;
+    if (skip_null && W.g_id[W.gidx[b + li]] == -1) continue;
+    const int t = __float_as_int(W.vel[b + li].w);
+    nt[t]++;
+    mts[t] += W.pos[b + li].w;
+  }
+  write_record(W, P, S, v[0], v[1], v[2], v[3], v[4], v[5], nt, mts);
+}
+
+__global__ void output_record_kernel(Work W, DevParams P) {
   SEG_LOOP(k, W) {
     Seg &S = W.seg[k];
-    const bool fin = early ? (S.flags & F_EARLY) != 0 : (S.flags & F_FINAL) != 0;
-    if (!fin) continue;
-    const int64_t b = S.ibase;
-    const bool conv = (S.flags & F_CONV) != 0;
-    const int nb = S.nbound;
-    const bool skip_null = !(S.flags & F_EARLY) && nb <= 100;
-    double v[6] = {0, 0, 0, 0, 0, 0};
-    int nt[HBT_TYPE_MAX] = {0, 0, 0, 0, 0, 0};
-    float mts[HBT_TYPE_MAX] = {0, 0, 0, 0, 0, 0};
-    for (int i = 0; i < nb; i++) {
-      const int li = conv ? W.el[b + i] : i;
-      if (nb > 1) kin_accum(W, P, S, li, v);
-    }
-    for (int i = 0; i < nb; i++) {
-      const int li = conv ? W.el[b + i] : i;
-      if (skip_null && W.g_id[W.gidx[b + li]] == -1) continue;
-      const int t = __float_as_int(W.vel[b + li].w);
-      nt[t]++;
-      mts[t] += W.pos[b + li].w;
-    }
-    write_record(W, P, S, v[0], v[1], v[2], v[3], v[4], v[5], nt, mts);
+    if (S.flags & F_FINAL) record_serial(W, P, S);
+  }
+}
+
+// Lists and records of the early exits (0 or 1 particles to unbind), a wave per
+// segment: over every slot they took 0.26 ms of a level of 54 million.
+__global__ void __launch_bounds__(BLOCK) output_early_kernel(Work W, DevParams P) {
+  WAVE_SEG_LOOP(k, W.nseg) {
+    Seg &S = W.seg[k];
+    if (!(S.flags & F_EARLY)) continue;  // uniform across the wave
+    const int lane = threadIdx.x & (WAVE - 1);
+    for (int l = lane; l < S.len; l += WAVE) output_entry(W, S, l, 0);  // (none of them converged)
+    if (lane == 0) record_serial(W, P, S);
   }
 }
 

@@ -526,14 +526,16 @@ __global__ void __launch_bounds__(BLOCK) fill_gaps_kernel(const hbt_subhalo *sub
   }
 }
 
-// Sum of n_evals over the records (one block).
+// Adds the sum of n_evals over the records to *out, which every level's
+// seg_init clears (one block over 200,000 of them took 0.46 ms).
 __global__ void __launch_bounds__(BLOCK) eval_sum_kernel(const hbt_subhalo *subs, int64_t nsub,
                                                          unsigned long long *out) {
   unsigned long long v = 0;
-  for (int64_t i = threadIdx.x; i < nsub; i += BLOCK) v += (unsigned long long)subs[i].n_evals;
+  for (int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x; i < nsub; i += (int64_t)gridDim.x * BLOCK)
+    v += (unsigned long long)subs[i].n_evals;
   unsigned long long tot;
   (void)block_exclusive_scan(v, &tot);
-  if (threadIdx.x == 0) *out = tot;
+  if (threadIdx.x == 0) atomicAdd(out, tot);
 }
 
 // Particle types outside [0, HBT_TYPE_MAX) (the per-type counts index by type).
@@ -924,10 +926,10 @@ struct Runner {
       merge_sorted(count_row(NC_SORT), nt_multi, RUN);
       RETCHK(sort_end(count_row(NC_SORT), TILE, RUN));
       if (max_n > RUN) energy_writeback_kernel<<<gmulti(), BLOCK, 0, c->stream>>>(M, RUN);
-      output_list_kernel<<<gmulti(), BLOCK, 0, c->stream>>>(M, 0);
+      output_list_kernel<<<gmulti(), BLOCK, 0, c->stream>>>(M);
       if (!P.replay) output_records(W.nmulti, nt_multi);
     }
-    if (P.replay) output_record_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P, 0);
+    if (P.replay) output_record_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P);
     count_active_kernel<<<std::min(gseg, 64), BLOCK, 0, c->stream>>>(W);
     HIPCHK(hipGetLastError());
     return HBT_OK;
@@ -1000,8 +1002,8 @@ struct Runner {
     RETCHK(sort_pairs(count_row(NC_SORT), nt_cur));
     energy_writeback_kernel<<<gs, BLOCK, 0, c->stream>>>(W, 0);
     refine_done_kernel<<<gseg, BLOCK, 0, c->stream>>>(W);
-    output_list_kernel<<<gs, BLOCK, 0, c->stream>>>(W, 0);
-    if (P.replay) output_record_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P, 0);
+    output_list_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
+    if (P.replay) output_record_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P);
     else output_records(W.nseg, nt_cur);
     HIPCHK(hipGetLastError());
     return HBT_OK;
@@ -1162,10 +1164,8 @@ int run_level(hbt_ctx *c, Level &L, const hbt_particles *parts, hbt_subhalo *sub
   } else {
     gather_kernel<<<R.gs, BLOCK, 0, c->stream>>>(R.W, 3);
   }
-  el_init_kernel<<<R.gs, BLOCK, 0, c->stream>>>(R.W);
   RETCHK(R.prelude());
-  output_list_kernel<<<R.gs, BLOCK, 0, c->stream>>>(R.W, 1);
-  output_record_kernel<<<R.gseg, BLOCK, 0, c->stream>>>(R.W, R.P, 1);
+  output_early_kernel<<<grid_for(nseg * WAVE, c->cus), BLOCK, 0, c->stream>>>(R.W, R.P);
   HIPCHK(hipGetLastError());
   if (getenv("HBT_PASS_TIMES") && atoi(getenv("HBT_PASS_TIMES"))) {
     HIPCHK(hipStreamSynchronize(c->stream));
@@ -1875,7 +1875,8 @@ static int unbind_batch_impl(hbt_ctx *ctx, const hbt_particles *particles, int64
   HIPCHK(hipEventRecord(ctx->ev1, ctx->stream));
   // evaluation count, summed on the device after the timed work
   long long *h_ev = (long long *)(ctx->h_active + 4);
-  eval_sum_kernel<<<1, BLOCK, 0, ctx->stream>>>(subs, nsub, ctx->counters.as<unsigned long long>() + 4);
+  eval_sum_kernel<<<std::min(grid_for(nsub, ctx->cus), ctx->cus), BLOCK, 0, ctx->stream>>>(
+      subs, nsub, ctx->counters.as<unsigned long long>() + 4);
   HIPCHK(hipMemcpyAsync(h_ev, ctx->counters.as<unsigned long long>() + 4, 8, hipMemcpyDeviceToHost,
                         ctx->stream));
   HIPCHK(hipStreamSynchronize(ctx->stream));
