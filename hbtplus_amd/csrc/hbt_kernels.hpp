@@ -74,7 +74,9 @@ struct Work {
   int *tcount;               // per tile of the pass's table: list length of the super-tile it starts
   Item *items;               // [2*nslots] tree items in pre-order
   unsigned char *isb;
-  int *active;               // [4]: segments active after the pass, the largest Nlast among them
+  int *active;               // [4]: segments active after the pass, the largest Nlast among them, blocks that
+                             // have counted, refinements pending in the level
+  int *host_active;          // the same for the host (pinned)
   unsigned long long *counters;  // interactions, opened nodes, targets (instrumented passes); [4] evaluations
   // caller outputs
   hbt_subhalo *subs;
@@ -192,9 +194,52 @@ __global__ void __launch_bounds__(BLOCK) seg_of_chunk_kernel(int nseg, const int
   }
 }
 
-// The level's segment records: zero, then the host's fixed fields.
-__global__ void __launch_bounds__(BLOCK) seg_expand_kernel(Seg *seg, const SegIn *in, int n) {
-  for (int k = blockIdx.x * BLOCK + threadIdx.x; k < n; k += gridDim.x * BLOCK) {
+// Unbind entry (src/subhalo_unbind.cpp:263-309): early exits, initial Elist;
+// the shuffle's sort count (steps 1..ulen-1) of a shuffled list.
+__device__ __forceinline__ void init_segment(const Work &W, const DevParams &P, Seg &S, int k) {
+  hbt_subhalo &r = W.subs[S.sub];
+  const bool orphan = S.nbprev <= 1;
+  S.ulen = orphan ? S.count : S.len;
+  S.flags = orphan ? F_ORPHAN : 0;
+  S.iter = 0;
+  S.evals = 0;
+  for (int j = 0; j < 3; j++) { S.ref_pos[j] = r.ref_pos[j]; S.ref_vel[j] = r.ref_vel[j]; }
+  if (S.ulen < P.min_part && r.snapshot_index_of_death == -1) r.snapshot_index_of_death = P.snap;
+  if (S.ulen <= 1) {
+    S.flags |= F_EARLY;
+    S.nbound = S.ulen;
+    S.nlast = S.ulen;
+  } else {
+    S.flags |= F_ACTIVE;
+    S.nbound = S.ulen;
+    S.nlast = S.ulen;
+  }
+  // the host shuffles exactly the lists longer than the sample (:302), with
+  // draws counted for the same length (a list of another length would read
+  // other segments' draws: it is not shuffled, and parity tests show it)
+  if (S.draw_off >= 0 && S.ulen > P.max_sample && P.max_sample > 0 && S.ulen == S.shuf_len) S.flags |= F_SHUF;
+  else S.draw_off = -1;
+  W.ncount[NC_SRC * W.nseg + k] = S.draw_off >= 0 ? S.ulen - 1 : 0;
+}
+
+__device__ __forceinline__ void clear_level_counts(const Work &W) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    W.active[3] = 0;    // refinements pending in the level
+    W.counters[4] = 0;  // evaluations, summed after the last level
+  }
+}
+
+// After build_lists_kernel (a level with nested subhalos' tails).
+__global__ void seg_init_kernel(Work W, DevParams P) {
+  clear_level_counts(W);
+  SEG_LOOP(k, W) init_segment(W, P, W.seg[k], k);
+}
+
+// The level's segment records: zero, then the host's fixed fields.  begin: the
+// lists are the segments' own, and their unbinding starts here too.
+__global__ void __launch_bounds__(BLOCK) seg_expand_kernel(Work W, DevParams P, const SegIn *in, int begin) {
+  if (begin) clear_level_counts(W);
+  SEG_LOOP(k, W) {
     const SegIn a = in[k];
     Seg S{};
     S.ibase = a.ibase;
@@ -209,7 +254,11 @@ __global__ void __launch_bounds__(BLOCK) seg_expand_kernel(Seg *seg, const SegIn
     S.shuf_len = a.shuf_len;
     S.mf = 1.f;
     S.swapq = INT_MAX;
-    seg[k] = S;
+    if (begin) {
+      S.len = S.count;
+      init_segment(W, P, S, k);
+    }
+    W.seg[k] = S;
   }
 }
 
@@ -274,41 +323,6 @@ __global__ void __launch_bounds__(BLOCK) gather_kernel(Work W, int phase) {
       W.pos[s] = make_float4(W.g_x[g], W.g_y[g], W.g_z[g], W.g_m[g]);
       W.vel[s] = make_float4(W.g_vx[g], W.g_vy[g], W.g_vz[g], __int_as_float(W.g_type ? W.g_type[g] : 1));
     }
-  }
-}
-
-// Unbind entry (src/subhalo_unbind.cpp:263-309): early exits, initial Elist;
-// the shuffle's sort count (steps 1..ulen-1) of a shuffled list.
-__global__ void seg_init_kernel(Work W, DevParams P) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    W.active[3] = 0;    // refinements pending in the level
-    W.counters[4] = 0;  // evaluations, summed after the last level
-  }
-  SEG_LOOP(k, W) {
-    Seg &S = W.seg[k];
-    hbt_subhalo &r = W.subs[S.sub];
-    const bool orphan = S.nbprev <= 1;
-    S.ulen = orphan ? S.count : S.len;
-    S.flags = orphan ? F_ORPHAN : 0;
-    S.iter = 0;
-    S.evals = 0;
-    for (int j = 0; j < 3; j++) { S.ref_pos[j] = r.ref_pos[j]; S.ref_vel[j] = r.ref_vel[j]; }
-    if (S.ulen < P.min_part && r.snapshot_index_of_death == -1) r.snapshot_index_of_death = P.snap;
-    if (S.ulen <= 1) {
-      S.flags |= F_EARLY;
-      S.nbound = S.ulen;
-      S.nlast = S.ulen;
-    } else {
-      S.flags |= F_ACTIVE;
-      S.nbound = S.ulen;
-      S.nlast = S.ulen;
-    }
-    // the host shuffles exactly the lists longer than the sample (:302), with
-    // draws counted for the same length (a list of another length would read
-    // other segments' draws: it is not shuffled, and parity tests show it)
-    if (S.draw_off >= 0 && S.ulen > P.max_sample && P.max_sample > 0 && S.ulen == S.shuf_len) S.flags |= F_SHUF;
-    else S.draw_off = -1;
-    W.ncount[NC_SRC * W.nseg + k] = S.draw_off >= 0 ? S.ulen - 1 : 0;
   }
 }
 
@@ -3080,7 +3094,9 @@ __global__ void __launch_bounds__(BLOCK, 4) post_one_kernel(Work W, DevParams P,
 }
 
 // Segments active after the pass, and the largest Nlast among them: by blocks,
-// since the atomics on two addresses are served one after another.
+// since the atomics on two addresses are served one after another.  The last
+// block writes them where the host reads them, which saves the copy that
+// followed.
 __global__ void __launch_bounds__(BLOCK) count_active_kernel(Work W) {
   int cnt = 0, most = 0;
   SEG_LOOP(k, W) {
@@ -3095,6 +3111,14 @@ __global__ void __launch_bounds__(BLOCK) count_active_kernel(Work W) {
   if ((threadIdx.x & (WAVE - 1)) == 0 && cnt) {
     atomicAdd(&W.active[0], cnt);
     atomicMax(&W.active[1], most);  // bounds every count of the next pass
+  }
+  __threadfence();
+  __syncthreads();
+  if (threadIdx.x == 0 && atomicAdd(&W.active[2], 1) == (int)gridDim.x - 1) {
+    __threadfence();
+    for (int i = 0; i < 4; i++)
+      if (i != 2) W.host_active[i] = __hip_atomic_load(&W.active[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __threadfence_system();
   }
 }
 

@@ -1114,6 +1114,7 @@ Work make_work(hbt_ctx *c, const Level &L, const hbt_particles *parts, hbt_subha
   W.tcount = c->tcount.as<int>();
   W.isb = c->isb.as<unsigned char>();
   W.active = c->active.as<int>();
+  W.host_active = c->h_active;
   W.counters = c->counters.as<unsigned long long>();
   W.subs = subs;
   W.out_index = out_index;
@@ -1124,8 +1125,6 @@ Work make_work(hbt_ctx *c, const Level &L, const hbt_particles *parts, hbt_subha
 // After a level's passes: the refinements that wait for them.
 int finish_level(hbt_ctx *c, Runner &R) {
   if (!R.P.refine) return HBT_OK;
-  HIPCHK(hipMemcpyAsync(c->h_active + 3, R.W.active + 3, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
   if (c->h_active[3] == 0) return HBT_OK;
   RETCHK(R.refine());
   HIPCHK(hipStreamSynchronize(c->stream));
@@ -1151,11 +1150,14 @@ int run_level(hbt_ctx *c, Level &L, const hbt_particles *parts, hbt_subhalo *sub
   R.gseg = grid_for(nseg, c->cus);
   const int gsb = (int)std::min<int64_t>(nseg, (int64_t)c->cus * 8);
   R.gblk = gsb;
-  seg_expand_kernel<<<R.gseg, BLOCK, 0, c->stream>>>(R.W.seg, c->segin.as<SegIn>(), (int)nseg);
+  const bool flat = L.child_list.empty();
+  seg_expand_kernel<<<R.gseg, BLOCK, 0, c->stream>>>(R.W, R.P, c->segin.as<SegIn>(), flat ? 1 : 0);
   // segment bases are multiples of WAVE (capacities are rounded up to it)
   seg_of_chunk_kernel<<<R.gs, BLOCK, 0, c->stream>>>((int)nseg, R.W.ibase, L.nslots, c->seg_of_slot.as<int>());
-  build_lists_kernel<<<gsb, BLOCK, 0, c->stream>>>(R.W, c->child_ptr.as<int>(), c->child_list.as<int>());
-  seg_init_kernel<<<R.gseg, BLOCK, 0, c->stream>>>(R.W, R.P);
+  if (!flat) {
+    build_lists_kernel<<<gsb, BLOCK, 0, c->stream>>>(R.W, c->child_ptr.as<int>(), c->child_list.as<int>());
+    seg_init_kernel<<<R.gseg, BLOCK, 0, c->stream>>>(R.W, R.P);
+  }
   if (L.ndraws > 0) {
     // shuffled lists: positions, the shuffle, then the columns in shuffled order
     gather_kernel<<<R.gs, BLOCK, 0, c->stream>>>(R.W, 1);
@@ -1175,8 +1177,8 @@ int run_level(hbt_ctx *c, Level &L, const hbt_particles *parts, hbt_subhalo *sub
   // every pass that does not converge removes at least one particle
   static const bool debug = getenv("HBT_DEBUG") != nullptr;
   // The pass sequence has static launch shapes and arguments for the whole
-  // level, so it is captured once as a hipGraph (graph_passes passes plus the
-  // read-back of the active count) and replayed until no segment is active.
+  // level, so it is captured once as a hipGraph (graph_passes passes, whose last
+  // kernel writes the active count where the host reads it) and replayed until no segment is active.
   // the plain form (one subhalo per level) launches directly, as a per-subhalo
   // Unbind loop does; graphs serve the batched form
   const bool graph = c->tune.use_graph && c->prof_mode == 0 && !debug && L.seg.size() > 1;
@@ -1192,9 +1194,8 @@ int run_level(hbt_ctx *c, Level &L, const hbt_particles *parts, hbt_subhalo *sub
     HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     int rc = HBT_OK;
     for (int p = 0; p < graph_passes && rc == HBT_OK; p++) rc = R.pass();
-    hipError_t e1 = hipMemcpyAsync(c->h_active, R.W.active, sizeof(int), hipMemcpyDeviceToHost, c->stream);
     hipError_t e2 = hipStreamEndCapture(c->stream, &g);
-    if (rc != HBT_OK || e1 != hipSuccess || e2 != hipSuccess) {
+    if (rc != HBT_OK || e2 != hipSuccess) {
       release();
       return rc != HBT_OK ? rc : fail(HBT_ERR_DEVICE, "pass graph capture failed");
     }
@@ -1257,7 +1258,6 @@ int run_level(hbt_ctx *c, Level &L, const hbt_particles *parts, hbt_subhalo *sub
       for (size_t i = 0; i < el.size(); i++) fprintf(stderr, " %d", el[i]);
       fprintf(stderr, "\n");
     }
-    HIPCHK(hipMemcpyAsync(c->h_active, R.W.active, 4 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     if (pass_times) {
       float ms = 0;
