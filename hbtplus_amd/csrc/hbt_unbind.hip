@@ -160,7 +160,8 @@ struct hbt_ctx {
   double sort_ms = 0;
   int64_t sort_calls = 0;
   // staging for hbt_unbind_one / hbt_tree_potential
-  DBuf st_cols, st_subs, st_out_i, st_out_e, st_phi;
+  DBuf st_one, st_phi;
+  HBuf h_one;           // pinned: hbt_unbind_one's columns and results
   int *h_active = nullptr;  // pinned
   const int64_t *list_index = nullptr;  // set for the duration of hbt_unbind_batch_indexed
   const float4 *packed = nullptr;       // likewise, when the snapshot is gathered from packed records
@@ -180,12 +181,13 @@ struct hbt_ctx {
   ~hbt_ctx() {
     for (DBuf *b : {&gidx, &pos, &vel, &E, &el, &el2, &sp, &k0, &k1, &v0, &v1, &dl,
                     &bits, &pre, &nlo, &nhi, &npos, &items, &scan64, &isb, &seg_of_slot, &cross, &cross2, &tcount, &seg, &lvlbuf, &ncount, &tsum, &tpart, &active, &counters,
-                    &st_cols, &st_subs, &st_out_i, &st_out_e, &st_phi, &segact, &actbuf, &gaps, &pack, &idtab, &idpart, &idcnt,
+                    &st_one, &st_phi, &segact, &actbuf, &gaps, &pack, &idtab, &idpart, &idcnt,
                     &Er, &draws, &randtab, &tgt, &kick, &kickin, &kickcnt})
       b->release();
     if (h_active) (void)hipHostFree(h_active);
     if (h_stage) (void)hipHostFree(h_stage);
     h_list.release();
+    h_one.release();
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     if (evw0) (void)hipEventDestroy(evw0);
@@ -1501,7 +1503,7 @@ int hbt_plan_batch(hbt_subhalo *subs, int64_t nsub, int64_t *total) {
 static int unbind_batch_impl(hbt_ctx *ctx, const hbt_particles *particles, int64_t n_list,
                              hbt_subhalo *subs, const hbt_subhalo *subs_host, int64_t nsub,
                              int64_t *out_index, float *out_energy, int plain, const int64_t *out_cap,
-                             bool planned);
+                             bool planned, bool one = false);
 
 // The host plan of the last batch (memory reused from call to call, so a
 // repeated batch pays no page faults for it).
@@ -1725,17 +1727,19 @@ int hbt_unbind_batch_indexed(hbt_ctx *ctx, const hbt_particles *snapshot, const 
 
 // out_cap: the output capacity the caller planned per subhalo when it exceeds
 // what the lists now need (lists compacted by KickNullParticles), or null.
+// one: the caller has checked the particle types, takes the evaluations from the
+// record it reads back, and waits for the stream itself.
 static int unbind_batch_impl(hbt_ctx *ctx, const hbt_particles *particles, int64_t n_list,
                              hbt_subhalo *subs, const hbt_subhalo *subs_host, int64_t nsub,
                              int64_t *out_index, float *out_energy, int plain, const int64_t *out_cap,
-                             bool planned) {
+                             bool planned, bool one) {
   if (nsub > 0 && (!subs || !subs_host || !out_index || !out_energy))
     return fail(HBT_ERR_INVALID_ARG, "null argument");
   if (nsub == 0) return HBT_OK;
   if (particles->n >= (int64_t)INT32_MAX) return fail(HBT_ERR_UNSUPPORTED, "more than 2^31 particles");
   HIPCHK(hipSetDevice(ctx->device));
   // the type check runs on the device while the host plans the nests
-  const bool check_types = particles->type && particles->n > 0;
+  const bool check_types = !one && particles->type && particles->n > 0;
   if (check_types) {
     RETCHK(ctx->active.ensure(32));
     int *dbad = ctx->active.as<int>() + 6;
@@ -1873,6 +1877,8 @@ static int unbind_batch_impl(hbt_ctx *ctx, const hbt_particles *particles, int64
     HIPCHK(hipGetLastError());
   }
   HIPCHK(hipEventRecord(ctx->ev1, ctx->stream));
+  ctx->last_passes = passes;
+  if (one) return HBT_OK;
   // evaluation count, summed on the device after the timed work
   long long *h_ev = (long long *)(ctx->h_active + 4);
   eval_sum_kernel<<<std::min(grid_for(nsub, ctx->cus), ctx->cus), BLOCK, 0, ctx->stream>>>(
@@ -1883,7 +1889,6 @@ static int unbind_batch_impl(hbt_ctx *ctx, const hbt_particles *particles, int64
   float ms = 0;
   HIPCHK(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
   ctx->last_ms = ms;
-  ctx->last_passes = passes;
   ctx->last_evals = *h_ev;
   return HBT_OK;
 }
@@ -1948,6 +1953,14 @@ int hbt_profile_sorts(hbt_ctx *ctx, double *sort_ms, int64_t *sort_calls, int64_
   return HBT_OK;
 }
 
+// The columns go up and the results come down through pinned memory in one copy
+// each for lists of up to ONE_STAGED particles: nine copies from pageable memory
+// and three back cost 0.07 ms of a call of 300 particles (0.32 ms; 0.25 now) and
+// 0.1 of one of 24,000 (0.79; 0.69) or 90,000 (1.59; 1.49), but of 350,000 only
+// 0.04 of 3.72 ms.  Larger lists copy straight from and to the caller's columns,
+// which bounds the pinned block at 7 MB.
+constexpr int64_t ONE_STAGED = 131072;
+
 int hbt_unbind_one(hbt_ctx *ctx, const hbt_particles *particles, hbt_subhalo *sub,
                    int64_t *out_index, float *out_energy) {
   if (!ctx || !particles || !sub || !out_index || !out_energy)
@@ -1956,48 +1969,75 @@ int hbt_unbind_one(hbt_ctx *ctx, const hbt_particles *particles, hbt_subhalo *su
   if (n < 0 || n > particles->n) return fail(HBT_ERR_INVALID_ARG, "bad count");
   HIPCHK(hipSetDevice(ctx->device));
   const size_t nn = (size_t)std::max<int64_t>(n, 1);
-  RETCHK(ctx->st_cols.ensure(nn * (8 + 7 * 4 + 4)));
-  RETCHK(ctx->st_subs.ensure(sizeof(hbt_subhalo)));
-  RETCHK(ctx->st_out_i.ensure(nn * 8));
-  RETCHK(ctx->st_out_e.ensure(nn * 4));
-  char *base = ctx->st_cols.as<char>();
+  const bool staged = n <= ONE_STAGED;
+  // device and pinned layout: IDs, seven float columns, types | record | list,
+  // energies; the first two go up, the last two come down
+  const size_t cols = (nn * (8 + 7 * 4 + 4) + 255) & ~(size_t)255;
+  const size_t list = cols + ((sizeof(hbt_subhalo) + 255) & ~(size_t)255), end = list + nn * (8 + 4);
+  RETCHK(ctx->st_one.ensure(end));
+  if (staged) RETCHK(ctx->h_one.ensure(end));
+  char *d = ctx->st_one.as<char>(), *h = (char *)ctx->h_one.p;
   hbt_particles D;
   D.n = n;
-  int64_t *did = (int64_t *)base;
-  float *f = (float *)(base + nn * 8);
+  int64_t *did = (int64_t *)d;
+  float *f = (float *)(did + nn);
   D.id = did;
   D.x = f; D.y = f + nn; D.z = f + 2 * nn; D.vx = f + 3 * nn; D.vy = f + 4 * nn; D.vz = f + 5 * nn;
   D.mass = f + 6 * nn;
-  D.type = (int32_t *)(f + 7 * nn);
-  hipStream_t st = ctx->stream;
-  if (n > 0) {
-    HIPCHK(hipMemcpyAsync((void *)D.id, particles->id, n * 8, hipMemcpyHostToDevice, st));
-    const float *src[7] = {particles->x, particles->y, particles->z, particles->vx, particles->vy,
-                           particles->vz, particles->mass};
-    const float *dst[7] = {D.x, D.y, D.z, D.vx, D.vy, D.vz, D.mass};
-    for (int i = 0; i < 7; i++)
-      HIPCHK(hipMemcpyAsync((void *)dst[i], src[i], n * 4, hipMemcpyHostToDevice, st));
-    if (particles->type)
-      HIPCHK(hipMemcpyAsync((void *)D.type, particles->type, n * 4, hipMemcpyHostToDevice, st));
-    else
-      D.type = nullptr;
+  D.type = particles->type && n > 0 ? (int32_t *)(f + 7 * nn) : nullptr;
+  const void *src[9] = {particles->id, particles->x, particles->y, particles->z, particles->vx,
+                        particles->vy, particles->vz, particles->mass, D.type ? particles->type : nullptr};
+  for (int i = 0; i < 8; i++)
+    if (!src[i] && n > 0) return fail(HBT_ERR_INVALID_ARG, "null argument");
+  if (D.type) {
+    int64_t bad = 0;
+    for (int64_t i = 0; i < n; i++) bad += particles->type[i] < 0 || particles->type[i] >= HBT_TYPE_MAX;
+    if (bad) return fail(HBT_ERR_INVALID_ARG, std::to_string(bad) + " particle types outside [0, 6)");
   }
   const hbt_subhalo keep = *sub;
-  hbt_subhalo h = *sub;
-  h.offset = 0;
-  h.parent = -1;
-  h.out_offset = 0;
+  hbt_subhalo r = *sub;
+  r.offset = 0;
+  r.parent = -1;
+  r.out_offset = 0;
   // Subhalo_t::Unbind has no orphan rule (that belongs to RecursiveUnbind)
-  h.nbound_prev = INT64_MAX;
-  HIPCHK(hipMemcpyAsync(ctx->st_subs.p, &h, sizeof(h), hipMemcpyHostToDevice, st));
-  RETCHK(hbt_unbind_batch(ctx, &D, ctx->st_subs.as<hbt_subhalo>(), &h, 1, ctx->st_out_i.as<int64_t>(),
-                          ctx->st_out_e.as<float>(), 1));
-  HIPCHK(hipMemcpyAsync(sub, ctx->st_subs.p, sizeof(hbt_subhalo), hipMemcpyDeviceToHost, st));
-  if (n > 0) {
-    HIPCHK(hipMemcpyAsync(out_index, ctx->st_out_i.p, n * 8, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(out_energy, ctx->st_out_e.p, n * 4, hipMemcpyDeviceToHost, st));
+  r.nbound_prev = INT64_MAX;
+  hipStream_t st = ctx->stream;
+  hbt_subhalo *dsub = (hbt_subhalo *)(d + cols);
+  int64_t *out_i = (int64_t *)(d + list);
+  float *out_e = (float *)(out_i + nn);
+  size_t at = 0;
+  for (int i = 0; i < 9; i++) {
+    const size_t width = i == 0 ? 8 : 4;
+    if (src[i] && n > 0) {
+      if (staged) memcpy(h + at, src[i], n * width);
+      else HIPCHK(hipMemcpyAsync(d + at, src[i], n * width, hipMemcpyHostToDevice, st));
+    }
+    at += nn * width;
   }
-  HIPCHK(hipStreamSynchronize(st));
+  if (staged) {
+    memcpy(h + cols, &r, sizeof r);
+    HIPCHK(hipMemcpyAsync(d, h, list, hipMemcpyHostToDevice, st));
+  } else {
+    HIPCHK(hipMemcpyAsync(dsub, &r, sizeof r, hipMemcpyHostToDevice, st));
+  }
+  ctx->list_index = nullptr;
+  RETCHK(unbind_batch_impl(ctx, &D, n, dsub, &r, 1, out_i, out_e, 1, nullptr, false, true));
+  if (staged) {
+    HIPCHK(hipMemcpyAsync(h + cols, dsub, end - cols, hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    memcpy(sub, h + cols, sizeof *sub);
+    memcpy(out_index, h + list, n * 8);
+    memcpy(out_energy, h + list + nn * 8, n * 4);
+  } else {
+    HIPCHK(hipMemcpyAsync(sub, dsub, sizeof *sub, hipMemcpyDeviceToHost, st));
+    HIPCHK(hipMemcpyAsync(out_index, out_i, n * 8, hipMemcpyDeviceToHost, st));
+    HIPCHK(hipMemcpyAsync(out_energy, out_e, n * 4, hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+  }
+  float ms = 0;
+  HIPCHK(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
+  ctx->last_ms = ms;
+  ctx->last_evals = sub->n_evals;
   sub->offset = keep.offset;
   sub->parent = keep.parent;
   sub->out_offset = keep.out_offset;

@@ -222,3 +222,29 @@ def test_digit_sorts(gpu, softening):
     p["precision"], p["softening"] = abi.HBT_PREC_REPLAY, softening
     cat = synth.Catalogue(cols, subs, p, "digit sorts")
     assert_exact(oracle.unbind_batch(cat, nthreads=8), gpu(p).unbind_batch(cat))
+
+
+def test_single_call_staging(gpu):
+    """the single call sends its columns through pinned memory up to 131,072
+    particles and straight from the caller's arrays above: both give the batched
+    bytes, as do a list of one particle and one without types; a type out of range
+    and a missing column are errors either way"""
+    base = synth.config1(seed=98, n_nfw=120000, n_cont=11073)
+    U = gpu(base.params)
+    for n in (1, 131072, 131073):
+        for types in (True, False):
+            cols = {c: a[:n] for c, a in base.cols.items() if types or c != "type"}
+            sub = base.subs[:1].copy()
+            sub["count"] = n
+            # (a batch of one list unbinds one that had a single particle as an orphan)
+            sub["nbound_prev"] = max(n, 2)
+            rec, idx, e = U.unbind_one(cols, sub)
+            full = dict(cols, type=np.ones(n, np.int32))
+            r, i, f = U.unbind_batch(synth.Catalogue(full, sub, base.params, "one"))
+            assert np.array_equal(i, idx) and np.array_equal(f.view(np.uint32), e.view(np.uint32))
+            assert np.array_equal(r.view(np.uint8), rec.view(np.uint8))
+        bad = dict(base.cols, type=np.full(n, 6, np.int32))
+        with pytest.raises(RuntimeError, match="particle types outside"):
+            U.unbind_one({c: a[:n] for c, a in bad.items()}, sub)
+        with pytest.raises(RuntimeError, match="null argument"):
+            U.unbind_one({c: a[:n] for c, a in base.cols.items() if c != "vx"}, sub)
