@@ -717,32 +717,8 @@ __device__ __forceinline__ int prefix_lower(const u64 *key, int lo, int hi, int 
   return lo;
 }
 
-// The keys of a tile (and one on either side) are staged in LDS, so the
-// binary searches for a node's first and last sources run there; a search
-// goes to device memory only for the part of its range outside the tile (the
-// nodes that extend past it).  KeyWin is that window: sources w_lo..w_hi.
-struct KeyWin {
-  const u64 *sk;   // LDS: keys of sources w_lo..w_hi
-  const u64 *key;  // the segment's keys in device memory
-  int w_lo, w_hi;
-  __device__ __forceinline__ u64 at(int i) const { return (i >= w_lo && i <= w_hi) ? sk[i - w_lo] : key[i]; }
-  // first index in [a, h + 1] whose v-digit prefix is >= p (keys ascending)
-  __device__ __forceinline__ int lower(int a, int h, int v, u64 p) const {
-    const int wa = a > w_lo ? a : w_lo, wh = h < w_hi ? h : w_hi;
-    if (wa > wh) return prefix_lower(key, a, h, v, p);
-    if (key_prefix(sk[wa - w_lo], v) >= p) return wa == a ? a : prefix_lower(key, a, wa - 1, v, p);
-    if (key_prefix(sk[wh - w_lo], v) < p) return wh == h ? h + 1 : prefix_lower(key, wh + 1, h, v, p);
-    int lo = wa + 1, hi = wh - 1;  // the answer is in [wa + 1, wh]
-    while (lo <= hi) {
-      const int m = (lo + hi) >> 1;
-      if (key_prefix(sk[m - w_lo], v) < p) lo = m + 1;
-      else hi = m - 1;
-    }
-    return lo;
-  }
-};
-
-// The same interface over keys that are all in LDS.
+// Keys 0 .. n-1 at sk: sk(i), and the first index in [a, h + 1] whose v-digit
+// prefix is >= p.
 struct KeyAll {
   const u64 *sk;
   __device__ __forceinline__ u64 at(int i) const { return sk[i]; }
@@ -771,33 +747,105 @@ __device__ __forceinline__ bool node_of_pair(const Keys &K, int l, int n, int D,
   return true;
 }
 
+// A tile's keys and those around them, w_lo .. w_hi of the segment's n, in LDS;
+// every pair of the tile has its neighbours' keys there.  `inside` is cleared by
+// a search whose answer lies beyond the window.
+struct KeyWin {
+  const u64 *sk;
+  int w_lo, w_hi, n;
+  mutable bool inside = true;
+  __device__ __forceinline__ u64 at(int i) const { return sk[max(i, w_lo) - w_lo]; }
+  __device__ __forceinline__ int lower(int a, int h, int v, u64 p) const {
+    const int wa = max(a, w_lo), wh = min(h, w_hi);
+    const int i = prefix_lower(sk, wa - w_lo, wh - w_lo, v, p) + w_lo;
+    if ((i == wa && wa > a) || (i > wh && wh < h)) inside = false;
+    return i;
+  }
+};
+
+// A pair's node that reaches beyond the window: both of its ends searched
+// together in device memory, where one step waits on the other.
+__device__ __forceinline__ bool node_of_pair_far(const u64 *sk, int w_lo, int w_hi, const u64 *key, int l, int n,
+                                                 int D, int &lo, int &hi) {
+  auto win = [&](int i) { return sk[i - w_lo]; };
+  const u64 kl = win(l);
+  const int v = key_delta(kl, win(l + 1), D);
+  const int vl = l > 0 ? key_delta(win(l - 1), kl, D) : -1;
+  const int vr = l + 2 < n ? key_delta(win(l + 1), win(l + 2), D) : -1;
+  const u64 p = key_prefix(kl, v);
+  // first source of [a0, a1 + 1] with prefix p, first of [b0, b1 + 1] beyond it
+  int a0 = l, a1 = l - 1, b0 = l + 2, b1 = l + 1;
+  if (vl > v) {
+    if (w_lo == 0 || key_prefix(win(w_lo), v) < p) { a0 = prefix_lower(sk, 0, l - 1 - w_lo, v, p) + w_lo; a1 = a0 - 1; }
+    else { a0 = 0; a1 = w_lo - 1; }
+  }
+  if (vr >= v) {
+    if (w_hi == n - 1 || key_prefix(win(w_hi), v) > p) { b0 = prefix_lower(sk, l + 2 - w_lo, w_hi - w_lo, v, p + 1) + w_lo; b1 = b0 - 1; }
+    else { b0 = w_hi + 1; b1 = n - 1; }
+  }
+  while (a0 <= a1 || b0 <= b1) {
+    const int ma = (a0 + a1) >> 1, mb = (b0 + b1) >> 1;
+    const u64 xa = a0 <= a1 ? key[ma] : 0ull, xb = b0 <= b1 ? key[mb] : 0ull;
+    if (a0 <= a1) { if (key_prefix(xa, v) < p) a0 = ma + 1; else a1 = ma - 1; }
+    if (b0 <= b1) { if (key_prefix(xb, v) < p + 1) b0 = mb + 1; else b1 = mb - 1; }
+  }
+  lo = a0;
+  hi = vr >= v ? b0 - 1 : l + 1;
+  return !(vl > v) || key_delta(lo >= w_lo ? win(lo) : key[lo], kl, D) > v;
+}
+
 // Per pair l of sorted sources: its delta, and the node of which it is the
 // leftmost split.  In a full pass the sorted order also becomes the spatial
-// target order.  One tile of TILE sources, window t0 - 1 .. t0 + TILE + 1.
+// target order.  A tile's keys are in LDS (window t0 - 1 .. t0 + TILE + 1), so
+// the searches for a node's ends run there; the pairs whose nodes reach beyond
+// it, a few per depth, are listed and searched together at the end: among the
+// others, each of a thread's four pairs could wait on two chains of loads: one
+// list of 24,000 took 25 us (19 now), 200,000 subhalos' passes 1.27 ms (0.94).
 __global__ void __launch_bounds__(BLOCK) emit_kernel(Work W, const Tile *__restrict__ tiles, int ntiles,
                                                      int full_copy_sp) {
   __shared__ u64 sk[TILE + 3];
+  __shared__ unsigned short far[TILE];
+  __shared__ int nfar;
   for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
     const Tile tl = tiles[t];
     const Seg &S = W.seg[tl.seg];
     const int n = S.n_src;
     const int cnt = min(TILE, n - tl.start);
     if (cnt <= 0) continue;  // uniform across the block
+    const int64_t b = S.ibase;
     const bool copy_sp = full_copy_sp && !(S.flags & (F_CORR | F_SAMP | F_REFINE));
-    KeyWin K{sk, W.k0 + S.ibase, tl.start > 0 ? tl.start - 1 : 0, min(n - 1, tl.start + TILE + 1)};
-    for (int i = K.w_lo + (int)threadIdx.x; i <= K.w_hi; i += BLOCK) sk[i - K.w_lo] = K.key[i];
+    const int D = S.D, w_lo = tl.start > 0 ? tl.start - 1 : 0, w_hi = min(n - 1, tl.start + TILE + 1);
+    const u64 *key = W.k0 + b;
+    for (int i = w_lo + (int)threadIdx.x; i <= w_hi; i += BLOCK) sk[i - w_lo] = key[i];
+    if (threadIdx.x == 0) nfar = 0;
     __syncthreads();
     for (int i = threadIdx.x; i < cnt; i += BLOCK) {
       const int l = tl.start + i;
-      const int64_t s = S.ibase + l;
+      const int64_t s = b + l;
       if (copy_sp) W.sp[s] = (int)W.v0[s];
+      KeyWin K{sk, w_lo, w_hi, n};
       int lo, hi, v;
-      const bool node = node_of_pair(K, l, n, S.D, lo, hi, v);
+      const bool node = node_of_pair(K, l, n, D, lo, hi, v);
       W.dl[s] = (signed char)v;
+      if (!K.inside) {
+        far[atomicAdd(&nfar, 1)] = (unsigned short)i;
+        continue;
+      }
       W.nlo[s] = node ? lo : -1;
       if (node) {
         W.nhi[s] = hi;
-        atomicOr(&W.bits[S.ibase + lo], 1u << v);
+        atomicOr(&W.bits[b + lo], 1u << v);
+      }
+    }
+    __syncthreads();
+    for (int f = threadIdx.x; f < nfar; f += BLOCK) {
+      const int l = tl.start + far[f];
+      int lo, hi;
+      const bool node = node_of_pair_far(sk, w_lo, w_hi, key, l, n, D, lo, hi);
+      W.nlo[b + l] = node ? lo : -1;
+      if (node) {
+        W.nhi[b + l] = hi;
+        atomicOr(&W.bits[b + lo], 1u << key_delta(sk[l - w_lo], sk[l + 1 - w_lo], D));
       }
     }
     __syncthreads();  // the next tile restages sk
@@ -1244,37 +1292,116 @@ __global__ void __launch_bounds__(BLOCK, 4) items_tile_kernel(Work W, DevParams 
   }
 }
 
-// The nodes of a list (pairs at list[0..ng)) of segment S, deepest first.
-__device__ __forceinline__ void moments_of_list(const Work &W, const Seg &S, const int *list, int ng) {
+// The nodes of a list (pairs at list[0..ng)) of segment S, deepest first.  Where
+// the list fits in LDS its nodes are grouped by depth and their children's places
+// found for all of them at once: one after another down the skips, child after
+// child and depth after depth, the loads of a list's nodes were a chain that took
+// 24 us for one list of 24,000 (14 now).
+constexpr int LISTED = 1024, SONS = 8;  // nodes, children of a node (more only where digits are equal)
+struct ListNodes {
+  int son[SONS][LISTED];
+  unsigned short node[LISTED];  // grouped by depth, deepest first
+  unsigned char sons[LISTED];
+  int count[NLEVEL], first[NLEVEL + 1];
+};
+
+__device__ __forceinline__ void moments_of_list(const Work &W, const Seg &S, const int *list, int ng, ListNodes &L) {
+#pragma clang fp contract(off)
   const int64_t b = S.ibase, ib = 2 * b;
-  for (int v = min(max(S.D, S.Dfull), MAX_DEPTH); v >= 0; v--) {
-    for (int i = threadIdx.x; i < ng; i += BLOCK) {
-      const int64_t s = b + list[i];
-      if (W.dl[s] == v) node_moments(W, ib, W.npos[s]);
+  if (ng > LISTED) {
+    for (int v = min(max(S.D, S.Dfull), MAX_DEPTH); v >= 0; v--) {
+      for (int i = threadIdx.x; i < ng; i += BLOCK) {
+        const int64_t s = b + list[i];
+        if (W.dl[s] == v) node_moments(W, ib, W.npos[s]);
+      }
+      __syncthreads();
+    }
+    return;
+  }
+  constexpr int PER = LISTED / BLOCK;
+  Item *it = W.items + ib;
+  for (int d = threadIdx.x; d < NLEVEL; d += BLOCK) L.count[d] = 0;
+  __syncthreads();
+  int pos[PER], depth[PER], rank[PER];
+#pragma unroll
+  for (int r = 0; r < PER; r++) {
+    const int i = (int)threadIdx.x + BLOCK * r;
+    if (i >= ng) continue;
+    const int64_t s = b + list[i];
+    pos[r] = (int)(W.npos[s] - ib);
+    depth[r] = W.dl[s];
+    rank[r] = atomicAdd(&L.count[depth[r]], 1);
+    const int end = it[pos[r]].ax.y;
+    int c = pos[r] + 1, k = 0;
+    for (; c < end && k < SONS; k++) {
+      L.son[k][i] = c;
+      const int nx = it[c].ax.y;
+      c = nx > c ? nx : end;  // skips always advance
+    }
+    L.sons[i] = (unsigned char)(c < end ? SONS + 1 : k);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int o = 0;
+    for (int d = MAX_DEPTH; d >= 0; d--) { L.first[d] = o; o += L.count[d]; }
+    L.first[NLEVEL] = o;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < PER; r++) {
+    const int i = (int)threadIdx.x + BLOCK * r;
+    if (i < ng) L.node[L.first[depth[r]] + rank[r]] = (unsigned short)i;
+  }
+  __syncthreads();
+  for (int d = MAX_DEPTH; d >= 0; d--) {
+    const int p0 = L.first[d], p1 = d > 0 ? L.first[d - 1] : L.first[NLEVEL];
+    if (p0 == p1) continue;  // uniform
+    for (int p = p0 + (int)threadIdx.x; p < p1; p += BLOCK) {
+      const int i = L.node[p], n = L.sons[i], g = L.son[0][i] - 1;
+      if (n > SONS) {
+        node_moments(W, ib, ib + g);
+        continue;
+      }
+      float4 q[SONS];
+#pragma unroll
+      for (int k = 0; k < SONS; k++) q[k] = it[L.son[k < n ? k : 0][i]].pm;
+      double mass = 0., cx = 0., cy = 0., cz = 0.;  // as sum_children
+#pragma unroll
+      for (int k = 0; k < SONS; k++)
+        if (k < n) {
+          const double m = q[k].w;
+          mass += m;
+          cx += (double)q[k].x * m;
+          cy += (double)q[k].y * m;
+          cz += (double)q[k].z * m;
+        }
+      it[g].pm = make_float4((float)(cx / mass), (float)(cy / mass), (float)(cz / mass), (float)mass);
     }
     __syncthreads();
   }
 }
 
 __global__ void __launch_bounds__(BLOCK) moments_super_kernel(Work W, const Tile *__restrict__ tiles, int ntiles) {
+  __shared__ ListNodes L;
   for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
     const Tile tl = tiles[t];
     if (tl.start % SUPER != 0) continue;  // a super-tile's first tile stands for it
     const int ng = W.tcount[t];
     if (ng == 0) continue;  // uniform
     const Seg &S = W.seg[tl.seg];
-    moments_of_list(W, S, W.cross + S.ibase + tl.start, ng);
+    moments_of_list(W, S, W.cross + S.ibase + tl.start, ng, L);
   }
 }
 
 __global__ void __launch_bounds__(BLOCK) moments_cross_kernel(Work W, const Tile *__restrict__ tiles, int ntiles) {
+  __shared__ ListNodes L;
   for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
     const Tile tl = tiles[t];
     if (tl.start != 0) continue;  // the segment's first tile stands for it
     const int ng = W.ncount[NC_CROSS * W.nseg + tl.seg];
     if (ng == 0) continue;  // uniform
     const Seg &S = W.seg[tl.seg];
-    moments_of_list(W, S, W.cross2 + S.ibase, ng);
+    moments_of_list(W, S, W.cross2 + S.ibase, ng, L);
   }
 }
 
