@@ -2485,19 +2485,6 @@ __global__ void __launch_bounds__(RUN_THREADS, 8) energy_sort_kernel(Work W, con
   });
 }
 
-// The merged order into Elist, for segments that more than `run` elements were
-// sorted of.
-__global__ void __launch_bounds__(BLOCK) energy_writeback_kernel(Work W, int run) {
-  SLOT_LOOP(s, W) {
-    int k;
-    int l = seg_lane_local(W, s, k);
-    if (l < 0) continue;
-    const Seg &S = W.seg[k];
-    if (l >= S.nsort || S.nsort <= run) continue;
-    W.el[S.ibase + S.sort_lo + l] = (int)W.v0[s];
-  }
-}
-
 // ---------------------------------------------------------------------------
 // FAST frame sums, tile-parallel: every tile of an active segment sums its part
 // of the bound block in FP64 (mass, m*v, m*x relative to the periodic origin,
@@ -2737,32 +2724,29 @@ __global__ void frames_serial_kernel(Work W, DevParams P) {
 // Outputs for segments that finished in this pass, early exits and orphans.
 
 // Output list and energies of entry l.  li: Elist's entry at l, for l < ulen.
-__device__ __forceinline__ void output_entry(const Work &W, const Seg &S, int l, int li) {
-  const int64_t o = S.out_off + l;
-  if ((S.flags & F_CONV) && !(S.flags & F_ORPHAN)) {
-    if (l >= S.ulen) li = l;
-    W.out_index[o] = W.gidx[S.ibase + li];
-    W.out_energy[o] = l < S.ulen ? W.E[S.ibase + li] : __builtin_nanf("");
-  } else {
-    // disrupted, early, orphan: the list keeps its order -- an orphan's
-    // own list as it came in, even when a shuffled copy of it was unbound
-    // (:434-446)
-    const bool orig = (S.flags & F_ORPHAN) && (S.flags & F_SHUF) && l < S.count;
-    W.out_index[o] = orig ? own_entry(W, S, l) : W.gidx[S.ibase + l];
-    W.out_energy[o] = __builtin_nanf("");
-  }
+// Split in what is read and what is written, so that a thread's entries load
+// together.
+struct OutEntry {
+  int64_t index;
+  float energy;
+};
+template <class Energy>
+__device__ __forceinline__ OutEntry output_entry(const Work &W, const Seg &S, int l, int li, Energy energy) {
+  const bool sorted = (S.flags & F_CONV) && !(S.flags & F_ORPHAN) && l < S.ulen;
+  OutEntry e;
+  e.index = W.gidx[S.ibase + (sorted ? li : l)];
+  e.energy = sorted ? energy() : __builtin_nanf("");
+  // disrupted, early, orphan: the list keeps its order -- an orphan's own list
+  // as it came in, even when a shuffled copy of it was unbound (:434-446)
+  if ((S.flags & F_ORPHAN) && (S.flags & F_SHUF) && l < S.count) e.index = own_entry(W, S, l);
+  return e;
 }
-
-// Lists of the segments that finished in the pass.
-__global__ void __launch_bounds__(BLOCK) output_list_kernel(Work W) {
-  SLOT_LOOP(s, W) {
-    int k;
-    int l = seg_lane_local(W, s, k);
-    if (l < 0) continue;
-    const Seg &S = W.seg[k];
-    if (!(S.flags & F_FINAL) || l >= S.len) continue;
-    output_entry(W, S, l, W.el[s]);
-  }
+__device__ __forceinline__ OutEntry output_entry(const Work &W, const Seg &S, int l, int li) {
+  return output_entry(W, S, l, li, [&]() { return W.E[S.ibase + li]; });
+}
+__device__ __forceinline__ void write_entry(const Work &W, const Seg &S, int l, const OutEntry &e) {
+  W.out_index[S.out_off + l] = e.index;
+  W.out_energy[S.out_off + l] = e.energy;
 }
 
 // Writes the record of a segment that finished, from its sums over the bound
@@ -2888,7 +2872,7 @@ __global__ void __launch_bounds__(BLOCK) output_early_kernel(Work W, DevParams P
     Seg &S = W.seg[k];
     if (!(S.flags & F_EARLY)) continue;  // uniform across the wave
     const int lane = threadIdx.x & (WAVE - 1);
-    for (int l = lane; l < S.len; l += WAVE) output_entry(W, S, l, 0);  // (none of them converged)
+    for (int l = lane; l < S.len; l += WAVE) write_entry(W, S, l, output_entry(W, S, l, 0));  // (none of them converged)
     if (lane == 0) record_serial(W, P, S);
   }
 }
@@ -2917,6 +2901,54 @@ __device__ __forceinline__ void record_accum(const Work &W, const DevParams &P, 
     const bool hit = q == ty;
     v[6 + q] += hit ? 1.0 : 0.0;
     v[12 + q] += hit ? (double)m : 0.0;
+  }
+}
+
+// After the energy sort, a workgroup per tile: the merged order into Elist where
+// more than `run` elements were sorted (shorter ones are there), and the lists of
+// the segments that finished.  keyed: the merged keys hold the entries' energies,
+// which are then not gathered.  As two launches over the slots, a thread's entries
+// one after another, 1.24 ms of 200,000 subhalos' passes, 0.76 now; with the
+// record sums in the same launch, whose registers leave five waves per SIMD, both
+// took 1.6 together (1.4 apart).
+__global__ void __launch_bounds__(BLOCK)
+output_tile_kernel(Work W, const Tile *__restrict__ tiles, int ntiles, int run, bool keyed) {
+  for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    const Tile tl = tiles[t];
+    const Seg &S = W.seg[tl.seg];
+    const bool fin = (S.flags & F_FINAL) != 0;
+    const int lo = S.sort_lo, nsort = S.nsort;
+    const bool merged = nsort > run;
+    const int end = fin ? S.len : merged ? lo + nsort : 0;
+    const int cnt = min(TILE, end - tl.start);
+    if (cnt <= 0) continue;  // uniform
+    const int64_t b = S.ibase;
+    int li[ITEMS];
+    OutEntry e[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++) {
+      const int i = (int)threadIdx.x + BLOCK * r, l = tl.start + i;
+      const bool in = merged && l >= lo && l < lo + nsort;
+      li[r] = i >= cnt ? 0 : in ? (int)W.v0[b + l - lo] : W.el[b + l];
+    }
+    if (fin) {
+#pragma unroll
+      for (int r = 0; r < ITEMS; r++) {
+        const int i = (int)threadIdx.x + BLOCK * r, l = tl.start + i;
+        const bool key = keyed && merged && l >= lo && l < lo + nsort;
+        if (i < cnt)
+          e[r] = output_entry(W, S, l, li[r], [&]() {
+            return key ? ord2f((u32)(W.k0[b + l - lo] >> 31)) : W.E[b + li[r]];
+          });
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++) {
+      const int i = (int)threadIdx.x + BLOCK * r, l = tl.start + i;
+      if (i >= cnt) continue;
+      if (merged && l >= lo && l < lo + nsort) W.el[b + l] = li[r];
+      if (fin) write_entry(W, S, l, e[r]);
+    }
   }
 }
 
@@ -3189,7 +3221,7 @@ __device__ __forceinline__ void post_one(Work &W, const DevParams &P, const Tile
   for (int l = id; l < n; l += T) W.el[b + l] = L.el[l];
   if constexpr ((STAGE & POST_SORT) != 0) {
     if (S.flags & F_FINAL) {  // uniform across the team
-      for (int l = id; l < S.len; l += T) output_entry(W, S, l, l < n ? L.el[l] : l < S.ulen ? W.el[b + l] : 0);
+      for (int l = id; l < S.len; l += T) write_entry(W, S, l, output_entry(W, S, l, l < n ? L.el[l] : l < S.ulen ? W.el[b + l] : 0));
       if constexpr ((STAGE & POST_RECORD) != 0) {
         const bool conv = (S.flags & F_CONV) != 0;
         const int nb = S.nbound;

@@ -922,14 +922,11 @@ struct Runner {
     }
     if (nt_multi > 0) {
       // energy sort of the removed block, and of the bound block on convergence
-      Work M = multi();
       RETCHK(sort_begin());
       energy_sort_kernel<<<tile_grid(nt_multi, 1), RUN_THREADS, 0, c->stream>>>(W, tl_cur, nt_multi);
       merge_sorted(count_row(NC_SORT), nt_multi, RUN);
       RETCHK(sort_end(count_row(NC_SORT), TILE, RUN));
-      if (max_n > RUN) energy_writeback_kernel<<<gmulti(), BLOCK, 0, c->stream>>>(M, RUN);
-      output_list_kernel<<<gmulti(), BLOCK, 0, c->stream>>>(M);
-      if (!P.replay) output_records(W.nmulti, nt_multi);
+      output_tiles(W.nmulti, nt_multi, RUN, true);
     }
     if (P.replay) output_record_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P);
     count_active_kernel<<<std::min(gseg, 64), BLOCK, 0, c->stream>>>(W);
@@ -981,9 +978,11 @@ struct Runner {
     frames_combine_kernel<<<gmseg(), BLOCK, 0, c->stream>>>(W, P, ft_cur, part, gpart);
   }
 
-  // The records of the finished ones among the first nseg segments, which hold
-  // the first nt tiles.
-  void output_records(int nseg, int nt) {
+  // The merged energy order, the lists and (FAST) the records of the finished
+  // ones among the first nseg segments, which hold the first nt tiles.
+  void output_tiles(int nseg, int nt, int run, bool keyed) {
+    output_tile_kernel<<<tile_grid(nt), BLOCK, 0, c->stream>>>(W, tl_cur, nt, run, keyed);
+    if (P.replay) return;
     double *part = c->tpart.as<double>();
     output_partial_kernel<<<tile_grid(nt), BLOCK, 0, c->stream>>>(W, P, tl_cur, nt, part);
     output_combine_kernel<<<grid_for((int64_t)nseg * WAVE, c->cus), BLOCK, 0, c->stream>>>(W, P, nseg, ft_cur, part);
@@ -1002,11 +1001,9 @@ struct Runner {
     launch_walk(false);
     refine_keys_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
     RETCHK(sort_pairs(count_row(NC_SORT), nt_cur));
-    energy_writeback_kernel<<<gs, BLOCK, 0, c->stream>>>(W, 0);
     refine_done_kernel<<<gseg, BLOCK, 0, c->stream>>>(W);
-    output_list_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
+    output_tiles(W.nseg, nt_cur, 0, false);
     if (P.replay) output_record_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P);
-    else output_records(W.nseg, nt_cur);
     HIPCHK(hipGetLastError());
     return HBT_OK;
   }
