@@ -2492,12 +2492,11 @@ __global__ void __launch_bounds__(RUN_THREADS, 8) energy_sort_kernel(Work W, con
 // result does not depend on scheduling.
 constexpr int FRAME_SUMS = 7;
 
-// The frame sums of bound entry li: mass, momentum, mass-weighted position
+// The frame sums of a bound entry at q, w: mass, momentum, mass-weighted position
 // (relative to the most-bound entry o when periodic).
-__device__ __forceinline__ void frame_accum(const Work &W, const DevParams &P, int64_t b, int li,
-                                            const double o[3], double v[FRAME_SUMS]) {
+__device__ __forceinline__ void frame_accum(const DevParams &P, const float4 &q, const float4 &w, const double o[3],
+                                            double v[FRAME_SUMS]) {
 #pragma clang fp contract(off)
-  const float4 q = W.pos[b + li], w = W.vel[b + li];
   const float m = q.w;
   v[0] += m;
   v[1] += w.x * m; v[2] += w.y * m; v[3] += w.z * m;
@@ -2551,6 +2550,12 @@ __global__ void __launch_bounds__(BLOCK) part_finish_kernel(Work W, DevParams P,
     const double o[3] = {p0.x, p0.y, p0.z};
     const int bound = min(TILE, S.nbound - tl.start);
     double v[FRAME_SUMS] = {0, 0, 0, 0, 0, 0, 0};
+    float4 pos[ITEMS], vel[ITEMS];  // before the stores, so that they load together
+    if (SUMS) {
+#pragma unroll
+      for (int r = 0; r < ITEMS; r++)
+        if ((int)threadIdx.x + BLOCK * r < bound) { pos[r] = W.pos[b + li[r]]; vel[r] = W.vel[b + li[r]]; }
+    }
 #pragma unroll
     for (int r = 0; r < ITEMS; r++) {
       const int i = (int)threadIdx.x + BLOCK * r;
@@ -2558,7 +2563,7 @@ __global__ void __launch_bounds__(BLOCK) part_finish_kernel(Work W, DevParams P,
       const int w = i / WAVE;
       if ((mask[w] >> lane) & 1ull) sp_out[b + first[w] + __popcll(mask[w] & ((1ull << lane) - 1ull))] = q[r];
       W.el[s0 + i] = li[r];
-      if (SUMS && i < bound) frame_accum(W, P, b, li[r], o, v);
+      if (SUMS && i < bound) frame_accum(P, pos[r], vel[r], o, v);
     }
     if (SUMS) {
       for (int c = 0; c < FRAME_SUMS; c++) {
@@ -3173,7 +3178,9 @@ __device__ __forceinline__ void post_one(Work &W, const DevParams &P, const Tile
         const double o[3] = {p0.x, p0.y, p0.z};
         double v[FRAME_SUMS];
         tile_sums<TM, FRAME_SUMS>(nb, v, L.sums,
-                                  [&](int i, double (&x)[FRAME_SUMS]) { frame_accum(W, P, b, L.el[i], o, x); });
+                                  [&](int i, double (&x)[FRAME_SUMS]) {
+                                    frame_accum(P, W.pos[b + L.el[i]], W.vel[b + L.el[i]], o, x);
+                                  });
         if (id == 0) frame_update(W, P, S, l0, v[0], v[1], v[2], v[3], v[4], v[5], v[6]);
       }
     }
