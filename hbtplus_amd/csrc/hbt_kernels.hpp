@@ -2,8 +2,9 @@
 //
 // One pass of the reference's Unbind loop (src/subhalo_unbind.cpp:310-422)
 // runs for every active segment (subhalo) of a level at once:
-//   pass_setup        full pass over Elist[0,Nlast) or correction pass over the
-//                     freshly removed block Elist[Nbound,Nlast) (:312-356)
+//   begin_pass        full pass over Elist[0,Nlast) or correction pass over the
+//                     freshly removed block Elist[Nbound,Nlast) (:312-356), set
+//                     up at the end of the pass before
 //   tree_one          a segment of one tile: its whole tree in one launch
 //   bbox / keys_sort / (merge levels) / emit / items_tile / moments_super, _cross
 //                     the others: root cube and per-particle octant digits
@@ -26,7 +27,7 @@ namespace hbt {
 // One tree item (leaf or node) in DFS pre-order, one 32-byte record: the
 // walk reads both halves of an item at once.
 // Rows of Work::ncount, each written by the kernel that decides the count:
-// sources of the tree (pass setup), the energy sort (frames), the tree's nodes
+// sources of the tree (begin_pass), the energy sort (frames), the tree's nodes
 // that span super-tiles (bbox, items).
 enum { NC_SRC = 0, NC_SORT = 1, NC_CROSS = 2, NC_ROWS = 3 };
 
@@ -47,7 +48,7 @@ struct Work {
   // wave-sized chunks of the segments still active (nact = 64 * chunks)
   const int *act_chunk;
   int64_t nact;
-  int *segact;               // [nseg] nonzero: the segment stays active after the pass (its Nlast)
+  int *segact;               // [nseg] nonzero: the segment stays active after the pass
   const int *seg_of_slot;
   const int64_t *ibase;
   int *ncount;               // [NC_ROWS][nseg] element counts of the pass's scans and sorts
@@ -222,9 +223,48 @@ __device__ __forceinline__ void init_segment(const Work &W, const DevParams &P, 
   W.ncount[NC_SRC * W.nseg + k] = S.draw_off >= 0 ? S.ulen - 1 : 0;
 }
 
+// Setup of a segment's next pass: full over Elist[0, Nbound), or a correction
+// over the block just removed.
+__device__ __forceinline__ void begin_pass(const Work &W, const DevParams &P, Seg &S, int k) {
+  S.flags &= ~(F_FINAL | F_SAMP);
+  S.mf = 1.f;
+  S.n_src = 0; S.n_tgt = 0; S.src_lo = 0; S.nsort = 0; S.sort_lo = 0; S.n_items = 0;
+  S.K = 0; S.nP = 0; S.nG = 0;
+  if (S.flags & F_ACTIVE) {
+    S.iter++;
+    if (S.flags & F_CORR) {
+      // RelativeVelocity(OldRefPos, OldRefVel, RefPos, RefVel), dK (:314-316)
+      rel_vel(P, S.old_pos[0], S.old_pos[1], S.old_pos[2], S.old_vel[0], S.old_vel[1],
+              S.old_vel[2], S.ref_pos, S.ref_vel, S.rvd);
+      S.dK = (float)(0.5 * (double)vnorm_f(S.rvd));
+      S.src_lo = S.nbound;
+      S.n_src = S.nlast - S.nbound;
+      S.n_tgt = S.nbound;
+      S.nlast = S.nbound;  // Nlast=Nbound after the correction loop (:329)
+    } else {
+      S.nlast = S.nbound;
+      S.src_lo = 0;
+      S.n_src = S.nlast;
+      S.n_tgt = S.nlast;
+      if (P.max_sample > 0 && S.nlast > P.max_sample) {
+        // sampled tree: the first MaxSampleSize entries with their masses
+        // scaled by Nlast / MaxSampleSize (float / long -> float, :334-339)
+        S.n_src = P.max_sample;
+        S.mf = (float)S.nlast / (float)P.max_sample;
+        S.flags |= F_SAMP;
+      }
+    }
+    S.evals += S.n_tgt;
+    S.nsort = S.n_src;
+    for (int j = 0; j < 3; j++) { S.bmin[j] = 0xffffffffu; S.bmax[j] = 0u; }
+  }
+  W.ncount[NC_SRC * W.nseg + k] = S.n_src;
+  W.ncount[NC_SORT * W.nseg + k] = 0;
+}
+
 __device__ __forceinline__ void clear_level_counts(const Work &W) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    W.active[3] = 0;    // refinements pending in the level
+    for (int i = 0; i < 4; i++) W.active[i] = 0;
     W.counters[4] = 0;  // evaluations, summed after the last level
   }
 }
@@ -235,8 +275,9 @@ __global__ void seg_init_kernel(Work W, DevParams P) {
   SEG_LOOP(k, W) init_segment(W, P, W.seg[k], k);
 }
 
-// The level's segment records: zero, then the host's fixed fields.  begin: the
-// lists are the segments' own, and their unbinding starts here too.
+// The level's segment records: zero, then the host's fixed fields.  begin: 1, the
+// lists are the segments' own, and their unbinding starts here too; 2, and
+// none is shuffled: their first pass also.
 __global__ void __launch_bounds__(BLOCK) seg_expand_kernel(Work W, DevParams P, const SegIn *in, int begin) {
   if (begin) clear_level_counts(W);
   SEG_LOOP(k, W) {
@@ -257,7 +298,9 @@ __global__ void __launch_bounds__(BLOCK) seg_expand_kernel(Work W, DevParams P, 
     if (begin) {
       S.len = S.count;
       init_segment(W, P, S, k);
+      if (begin == 2) begin_pass(W, P, S, k);
     }
+    W.segact[k] = 1;
     W.seg[k] = S;
   }
 }
@@ -441,50 +484,10 @@ __global__ void __launch_bounds__(BLOCK) prelude_sp_kernel(Work W) {
   }
 }
 
-// ---------------------------------------------------------------------------
-// Pass: setup
-
-__global__ void pass_setup_kernel(Work W, DevParams P) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) { W.active[0] = 0; W.active[1] = 0; W.active[2] = 0; }
-  SEG_LOOP(k, W) {
-    Seg &S = W.seg[k];
-    W.segact[k] = 0;
-    S.flags &= ~(F_FINAL | F_SAMP);
-    S.mf = 1.f;
-    S.n_src = 0; S.n_tgt = 0; S.src_lo = 0; S.nsort = 0; S.sort_lo = 0; S.n_items = 0;
-    S.K = 0; S.nP = 0; S.nG = 0;
-    if (!(S.flags & F_ACTIVE)) continue;
-    S.iter++;
-    if (S.flags & F_CORR) {
-      // RelativeVelocity(OldRefPos, OldRefVel, RefPos, RefVel), dK (:314-316)
-      rel_vel(P, S.old_pos[0], S.old_pos[1], S.old_pos[2], S.old_vel[0], S.old_vel[1],
-              S.old_vel[2], S.ref_pos, S.ref_vel, S.rvd);
-      S.dK = (float)(0.5 * (double)vnorm_f(S.rvd));
-      S.src_lo = S.nbound;
-      S.n_src = S.nlast - S.nbound;
-      S.n_tgt = S.nbound;
-      S.nlast = S.nbound;  // Nlast=Nbound after the correction loop (:329)
-    } else {
-      S.nlast = S.nbound;
-      S.src_lo = 0;
-      S.n_src = S.nlast;
-      S.n_tgt = S.nlast;
-      if (P.max_sample > 0 && S.nlast > P.max_sample) {
-        // sampled tree: the first MaxSampleSize entries with their masses
-        // scaled by Nlast / MaxSampleSize (float / long -> float, :334-339)
-        S.n_src = P.max_sample;
-        S.mf = (float)S.nlast / (float)P.max_sample;
-        S.flags |= F_SAMP;
-      }
-    }
-    S.evals += S.n_tgt;
-    S.nsort = S.n_src;
-    for (int j = 0; j < 3; j++) { S.bmin[j] = 0xffffffffu; S.bmax[j] = 0u; }
-  }
-  SEG_LOOP(k, W) {
-    W.ncount[NC_SRC * W.nseg + k] = W.seg[k].n_src;
-    W.ncount[NC_SORT * W.nseg + k] = 0;
-  }
+// First pass of a level whose lists were shuffled or hold nested tails (else
+// seg_expand_kernel sets it up; pass_end_kernel sets up the later ones).
+__global__ void pass_begin_kernel(Work W, DevParams P) {
+  SEG_LOOP(k, W) begin_pass(W, P, W.seg[k], k);
 }
 
 // ---------------------------------------------------------------------------
@@ -2627,7 +2630,6 @@ __device__ void frame_update(Work &W, const DevParams &P, Seg &S, int l0, double
   } else {
     S.sort_lo = nb;
     S.nsort = S.nlast - nb;
-    W.segact[&S - W.seg] = max(1, S.nlast);
   }
   W.ncount[NC_SORT * W.nseg + (int)(&S - W.seg)] = S.nsort;
 }
@@ -3259,33 +3261,50 @@ __global__ void __launch_bounds__(BLOCK, 4) post_one_kernel(Work W, DevParams P,
   for (int t = t0 + (int)blockIdx.x; t < ntiles; t += gridDim.x) post_one<TM, STAGE>(W, P, tiles[t], sp_out, L);
 }
 
-// Segments active after the pass, and the largest Nlast among them: by blocks,
-// since the atomics on two addresses are served one after another.  The last
-// block writes them where the host reads them, which saves the copy that
-// followed.
-__global__ void __launch_bounds__(BLOCK) count_active_kernel(Work W) {
+// The end of a pass: the segments still active and the largest Nlast among them,
+// and the setup of their next pass.  A segment that was not active before is not
+// read.  Counted by blocks, since atomics on one address are served one after
+// another; the last block writes the counts where the host reads them and clears
+// them.  Setup, count and copy as three launches took 14 us of a 300-particle
+// list's pass of 60.
+__global__ void __launch_bounds__(BLOCK) pass_end_kernel(Work W, DevParams P) {
+  __shared__ int sh[2][BLOCK / WAVE];
   int cnt = 0, most = 0;
   SEG_LOOP(k, W) {
-    const int a = W.segact[k];
-    cnt += a > 0 ? 1 : 0;
-    most = max(most, a);
+    if (W.segact[k] == 0) continue;
+    Seg &S = W.seg[k];
+    const bool active = (S.flags & F_ACTIVE) != 0;
+    if (active) {
+      cnt++;
+      most = max(most, S.nlast);
+    }
+    W.segact[k] = active ? 1 : 0;
+    begin_pass(W, P, S, k);
   }
   for (int d = WAVE / 2; d > 0; d >>= 1) {
     cnt += __shfl_xor(cnt, d, WAVE);
     most = max(most, __shfl_xor(most, d, WAVE));
   }
-  if ((threadIdx.x & (WAVE - 1)) == 0 && cnt) {
+  if ((threadIdx.x & (WAVE - 1)) == 0) { sh[0][threadIdx.x / WAVE] = cnt; sh[1][threadIdx.x / WAVE] = most; }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int w = 1; w < BLOCK / WAVE; w++) {
+    cnt += sh[0][w];
+    most = max(most, sh[1][w]);
+  }
+  if (cnt) {
     atomicAdd(&W.active[0], cnt);
     atomicMax(&W.active[1], most);  // bounds every count of the next pass
   }
   __threadfence();
-  __syncthreads();
-  if (threadIdx.x == 0 && atomicAdd(&W.active[2], 1) == (int)gridDim.x - 1) {
-    __threadfence();
-    for (int i = 0; i < 4; i++)
-      if (i != 2) W.host_active[i] = __hip_atomic_load(&W.active[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __threadfence_system();
+  if (atomicAdd(&W.active[2], 1) != (int)gridDim.x - 1) return;
+  __threadfence();
+  for (int i = 0; i < 4; i++) {
+    if (i == 2) continue;
+    W.host_active[i] = __hip_atomic_load(&W.active[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
+  for (int i = 0; i < 3; i++) __hip_atomic_store(&W.active[i], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __threadfence_system();
 }
 
 // ---------------------------------------------------------------------------

@@ -898,7 +898,6 @@ struct Runner {
   }
 
   int pass() {
-    pass_setup_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P);
     if (P.max_sample > 0) sample_flags_kernel<<<gs, BLOCK, 0, c->stream>>>(W);
     RETCHK(build_tree(true));
     if (c->prof_mode == 1) HIPCHK(hipEventRecord(c->evw0, c->stream));
@@ -929,7 +928,7 @@ struct Runner {
       output_tiles(W.nmulti, nt_multi, RUN, true);
     }
     if (P.replay) output_record_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P);
-    count_active_kernel<<<std::min(gseg, 64), BLOCK, 0, c->stream>>>(W);
+    pass_end_kernel<<<std::min(gseg, c->cus), BLOCK, 0, c->stream>>>(W, P);
     HIPCHK(hipGetLastError());
     return HBT_OK;
   }
@@ -1150,7 +1149,8 @@ int run_level(hbt_ctx *c, Level &L, const hbt_particles *parts, hbt_subhalo *sub
   const int gsb = (int)std::min<int64_t>(nseg, (int64_t)c->cus * 8);
   R.gblk = gsb;
   const bool flat = L.child_list.empty();
-  seg_expand_kernel<<<R.gseg, BLOCK, 0, c->stream>>>(R.W, R.P, c->segin.as<SegIn>(), flat ? 1 : 0);
+  seg_expand_kernel<<<R.gseg, BLOCK, 0, c->stream>>>(R.W, R.P, c->segin.as<SegIn>(),
+                                                    !flat ? 0 : L.ndraws > 0 ? 1 : 2);
   // segment bases are multiples of WAVE (capacities are rounded up to it)
   seg_of_chunk_kernel<<<R.gs, BLOCK, 0, c->stream>>>((int)nseg, R.W.ibase, L.nslots, c->seg_of_slot.as<int>());
   if (!flat) {
@@ -1166,6 +1166,7 @@ int run_level(hbt_ctx *c, Level &L, const hbt_particles *parts, hbt_subhalo *sub
     gather_kernel<<<R.gs, BLOCK, 0, c->stream>>>(R.W, 3);
   }
   RETCHK(R.prelude());
+  if (!flat || L.ndraws > 0) pass_begin_kernel<<<R.gseg, BLOCK, 0, c->stream>>>(R.W, R.P);
   output_early_kernel<<<grid_for(nseg * WAVE, c->cus), BLOCK, 0, c->stream>>>(R.W, R.P);
   HIPCHK(hipGetLastError());
   if (getenv("HBT_PASS_TIMES") && atoi(getenv("HBT_PASS_TIMES"))) {
