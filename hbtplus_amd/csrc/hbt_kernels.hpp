@@ -653,7 +653,7 @@ __device__ __forceinline__ void for_runs(const Tile *__restrict__ tiles, int nti
 // run.  In one kernel the keys reach memory sorted: digits and sort in kernels
 // of their own wrote and read 12 bytes per source in between.
 __global__ void __launch_bounds__(RUN_THREADS, 8) keys_sort_kernel(Work W, DevParams P, const Tile *__restrict__ tiles,
-                                                                   int ntiles) {
+                                                                   int ntiles, bool ranked) {
   __shared__ u64 sk[RUN];
   __shared__ u32 sv[RUN];
   __shared__ RootCube cube;
@@ -682,7 +682,7 @@ __global__ void __launch_bounds__(RUN_THREADS, 8) keys_sort_kernel(Work W, DevPa
     for (int r = 0; r < ITEMS; r++)
       k[r] = v[r] != ~0u ? octant_key(cube.center, cube.Len, cube.D, q[r].x, q[r].y, q[r].z) : ~0ull;
     sort_tile_spare<RUN_THREADS>(k, v, cnt, 3 * (MAX_DEPTH - cube.D), sk, sv);
-    const bool odd = (merge_levels(n, RUN) & 1) != 0;
+    const bool odd = (merge_levels(n, RUN, ranked) & 1) != 0;
     u64 *kout = odd ? W.k1 : W.k0;
     u32 *vout = odd ? W.v1 : W.v0;
     for (int i = threadIdx.x; i < cnt; i += RUN_THREADS) {
@@ -2102,12 +2102,12 @@ __global__ void __launch_bounds__(PARTS *WAVE) walk_split_kernel(Work W, DevPara
 
 // Instrumented passes: the elements a segmented sort ordered (counters[8])
 // and the elements times the merge levels each needed (counters[9]).
-__global__ void sort_count_kernel(Work W, const int *n, int above, int run) {
+__global__ void sort_count_kernel(Work W, const int *n, int above, int run, bool ranked) {
   unsigned long long e = 0, el = 0;
   SEG_LOOP(k, W) {
     const int c = W.seg[k].cap > above && n[k] > 0 ? n[k] : 0;
     e += (unsigned long long)c;
-    el += (unsigned long long)c * (unsigned long long)merge_levels(c, run);
+    el += (unsigned long long)c * (unsigned long long)merge_levels(c, run, ranked);
   }
   e = wave_reduce_sum(e);
   el = wave_reduce_sum(el);
@@ -2453,7 +2453,7 @@ __device__ __forceinline__ u64 energy_key(u64 w, int first) {
 // Energies of Elist[sort_lo, sort_lo + nsort), sorted by runs: into Elist where
 // that is all, else into the buffer from which the merge levels end in (k0, v0).
 __global__ void __launch_bounds__(RUN_THREADS, 8) energy_sort_kernel(Work W, const Tile *__restrict__ tiles,
-                                                                     int ntiles) {
+                                                                     int ntiles, bool ranked) {
   constexpr int BITS = log2_of(RUN);
   __shared__ u64 sk[RUN];
   __shared__ int sv[RUN];
@@ -2471,7 +2471,7 @@ __global__ void __launch_bounds__(RUN_THREADS, 8) energy_sort_kernel(Work W, con
       x[r] = e < cnt ? energy_word<BITS>(first + e, first, nb, W.E[b + li]) : ~0ull;
     }
     sort_tile_words<RUN_THREADS>(x, cnt, sk);
-    const int m = merge_levels(n, RUN);
+    const int m = merge_levels(n, RUN, ranked);
     u64 *kout = (m & 1) != 0 ? W.k1 : W.k0;
     u32 *vout = (m & 1) != 0 ? W.v1 : W.v0;
     for (int i = threadIdx.x; i < cnt; i += RUN_THREADS) {

