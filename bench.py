@@ -223,7 +223,7 @@ def sort_roofline(sort_t, sort_c, ms_per_step):
     s = sort_t["sort_ms"] / 1e3
     achieved = alg / s / 1e9 if s > 0 else 0.0
     return dict(bound="hbm", achieved=round(achieved, 1), peak=PEAK_HBM_GBS, unit="GB/s",
-                frac=round(achieved / PEAK_HBM_GBS, 4), kernels="tile_sort_kernel + keys_sort_kernel + merge_pass_kernel",
+                frac=round(achieved / PEAK_HBM_GBS, 4), kernels="keys_sort_kernel + energy_sort_kernel + merge_pass_kernel",
                 sorts_per_step=sort_t["sort_calls"], ms_per_step=round(sort_t["sort_ms"], 3),
                 elements_per_step=sort_c["elements"], element_levels_per_step=sort_c["element_levels"],
                 algorithmic_bytes_per_step=int(alg), share_of_step=round(sort_t["sort_ms"] / ms_per_step, 3))

@@ -495,8 +495,8 @@ __global__ void pass_begin_kernel(Work W, DevParams P) {
 // or a workgroup each, everything between the sources and the finished items in
 // LDS (tree_one_kernel).  Larger ones go through their tiles: box, digits and
 // tile sort, merge levels, nodes, pre-order positions, items and moments.  The
-// trees of 200,000 subhalos' passes take 9.1 ms this way (5.5 of it the larger
-// segments'), 50,000 small ones' 6.1; with every stage a launch over all
+// trees of 200,000 subhalos' passes take 8.7 ms this way, without the merge levels
+// (5.8 of it the larger segments'), 50,000 small ones' 5.8; with every stage a launch over all
 // segments, through memory, 12.4 and 8.4.
 
 // Folds every thread's box (ordered-integer encoding of the floats) over the
@@ -2181,7 +2181,7 @@ __global__ void __launch_bounds__(BLOCK) walk_kernel(Work W, DevParams P) {
 // word between these launches, and ranks are found again from them: stored as
 // 64-bit prefixes that every later launch read again, in fourteen launches, the
 // larger segments' part of 200,000 subhalos' passes took 7.2 ms here and, with
-// the frame sums it includes, takes 3.2 (37 million entries in the first pass).
+// the frame sums it includes, takes 3.1 (37 million entries in the first pass).
 //
 // The tree's scratch is free after the walk: nlo holds the positions p_k (at
 // k), nhi those of E<0 from the front (the j-th at j), npos the new Elist, dl
@@ -3018,8 +3018,8 @@ __global__ void __launch_bounds__(BLOCK) output_combine_kernel(Work W, DevParams
 // tree_one), Elist and energies in LDS in between.  REPLAY sums in the
 // reference's order between two stages of it.  As fifteen launches over every
 // slot, each behind its own loads of segment, list and record, this took 7.0 ms
-// of a batch of 200,000 subhalos' passes (3.8 now) and 35 of a 300-particle
-// list's 50 us a pass (15 now); the record's 18 FP64 sums bound it, so their
+// of a batch of 200,000 subhalos' passes (3.4 now) and 35 us of a pass of a
+// 300-particle list (12 now); the record's 18 FP64 sums bound it, so their
 // registers are kept to four waves per SIMD.
 enum { POST_PART = 1, POST_FRAME = 2, POST_SORT = 4, POST_RECORD = 8 };
 constexpr int POST_ALL = POST_PART | POST_FRAME | POST_SORT | POST_RECORD;

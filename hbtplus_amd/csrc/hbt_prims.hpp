@@ -9,8 +9,11 @@
 //
 // Primitives:
 //   segmented sort of (u64 key, u32 value) pairs by (key, value):
-//     tile_sort_kernel    : LDS bitonic sort of each tile
+//     sort_tile, sort_tile_spare, sort_tile_words : a workgroup's run, as pairs or
+//                           as words that carry their place
+//     tile_sort_kernel    : each tile's pairs
 //     merge_pass_kernel   : one bottom-up merge level (co-rank by binary search)
+//     rank_merge_kernel   : a level of 16 runs, for launches of few tiles
 //   segmented exclusive scan (load/store functors):
 //     scan_tiles_kernel / scan_add_kernel
 #pragma once
