@@ -9,10 +9,12 @@
 // its claim order.  On the device:
 //   mask_gather   key = particle ID (sign bit flipped: unsigned order =
 //                 signed order), value = claim order
-//   segmented sort by (ID, claim order) per group
-//   mask_owner    the first entry of every run of equal IDs keeps its particle
-//   segmented scan of the keep flags per group, mask_write: each subhalo's
-//   kept entries in list order at the front of its range
+//   groups of up to CLAIM_CAP entries, mask_claim: a table in LDS holds the
+//   first claim of each ID; the keep flags and their scan
+//   larger ones: segmented sort by (ID, claim order), mask_owner (the first
+//   entry of every run of equal IDs keeps its particle), segmented scan
+//   mask_write    each subhalo's kept entries in list order at the front of its
+//                 range
 // Subhalos that do not claim (orphans, field) keep their lists (mask_copy).
 #pragma once
 
@@ -25,14 +27,16 @@ struct MaskSub {
   int gstart;      // first claim position in the group segment
 };
 
+// Groups whose first claims a workgroup finds in LDS: of up to CLAIM_SMALL
+// entries by one of 256 threads, of up to CLAIM_CAP by one of 1,024.
+constexpr int CLAIM_SMALL = 1024, CLAIM_CAP = 8192;
+
 struct MaskArgs {
   const MaskSub *sub;
   int nsub;
   const int64_t *gbase;  // first slot of each group segment
   const int *gn;         // entries per group segment
   int ngrp;
-  int64_t nslots;
-  const int *seg_of_slot;
   const int64_t *id;
   u64 *k0;
   u32 *v0;
@@ -56,23 +60,92 @@ __global__ void __launch_bounds__(BLOCK) mask_gather_kernel(MaskArgs A) {
     const MaskSub m = A.sub[s];
     if (m.grp < 0) continue;
     const int64_t b = A.gbase[m.grp] + m.gstart;
+    const bool sorted = A.gn[m.grp] > CLAIM_CAP;
     for (int64_t l = threadIdx.x; l < m.count; l += BLOCK) {
       A.k0[b + l] = (u64)A.id[m.offset + l] ^ (1ull << 63);
-      A.v0[b + l] = (u32)(m.gstart + l);
+      if (sorted) A.v0[b + l] = (u32)(m.gstart + l);
     }
   }
 }
 
-// sorted position i of a group: owner iff its ID differs from position i-1
-__global__ void __launch_bounds__(BLOCK) mask_owner_kernel(MaskArgs A) {
-  for (int64_t s = (int64_t)blockIdx.x * BLOCK + threadIdx.x; s < A.nslots; s += (int64_t)gridDim.x * BLOCK) {
-    const int g = A.seg_of_slot[s];
-    if (g < 0) continue;
-    const int64_t b = A.gbase[g];
-    const int i = (int)(s - b);
-    if (i >= A.gn[g]) continue;
-    const bool owner = i == 0 || A.k0[s - 1] != A.k0[s];
-    A.keep[b + A.v0[s]] = owner ? 1 : 0;
+// The first claims of a group of n <= T PER entries, a workgroup's: a table of
+// twice as many places holds a claim for each ID, the smallest once all are in.  A
+// place keeps the ID it was taken for, so a claim is compared with whichever
+// claim of that ID stands there, and half of the places stay empty, so every
+// probe ends.
+// The IDs themselves stay in memory: a probe of a taken place reads one through
+// the L2, which bounds the kernel, and the table of a group of 8,192 leaves room
+// for a second workgroup on the CU.
+template <int T, int PER>
+__global__ void __launch_bounds__(T) mask_claim_kernel(MaskArgs A, const int *groups, int ngroups) {
+  constexpr u32 SLOTS = 2u * T * PER, EMPTY = ~0u;
+  __shared__ u32 claim[SLOTS];
+  __shared__ u32 wsum[T / WAVE];
+  const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+  for (int i = blockIdx.x; i < ngroups; i += gridDim.x) {
+    const int n = A.gn[groups[i]];
+    const int64_t b = A.gbase[groups[i]];
+    const u64 *id = A.k0 + b;
+    u32 slots = 2 * WAVE;  // no more than needed: they are cleared
+    while (slots < 2 * (u32)n) slots *= 2;
+    for (u32 h = threadIdx.x; h < slots; h += T) claim[h] = EMPTY;
+    u64 key[PER];
+    const int c0 = PER * (int)threadIdx.x;
+#pragma unroll
+    for (int r = 0; r < PER; r++) key[r] = id[min(c0 + r, n - 1)];
+    __syncthreads();
+    u32 at[PER];
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+      const u32 c = (u32)(c0 + r);
+      at[r] = 0;
+      if (c >= (u32)n) continue;
+      u32 h = (u32)id_hash((long long)key[r]) & (slots - 1);
+      for (;;) {
+        const u32 p = atomicCAS(&claim[h], EMPTY, c);
+        if (p == EMPTY) break;
+        if (id[p] == key[r]) {
+          if (c < p) atomicMin(&claim[h], c);
+          break;
+        }
+        h = (h + 1) & (slots - 1);
+      }
+      at[r] = h;
+    }
+    __syncthreads();
+    u32 kept = 0, mine = 0;
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+      const bool first = c0 + r < n && claim[at[r]] == (u32)(c0 + r);
+      mine |= (u32)first << r;
+      kept += first;
+    }
+    u32 ex = wave_inclusive_scan(kept);
+    if (lane == WAVE - 1) wsum[w] = ex;
+    __syncthreads();
+    ex -= kept;
+    for (int u = 0; u < w; u++) ex += wsum[u];
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+      if (c0 + r >= n) continue;
+      A.keep[b + c0 + r] = mine >> r & 1;
+      A.scan[b + c0 + r] = ex;
+      ex += mine >> r & 1;
+    }
+    __syncthreads();  // the table and wsum are written again
+  }
+}
+
+// sorted position i of a larger group: owner iff its ID differs from position i-1
+__global__ void __launch_bounds__(BLOCK) mask_owner_kernel(MaskArgs A, const Tile *tiles, int ntiles) {
+  for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    const Tile tl = tiles[t];
+    const int64_t b = A.gbase[tl.seg];
+    const int end = min(tl.start + TILE, A.gn[tl.seg]);
+    for (int i = tl.start + (int)threadIdx.x; i < end; i += BLOCK) {
+      const bool owner = i == 0 || A.k0[b + i - 1] != A.k0[b + i];
+      A.keep[b + A.v0[b + i]] = owner ? 1 : 0;
+    }
   }
 }
 
@@ -154,8 +227,8 @@ extern "C" int hbt_mask_subhalos(hbt_ctx *ctx, const hbt_particles *particles, c
   std::vector<MaskSub> ms(nsub);
   for (int64_t s = 0; s < nsub; s++) ms[s] = MaskSub{subs_host[s].offset, subs_host[s].count, -1, 0};
   std::vector<int64_t> gbase;
-  std::vector<int> gn, capal, first_tile, ntile;
-  std::vector<Tile> tiles;
+  std::vector<int> gn, claims[2];
+  std::vector<Tile> tiles;  // of the groups that are sorted
   std::vector<char> seen(nsub, 0);
   int64_t off = 0;
   int maxn = 0;
@@ -189,13 +262,13 @@ extern "C" int hbt_mask_subhalos(hbt_ctx *ctx, const hbt_particles *particles, c
     const int k = (int)gbase.size();
     gbase.push_back(off);
     gn.push_back((int)pos);
-    const int ca = (int)((pos + WAVE - 1) / WAVE * WAVE);
-    capal.push_back(ca);
-    first_tile.push_back((int)tiles.size());
+    off += (pos + WAVE - 1) / WAVE * WAVE;
+    if (pos <= CLAIM_CAP) {
+      claims[pos <= CLAIM_SMALL ? 0 : 1].push_back(k);
+      continue;
+    }
     const int nt = (int)((pos + TILE - 1) / TILE);
-    ntile.push_back(nt);
     for (int t = 0; t < nt; t++) tiles.push_back(Tile{k, t * TILE});
-    off += ca;
     maxn = std::max(maxn, (int)pos);
   }
   // groups whose central never got a segment keep -1; map group ids for subhalos
@@ -209,8 +282,8 @@ extern "C" int hbt_mask_subhalos(hbt_ctx *ctx, const hbt_particles *particles, c
   int rc = stage_blobs(ctx, {{ms.data(), ms.size() * sizeof(MaskSub)},
                              {gbase.data(), gbase.size() * 8},
                              {gn.data(), gn.size() * 4},
-                             {capal.data(), capal.size() * 4},
-                             {first_tile.data(), first_tile.size() * 4},
+                             {claims[0].data(), claims[0].size() * 4},
+                             {claims[1].data(), claims[1].size() * 4},
                              {tiles.data(), tiles.size() * sizeof(Tile)}},
                        d);
   if (rc != HBT_OK) { dcnt.release(); return rc; }
@@ -220,8 +293,6 @@ extern "C" int hbt_mask_subhalos(hbt_ctx *ctx, const hbt_particles *particles, c
   A.gbase = (const int64_t *)d[1];
   A.gn = (const int *)d[2];
   A.ngrp = ngrp;
-  A.nslots = off;
-  A.seg_of_slot = ctx->seg_of_slot.as<int>();
   A.id = particles->id;
   A.k0 = ctx->k0.as<u64>();
   A.v0 = ctx->v0.as<u32>();
@@ -232,22 +303,26 @@ extern "C" int hbt_mask_subhalos(hbt_ctx *ctx, const hbt_particles *particles, c
   const int gsub = (int)std::min<int64_t>(nsub, (int64_t)ctx->cus * 8);
   mask_copy_kernel<<<gsub, BLOCK, 0, st>>>(A);
   if (ngrp > 0) {
-    const Tile *dt = (const Tile *)d[5];
-    const int nt = (int)tiles.size();
-    const int gt = (int)std::max<int64_t>(1, std::min<int64_t>(nt, (int64_t)ctx->cus * 8));
-    const int gm = (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)nt * (TILE / BLOCK), (int64_t)ctx->cus * 16));
-    fill_seg_of_slot_kernel<<<std::min(ngrp, ctx->cus * 8), BLOCK, 0, st>>>(ngrp, A.gbase, (const int *)d[3],
-                                                                            ctx->seg_of_slot.as<int>());
     mask_gather_kernel<<<gsub, BLOCK, 0, st>>>(A);
-    tile_sort_kernel<<<gt, BLOCK, 0, st>>>(dt, nt, A.gbase, A.gn, A.k0, A.v0, ctx->k1.as<u64>(), ctx->v1.as<u32>());
-    int level = 0;
-    for (int w = TILE; w < maxn; w *= 2, level++)
-      merge_pass_kernel<<<gm, BLOCK, 0, st>>>(dt, nt, A.gbase, A.gn, TILE, level, A.k0, A.v0, ctx->k1.as<u64>(),
-                                              ctx->v1.as<u32>());
-    mask_owner_kernel<<<grid_for(off, ctx->cus), BLOCK, 0, st>>>(A);
-    u64 *ts = ctx->tsum.as<u64>();
-    scan_tiles_kernel<u64><<<gt, BLOCK, 0, st>>>(dt, nt, A.gn, ts, KeepLoad{A.gbase, A.keep}, KeepStore{A.gbase, A.scan});
-    scan_add_kernel<u64><<<gt, BLOCK, 0, st>>>(dt, nt, A.gn, ts, KeepAdd{A.gbase, A.scan});
+    const int nc0 = (int)claims[0].size(), nc1 = (int)claims[1].size(), nt = (int)tiles.size();
+    if (nc0 > 0)
+      mask_claim_kernel<BLOCK, CLAIM_SMALL / BLOCK><<<std::min(nc0, ctx->cus * 8), BLOCK, 0, st>>>(A, (const int *)d[3], nc0);
+    if (nc1 > 0)
+      mask_claim_kernel<1024, CLAIM_CAP / 1024><<<std::min(nc1, ctx->cus * 2), 1024, 0, st>>>(A, (const int *)d[4], nc1);
+    if (nt > 0) {
+      const Tile *dt = (const Tile *)d[5];
+      const int gt = std::min(nt, ctx->cus * 8);
+      const int gm = (int)std::min<int64_t>((int64_t)nt * (TILE / BLOCK), (int64_t)ctx->cus * 16);
+      tile_sort_kernel<<<gt, BLOCK, 0, st>>>(dt, nt, A.gbase, A.gn, A.k0, A.v0, ctx->k1.as<u64>(), ctx->v1.as<u32>());
+      int level = 0;
+      for (int64_t w = TILE; w < maxn; w *= 2, level++)
+        merge_pass_kernel<<<gm, BLOCK, 0, st>>>(dt, nt, A.gbase, A.gn, TILE, level, A.k0, A.v0, ctx->k1.as<u64>(),
+                                                ctx->v1.as<u32>());
+      mask_owner_kernel<<<gt, BLOCK, 0, st>>>(A, dt, nt);
+      u64 *ts = ctx->tsum.as<u64>();
+      scan_tiles_kernel<u64><<<gt, BLOCK, 0, st>>>(dt, nt, A.gn, ts, KeepLoad{A.gbase, A.keep}, KeepStore{A.gbase, A.scan});
+      scan_add_kernel<u64><<<gt, BLOCK, 0, st>>>(dt, nt, A.gn, ts, KeepAdd{A.gbase, A.scan});
+    }
     mask_write_kernel<<<gsub, BLOCK, 0, st>>>(A);
   }
   hipError_t e = hipGetLastError();

@@ -275,3 +275,42 @@ def test_ranked_runs(gpu, sizes):
     assert_tolerant(oracle.unbind_batch(cat, nthreads=8), got)
     for a, b in zip(got, U.unbind_batch(cat, plain=True)):
         assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
+
+
+@pytest.mark.parametrize("ids", ["mixed", "one", "high_bits"])
+def test_mask_claims(gpu, ids):
+    """groups of 1 to 9,000 entries in several subhalos: first claims in a table
+    of one workgroup (up to 1,024 and 8,192 entries) and by sorting; IDs repeated
+    in and across lists, one ID alone, IDs that differ in their high bits only"""
+    rng = np.random.default_rng(41)
+    sizes = [1, 2, 63, 64, 65, 255, 256, 257, 1023, 1024, 1025, 2049, 8191, 8192, 8193, 9000]
+    counts, grp, parent, pool = [], [], [], []
+    for g, n in enumerate(sizes):
+        cuts = np.sort(rng.integers(0, n + 1, min(n - 1, 6)))
+        part = np.diff(np.concatenate([[0], cuts, [n]]))  # some lists empty
+        first = len(counts)
+        counts += list(part)
+        grp += [g] * len(part)
+        parent += [-1] + [int(rng.integers(first, first + i)) if i % 2 else -1 for i in range(1, len(part))]
+        pool.append(rng.integers(0, max(1, n * 2 // 3), n))
+    ident = np.concatenate(pool).astype(np.int64)
+    if ids == "mixed":
+        ident = np.where(rng.random(len(ident)) < 0.1, np.int64(-1), ident - 500)
+    elif ids == "one":
+        ident[:] = 7
+    else:
+        ident = (ident << 48) ^ np.int64(1)
+    subs = np.zeros(len(counts), abi.SUB_DTYPE)
+    subs["count"] = subs["nbound_prev"] = counts
+    subs["offset"] = np.cumsum([0] + counts[:-1])
+    subs["parent"] = parent
+    subs["nbound_prev"][5::9] = 1  # claim nothing
+    n = len(ident)
+    cols = {k: np.zeros(n, np.float32) for k in ("x", "y", "z", "vx", "vy", "vz", "mass")}
+    cols.update(id=ident, type=np.ones(n, np.int32))
+    grp = np.array(grp, np.int64)
+    out, cnt = gpu(abi.make_params()).mask_subhalos(cols, subs, grp)
+    ref_out, ref_cnt = oracle.mask_subhalos(cols, subs, grp)
+    assert np.array_equal(cnt, ref_cnt)
+    for o, c in zip(subs["offset"], cnt):
+        assert np.array_equal(out[o:o + c], ref_out[o:o + c])
