@@ -72,10 +72,12 @@ __global__ void __launch_bounds__(BLOCK) mask_gather_kernel(MaskArgs A) {
 // twice as many places holds a claim for each ID, the smallest once all are in.  A
 // place keeps the ID it was taken for, so a claim is compared with whichever
 // claim of that ID stands there, and half of the places stay empty, so every
-// probe ends.
-// The IDs themselves stay in memory: a probe of a taken place reads one through
-// the L2, which bounds the kernel, and the table of a group of 8,192 leaves room
-// for a second workgroup on the CU.
+// probe ends.  The IDs themselves stay in memory: a probe of a taken place reads
+// one through the L2, which bounds the kernel, and the table of a group of 8,192
+// leaves room for a second workgroup on the CU.  1,000 groups (4.0 M entries)
+// take 54 us in both sizes where their sort, owners and scan took 190; the call
+// 0.67 -> 0.44 ms, with 20 groups 0.20 -> 0.08.  A table for 16,384 would leave
+// one workgroup of 16 waves on a CU.
 template <int T, int PER>
 __global__ void __launch_bounds__(T) mask_claim_kernel(MaskArgs A, const int *groups, int ngroups) {
   constexpr u32 SLOTS = 2u * T * PER, EMPTY = ~0u;
