@@ -38,6 +38,8 @@ struct __align__(32) Item {
                // squared distance below which the FP32 walk opens the node (0 for a leaf)
 };
 
+static_assert(sizeof(Item) == 32, "the walks step by 32 bytes");
+
 struct Work {
   // per level
   Seg *seg;
@@ -899,17 +901,19 @@ struct DepthTable {
   }
 };
 
+// (not read in trees that are too large for it)
+__device__ __forceinline__ int byte_offset(int item) { return (int)((u32)sizeof(Item) * (u32)item); }
 __device__ __forceinline__ Item leaf_item(const float4 &pm, int pos) {
-  return Item{pm, make_int2(0, pos + 1), make_int2(32 * (pos + 1), 0)};
+  return Item{pm, make_int2(0, pos + 1), make_int2(byte_offset(pos + 1), 0)};
 }
 __device__ __forceinline__ Item node_item(const float4 &pm, int skip, float lsq, float below) {
-  return Item{pm, make_int2(__float_as_int(lsq), skip), make_int2(32 * skip, __float_as_int(below))};
+  return Item{pm, make_int2(__float_as_int(lsq), skip), make_int2(byte_offset(skip), __float_as_int(below))};
 }
 // Sentinel after the last item: massless, far from every target, never
 // opened, its skip is itself, so a group walk that has finished reads it, adds
 // nothing and stays put.
 __device__ __forceinline__ Item sentinel_item(int pos) {
-  return Item{make_float4(1e18f, 1e18f, 1e18f, 0.f), make_int2(0, pos), make_int2(32 * pos, 0)};
+  return Item{make_float4(1e18f, 1e18f, 1e18f, 0.f), make_int2(0, pos), make_int2(byte_offset(pos), 0)};
 }
 
 // A leaf: a sampled tree's leaves carry mass * MassFactor (EnergySnapshot_t::GetMass, :79).
@@ -1898,8 +1902,8 @@ __device__ __forceinline__ double walk_group_dispatch(const Item *__restrict__ i
   return walk_group<GROUP, COUNT, FastTerm<false, true>>(it, P, ib, end, live, x, y, z, tm, wc);
 }
 
-// Lanes per group chosen per segment (S.wgroup, set from its size bin).  The
-// straddling and uncompensated forms (rare; precision study) keep 64.
+// Lanes per group chosen per segment (S.wgroup, set from its size: 64 where
+// 32-bit byte offsets do not reach).  The straddling and uncompensated forms (rare; precision study) keep 64.
 template <bool COUNT, bool REPLAY>
 __device__ __forceinline__ double walk_binned(const Item *__restrict__ it, const DevParams &P,
                                               const Seg &S, int ib, int end, bool live, float x,

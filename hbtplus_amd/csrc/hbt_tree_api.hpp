@@ -123,7 +123,9 @@ __device__ __forceinline__ bool targets_wrap(const Seg &S, const DevParams &P, c
   return wrap;
 }
 
-// One target per lane, in tree order.
+// One target per lane, in tree order, GROUP lanes together: 16, or 64 in trees
+// beyond byte_walk.
+template <int GROUP>
 __global__ void __launch_bounds__(BLOCK) walk_points_kernel(Work W, DevParams P, TgtArgs A,
                                                             const Item *__restrict__ it) {
   Seg S = W.seg[0];
@@ -134,8 +136,8 @@ __global__ void __launch_bounds__(BLOCK) walk_points_kernel(Work W, DevParams P,
     const bool live = i < A.n;
     const int t = live ? A.order[i] : 0;
     const float x = A.x[t], y = A.y[t], z = A.z[t], tm = A.m ? A.m[t] : 0.f;
-    const double pot = P.replay ? walk_group_dispatch<16, false, true>(it, P, S, 0, S.n_items, live, x, y, z, tm, wc)
-                                : walk_group_dispatch<16, false, false>(it, P, S, 0, S.n_items, live, x, y, z, tm, wc);
+    const double pot = P.replay ? walk_group_dispatch<GROUP, false, true>(it, P, S, 0, S.n_items, live, x, y, z, tm, wc)
+                                : walk_group_dispatch<GROUP, false, false>(it, P, S, 0, S.n_items, live, x, y, z, tm, wc);
     if (live) A.out[t] = pot * (double)P.G / (double)P.a;
   }
 }
@@ -220,13 +222,17 @@ extern "C" int hbt_tree_potential(hbt_ctx *ctx, int64_t n_src, const float *sx, 
     if (nt > 1) scan_add_kernel<u64><<<g, BLOCK, 0, st>>>(R.tl_cur, nt, n, ctx->tsum.as<u64>(), TgtAdd{A.first});
     tgt_order_kernel<<<grid_for(A.n, ctx->cus), BLOCK, 0, st>>>(A);
     const int chunks = (A.n + WAVE - 1) / WAVE;
+    if (!byte_walk(n_src)) {
+      walk_points_kernel<64><<<(A.n + BLOCK - 1) / BLOCK, BLOCK, 0, st>>>(R.W, R.P, A, R.W.items);
+      continue;
+    }
     switch (R.P.replay || !R.P.wide_sum ? 1 : walk_parts(chunks, ctx->cus)) {
       case 16: walk_points_split_kernel<16><<<chunks, 16 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items); break;
       case 8: walk_points_split_kernel<8><<<chunks, 8 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items); break;
       case 4: walk_points_split_kernel<4><<<chunks, 4 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items); break;
       case 2: walk_points_split_kernel<2><<<chunks, 2 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items); break;
       default:
-        walk_points_kernel<<<(A.n + BLOCK - 1) / BLOCK, BLOCK, 0, st>>>(R.W, R.P, A, R.W.items);
+        walk_points_kernel<16><<<(A.n + BLOCK - 1) / BLOCK, BLOCK, 0, st>>>(R.W, R.P, A, R.W.items);
     }
   }
   HIPCHK(hipGetLastError());

@@ -23,6 +23,7 @@
 
 #include "../../include/hbt_unbind.h"
 #include "hbt_kernels.hpp"
+#include "hbt_walk_rules.hpp"
 
 using namespace hbt;
 
@@ -219,10 +220,6 @@ struct Level {
   int64_t ndraws = 0;                 // rand() values the level's shuffles take
   uint32_t win[31] = {};              // the stream's window before the first of them
 };
-
-int walk_group_for(const hbt_tuning &t, int64_t len) {
-  return len < t.bin_edge[0] ? t.walk_group[0] : (len < t.bin_edge[1] ? t.walk_group[1] : t.walk_group[2]);
-}
 
 // The batch's nest structure on the host, with the record fields the
 // planning reads gathered once (a record is 240 bytes, the planning needs 40
@@ -471,19 +468,6 @@ int walk_grid(int64_t nslots, int xcd_run) {
   const int64_t m = (int64_t)NXCD * std::max(1, xcd_run);
   g = (g + m - 1) / m * m;
   return (int)std::max<int64_t>(g, 1);
-}
-
-// Waves that share a chunk's walk (1, 2, 4, 8 or 16): about eight waves per
-// SIMD.  From six without sharing on a second wave no longer pays: a list of
-// 420,000 (6,563 chunks) walks 1.71 ms alone and 1.78 shared by two, 50 lists of
-// together 5,900 chunks 0.81 and 0.62, one list of 24,000 (375) 0.53 and, by 16,
-// 0.147.
-int walk_parts(int64_t chunks, int cus) {
-  const int64_t simds = 4 * (int64_t)cus;
-  if (chunks >= 6 * simds) return 1;
-  int parts = 2;
-  while (parts < 16 && chunks * parts < 8 * simds) parts *= 2;
-  return parts;
 }
 
 int grid_for(int64_t n, int cus) {
@@ -896,9 +880,9 @@ struct Runner {
       else if (parts == 8) launch_split_walk<8>();
       else launch_split_walk<16>();
     } else if (c->walk_mode == 0) {
-      const int *g = c->tune.walk_group;
-      const int uniform = (g[0] == g[1] && g[1] == g[2]) ? g[0] : 0;
-      switch (uniform) {
+      // (segments are listed largest first; one too large for byte offsets has
+      // chunks enough never to be split)
+      switch (launch_group(c->tune, cur_cap.empty() ? 0 : cur_cap[0])) {
         case 0: launch_shared_walk<0>(count); break;  // per-segment bins
         case 8: launch_shared_walk<8>(count); break;
         case 16: launch_shared_walk<16>(count); break;
