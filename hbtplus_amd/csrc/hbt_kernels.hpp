@@ -945,12 +945,10 @@ __device__ __forceinline__ float4 sum_children(Pm pm, Skip skip, int g, int end)
   return make_float4((float)(cx / mass), (float)(cy / mass), (float)(cz / mass), (float)mass);
 }
 
-// The same over the items in device memory.  Skips are segment-local item
-// positions; ib is the segment's first item.
-__device__ __forceinline__ void node_moments(const Work &W, int64_t ib, int g) {
-  const Item *it = W.items;
-  W.items[g].pm = sum_children([&](int c) { return it[c].pm; }, [&](int c) { return (int)(ib + it[c].ax.y); },
-                               g, (int)(ib + W.items[g].ax.y));
+// The same over a segment's items in device memory (positions and skips are
+// segment-local: a level's items may number more than 2^31).
+__device__ __forceinline__ void node_moments(Item *it, int g) {
+  it[g].pm = sum_children([&](int c) { return it[c].pm; }, [&](int c) { return it[c].ax.y; }, g, it[g].ax.y);
 }
 
 // A team: the threads that build one tile's tree (one wave, or the workgroup),
@@ -1269,7 +1267,7 @@ __global__ void __launch_bounds__(BLOCK, 4) items_tile_kernel(Work W, DevParams 
         at[j] = pos - first;
       } else {
         W.items[ib + pos] = node_item(make_float4(0.f, 0.f, 0.f, 0.f), nskip[j], depth.lsq[pdl[j]], depth.below[pdl[j]]);
-        W.npos[b + l] = (int)(ib + pos);
+        W.npos[b + l] = pos;
         list_crossing(W, t, tl, b, l, plo[j], phi[j], ncross);
       }
     }
@@ -1314,19 +1312,19 @@ struct ListNodes {
 
 __device__ __forceinline__ void moments_of_list(const Work &W, const Seg &S, const int *list, int ng, ListNodes &L) {
 #pragma clang fp contract(off)
-  const int64_t b = S.ibase, ib = 2 * b;
+  const int64_t b = S.ibase;
+  Item *it = W.items + 2 * b;
   if (ng > LISTED) {
     for (int v = min(max(S.D, S.Dfull), MAX_DEPTH); v >= 0; v--) {
       for (int i = threadIdx.x; i < ng; i += BLOCK) {
         const int64_t s = b + list[i];
-        if (W.dl[s] == v) node_moments(W, ib, W.npos[s]);
+        if (W.dl[s] == v) node_moments(it, W.npos[s]);
       }
       __syncthreads();
     }
     return;
   }
   constexpr int PER = LISTED / BLOCK;
-  Item *it = W.items + ib;
   for (int d = threadIdx.x; d < NLEVEL; d += BLOCK) L.count[d] = 0;
   __syncthreads();
   int pos[PER], depth[PER], rank[PER];
@@ -1335,7 +1333,7 @@ __device__ __forceinline__ void moments_of_list(const Work &W, const Seg &S, con
     const int i = (int)threadIdx.x + BLOCK * r;
     if (i >= ng) continue;
     const int64_t s = b + list[i];
-    pos[r] = (int)(W.npos[s] - ib);
+    pos[r] = W.npos[s];
     depth[r] = W.dl[s];
     rank[r] = atomicAdd(&L.count[depth[r]], 1);
     const int end = it[pos[r]].ax.y;
@@ -1366,7 +1364,7 @@ __device__ __forceinline__ void moments_of_list(const Work &W, const Seg &S, con
     for (int p = p0 + (int)threadIdx.x; p < p1; p += BLOCK) {
       const int i = L.node[p], n = L.sons[i], g = L.son[0][i] - 1;
       if (n > SONS) {
-        node_moments(W, ib, ib + g);
+        node_moments(it, g);
         continue;
       }
       float4 q[SONS];
@@ -1420,24 +1418,22 @@ __global__ void __launch_bounds__(BLOCK) moments_cross_kernel(Work W, const Tile
 
 // Reference arithmetic (src/gravity_tree.cpp:79-164): FP64 walk over float data.
 template <bool COUNT>
-__device__ double walk_replay(const Work &W, const DevParams &P, int64_t ib, int n_items, float tx,
-                              float ty, float tz, float tmass, unsigned &ni, unsigned &no) {
+__device__ double walk_replay(const Item *it, const DevParams &P, int end, float tx, float ty, float tz, float tmass,
+                              unsigned &ni, unsigned &no) {
 #pragma clang fp contract(off)
   const double h = 2.8 * (double)P.eps, hinv = 1.0 / h;
   double pot = (double)(float)(tmass / P.eps);
   const double x = tx, y = ty, z = tz;
-  const int end = (int)(ib + n_items);
-  int j = (int)ib;
+  int j = 0;
   while (j < end) {
-    const float4 q = W.items[j].pm;
-    const int2 a = W.items[j].ax;
+    const float4 q = it[j].pm;
+    const int2 a = it[j].ax;
     double dx = (double)q.x - x, dy = (double)q.y - y, dz = (double)q.z - z;
     if (P.periodic) { dx = nearest_d(dx, P); dy = nearest_d(dy, P); dz = nearest_d(dz, P); }
     const double r2 = dx * dx + dy * dy + dz * dz;
     const float lsq = __int_as_float(a.x);
     if ((double)lsq > r2 * (double)P.theta2) { j++; if (COUNT) no++; continue; }
-    const int nj = (int)(ib + a.y);
-    j = nj > j ? nj : end;  // skips always advance
+    j = a.y > j ? a.y : end;  // skips always advance
     if (COUNT) ni++;
     pot += kernel_term_d((double)q.w, sqrt(r2), h, hinv);
   }
@@ -1448,18 +1444,17 @@ __device__ double walk_replay(const Work &W, const DevParams &P, int64_t ib, int
 // group walk's FastTerm sums them.  Straddling segments (a periodic subhalo
 // wider than a quarter box) form the separation in double.
 template <bool STRADDLE, bool COUNT>
-__device__ double walk_fast(const Work &W, const DevParams &P, int64_t ib, int n_items, float tx,
-                            float ty, float tz, float tmass, unsigned &ni, unsigned &no) {
+__device__ double walk_fast(const Item *it, const DevParams &P, int end, float tx, float ty, float tz, float tmass,
+                            unsigned &ni, unsigned &no) {
 #pragma clang fp contract(off)
   const float h = 2.8f * P.eps, h2 = h * h, hinv = 1.0f / h;
   const float self = tmass / P.eps;
   double accd = self;
   float accf = self;
-  const int end = (int)(ib + n_items);
-  int j = (int)ib;
+  int j = 0;
   while (j < end) {
-    const float4 q = W.items[j].pm;
-    const int2 a = W.items[j].ax;
+    const float4 q = it[j].pm;
+    const int2 a = it[j].ax;
     float dx, dy, dz;
     if (STRADDLE) {
       dx = (float)nearest_d((double)q.x - (double)tx, P);
@@ -1470,8 +1465,7 @@ __device__ double walk_fast(const Work &W, const DevParams &P, int64_t ib, int n
     }
     const float r2 = pair_r2(dx, dy, dz);
     if (__int_as_float(a.x) > r2 * P.theta2) { j++; if (COUNT) no++; continue; }
-    const int nj = (int)(ib + a.y);
-    j = nj > j ? nj : end;  // skips always advance
+    j = a.y > j ? a.y : end;  // skips always advance
     if (COUNT) ni++;
     const float t = kernel_term_f(q.w, r2, h2, hinv);
     if (P.wide_sum) accd += t;
@@ -1484,10 +1478,10 @@ template <bool COUNT>
 __device__ __forceinline__ double walk_dispatch(const Work &W, const DevParams &P, const Seg &S,
                                                 float tx, float ty, float tz, float tmass,
                                                 unsigned &ni, unsigned &no) {
-  const int64_t ib = 2 * S.ibase;
-  if (P.replay) return walk_replay<COUNT>(W, P, ib, S.n_items, tx, ty, tz, tmass, ni, no);
-  if (S.straddle) return walk_fast<true, COUNT>(W, P, ib, S.n_items, tx, ty, tz, tmass, ni, no);
-  return walk_fast<false, COUNT>(W, P, ib, S.n_items, tx, ty, tz, tmass, ni, no);
+  const Item *it = W.items + 2 * S.ibase;  // positions and skips are segment-local
+  if (P.replay) return walk_replay<COUNT>(it, P, S.n_items, tx, ty, tz, tmass, ni, no);
+  if (S.straddle) return walk_fast<true, COUNT>(it, P, S.n_items, tx, ty, tz, tmass, ni, no);
+  return walk_fast<false, COUNT>(it, P, S.n_items, tx, ty, tz, tmass, ni, no);
 }
 
 __device__ __forceinline__ void flush_counts(const Work &W, unsigned ni, unsigned no, unsigned nt,
