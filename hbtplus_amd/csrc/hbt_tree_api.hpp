@@ -65,7 +65,56 @@ __global__ void __launch_bounds__(BLOCK) tgt_clear_kernel(Work W, TgtArgs A, int
   for (int j = i; j < nb; j += gridDim.x * BLOCK) A.count[j] = 0;
 }
 
+// The target's bucket: the place of the first source whose digits are not below
+// its own.
+__device__ __forceinline__ int tgt_bucket(const Work &W, const Seg &S, float x, float y, float z) {
+  const u64 key = octant_key(S.center, S.Len, S.D, x, y, z);
+  int lo = 0, hi = S.n_src;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (W.k0[mid] < key) lo = mid + 1; else hi = mid;
+  }
+  return lo >> BUCKET_BITS;
+}
+
+// Folds a position into a thread's box (ordered-integer encoding).
+__device__ __forceinline__ void box_take(u32 mn[3], u32 mx[3], float x, float y, float z) {
+  const u32 o[3] = {f2ord(x), f2ord(y), f2ord(z)};
+  for (int j = 0; j < 3; j++) { mn[j] = min(mn[j], o[j]); mx[j] = max(mx[j], o[j]); }
+}
+
 // Bucket of each target, its place among the bucket's targets, the box of all.
+// Atomics on one address are served one after another, 28 ns each, and few buckets
+// hold many targets each: up to LDS_BUCKETS a block counts its run of the targets
+// in LDS and takes a range of each bucket with one atomic (2 million targets among
+// 100 sources 8.8 -> 0.33 ms a call, among 1,000 4.3 -> 0.91).  With more buckets a
+// wave takes its places in memory, one atomic for each bucket its targets are in
+// (2 million close to a few of a million sources: target by target 12.4 ms a call,
+// so 3.5).
+constexpr int LDS_BUCKETS = 4096;
+
+__global__ void __launch_bounds__(BLOCK) tgt_bucket_lds_kernel(Work W, TgtArgs A, int nb, int per_block) {
+  __shared__ int cnt[LDS_BUCKETS];
+  const Seg &S = W.seg[0];
+  u32 mn[3] = {0xffffffffu, 0xffffffffu, 0xffffffffu}, mx[3] = {0u, 0u, 0u};
+  const int i0 = blockIdx.x * per_block, i1 = min(A.n, i0 + per_block);
+  for (int j = threadIdx.x; j < nb; j += BLOCK) cnt[j] = 0;
+  __syncthreads();
+  for (int i = i0 + (int)threadIdx.x; i < i1; i += BLOCK) {
+    const float x = A.x[i], y = A.y[i], z = A.z[i];
+    box_take(mn, mx, x, y, z);
+    const int b = tgt_bucket(W, S, x, y, z);
+    A.bucket[i] = b;
+    A.rank[i] = atomicAdd(&cnt[b], 1);
+  }
+  __syncthreads();
+  for (int j = threadIdx.x; j < nb; j += BLOCK)
+    if (cnt[j]) cnt[j] = atomicAdd(&A.count[j], cnt[j]);
+  __syncthreads();
+  for (int i = i0 + (int)threadIdx.x; i < i1; i += BLOCK) A.rank[i] += cnt[A.bucket[i]];
+  fold_box(mn, mx, A.box, A.box + 3);
+}
+
 __global__ void __launch_bounds__(BLOCK) tgt_bucket_kernel(Work W, TgtArgs A) {
   const Seg &S = W.seg[0];
   u32 mn[3] = {0xffffffffu, 0xffffffffu, 0xffffffffu}, mx[3] = {0u, 0u, 0u};
@@ -74,32 +123,27 @@ __global__ void __launch_bounds__(BLOCK) tgt_bucket_kernel(Work W, TgtArgs A) {
     int b = -1;
     if (i < A.n) {
       const float x = A.x[i], y = A.y[i], z = A.z[i];
-      const u32 o[3] = {f2ord(x), f2ord(y), f2ord(z)};
-      for (int j = 0; j < 3; j++) { mn[j] = min(mn[j], o[j]); mx[j] = max(mx[j], o[j]); }
-      const u64 key = octant_key(S.center, S.Len, S.D, x, y, z);
-      int lo = 0, hi = S.n_src;  // first source whose digits are not below the target's
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (W.k0[mid] < key) lo = mid + 1; else hi = mid;
-      }
-      b = lo >> BUCKET_BITS;
+      box_take(mn, mx, x, y, z);
+      b = tgt_bucket(W, S, x, y, z);
       A.bucket[i] = b;
     }
-    // the lanes in the first lane's bucket take their places with one atomic
-    const int lead = __builtin_amdgcn_readfirstlane(b);
-    const u64 same = __ballot(b == lead && b >= 0);
-    if (b >= 0) {
-      const int lane = threadIdx.x & (WAVE - 1);
-      int r = 0;
-      if (b == lead) {
-        const int head = __ffsll((long long)same) - 1;
-        if (lane == head) r = atomicAdd(&A.count[b], __popcll(same));
-        r = __shfl(r, head, WAVE) + __popcll(same & ((1ull << lane) - 1ull));
-      } else {
-        r = atomicAdd(&A.count[b], 1);
+    // the lanes of each bucket among the wave's: their first, how many, how many before
+    const int lane = threadIdx.x & (WAVE - 1);
+    int head = 0, size = 0, before = 0;
+    for (u64 todo = __ballot(b >= 0); todo != 0ull;) {  // uniform across the wave
+      const int first = __ffsll((long long)todo) - 1;
+      const u64 same = __ballot(b == __builtin_amdgcn_readlane(b, first));
+      if ((same >> lane) & 1ull) {
+        head = first;
+        size = __popcll(same);
+        before = __popcll(same & ((1ull << lane) - 1ull));
       }
-      A.rank[i] = r;
+      todo &= ~same;
     }
+    int r = 0;
+    if (size > 0 && lane == head) r = atomicAdd(&A.count[b], size);
+    r = __shfl(r, head, WAVE) + before;
+    if (b >= 0) A.rank[i] = r;
   }
   fold_box(mn, mx, A.box, A.box + 3);
 }
@@ -215,7 +259,12 @@ extern "C" int hbt_tree_potential(hbt_ctx *ctx, int64_t n_src, const float *sx, 
     A.order = A.rank + A.n;
     const int *n = R.count_row(NC_SORT);
     tgt_clear_kernel<<<grid_for(nb, ctx->cus), BLOCK, 0, st>>>(R.W, A, nb);
-    tgt_bucket_kernel<<<grid_for(A.n, ctx->cus), BLOCK, 0, st>>>(R.W, A);
+    if (nb <= LDS_BUCKETS) {
+      const int per = std::max((A.n + ctx->cus - 1) / ctx->cus, TILE);
+      tgt_bucket_lds_kernel<<<(A.n + per - 1) / per, BLOCK, 0, st>>>(R.W, A, nb, per);
+    } else {
+      tgt_bucket_kernel<<<grid_for(A.n, ctx->cus), BLOCK, 0, st>>>(R.W, A);
+    }
     // the level's tile table starts at the buckets' tiles (fewer buckets than sources)
     const int nt = (nb + TILE - 1) / TILE, g = std::min(nt, ctx->cus * 8);
     scan_tiles_kernel<u64><<<g, BLOCK, 0, st>>>(R.tl_cur, nt, n, ctx->tsum.as<u64>(), TgtLoad{A.count}, TgtStore{A.first});

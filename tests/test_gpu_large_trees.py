@@ -72,3 +72,29 @@ def test_walk_group_forms_of_many_chunks(gpu):
         for other in got[1:]:
             for x, y in zip(got[0], other):
                 assert np.array_equal(x.view(np.uint8), y.view(np.uint8)), prec
+
+
+@pytest.mark.parametrize("n_src", [1, 100, 65535, 65536])
+@pytest.mark.parametrize("n_tgt", [1, 1023, 1025, 263_001])
+def test_tree_targets_by_buckets(gpu, n_src, n_tgt):
+    """targets counted by buckets of 16 sources, in LDS up to 4,096 buckets (65,535
+    sources) by runs of 1,024 targets and more, and in memory beyond; half of the
+    targets stand in one place.  Any order of the targets gives the same bits, and a
+    sample of them the oracle's"""
+    rng = np.random.default_rng(n_src + n_tgt)
+    sp = rng.normal(size=(n_src, 3)) * 25.0 + 500.0
+    src = tuple(sp[:, j].astype(np.float32) for j in range(3)) + (rng.uniform(1e-4, 2e-4, n_src).astype(np.float32),)
+    tp = (rng.normal(size=(n_tgt, 3)) * 30.0 + 500.0).astype(np.float32)
+    tp[rng.random(n_tgt) < 0.5] = tp[0]
+    perm, some = rng.permutation(n_tgt), rng.integers(0, n_tgt, 200)
+    cols = lambda a: tuple(a[:, j].copy() for j in range(3))  # noqa: E731
+    for prec in (abi.HBT_PREC_REPLAY, abi.HBT_PREC_FAST):
+        p = abi.make_params(periodic=1, box_size=1.0e4, precision=prec)
+        U = gpu(p)
+        got = U.tree_potential(src, cols(tp))
+        assert np.array_equal(got[perm].view(np.uint64), U.tree_potential(src, cols(tp[perm])).view(np.uint64))
+        ref = oracle.tree_potential(p, src, cols(tp[some]))
+        if prec == abi.HBT_PREC_REPLAY:
+            assert np.array_equal(ref, got[some])
+        else:
+            assert np.abs(got[some] / ref - 1).max() < 1e-5
