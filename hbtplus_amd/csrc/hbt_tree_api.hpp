@@ -167,6 +167,20 @@ __device__ __forceinline__ bool targets_wrap(const Seg &S, const DevParams &P, c
   return wrap;
 }
 
+// Each lane walks a path of its own, over the targets in tree order or as they
+// came (then a periodic box always takes the wrapped separations, which give the
+// same bits where nothing wraps).
+template <bool ORDERED>
+__global__ void __launch_bounds__(BLOCK) walk_points_lane_kernel(Work W, DevParams P, TgtArgs A) {
+  Seg S = W.seg[0];
+  S.straddle = ORDERED ? (targets_wrap(S, P, A) ? 1 : 0) : P.periodic;
+  unsigned ni = 0, no = 0;
+  for (int i = blockIdx.x * BLOCK + threadIdx.x; i < A.n; i += gridDim.x * BLOCK) {
+    const int t = ORDERED ? A.order[i] : i;
+    A.out[t] = walk_dispatch<false>(W, P, S, A.x[t], A.y[t], A.z[t], A.m ? A.m[t] : 0.f, ni, no);
+  }
+}
+
 // One target per lane, in tree order, GROUP lanes together: 16, or 64 in trees
 // beyond byte_walk.
 template <int GROUP>
@@ -180,8 +194,7 @@ __global__ void __launch_bounds__(BLOCK) walk_points_kernel(Work W, DevParams P,
     const bool live = i < A.n;
     const int t = live ? A.order[i] : 0;
     const float x = A.x[t], y = A.y[t], z = A.z[t], tm = A.m ? A.m[t] : 0.f;
-    const double pot = P.replay ? walk_group_dispatch<GROUP, false, true>(it, P, S, 0, S.n_items, live, x, y, z, tm, wc)
-                                : walk_group_dispatch<GROUP, false, false>(it, P, S, 0, S.n_items, live, x, y, z, tm, wc);
+    const double pot = walk_group_dispatch<GROUP, false, false>(it, P, S, 0, S.n_items, live, x, y, z, tm, wc);
     if (live) A.out[t] = pot * (double)P.G / (double)P.a;
   }
 }
@@ -225,7 +238,8 @@ extern "C" int hbt_tree_potential(hbt_ctx *ctx, int64_t n_src, const float *sx, 
   Level L;
   build_level(N, std::vector<int>{0}, ctx->tune, nullptr, 1, L);
   RETCHK(ensure_slots(ctx, L.nslots, 1, (int64_t)L.tiles.size()));
-  if (n_tgt > 0)
+  const TargetWalk form = target_walk(n_src, n_tgt, ctx->params.precision);
+  if (n_tgt > 0 && form != TargetWalk::alone)
     RETCHK(ctx->tgt.ensure(((size_t)(n_src >> BUCKET_BITS) + 1) * 12 + 24 + (size_t)std::min(n_tgt, TGT_SLICE) * 12));
   RETCHK(stage_level(ctx, L));
   Runner R;
@@ -243,14 +257,18 @@ extern "C" int hbt_tree_potential(hbt_ctx *ctx, int64_t n_src, const float *sx, 
                                                                       ctx->seg_of_slot.as<int>());
   tree_only_setup_kernel<<<1, 1, 0, st>>>(R.W, (int)n_src);
   tree_sources_kernel<<<grid_for(n_src, ctx->cus), BLOCK, 0, st>>>(R.W, (int)n_src, sx, sy, sz, smass);
-  RETCHK(R.build_tree(false, true));  // the targets' order reads the sorted digits
+  RETCHK(R.build_tree(false, form != TargetWalk::alone));  // the targets' order reads the sorted digits
   const int nb = (int)(n_src >> BUCKET_BITS) + 1;  // a target's place among the sources is 0 .. n_src
   for (int64_t t0 = 0; t0 < n_tgt; t0 += TGT_SLICE) {
-    TgtArgs A;
+    TgtArgs A{};
     A.n = (int)std::min<int64_t>(TGT_SLICE, n_tgt - t0);
     A.x = tx + t0; A.y = ty + t0; A.z = tz + t0;
     A.m = target_mass ? target_mass + t0 : nullptr;
     A.out = out_phi + t0;
+    if (form == TargetWalk::alone) {
+      walk_points_lane_kernel<false><<<grid_for(A.n, ctx->cus), BLOCK, 0, st>>>(R.W, R.P, A);
+      continue;
+    }
     A.first = ctx->tgt.as<u64>();
     A.count = (int *)(A.first + nb);
     A.box = (u32 *)(A.count + nb);
@@ -270,12 +288,16 @@ extern "C" int hbt_tree_potential(hbt_ctx *ctx, int64_t n_src, const float *sx, 
     scan_tiles_kernel<u64><<<g, BLOCK, 0, st>>>(R.tl_cur, nt, n, ctx->tsum.as<u64>(), TgtLoad{A.count}, TgtStore{A.first});
     if (nt > 1) scan_add_kernel<u64><<<g, BLOCK, 0, st>>>(R.tl_cur, nt, n, ctx->tsum.as<u64>(), TgtAdd{A.first});
     tgt_order_kernel<<<grid_for(A.n, ctx->cus), BLOCK, 0, st>>>(A);
+    if (form == TargetWalk::alone_ordered) {
+      walk_points_lane_kernel<true><<<grid_for(A.n, ctx->cus), BLOCK, 0, st>>>(R.W, R.P, A);
+      continue;
+    }
     const int chunks = (A.n + WAVE - 1) / WAVE;
     if (!byte_walk(n_src)) {
       walk_points_kernel<64><<<(A.n + BLOCK - 1) / BLOCK, BLOCK, 0, st>>>(R.W, R.P, A, R.W.items);
       continue;
     }
-    switch (R.P.replay || !R.P.wide_sum ? 1 : walk_parts(chunks, ctx->cus)) {
+    switch (R.P.wide_sum ? walk_parts(chunks, ctx->cus) : 1) {
       case 16: walk_points_split_kernel<16><<<chunks, 16 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items); break;
       case 8: walk_points_split_kernel<8><<<chunks, 8 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items); break;
       case 4: walk_points_split_kernel<4><<<chunks, 4 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items); break;

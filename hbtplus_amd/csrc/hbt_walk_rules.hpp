@@ -41,4 +41,35 @@ inline int walk_parts(int64_t chunks, int cus) {
   return parts;
 }
 
+// How hbt_tree_potential walks its targets: each lane by itself, over the targets
+// as they came or in tree order, or lanes together (16 of them, or 64 beyond
+// byte_walk; FAST shares a chunk among several waves).  The bits are the same.
+// Lanes that walk together wait for the union of their paths, which is long where
+// few targets lie far apart in a large tree, and ordering the targets costs five
+// launches and the digits' sort.  ms a call, periodic box, alone / ordered /
+// together:
+//   REPLAY sums in the reference's order, so no chunk is shared: alone, in order
+//   from where two waves a SIMD hide each other's loads (20,000 to 1 million sources
+//   at 262,144 targets 1.20-4.57 / 1.10-3.52 / 1.42-3.63; 100,000 at 32,768 1.16 /
+//   1.19 / 1.60; 300 at any number fastest unordered).
+//   FP32 adds in one order too; together where targets are dense (10,000 sources,
+//   4,096 targets 0.69 / 0.69 / 0.57; 100,000 and 32,768 1.02 / 1.00 / 0.85), alone
+//   below a target in 16 sources (30,000 and 512 0.90 / 0.88 / 1.11; 1 million and
+//   64 1.64 / 1.45 / 4.77), up to two targets being paths of their own (0.70 together
+//   for one among a million, 1.08 alone).
+//   FAST, its chunks shared, only below one in 1,500 of a large tree (1 million
+//   and 64 1.64 / 1.45 / 3.14; 300,000 and 64 1.36 / 1.19 / 2.05, and 512 1.37 / 1.45
+//   / 1.30).
+//   Trees of a wave's sources are walked in less time than the ordering's launches
+//   take (16 sources, 4,096 targets 0.043 / 0.095 / 0.095).
+enum class TargetWalk { alone, alone_ordered, together };
+inline TargetWalk target_walk(int64_t n_src, int64_t n_tgt, int precision) {
+  if (precision == HBT_PREC_REPLAY)
+    return n_tgt >= 131072 && n_src >= 1000 ? TargetWalk::alone_ordered : TargetWalk::alone;
+  if (n_src <= 64) return TargetWalk::alone;
+  const bool sparse = precision == HBT_PREC_FP32 ? n_tgt > 2 && n_src > 16 * n_tgt
+                                                 : n_tgt > 8 && n_src > 1500 * n_tgt && n_src >= 131072;
+  return sparse ? TargetWalk::alone : TargetWalk::together;
+}
+
 }  // namespace hbt

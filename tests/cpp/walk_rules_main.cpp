@@ -3,7 +3,9 @@
 //    them below 2^32, from the root to the item after the sentinel;
 //  - larger ones, up to the longest list the library takes, go to 64 lanes by
 //    their segment and never to a launch's uniform group or to shared chunks,
-//    under every tuning.
+//    under every tuning;
+//  - targets whose potentials are summed in the reference's order (REPLAY) are
+//    walked by each lane alone, at any numbers of sources and targets.
 // Prints "ok" and exits 0, or names the first failed check and exits 1.
 #include <cstdio>
 #include <initializer_list>
@@ -45,8 +47,16 @@ static int check_walk_forms() {
   return 0;
 }
 
+static int check_target_walks() {
+  for (int64_t src = 1; src < (int64_t)1 << 30; src += 1 + src / 3)
+    for (int64_t tgt = 1; tgt < (int64_t)1 << 34; tgt += 1 + tgt / 3)
+      CHECK(target_walk(src, tgt, HBT_PREC_REPLAY) != TargetWalk::together, "REPLAY, %lld sources, %lld targets",
+            (long long)src, (long long)tgt);
+  return 0;
+}
+
 int main() {
-  if (check_walk_forms()) return 1;
+  if (check_walk_forms() || check_target_walks()) return 1;
   printf("ok\n");
   return 0;
 }

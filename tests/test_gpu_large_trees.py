@@ -1,4 +1,5 @@
-"""Trees beyond the reach of 32-bit byte offsets (2^27 items of 32 bytes)."""
+"""hbt_tree_potential at the sizes where its walk changes form, and trees beyond
+the reach of 32-bit byte offsets (2^27 items of 32 bytes)."""
 import numpy as np
 import pytest
 
@@ -98,3 +99,24 @@ def test_tree_targets_by_buckets(gpu, n_src, n_tgt):
             assert np.array_equal(ref, got[some])
         else:
             assert np.abs(got[some] / ref - 1).max() < 1e-5
+
+
+@pytest.mark.parametrize("n_src", [1, 64, 65, 1025, 5000, 200_000])
+@pytest.mark.parametrize("where", ["inside", "across_a_face", "not_periodic"])
+def test_target_walks_agree(gpu, n_src, where):
+    """a few targets and many of them take other forms of the walk (each lane alone,
+    the targets as they came or in tree order; lanes together; a chunk shared by
+    waves): the same target gets the same bits, in every precision"""
+    rng = np.random.default_rng(n_src)
+    box, n_tgt = 1.0e4, 140_000
+    at = {"inside": 500.0, "across_a_face": 0.0, "not_periodic": 0.0}[where]
+    wrap = (lambda a: (a % box).astype(np.float32)) if where != "not_periodic" else (lambda a: a.astype(np.float32))
+    sp, tp = wrap(rng.normal(size=(n_src, 3)) * 25.0 + at), wrap(rng.normal(size=(n_tgt, 3)) * 30.0 + at)
+    src = tuple(sp[:, j].copy() for j in range(3)) + (rng.uniform(1e-4, 2e-4, n_src).astype(np.float32),)
+    for prec in (abi.HBT_PREC_REPLAY, abi.HBT_PREC_FP32, abi.HBT_PREC_FAST):
+        U = gpu(abi.make_params(periodic=int(where != "not_periodic"), box_size=box, precision=prec))
+        full = U.tree_potential(src, tuple(tp[:, j].copy() for j in range(3)))
+        for n in (1, 4, 70, 3000):
+            some = rng.permutation(n_tgt)[:n]
+            got = U.tree_potential(src, tuple(tp[some, j].copy() for j in range(3)))
+            assert np.array_equal(got.view(np.uint64), full[some].view(np.uint64)), (prec, n)
