@@ -43,6 +43,7 @@ struct TgtArgs {
   int *count;                  // [buckets] targets per bucket
   u64 *first;                  // [buckets] exclusive prefix of count
   u32 *box;                    // [6] targets' bounding box, ordered-integer encoding
+  int *apart;                  // chunks whose lanes walk alone
 };
 
 struct TgtLoad {
@@ -61,13 +62,19 @@ struct TgtAdd {
 __global__ void __launch_bounds__(BLOCK) tgt_clear_kernel(Work W, TgtArgs A, int nb) {
   const int i = blockIdx.x * BLOCK + threadIdx.x;
   if (i < 6) A.box[i] = i < 3 ? 0xffffffffu : 0u;
-  if (i == 0) W.ncount[NC_SORT * W.nseg] = nb;  // the scan's element count
+  if (i == 0) {
+    W.ncount[NC_SORT * W.nseg] = nb;  // the scan's element count
+    *A.apart = 0;
+  }
   for (int j = i; j < nb; j += gridDim.x * BLOCK) A.count[j] = 0;
 }
 
 // The target's bucket: the place of the first source whose digits are not below
-// its own.
-__device__ __forceinline__ int tgt_bucket(const Work &W, const Seg &S, float x, float y, float z) {
+// its own; the last one outside the sources' cube, whose outermost sources' digits
+// would bring targets from everywhere together.
+__device__ __forceinline__ int tgt_bucket(const Work &W, const Seg &S, int outside, float x, float y, float z) {
+  const double half = 0.5 * S.Len;
+  if (fabs(x - S.center[0]) > half || fabs(y - S.center[1]) > half || fabs(z - S.center[2]) > half) return outside;
   const u64 key = octant_key(S.center, S.Len, S.D, x, y, z);
   int lo = 0, hi = S.n_src;
   while (lo < hi) {
@@ -103,7 +110,7 @@ __global__ void __launch_bounds__(BLOCK) tgt_bucket_lds_kernel(Work W, TgtArgs A
   for (int i = i0 + (int)threadIdx.x; i < i1; i += BLOCK) {
     const float x = A.x[i], y = A.y[i], z = A.z[i];
     box_take(mn, mx, x, y, z);
-    const int b = tgt_bucket(W, S, x, y, z);
+    const int b = tgt_bucket(W, S, nb - 1, x, y, z);
     A.bucket[i] = b;
     A.rank[i] = atomicAdd(&cnt[b], 1);
   }
@@ -115,7 +122,7 @@ __global__ void __launch_bounds__(BLOCK) tgt_bucket_lds_kernel(Work W, TgtArgs A
   fold_box(mn, mx, A.box, A.box + 3);
 }
 
-__global__ void __launch_bounds__(BLOCK) tgt_bucket_kernel(Work W, TgtArgs A) {
+__global__ void __launch_bounds__(BLOCK) tgt_bucket_kernel(Work W, TgtArgs A, int nb) {
   const Seg &S = W.seg[0];
   u32 mn[3] = {0xffffffffu, 0xffffffffu, 0xffffffffu}, mx[3] = {0u, 0u, 0u};
   for (int i0 = blockIdx.x * BLOCK; i0 < A.n; i0 += gridDim.x * BLOCK) {  // uniform across the block
@@ -124,13 +131,14 @@ __global__ void __launch_bounds__(BLOCK) tgt_bucket_kernel(Work W, TgtArgs A) {
     if (i < A.n) {
       const float x = A.x[i], y = A.y[i], z = A.z[i];
       box_take(mn, mx, x, y, z);
-      b = tgt_bucket(W, S, x, y, z);
+      b = tgt_bucket(W, S, nb - 1, x, y, z);
       A.bucket[i] = b;
     }
-    // the lanes of each bucket among the wave's: their first, how many, how many before
+    // the lanes of each bucket among the wave's: their first, how many, how many before;
+    // four buckets with one lane each, and the rest are taken to be so too
     const int lane = threadIdx.x & (WAVE - 1);
-    int head = 0, size = 0, before = 0;
-    for (u64 todo = __ballot(b >= 0); todo != 0ull;) {  // uniform across the wave
+    int head = lane, size = b >= 0 ? 1 : 0, before = 0, lone = 0;
+    for (u64 todo = __ballot(b >= 0); todo != 0ull && lone < 4;) {  // uniform across the wave
       const int first = __ffsll((long long)todo) - 1;
       const u64 same = __ballot(b == __builtin_amdgcn_readlane(b, first));
       if ((same >> lane) & 1ull) {
@@ -138,6 +146,7 @@ __global__ void __launch_bounds__(BLOCK) tgt_bucket_kernel(Work W, TgtArgs A) {
         size = __popcll(same);
         before = __popcll(same & ((1ull << lane) - 1ull));
       }
+      lone += __popcll(same) == 1 ? 1 : 0;
       todo &= ~same;
     }
     int r = 0;
@@ -167,6 +176,35 @@ __device__ __forceinline__ bool targets_wrap(const Seg &S, const DevParams &P, c
   return wrap;
 }
 
+// Whether the lanes of a chunk of 64 ordered targets walk alone, as target_walk
+// decides for a call's sizes: most of its targets lie outside the sources' cube, or
+// the buckets between neighbours add up to more than `reach` (a step counts for a
+// quarter of it at most: one from an octant to the next passes over any number),
+// and their paths have little in common.  Targets spread over the box of one halo,
+// together / so / each lane alone as they came (ms a call, FAST): a million sources
+// and as many targets 4.4 / 2.3 / 2.5, 262,144 targets 3.2 / 1.7 / 1.9, 100,000
+// sources and a million targets 2.6 / 1.9 / 1.6.  A chunk that four waves or more share
+// is walked together: they are the chunks of calls with few targets, whose longest
+// path alone would be the call.  Called by whole waves; t: the lane's target.
+__device__ __forceinline__ bool chunk_alone(const TgtArgs &A, bool live, int t, int nb, int reach) {
+  const int b = live ? A.bucket[t] : nb - 1;
+  const int next = __shfl_down(b, 1, WAVE);
+  const bool last = (threadIdx.x & (WAVE - 1)) == WAVE - 1;
+  int apart = last || next == nb - 1 ? 0 : min(next - b, reach / 4);
+  for (int d = WAVE / 2; d > 0; d >>= 1) apart += __shfl_xor(apart, d, WAVE);
+  return 2 * __popcll(__ballot(live && b == nb - 1)) > __popcll(__ballot(live)) || apart > reach;
+}
+
+// The chunks that walk alone, counted.
+__global__ void __launch_bounds__(BLOCK) tgt_apart_kernel(TgtArgs A, int nb, int reach) {
+  int n = 0;
+  for (int i0 = blockIdx.x * BLOCK + (threadIdx.x & ~(WAVE - 1)); i0 < A.n; i0 += gridDim.x * BLOCK) {
+    const int i = i0 + (int)(threadIdx.x & (WAVE - 1));
+    n += chunk_alone(A, i < A.n, i < A.n ? A.order[i] : 0, nb, reach) ? 1 : 0;
+  }
+  if (n > 0 && (threadIdx.x & (WAVE - 1)) == 0) atomicAdd(A.apart, n);
+}
+
 // Each lane walks a path of its own, over the targets in tree order or as they
 // came (then a periodic box always takes the wrapped separations, which give the
 // same bits where nothing wraps).
@@ -182,10 +220,13 @@ __global__ void __launch_bounds__(BLOCK) walk_points_lane_kernel(Work W, DevPara
 }
 
 // One target per lane, in tree order, GROUP lanes together: 16, or 64 in trees
-// beyond byte_walk.
-template <int GROUP>
+// beyond byte_walk.  MIXED: some chunks' lanes alone.  Both forms are launched and
+// one runs, the mixed one where more than one chunk in 20 is to walk alone: with
+// both walks in one kernel the walk together takes 8% longer.
+template <int GROUP, bool MIXED>
 __global__ void __launch_bounds__(BLOCK) walk_points_kernel(Work W, DevParams P, TgtArgs A,
-                                                            const Item *__restrict__ it) {
+                                                            const Item *__restrict__ it, int nb, int reach) {
+  if ((*A.apart > A.n / (20 * WAVE)) != MIXED) return;
   Seg S = W.seg[0];
   S.straddle = targets_wrap(S, P, A) ? 1 : 0;
   WalkCount wc;
@@ -194,6 +235,11 @@ __global__ void __launch_bounds__(BLOCK) walk_points_kernel(Work W, DevParams P,
     const bool live = i < A.n;
     const int t = live ? A.order[i] : 0;
     const float x = A.x[t], y = A.y[t], z = A.z[t], tm = A.m ? A.m[t] : 0.f;
+    if (MIXED && chunk_alone(A, live, t, nb, reach)) {  // uniform across the wave
+      unsigned ni = 0, no = 0;
+      if (live) A.out[t] = walk_dispatch<false>(W, P, S, x, y, z, tm, ni, no);
+      continue;
+    }
     const double pot = walk_group_dispatch<GROUP, false, false>(it, P, S, 0, S.n_items, live, x, y, z, tm, wc);
     if (live) A.out[t] = pot * (double)P.G / (double)P.a;
   }
@@ -202,7 +248,8 @@ __global__ void __launch_bounds__(BLOCK) walk_points_kernel(Work W, DevParams P,
 // The same with PARTS waves to 64 targets, one chunk per workgroup.
 template <int PARTS>
 __global__ void __launch_bounds__(PARTS *WAVE) walk_points_split_kernel(Work W, DevParams P, TgtArgs A,
-                                                                        const Item *__restrict__ it) {
+                                                                        const Item *__restrict__ it, int nb,
+                                                                        int reach) {
   __shared__ double part[PARTS - 1][WAVE];
   const Seg &S = W.seg[0];
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
@@ -210,6 +257,13 @@ __global__ void __launch_bounds__(PARTS *WAVE) walk_points_split_kernel(Work W, 
   const bool live = i < A.n;
   const int t = live ? A.order[i] : 0;
   const float x = A.x[t], y = A.y[t], z = A.z[t], tm = A.m ? A.m[t] : 0.f;
+  if (PARTS == 2 && chunk_alone(A, live, t, nb, reach)) {  // uniform across the workgroup; each wave takes a part of the targets
+    Seg T = S;
+    T.straddle = targets_wrap(S, P, A) ? 1 : 0;
+    unsigned ni = 0, no = 0;
+    if (live && (int)(threadIdx.x & (WAVE - 1)) / (WAVE / PARTS) == w) A.out[t] = walk_dispatch<false>(W, P, T, x, y, z, tm, ni, no);
+    return;
+  }
   const int M = S.n_items;
   const int mid = A.bucket[A.order[min((int)blockIdx.x * WAVE + WAVE / 2, A.n - 1)]] << BUCKET_BITS;
   const int own = __builtin_amdgcn_readfirstlane((int)((int64_t)M * min(mid, S.n_src) / S.n_src));
@@ -240,7 +294,7 @@ extern "C" int hbt_tree_potential(hbt_ctx *ctx, int64_t n_src, const float *sx, 
   RETCHK(ensure_slots(ctx, L.nslots, 1, (int64_t)L.tiles.size()));
   const TargetWalk form = target_walk(n_src, n_tgt, ctx->params.precision);
   if (n_tgt > 0 && form != TargetWalk::alone)
-    RETCHK(ctx->tgt.ensure(((size_t)(n_src >> BUCKET_BITS) + 1) * 12 + 24 + (size_t)std::min(n_tgt, TGT_SLICE) * 12));
+    RETCHK(ctx->tgt.ensure(((size_t)(n_src >> BUCKET_BITS) + 2) * 12 + 28 + (size_t)std::min(n_tgt, TGT_SLICE) * 12));
   RETCHK(stage_level(ctx, L));
   Runner R;
   R.c = ctx;
@@ -258,7 +312,7 @@ extern "C" int hbt_tree_potential(hbt_ctx *ctx, int64_t n_src, const float *sx, 
   tree_only_setup_kernel<<<1, 1, 0, st>>>(R.W, (int)n_src);
   tree_sources_kernel<<<grid_for(n_src, ctx->cus), BLOCK, 0, st>>>(R.W, (int)n_src, sx, sy, sz, smass);
   RETCHK(R.build_tree(false, form != TargetWalk::alone));  // the targets' order reads the sorted digits
-  const int nb = (int)(n_src >> BUCKET_BITS) + 1;  // a target's place among the sources is 0 .. n_src
+  const int nb = (int)(n_src >> BUCKET_BITS) + 2;  // a target's place among the sources is 0 .. n_src, or far from them
   for (int64_t t0 = 0; t0 < n_tgt; t0 += TGT_SLICE) {
     TgtArgs A{};
     A.n = (int)std::min<int64_t>(TGT_SLICE, n_tgt - t0);
@@ -272,16 +326,17 @@ extern "C" int hbt_tree_potential(hbt_ctx *ctx, int64_t n_src, const float *sx, 
     A.first = ctx->tgt.as<u64>();
     A.count = (int *)(A.first + nb);
     A.box = (u32 *)(A.count + nb);
-    A.bucket = (int *)(A.box + 6);
+    A.apart = (int *)(A.box + 6);
+    A.bucket = A.apart + 1;
     A.rank = A.bucket + A.n;
     A.order = A.rank + A.n;
     const int *n = R.count_row(NC_SORT);
     tgt_clear_kernel<<<grid_for(nb, ctx->cus), BLOCK, 0, st>>>(R.W, A, nb);
     if (nb <= LDS_BUCKETS) {
-      const int per = std::max((A.n + ctx->cus - 1) / ctx->cus, TILE);
+      const int per = std::max((A.n + ctx->cus - 1) / ctx->cus, BLOCK);
       tgt_bucket_lds_kernel<<<(A.n + per - 1) / per, BLOCK, 0, st>>>(R.W, A, nb, per);
     } else {
-      tgt_bucket_kernel<<<grid_for(A.n, ctx->cus), BLOCK, 0, st>>>(R.W, A);
+      tgt_bucket_kernel<<<grid_for(A.n, ctx->cus), BLOCK, 0, st>>>(R.W, A, nb);
     }
     // the level's tile table starts at the buckets' tiles (fewer buckets than sources)
     const int nt = (nb + TILE - 1) / TILE, g = std::min(nt, ctx->cus * 8);
@@ -293,17 +348,23 @@ extern "C" int hbt_tree_potential(hbt_ctx *ctx, int64_t n_src, const float *sx, 
       continue;
     }
     const int chunks = (A.n + WAVE - 1) / WAVE;
-    if (!byte_walk(n_src)) {
-      walk_points_kernel<64><<<(A.n + BLOCK - 1) / BLOCK, BLOCK, 0, st>>>(R.W, R.P, A, R.W.items);
-      continue;
-    }
-    switch (R.P.wide_sum ? walk_parts(chunks, ctx->cus) : 1) {
-      case 16: walk_points_split_kernel<16><<<chunks, 16 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items); break;
-      case 8: walk_points_split_kernel<8><<<chunks, 8 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items); break;
-      case 4: walk_points_split_kernel<4><<<chunks, 4 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items); break;
-      case 2: walk_points_split_kernel<2><<<chunks, 2 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items); break;
+    const int parts = byte_walk(n_src) && R.P.wide_sum ? walk_parts(chunks, ctx->cus) : 1;
+    const int reach = WAVE * target_reach(ctx->params.precision) >> BUCKET_BITS;
+    const int blocks = (A.n + BLOCK - 1) / BLOCK;
+    switch (parts) {
+      case 16: walk_points_split_kernel<16><<<chunks, 16 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items, nb, reach); break;
+      case 8: walk_points_split_kernel<8><<<chunks, 8 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items, nb, reach); break;
+      case 4: walk_points_split_kernel<4><<<chunks, 4 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items, nb, reach); break;
+      case 2: walk_points_split_kernel<2><<<chunks, 2 * WAVE, 0, st>>>(R.W, R.P, A, R.W.items, nb, reach); break;
       default:
-        walk_points_kernel<16><<<(A.n + BLOCK - 1) / BLOCK, BLOCK, 0, st>>>(R.W, R.P, A, R.W.items);
+        tgt_apart_kernel<<<grid_for(A.n, ctx->cus), BLOCK, 0, st>>>(A, nb, reach);
+        if (byte_walk(n_src)) {
+          walk_points_kernel<16, false><<<blocks, BLOCK, 0, st>>>(R.W, R.P, A, R.W.items, nb, reach);
+          walk_points_kernel<16, true><<<blocks, BLOCK, 0, st>>>(R.W, R.P, A, R.W.items, nb, reach);
+        } else {
+          walk_points_kernel<64, false><<<blocks, BLOCK, 0, st>>>(R.W, R.P, A, R.W.items, nb, reach);
+          walk_points_kernel<64, true><<<blocks, BLOCK, 0, st>>>(R.W, R.P, A, R.W.items, nb, reach);
+        }
     }
   }
   HIPCHK(hipGetLastError());

@@ -76,10 +76,10 @@ def test_walk_group_forms_of_many_chunks(gpu):
 
 
 @pytest.mark.parametrize("n_src", [1, 100, 65535, 65536])
-@pytest.mark.parametrize("n_tgt", [1, 1023, 1025, 263_001])
+@pytest.mark.parametrize("n_tgt", [1, 255, 257, 263_001])
 def test_tree_targets_by_buckets(gpu, n_src, n_tgt):
     """targets counted by buckets of 16 sources, in LDS up to 4,096 buckets (65,535
-    sources) by runs of 1,024 targets and more, and in memory beyond; half of the
+    sources) by runs of 256 targets and more, and in memory beyond; half of the
     targets stand in one place.  Any order of the targets gives the same bits, and a
     sample of them the oracle's"""
     rng = np.random.default_rng(n_src + n_tgt)
@@ -105,18 +105,21 @@ def test_tree_targets_by_buckets(gpu, n_src, n_tgt):
 @pytest.mark.parametrize("where", ["inside", "across_a_face", "not_periodic"])
 def test_target_walks_agree(gpu, n_src, where):
     """a few targets and many of them take other forms of the walk (each lane alone,
-    the targets as they came or in tree order; lanes together; a chunk shared by
-    waves): the same target gets the same bits, in every precision"""
+    the targets as they came or in tree order; lanes together, by chunks of dense
+    targets; a chunk shared by waves): the same target gets the same bits, in every
+    precision, among the sources, beside them and far away"""
     rng = np.random.default_rng(n_src)
     box, n_tgt = 1.0e4, 140_000
     at = {"inside": 500.0, "across_a_face": 0.0, "not_periodic": 0.0}[where]
     wrap = (lambda a: (a % box).astype(np.float32)) if where != "not_periodic" else (lambda a: a.astype(np.float32))
     sp, tp = wrap(rng.normal(size=(n_src, 3)) * 25.0 + at), wrap(rng.normal(size=(n_tgt, 3)) * 30.0 + at)
+    far = rng.random(n_tgt) < 0.3
+    tp[far] = wrap(rng.uniform(-4000, 4000, size=(int(far.sum()), 3)) + at)
     src = tuple(sp[:, j].copy() for j in range(3)) + (rng.uniform(1e-4, 2e-4, n_src).astype(np.float32),)
     for prec in (abi.HBT_PREC_REPLAY, abi.HBT_PREC_FP32, abi.HBT_PREC_FAST):
         U = gpu(abi.make_params(periodic=int(where != "not_periodic"), box_size=box, precision=prec))
         full = U.tree_potential(src, tuple(tp[:, j].copy() for j in range(3)))
-        for n in (1, 4, 70, 3000):
+        for n in (1, 4, 70, 3000, 30000):
             some = rng.permutation(n_tgt)[:n]
             got = U.tree_potential(src, tuple(tp[some, j].copy() for j in range(3)))
             assert np.array_equal(got.view(np.uint64), full[some].view(np.uint64)), (prec, n)
