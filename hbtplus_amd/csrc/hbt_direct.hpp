@@ -89,41 +89,82 @@ __device__ __forceinline__ void wave_min_max(float &mn, float &mx) {
   }
 }
 
-// The pairs of the staged sources sh[0, nj) with this lane's target; `self` is
+// The pairs of the sources src(0) .. src(nj - 1) with this lane's target; `self` is
 // the target's own place among them (left out), or outside [0, nj).  K pairs at
 // a time; the spline only where a lane of the wave is inside the softening
 // length, behind one scalar branch for the K.
-template <int K, int MODE, bool WRAP, bool SELF, class Real>
-__device__ __forceinline__ void direct_pairs(PairSum<MODE> &sum, const DevParams &P,
-                                             const typename SrcOf<MODE>::type *sh, int q, int self, Real tx, Real ty,
-                                             Real tz) {
+template <int K, int MODE, bool WRAP, bool SELF, class Real, class Source>
+__device__ __forceinline__ void direct_pairs(PairSum<MODE> &sum, const DevParams &P, Source src, int q, int self,
+                                             Real tx, Real ty, Real tz) {
   typename SrcOf<MODE>::type s[K];
   Real r2[K], t[K];
+  bool close[K];
   u64 near = 0;
 #pragma unroll
   for (int k = 0; k < K; k++) {
-    s[k] = sh[q + k];
+    s[k] = src(q + k);
     r2[k] = sum.template sep2<WRAP>(P, s[k], tx, ty, tz);
     t[k] = sum.far_term(s[k], r2[k]);
-    near |= __ballot(sum.near(r2[k]));
+    close[k] = sum.near(r2[k]) && !(SELF && q + k == self);  // (the target is its own nearest)
+    near |= __ballot(close[k]);
   }
   if (near != 0ull) {
 #pragma unroll
     for (int k = 0; k < K; k++)
-      if (sum.near(r2[k])) t[k] = sum.near_term(s[k], r2[k]);
+      if (close[k]) t[k] = sum.near_term(s[k], r2[k]);
   }
 #pragma unroll
   for (int k = 0; k < K; k++)
     if (!SELF || q + k != self) sum.add((q + k) & 3, t[k]);
 }
 
-template <int MODE, bool WRAP, bool SELF, class Real>
-__device__ __forceinline__ void direct_chunk(PairSum<MODE> &sum, const DevParams &P,
-                                             const typename SrcOf<MODE>::type *sh, int nj, int self, Real tx, Real ty,
-                                             Real tz) {
+template <int MODE, bool WRAP, bool SELF, class Real, class Source>
+__device__ __forceinline__ void direct_chunk(PairSum<MODE> &sum, const DevParams &P, Source src, int nj, int self,
+                                             Real tx, Real ty, Real tz) {
   int q = 0;
-  for (; q + 4 <= nj; q += 4) direct_pairs<4, MODE, WRAP, SELF, Real>(sum, P, sh, q, self, tx, ty, tz);
-  for (; q < nj; q++) direct_pairs<1, MODE, WRAP, SELF, Real>(sum, P, sh, q, self, tx, ty, tz);
+  for (; q + 4 <= nj; q += 4) direct_pairs<4, MODE, WRAP, SELF, Real>(sum, P, src, q, self, tx, ty, tz);
+  for (; q < nj; q++) direct_pairs<1, MODE, WRAP, SELF, Real>(sum, P, src, q, self, tx, ty, tz);
+}
+
+// The groups of at most a wave's particles, one to a wave: a particle to a lane,
+// the sources read from the lanes.  The wrap is left out where every particle lies
+// within a quarter box of the first (then no pair is half a box apart, and the
+// selects change nothing).  20,000 groups of 5 take 45 us a call in FP32 and 68 in
+// FP64, 20,000 of 20 69 and 110; as tiles, three of four waves idle and the boxes of
+// targets and sources to find for each, 98 to 127 and 159 to 189, 122 to 144 and 220
+// to 255.
+template <int MODE>
+__device__ __forceinline__ void direct_small(const int64_t *__restrict__ seg_offset, int64_t nseg, const float *x,
+                                             const float *y, const float *z, const float *m, const DevParams &P,
+                                             double *out) {
+  using Real = typename PairSum<MODE>::real;
+  using Src = typename SrcOf<MODE>::type;
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int64_t waves = (int64_t)gridDim.x * (BLOCK / WAVE);
+  for (int64_t s = (int64_t)blockIdx.x * (BLOCK / WAVE) + threadIdx.x / WAVE; s < nseg; s += waves) {  // uniform across the wave
+    const int64_t lo = seg_offset[s], len = seg_offset[s + 1] - lo;
+    if (len <= 0 || len > WAVE) continue;
+    const int n = __builtin_amdgcn_readfirstlane((int)len);
+    const int64_t i = lo + min(lane, n - 1);
+    const float px = x[i], py = y[i], pz = z[i], pm = m[i];
+    const auto lane_of = [](float v, int q) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), q)); };
+    const auto src = [&](int q) { return Src{lane_of(px, q), lane_of(py, q), lane_of(pz, q), lane_of(pm, q)}; };
+    const float near = 0.5f * P.box_half * (1.f - 1e-6f);
+    const bool inside = fabsf(px - lane_of(px, 0)) <= near && fabsf(py - lane_of(py, 0)) <= near &&
+                        fabsf(pz - lane_of(pz, 0)) <= near;
+    PairSum<MODE> sum;
+    sum.init(P);
+    if (P.periodic && __any(!inside)) direct_chunk<MODE, true, true, Real>(sum, P, src, n, lane, px, py, pz);
+    else direct_chunk<MODE, false, true, Real>(sum, P, src, n, lane, px, py, pz);
+    if (lane < n) out[i] = sum.result() * (double)P.G / (double)P.a;
+  }
+}
+
+template <int MODE>
+__global__ void __launch_bounds__(BLOCK)
+direct_small_kernel(const int64_t *__restrict__ seg_offset, int64_t nseg, const float *x, const float *y, const float *z,
+                    const float *m, DevParams P, double *out) {
+  direct_small<MODE>(seg_offset, nseg, x, y, z, m, P, out);
 }
 
 // One tile of targets (BLOCK consecutive particles of a group) against every
@@ -183,14 +224,15 @@ __device__ __forceinline__ void direct_tile(const DTile T, const float *x, const
         nan = nan || tx != tx || ty != ty || tz != tz;  // (a minimum passes over one)
         wrap = __any(nan || wrap);
       }
+      const auto src = [sh](int q) { return sh[q]; };
       const bool self = j0 < w0 + WAVE && w0 < j0 + nj;
       const int own = live ? (int)min<int64_t>(i - j0, BLOCK) : BLOCK;
       if (wrap) {
-        if (self) direct_chunk<MODE, true, true, Real>(sum, P, sh, nj, own, tx, ty, tz);
-        else direct_chunk<MODE, true, false, Real>(sum, P, sh, nj, own, tx, ty, tz);
+        if (self) direct_chunk<MODE, true, true, Real>(sum, P, src, nj, own, tx, ty, tz);
+        else direct_chunk<MODE, true, false, Real>(sum, P, src, nj, own, tx, ty, tz);
       } else {
-        if (self) direct_chunk<MODE, false, true, Real>(sum, P, sh, nj, own, tx, ty, tz);
-        else direct_chunk<MODE, false, false, Real>(sum, P, sh, nj, own, tx, ty, tz);
+        if (self) direct_chunk<MODE, false, true, Real>(sum, P, src, nj, own, tx, ty, tz);
+        else direct_chunk<MODE, false, false, Real>(sum, P, src, nj, own, tx, ty, tz);
       }
     }
     __syncthreads();
@@ -200,10 +242,11 @@ __device__ __forceinline__ void direct_tile(const DTile T, const float *x, const
 
 template <int MODE>
 __global__ void __launch_bounds__(BLOCK)
-direct_kernel(const DTile *tiles, int ntiles, const float *x, const float *y, const float *z,
-              const float *m, DevParams P, double *out) {
+direct_kernel(const DTile *tiles, int ntiles, const int64_t *__restrict__ seg_offset, int64_t nseg, const float *x,
+              const float *y, const float *z, const float *m, DevParams P, double *out) {
   __shared__ typename SrcOf<MODE>::type sh[BLOCK];
   for (int t = blockIdx.x; t < ntiles; t += gridDim.x) direct_tile<MODE>(tiles[t], x, y, z, m, P, out, sh);
+  direct_small<MODE>(seg_offset, nseg, x, y, z, m, P, out);
 }
 
 // ---- the entry point that allocates nothing ---------------------------------
@@ -232,8 +275,8 @@ int noalloc_scratch_setup(int device) {
   return HBT_OK;
 }
 
-// First tile of every group (ceil(len / BLOCK) tiles each, an exclusive scan
-// in one workgroup), the total at tstart[nseg], and *bad = 1 when a group's
+// First tile of every group of more than a wave's particles (ceil(len / BLOCK)
+// tiles each, an exclusive scan in one workgroup), the total at tstart[nseg], and *bad = 1 when a group's
 // offsets descend (such a group gets no tiles).
 __global__ void __launch_bounds__(BLOCK) direct_tile_starts_kernel(const int64_t *__restrict__ seg_offset,
                                                                    int64_t nseg, int64_t *tstart, int *bad) {
@@ -247,7 +290,7 @@ __global__ void __launch_bounds__(BLOCK) direct_tile_starts_kernel(const int64_t
     if (s < nseg) {
       const int64_t len = seg_offset[s + 1] - seg_offset[s];
       if (len < 0) atomicOr(&sbad, 1);
-      nt = len > 0 ? (len + BLOCK - 1) / BLOCK : 0;
+      nt = len > WAVE ? (len + BLOCK - 1) / BLOCK : 0;  // (direct_small takes the others)
     }
     unsigned long long tot;
     const unsigned long long ex = block_exclusive_scan((unsigned long long)nt, &tot);
@@ -277,6 +320,7 @@ direct_noalloc_kernel(const int64_t *__restrict__ seg_offset, int64_t nseg, cons
     const DTile T{seg_offset[lo], seg_offset[lo + 1], seg_offset[lo] + (t - tstart[lo]) * BLOCK};
     direct_tile<MODE>(T, x, y, z, m, P, out, sh);
   }
+  direct_small<MODE>(seg_offset, nseg, x, y, z, m, P, out);
 }
 
 }  // namespace
@@ -294,25 +338,38 @@ extern "C" int hbt_direct_potential(hbt_ctx *ctx, int64_t nseg, const int64_t *s
   HIPCHK(hipMemcpyAsync(off.data(), seg_offset, (nseg + 1) * 8, hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(hipStreamSynchronize(ctx->stream));
   std::vector<DTile> tiles;
+  bool small = false;
   for (int64_t s = 0; s < nseg; s++) {
     if (off[s + 1] < off[s]) return fail(HBT_ERR_INVALID_ARG, "seg_offset not ascending");
+    if (off[s + 1] - off[s] <= WAVE) {
+      small = small || off[s + 1] > off[s];
+      continue;
+    }
     for (int64_t t = off[s]; t < off[s + 1]; t += BLOCK) tiles.push_back(DTile{off[s], off[s + 1], t});
   }
-  if (tiles.empty()) return HBT_OK;
+  if (tiles.empty() && !small) return HBT_OK;
   DBuf tb;
-  RETCHK(tb.ensure(tiles.size() * sizeof(DTile)));
   hipStream_t st = ctx->stream;
-  hipError_t e = hipMemcpyAsync(tb.p, tiles.data(), tiles.size() * sizeof(DTile), hipMemcpyHostToDevice, st);
+  hipError_t e = hipSuccess;
+  if (!tiles.empty()) {
+    RETCHK(tb.ensure(tiles.size() * sizeof(DTile)));
+    e = hipMemcpyAsync(tb.p, tiles.data(), tiles.size() * sizeof(DTile), hipMemcpyHostToDevice, st);
+  }
   if (e == hipSuccess) {
     const DevParams P = make_dev_params(ctx->params);
     const int nt = (int)tiles.size();
-    const int g = std::min(nt, ctx->cus * 16);
-    if (mode == HBT_DIRECT_FP64)
-      direct_kernel<HBT_DIRECT_FP64><<<g, BLOCK, 0, st>>>(tb.as<DTile>(), nt, x, y, z, mass, P, out_phi);
+    // small groups alone: a kernel that leaves more waves to a SIMD; else after the tiles
+    const auto launch = [&](auto tile_kernel, auto small_kernel) {
+      const int64_t sb = small ? (nseg + BLOCK / WAVE - 1) / (BLOCK / WAVE) : 0;
+      const int g = (int)std::min<int64_t>(std::max<int64_t>(sb, nt), (int64_t)ctx->cus * 16);
+      if (nt == 0) small_kernel<<<g, BLOCK, 0, st>>>(seg_offset, nseg, x, y, z, mass, P, out_phi);
+      else
+        tile_kernel<<<g, BLOCK, 0, st>>>(tb.as<DTile>(), nt, seg_offset, small ? nseg : 0, x, y, z, mass, P, out_phi);
+    };
+    if (mode == HBT_DIRECT_FP64) launch(direct_kernel<HBT_DIRECT_FP64>, direct_small_kernel<HBT_DIRECT_FP64>);
     else if (mode == HBT_DIRECT_FP32_KAHAN)
-      direct_kernel<HBT_DIRECT_FP32_KAHAN><<<g, BLOCK, 0, st>>>(tb.as<DTile>(), nt, x, y, z, mass, P, out_phi);
-    else
-      direct_kernel<HBT_DIRECT_FP32><<<g, BLOCK, 0, st>>>(tb.as<DTile>(), nt, x, y, z, mass, P, out_phi);
+      launch(direct_kernel<HBT_DIRECT_FP32_KAHAN>, direct_small_kernel<HBT_DIRECT_FP32_KAHAN>);
+    else launch(direct_kernel<HBT_DIRECT_FP32>, direct_small_kernel<HBT_DIRECT_FP32>);
     e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(st);
   }
@@ -345,7 +402,7 @@ extern "C" int hbt_direct_potential_noalloc(hbt_ctx *ctx, int64_t nseg, const in
   hipStream_t st = ctx->stream;
   const DevParams P = make_dev_params(ctx->params);
   direct_tile_starts_kernel<<<1, BLOCK, 0, st>>>(seg_offset, nseg, tstart, bad);
-  const int g = ctx->cus * 16;
+  const int g = ctx->cus * 8;  // (twice what a CU holds of the FP64 form)
   if (mode == HBT_DIRECT_FP64)
     direct_noalloc_kernel<HBT_DIRECT_FP64><<<g, BLOCK, 0, st>>>(seg_offset, nseg, tstart, x, y, z, mass, P, out_phi);
   else if (mode == HBT_DIRECT_FP32_KAHAN)
