@@ -2871,14 +2871,28 @@ __global__ void output_record_kernel(Work W, DevParams P) {
 }
 
 // Lists and records of the early exits (0 or 1 particles to unbind), a wave per
-// segment: over every slot they took 0.26 ms of a level of 54 million.
+// segment: over every slot they took 0.26 ms of a level of 54 million.  An orphan
+// host's list holds its subhalos' tails too, whatever their number: of more than a
+// tile, it goes by tiles (early_tiles_kernel; ten tails of 300,000 by one wave took
+// 26 ms of a call, 10 without them).
 __global__ void __launch_bounds__(BLOCK) output_early_kernel(Work W, DevParams P) {
   WAVE_SEG_LOOP(k, W.nseg) {
     Seg &S = W.seg[k];
     if (!(S.flags & F_EARLY)) continue;  // uniform across the wave
     const int lane = threadIdx.x & (WAVE - 1);
-    for (int l = lane; l < S.len; l += WAVE) write_entry(W, S, l, output_entry(W, S, l, 0));  // (none of them converged)
+    if (S.len <= TILE)
+      for (int l = lane; l < S.len; l += WAVE) write_entry(W, S, l, output_entry(W, S, l, 0));  // (none of them converged)
     if (lane == 0) record_serial(W, P, S);
+  }
+}
+
+__global__ void __launch_bounds__(BLOCK) early_tiles_kernel(Work W, const Tile *__restrict__ tiles, int ntiles) {
+  for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    const Tile tl = tiles[t];
+    const Seg &S = W.seg[tl.seg];
+    if (!(S.flags & F_EARLY) || S.len <= TILE) continue;  // uniform
+    const int end = min(tl.start + TILE, S.len);
+    for (int l = tl.start + (int)threadIdx.x; l < end; l += BLOCK) write_entry(W, S, l, output_entry(W, S, l, 0));
   }
 }
 

@@ -1168,6 +1168,9 @@ int run_level(hbt_ctx *c, Level &L, const hbt_particles *parts, hbt_subhalo *sub
   RETCHK(R.prelude());
   if (!flat || L.ndraws > 0) pass_begin_kernel<<<R.gseg, BLOCK, 0, c->stream>>>(R.W, R.P);
   output_early_kernel<<<grid_for(nseg * WAVE, c->cus), BLOCK, 0, c->stream>>>(R.W, R.P);
+  // (a list without nested tails has at most the one particle)
+  if (!flat && R.nt_multi > 0)
+    early_tiles_kernel<<<R.tile_grid(R.nt_multi), BLOCK, 0, c->stream>>>(R.W, R.tl_cur, R.nt_multi);
   HIPCHK(hipGetLastError());
   if (getenv("HBT_PASS_TIMES") && atoi(getenv("HBT_PASS_TIMES"))) {
     HIPCHK(hipStreamSynchronize(c->stream));
