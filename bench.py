@@ -215,15 +215,15 @@ def walk_roofline(U, run, ms_per_step, config):
 def sort_roofline(sort_t, sort_c, ms_per_step):
     """HBM roofline of the segmented sorts of a step that are launches of their
     own (the octant digits of the trees of more than 1,024 sources, computed in
-    the tile sort; the energy order): the tile sort reads and writes each element's
-    12-byte key and value once, and every merge level once more, so the
-    algorithmic bytes are 24 B x (elements + elements x merge levels); timed
-    with HIP events around each sort (tile sort and its merge levels)."""
-    alg = 24.0 * (sort_c["elements"] + sort_c["element_levels"])
+    the sort of the runs; the energy order).  The library counts the algorithmic
+    bytes: per element 36 for the runs of digits, 12 for energies that are one run
+    and 20 where merge levels follow, and 24 for every merge level (key and value
+    in and out); timed with HIP events around each sort, runs and merge levels."""
+    alg = float(sort_c["bytes"])
     s = sort_t["sort_ms"] / 1e3
     achieved = alg / s / 1e9 if s > 0 else 0.0
     return dict(bound="hbm", achieved=round(achieved, 1), peak=PEAK_HBM_GBS, unit="GB/s",
-                frac=round(achieved / PEAK_HBM_GBS, 4), kernels="keys_sort_kernel + energy_sort_kernel + merge_pass_kernel",
+                frac=round(achieved / PEAK_HBM_GBS, 4), kernels="keys_sort_kernel + energy_sort_kernel + merge_pass_kernel + rank_merge_kernel",
                 sorts_per_step=sort_t["sort_calls"], ms_per_step=round(sort_t["sort_ms"], 3),
                 elements_per_step=sort_c["elements"], element_levels_per_step=sort_c["element_levels"],
                 algorithmic_bytes_per_step=int(alg), share_of_step=round(sort_t["sort_ms"] / ms_per_step, 3))

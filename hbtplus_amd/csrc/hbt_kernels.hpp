@@ -2098,20 +2098,34 @@ __global__ void __launch_bounds__(PARTS *WAVE) walk_split_kernel(Work W, DevPara
   if (w == 0 && live) finish_target<false>(W, P, S, b, li, q.x, q.y, q.z, pot);
 }
 
-// Instrumented passes: the elements a segmented sort ordered (counters[8])
-// and the elements times the merge levels each needed (counters[9]).
-__global__ void sort_count_kernel(Work W, const int *n, int above, int run, bool ranked) {
-  unsigned long long e = 0, el = 0;
+// What a sort's runs read and write per element: of lists that are one run, and
+// of those whose merge levels (24 bytes each: key and value in and out) follow.
+struct SortBytes {
+  int one_run, merged;
+};
+constexpr SortBytes SORT_DIGITS{20 + 16, 20 + 16};  // Elist entry, position; key, value, node mask
+constexpr SortBytes SORT_ENERGIES{8 + 4, 8 + 12};   // Elist entry, energy; the entry, or key and value
+constexpr SortBytes SORT_PAIRS{24, 24};
+
+// Instrumented passes: the elements a segmented sort ordered (counters[8]),
+// the elements times the merge levels each needed (counters[9]) and the bytes of
+// both (counters[10]).
+__global__ void sort_count_kernel(Work W, const int *n, int above, int run, bool ranked, SortBytes B) {
+  unsigned long long e = 0, el = 0, by = 0;
   SEG_LOOP(k, W) {
     const int c = W.seg[k].cap > above && n[k] > 0 ? n[k] : 0;
     e += (unsigned long long)c;
-    el += (unsigned long long)c * (unsigned long long)merge_levels(c, run, ranked);
+    const int levels = merge_levels(c, run, ranked);
+    el += (unsigned long long)c * (unsigned long long)levels;
+    by += (unsigned long long)c * (unsigned long long)(levels > 0 ? B.merged + 24 * levels : B.one_run);
   }
   e = wave_reduce_sum(e);
   el = wave_reduce_sum(el);
+  by = wave_reduce_sum(by);
   if ((threadIdx.x & (WAVE - 1)) == 0 && (e | el)) {
     atomicAdd(&W.counters[8], e);
     atomicAdd(&W.counters[9], el);
+    atomicAdd(&W.counters[10], by);
   }
 }
 

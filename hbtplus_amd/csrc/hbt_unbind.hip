@@ -763,7 +763,7 @@ struct Runner {
     RETCHK(sort_begin());
     tile_sort_kernel<<<tile_grid(nt), BLOCK, 0, c->stream>>>(tl_cur, nt, W.ibase, n, W.k0, W.v0, W.k1, W.v1);
     merge_sorted(n, nt, TILE);
-    return sort_end(n, 0, TILE, false);
+    return sort_end(n, 0, TILE, false, SORT_PAIRS);
   }
 
   // instrumentation: a sort's device time, or the elements it sorted and their
@@ -772,7 +772,7 @@ struct Runner {
     if (c->prof_mode == 1) HIPCHK(hipEventRecord(c->evs0, c->stream));
     return HBT_OK;
   }
-  int sort_end(const int *n, int above, int run, bool rk) {  // above: only segments of more slots were sorted
+  int sort_end(const int *n, int above, int run, bool rk, SortBytes bytes) {  // above: only segments of more slots were sorted
     if (c->prof_mode == 1) {
       HIPCHK(hipEventRecord(c->evs1, c->stream));
       HIPCHK(hipEventSynchronize(c->evs1));
@@ -781,7 +781,7 @@ struct Runner {
       c->sort_ms += ms;
       c->sort_calls++;
     } else if (c->prof_mode == 2) {
-      sort_count_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, n, above, run, rk);
+      sort_count_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, n, above, run, rk, bytes);
     }
     return HBT_OK;
   }
@@ -830,7 +830,7 @@ struct Runner {
     keys_sort_kernel<<<tile_grid(nt, 1), RUN_THREADS, 0, c->stream>>>(W, P, tl_cur, nt, rk);
     if (rk) rank_merge(count_row(NC_SRC), nt);
     else merge_sorted(count_row(NC_SRC), nt, RUN);
-    return sort_end(count_row(NC_SRC), nt < nt_cur ? TILE : 0, RUN, rk);
+    return sort_end(count_row(NC_SRC), nt < nt_cur ? TILE : 0, RUN, rk, SORT_DIGITS);
   }
 
   // Tree over the pass's sources.  Segments of at most one tile take one launch
@@ -924,7 +924,7 @@ struct Runner {
       energy_sort_kernel<<<tile_grid(nt_multi, 1), RUN_THREADS, 0, c->stream>>>(W, tl_cur, nt_multi, rk);
       if (rk) rank_merge(count_row(NC_SORT), nt_multi);
       else merge_sorted(count_row(NC_SORT), nt_multi, RUN);
-      RETCHK(sort_end(count_row(NC_SORT), TILE, RUN, rk));
+      RETCHK(sort_end(count_row(NC_SORT), TILE, RUN, rk, SORT_ENERGIES));
       output_tiles(W.nmulti, nt_multi, RUN, true);
     }
     if (P.replay) output_record_kernel<<<gseg, BLOCK, 0, c->stream>>>(W, P);
@@ -1951,6 +1951,19 @@ int hbt_profile_sorts(hbt_ctx *ctx, double *sort_ms, int64_t *sort_calls, int64_
   if (sort_calls) *sort_calls = ctx->sort_calls;
   if (elements) *elements = (int64_t)h[0];
   if (element_levels) *element_levels = (int64_t)h[1];
+  return HBT_OK;
+}
+
+int hbt_profile_sort_bytes(hbt_ctx *ctx, int64_t *bytes) {
+  if (!ctx || !bytes) return fail(HBT_ERR_INVALID_ARG, "null argument");
+  HIPCHK(hipSetDevice(ctx->device));
+  unsigned long long h = 0;
+  if (ctx->counters.p) {
+    HIPCHK(hipMemcpyAsync(&h, ctx->counters.as<unsigned long long>() + 10, sizeof(h), hipMemcpyDeviceToHost,
+                          ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+  }
+  *bytes = (int64_t)h;
   return HBT_OK;
 }
 

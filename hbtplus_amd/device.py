@@ -315,8 +315,10 @@ class GpuUnbinder:
         vals = [ctypes.c_int64() for _ in range(3)]
         check(self.lib.hbt_profile_sorts(self.ctx, ctypes.byref(ms), *[ctypes.byref(v) for v in vals]),
               "hbt_profile_sorts")
+        by = ctypes.c_int64()
+        check(self.lib.hbt_profile_sort_bytes(self.ctx, ctypes.byref(by)), "hbt_profile_sort_bytes")
         return dict(sort_ms=ms.value, sort_calls=vals[0].value, elements=vals[1].value,
-                    element_levels=vals[2].value)
+                    element_levels=vals[2].value, bytes=by.value)
 
     # per-subhalo form with host buffers --------------------------------------
     def unbind_one(self, cols: dict, sub: np.ndarray):

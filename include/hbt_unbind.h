@@ -447,14 +447,18 @@ int hbt_profile(hbt_ctx *ctx, int mode);
 int hbt_profile_read(hbt_ctx *ctx, double *walk_ms, int64_t *walk_launches,
                      int64_t *interactions, int64_t *opened, int64_t *targets,
                      int64_t *lane_slots, int64_t *tree_items, int64_t *wave_steps);
-/* The segmented sorts of the unbinding passes in launches of their own (the
- * octant digits of the lists of more than 1024 particles, computed in the tile
- * sort; the energy order): mode 1 times every sort (tile sort and its merge
- * levels) with HIP events, mode 2 counts the elements sorted and the elements
- * times the merge levels each needed (every level reads and writes each
- * element's 12-byte key and value once, the tile sort once more). */
+/* The segmented sorts of the unbinding passes in launches of their own (of the
+ * lists of more than 1024 particles the octant digits, computed in the sort of
+ * the runs, and the energy order; a sampled level's shuffles and refinements):
+ * mode 1 times every sort (runs and merge levels) with HIP events, mode 2 counts
+ * the elements sorted and the elements times the merge levels each needed. */
 int hbt_profile_sorts(hbt_ctx *ctx, double *sort_ms, int64_t *sort_calls, int64_t *elements,
                       int64_t *element_levels);
+/* Mode 2: the bytes those sorts need to read and write.  The runs of digits take
+ * 36 per element (list entry and position in; key, value and node mask out), those
+ * of energies 12 where the list is one run (list entry and energy in, the entry
+ * out) and 20 where merge levels follow, runs of pairs 24; every merge level 24. */
+int hbt_profile_sort_bytes(hbt_ctx *ctx, int64_t *bytes);
 
 #ifdef __cplusplus
 }
