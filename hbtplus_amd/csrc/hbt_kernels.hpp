@@ -2004,8 +2004,8 @@ __global__ void __launch_bounds__(BLOCK) walk_shared_kernel(Work W, DevParams P,
 // steps, one load after another (450 cycles a step at one wave per SIMD, 86
 // with the chip full).  PARTS waves then walk a part of the item array each for
 // the same 64 targets, and their sums are added.  The FP64 sum of FP32 terms
-// is exact while the terms spread over fewer than 2^29 (a list of millions of
-// equal masses spreads them over 2^25), so the parts change no bit of it there.
+// is exact while it is below 2^29 times its smallest term (a list of millions of
+// equal masses: 2^25), so the parts change no bit of it there; beyond it they may.
 // One list of 24,000 particles (375 chunks, 16 parts): walks 0.53 -> 0.147 ms.
 
 // First item of part w of PARTS for targets at item `own` of M: equal shares of

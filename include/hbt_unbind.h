@@ -399,7 +399,16 @@ int hbt_last_batch_stats(hbt_ctx *ctx, double *device_ms, int64_t *n_evals,
                          int64_t *n_passes);
 
 /* Execution tuning (no counterpart in the reference).  Results are identical
- * for every setting; only the speed changes.
+ * for every setting; only the speed changes.  HBT_PREC_FAST under one condition:
+ * a launch of few targets lets several waves sum parts of a potential, in FP64 of
+ * FP32 terms, which is exact, so that the parts change no bit, while the sum is
+ * below 2^29 times its smallest term (millions of equal masses spread their terms
+ * over 2^25).  Beyond that (masses tens of times apart in a list of millions, tens of
+ * thousands of times in one of a thousand) a potential's last FP64 bits, and rarely
+ * the float that holds it, can depend on how many targets the launch had: on
+ * use_graph, on the instrumentation's mode 2, and on which subhalos share a batch.
+ * Repeating a call with the same settings repeats its bits in any case.  HBT_PREC_REPLAY and HBT_PREC_FP32 sum in one
+ * order always.
  *   walk_group[b]: lanes that walk the tree together (8, 16, 32 or 64) for
  *                  subhalos of size bin b: list length < bin_edge[0] (b = 0),
  *                  < bin_edge[1] (b = 1), otherwise b = 2
@@ -424,12 +433,13 @@ int hbt_get_tuning(hbt_ctx *ctx, hbt_tuning *out);
 int hbt_set_tuning(hbt_ctx *ctx, const hbt_tuning *tuning);
 
 /* Autotuner: times hbt_unbind_batch (same arguments) under the context's
- * current tuning and then candidate tunings -- one group size for all bins, then a separate group for the small-subhalo
- * bin at two bin edges, then the XCD run length, then direct launches or a
- * graph and the passes per graph launch -- keeping at each
- * step the setting with the smallest device time over `reps` runs, sets the
- * winner on the context and returns it in *chosen.  The outputs of the last
- * run are left in subs/out_index/out_energy (identical for every tuning). */
+ * current tuning and then candidate tunings -- one group size for all bins, then a
+ * separate group for the small-subhalo bin at two bin edges, then the XCD run
+ * length, then direct launches or a graph and the passes per graph launch --
+ * keeping at each step the setting with the smallest device time over `reps` runs,
+ * sets the winner on the context and returns it in *chosen.  The outputs of the
+ * last run are left in subs/out_index/out_energy (identical for every tuning, under
+ * the condition above). */
 int hbt_autotune(hbt_ctx *ctx, const hbt_particles *particles, hbt_subhalo *subs,
                  const hbt_subhalo *subs_host, int64_t nsub, int64_t *out_index,
                  float *out_energy, int reps, hbt_tuning *chosen);
