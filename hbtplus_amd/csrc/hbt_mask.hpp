@@ -76,8 +76,13 @@ __global__ void __launch_bounds__(BLOCK) mask_gather_kernel(MaskArgs A) {
 // one through the L2, which bounds the kernel, and the table of a group of 8,192
 // leaves room for a second workgroup on the CU.  1,000 groups (4.0 M entries)
 // take 54 us in both sizes where their sort, owners and scan took 190; the call
-// 0.67 -> 0.44 ms, with 20 groups 0.20 -> 0.08.  A table for 16,384 would leave
-// one workgroup of 16 waves on a CU.
+// 0.67 -> 0.44 ms, with 20 groups 0.20 -> 0.08.
+// Both sides of the line, us a call with 400 groups (20 groups) of one size: 2,000
+// entries 123 by table, 185 sorted (58, 107); 4,096 128, 231 (61, 113); 8,192 153,
+// 330 (67, 128).  A table for 16,384, 128 KiB and one workgroup on a CU, in this
+// one's place costs groups of 8,192 180 (77) and gives those of 12,000 200 for 444
+// sorted (84, 146), of 16,384 221 for 554 (90, 147): it would pay as a third size
+// beside these two, which is not built.
 template <int T, int PER>
 __global__ void __launch_bounds__(T) mask_claim_kernel(MaskArgs A, const int *groups, int ngroups) {
   constexpr u32 SLOTS = 2u * T * PER, EMPTY = ~0u;
