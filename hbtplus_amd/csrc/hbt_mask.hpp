@@ -36,7 +36,6 @@ struct MaskArgs {
   int nsub;
   const int64_t *gbase;  // first slot of each group segment
   const int *gn;         // entries per group segment
-  int ngrp;
   const int64_t *id;
   u64 *k0;
   u32 *v0;
@@ -299,7 +298,6 @@ extern "C" int hbt_mask_subhalos(hbt_ctx *ctx, const hbt_particles *particles, c
   A.nsub = (int)nsub;
   A.gbase = (const int64_t *)d[1];
   A.gn = (const int *)d[2];
-  A.ngrp = ngrp;
   A.id = particles->id;
   A.k0 = ctx->k0.as<u64>();
   A.v0 = ctx->v0.as<u32>();

@@ -304,7 +304,6 @@ extern "C" int hbt_tree_potential(hbt_ctx *ctx, int64_t n_src, const float *sx, 
   R.max_n = L.maxcap;
   R.list_all();
   R.gseg = 1;
-  R.gblk = 1;
   hipStream_t st = ctx->stream;
   seg_expand_kernel<<<1, BLOCK, 0, st>>>(R.W, R.P, ctx->segin.as<SegIn>(), 0);
   seg_of_slot_kernel<<<grid_for(L.nslots, ctx->cus), BLOCK, 0, st>>>(1, R.W.ibase, L.nslots,

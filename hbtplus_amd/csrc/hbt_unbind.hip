@@ -599,7 +599,7 @@ struct Runner {
   Work W;
   DevParams P;
   Level *L;
-  int gs, gseg, gblk;          // slot, segment-thread and segment-block grids
+  int gs, gseg;                // slot and segment-thread grids
   bool swap_sp = true;         // swap the spatial list with its compacted copy (direct launches)
   int nt_multi = 0;            // tiles of segments of more than one (a prefix)
   int nt_big = 0;              // then those of segments of more than SMALL_CAP slots
@@ -1147,7 +1147,6 @@ int run_level(hbt_ctx *c, Level &L, const hbt_particles *parts, hbt_subhalo *sub
   R.list_all();
   R.gseg = grid_for(nseg, c->cus);
   const int gsb = (int)std::min<int64_t>(nseg, (int64_t)c->cus * 8);
-  R.gblk = gsb;
   const bool flat = L.child_list.empty();
   seg_expand_kernel<<<R.gseg, BLOCK, 0, c->stream>>>(R.W, R.P, c->segin.as<SegIn>(),
                                                     !flat ? 0 : L.ndraws > 0 ? 1 : 2);
