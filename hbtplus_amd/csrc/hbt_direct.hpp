@@ -174,8 +174,8 @@ direct_small_kernel(const int64_t *__restrict__ seg_offset, int64_t nseg, const 
 // half a box from one of its targets (boxes of its targets and of the chunk:
 // differences are monotonic, so the decision is exact), and looks for itself
 // only in chunks that hold it.  Vector issue bounds it: 1.25e9 pairs of 600
-// groups (20 to 4,700 particles, periodic) take 0.48 ms in FP32, 0.56 compensated
-// and 1.07 in FP64, where tests and wrap in every pair, a branch for its spline
+// groups (20 to 4,700 particles, periodic) take 0.47 ms in FP32, 0.54 compensated
+// and 1.03 in FP64, where tests and wrap in every pair, a branch for its spline
 // and FP64 by division and root took 1.64, 1.62 and 3.23.
 template <int MODE>
 __device__ __forceinline__ void direct_tile(const DTile T, const float *x, const float *y, const float *z,

@@ -43,7 +43,8 @@ inline int walk_parts(int64_t chunks, int cus) {
 
 // How hbt_tree_potential walks its targets: each lane by itself, over the targets
 // as they came or in tree order, or lanes together (16 of them, or 64 beyond
-// byte_walk; FAST shares a chunk among several waves).  The bits are the same.
+// byte_walk; FAST shares a chunk among several waves).  The bits are the same (in
+// FAST while its FP64 sums of FP32 terms are exact).
 // Lanes that walk together wait for the union of their paths, which is long where
 // few targets lie far apart in a large tree, and ordering the targets costs five
 // launches and the digits' sort.  ms a call, periodic box, alone / ordered /
